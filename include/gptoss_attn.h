@@ -108,7 +108,7 @@ typedef struct gptoss_attn_params {
     const void *d_o;
     void *dq, *dk, *dv;
     float *dsinks;          /* optional: NULL skips the sink gradient */
-    float *delta;           /* fp32 scratch of gptoss_attn_workspace_bytes() bytes */
+    float *delta;           /* fp32 scratch of gptoss_attn_workspace_bytes() bytes (forward: optional) */
 
     gptoss_attn_strides q_stride, k_stride, v_stride, o_stride;
     gptoss_attn_strides do_stride, dq_stride, dk_stride, dv_stride;
@@ -148,10 +148,18 @@ const char *gptoss_attn_status_string(int status);
 size_t gptoss_attn_workspace_bytes(const gptoss_attn_params *params);
 
 /*
+ * Bytes of scratch gptoss_attn_fwd can use for these shapes (0 for most): a few queries on a long key / value cache are
+ * cut over the keys, and the slices leave fp32 partial results there.  Given through `delta` (16-byte aligned);
+ * with delta == NULL the same kernel runs uncut.  Never more than gptoss_attn_workspace_bytes.  Host-only.
+ */
+size_t gptoss_attn_fwd_workspace_bytes(const gptoss_attn_params *params);
+
+/*
  * Forward: O and logsumexp.  Replaces the `_attn_fwd` launch in
  * `_attention.forward` (attention_kernel.py:11-100, 241-262) including the
  * output transpose copy at :272 (O is written directly in the caller's layout).
- * Reads q,k,v,sinks,seqlens,doc_start; writes o,lse.
+ * Reads q,k,v,sinks,seqlens,doc_start; writes o,lse (and delta, where
+ * gptoss_attn_fwd_workspace_bytes asks for it).
  */
 int gptoss_attn_fwd(const gptoss_attn_params *params, void *stream);
 

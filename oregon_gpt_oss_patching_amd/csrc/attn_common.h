@@ -55,6 +55,8 @@ struct KArgs {
     float scale_log2;    // scale * log2(e)
     int dkdv_parts;      // dK/dV kernel: workgroups that share one key block, each taking a slice of its query tiles
     float *dkdv_partial; // dkdv_parts > 1: fp32 partial sums, [part][dK, dV][B][G][Skv][64]
+    int kv_splits;       // forward: workgroups that share one query block, each taking a slice of its keys
+    float *fwd_partial;  // kv_splits > 1: fp32 partial results of the slices
     int chunk_tiles;     // single-pass window backward: 64-row query tiles per workgroup
     float *dsink_partial; // single-pass window backward: dSinks partial sums, [B][chunk][H][2]
     float *boundary_partial; // single-pass window backward: fp32 dK / dV shares of the tiles on chunk seams, or NULL

@@ -11,6 +11,7 @@
 #include "attn_bwd_dkdv64.h"
 #include "attn_bwd_window.h"
 #include "attn_common.h"
+#include "attn_decode.h"
 #include "attn_f32.h"
 #include "attn_fwd.h"
 #include "attn_fwd_pipe.h"
@@ -77,6 +78,8 @@ KArgs make_args(const gptoss_attn_params *p) {
     a.scale = p->scale;
     a.scale_log2 = p->scale * kLog2e;
     a.dkdv_parts = 1;
+    a.kv_splits = 1;
+    a.fwd_partial = nullptr;
     a.chunk_tiles = 0;
     a.dsink_partial = nullptr;
     a.boundary_partial = nullptr;
@@ -153,6 +156,21 @@ bool fwd_window_route(const gptoss_attn_params *p) {
     if ((int64_t)(p->H / p->G / 4) * p->B > 65535 || p->Sq / 32 > 65535) return false;
     return p->dtype == GPTOSS_ATTN_BF16 && w >= 32 && w <= 128 && w % 32 == 0 && !p->doc_start &&
            p->q_offset == 0 && !p->q_offset_dev && p->Sq == p->Skv && p->Sq % 32 == 0 && (p->H / p->G) % 4 == 0;
+}
+
+// A few queries on a long cache (attn_decode.h): all (query, head) pairs of a KV head fit two 32-column blocks.
+bool decode_route(const gptoss_attn_params *p) {
+    return p->dtype == GPTOSS_ATTN_BF16 && !p->doc_start && (int64_t)p->Sq * (p->H / p->G) <= Decode::kMaxPairs;
+}
+// Slices of the keys: about two workgroups per compute unit of a 256-CU part (so that the scratch does not depend on the
+// device), each wavefront of a slice with a tile of its own at least.
+int decode_splits(const gptoss_attn_params *p) {
+    const int64_t keys = p->window > 0 && (int64_t)p->window + p->Sq < p->Skv ? (int64_t)p->window + p->Sq : p->Skv;
+    const int64_t groups = (int64_t)p->B * p->G;
+    int64_t n = (512 + groups - 1) / groups;
+    const int64_t most = keys / (4 * Decode::kKeys);
+    if (n > most) n = most;
+    return (int)(n < 1 ? 1 : n);
 }
 
 // workgroups of four independent wavefronts for the float32 kernels
@@ -348,9 +366,19 @@ static size_t stats_bytes(const gptoss_attn_params *p) {
     return fp32_stats_bytes(p) + (size_t)16 * (size_t)p->B * (size_t)p->H * (size_t)p->Sq;
 }
 
+size_t gptoss_attn_fwd_workspace_bytes(const gptoss_attn_params *p) {
+    if (!p || p->B <= 0 || p->H <= 0 || p->G <= 0 || p->Sq <= 0 || p->Skv <= 0) return 0;
+    if (decode_route(p)) {
+        const int splits = decode_splits(p);
+        if (splits > 1) return (size_t)p->B * p->G * splits * decode_partial_floats(p->Sq * (p->H / p->G)) * sizeof(float);
+    }
+    return 0;
+}
+
 size_t gptoss_attn_workspace_bytes(const gptoss_attn_params *p) {
     if (!p || p->B <= 0 || p->H <= 0 || p->Sq <= 0) return 0;
     size_t n = stats_bytes(p);
+    if (gptoss_attn_fwd_workspace_bytes(p) > n) n = gptoss_attn_fwd_workspace_bytes(p);
     if (p->G > 0 && p->Skv > 0) {
         const int parts = dkdv_parts_for(p);
         if (parts > 1) n += (size_t)parts * 2 * sizeof(float) * (size_t)p->B * (size_t)p->G * (size_t)p->Skv * kD;
@@ -368,8 +396,17 @@ size_t gptoss_attn_workspace_bytes(const gptoss_attn_params *p) {
 int gptoss_attn_fwd(const gptoss_attn_params *p, void *stream) {
     const int rc = gptoss_attn_validate(p, 0);
     if (rc) return rc;
-    const KArgs a = make_args(p);
+    KArgs a = make_args(p);
     hipStream_t st = static_cast<hipStream_t>(stream);
+    if (p->delta && !aligned16(p->delta)) return GPTOSS_ATTN_ERR_ALIGNMENT;
+    if (decode_route(p)) {
+        if (p->delta) { a.kv_splits = decode_splits(p); a.fwd_partial = p->delta; }
+        const int pairs = a.Sq * a.r;
+        const int64_t wgs = (int64_t)a.G * a.B * a.kv_splits;
+        const int s = pairs <= 32 ? launch(attn_decode_kernel<1>, wgs, 256, st, a) : launch(attn_decode_kernel<2>, wgs, 256, st, a);
+        if (s || a.kv_splits == 1) return s;
+        return launch(attn_decode_combine_kernel, ((int64_t)a.B * a.G * pairs + 3) / 4, 256, st, a);
+    }
     if (p->dtype == GPTOSS_ATTN_FP32)
         return launch(attn_f32_fwd_kernel, f32_grid((int64_t)a.B * a.H * ((a.Sq + 31) / 32)), 256, st, a);
     const int hpb = hpb_for(a.r), qb = query_blocks_for(a.window);
