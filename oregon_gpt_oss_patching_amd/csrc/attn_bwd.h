@@ -278,6 +278,23 @@ __device__ __forceinline__ void dkdv_tile(uint32_t qsm, uint32_t gsm, uint32_t s
     }
 }
 
+// First row behind key j whose document starts behind key j (S if there is none): the rows that can see key j end there.
+// Document starts never decrease along a row; a wavefront narrows the range 64-fold per round (two rounds at S = 4096, three
+// to 262144).
+__device__ __forceinline__ int document_end(const int32_t *dsrow, int S, int j, int lane) {
+    int lo = j + 1, hi = S;                    // the answer is in [lo, hi]; dsrow[hi] > j or hi == S
+    while (lo < hi) {
+        const int step = (hi - lo + 63) >> 6;
+        const int i = lo + (lane + 1) * step - 1;
+        const uint64_t past = __builtin_amdgcn_ballot_w64(i >= hi || dsrow[min(i, S - 1)] > j);   // (lane 63's i is hi - 1 or more)
+        const int first = past ? __builtin_ctzll(past) : 64;
+        hi = min(hi, lo + (first + 1) * step - 1);
+        lo += first * step;
+        if (step == 1) break;
+    }
+    return __builtin_amdgcn_readfirstlane(hi);
+}
+
 template <int NW, int NB, bool DOCS>  // NB = 32-key blocks per wavefront; DOCS = packed rows (doc_start given)
 __global__ __launch_bounds__(NW * 64, (NB == 1 ? 2 : 1)) void attn_bwd_dkdv_kernel(const KArgs a) {
     const int q_offset = query_offset(a);
@@ -294,9 +311,10 @@ __global__ __launch_bounds__(NW * 64, (NB == 1 ? 2 : 1)) void attn_bwd_dkdv_kern
 
     int bid = blockIdx.x;
     const int g = bid % a.G; bid /= a.G;
-    const int b = bid % a.B; bid /= a.B;
+    const int bi = bid % a.B; bid /= a.B;
     const int part = bid % a.dkdv_parts; bid /= a.dkdv_parts;
     const int kt = bid;                                   // ascending: most work first
+    const int b = rotated_batch_row(bi, kt, a.B);
     const int j0 = kt * BN;                               // first key of the workgroup
     const int wj0 = j0 + WK * w;                          // first key of the wavefront
 
@@ -309,7 +327,12 @@ __global__ __launch_bounds__(NW * 64, (NB == 1 ? 2 : 1)) void attn_bwd_dkdv_kern
     const int i_lo = max(0, j0 - q_offset);
     int64_t i_hi64 = min((int64_t)a.Sq, (int64_t)q_len - q_offset);
     i_hi64 = min(i_hi64, (int64_t)j1 + weff - q_offset);
-    const int i_hi = (j1 >= j0) ? (int)max((int64_t)0, i_hi64) : 0;
+    int i_hi = (j1 >= j0) ? (int)max((int64_t)0, i_hi64) : 0;
+    // packed rows: nobody behind the document of the workgroup's last key sees any of its keys (without this bound the
+    // walk went on to the row's end, loading and skipping tile after tile: 0.96 ms against 0.54 for seven documents
+    // in a row of 8192)
+    if constexpr (DOCS)
+        if (i_hi > i_lo) i_hi = min(i_hi, document_end(a.doc_start + (int64_t)b * a.Sq, a.Sq, j1, lane));
     // With dkdv_parts > 1 the query tiles of the key block (walked from the last one down) are cut
     // into dkdv_parts consecutive slices, one per workgroup; each leaves an fp32 partial sum and
     // attn_bwd_dkdv_reduce_kernel adds them in a fixed order.
@@ -639,7 +662,8 @@ __global__ __launch_bounds__(256, (NQB == 1 ? 3 : 2)) void attn_bwd_dq_kernel(co
     int bid = blockIdx.x;
     const int g = bid % a.G; bid /= a.G;
     const int hc = bid % n_hc; bid /= n_hc;
-    const int b = bid % a.B; bid /= a.B;
+    const int bi = bid % a.B; bid /= a.B;
+    const int b = rotated_batch_row(bi, bid, a.B);
     const int n_qt = (a.Sq + BM - 1) / BM;
     const int qt = n_qt - 1 - bid;
 

@@ -56,9 +56,10 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv64_kernel(const KArgs a) 
 
     int bid = blockIdx.x;
     const int g = bid % a.G; bid /= a.G;
-    const int b = bid % a.B; bid /= a.B;
+    const int bi = bid % a.B; bid /= a.B;
     const int part = bid % a.dkdv_parts; bid /= a.dkdv_parts;
     const int kt = bid;                                   // ascending: most work first
+    const int b = rotated_batch_row(bi, kt, a.B);
     const int j0 = kt * BN;                               // first key of the workgroup
     const int wj0 = j0 + WK * w;                          // first key of the wavefront
 

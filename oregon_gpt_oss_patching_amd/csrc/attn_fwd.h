@@ -200,7 +200,8 @@ __global__ __launch_bounds__(256, (NQB == 1 ? 3 : 2)) void attn_fwd_kernel(const
     int bid = blockIdx.x;
     const int g = bid % a.G; bid /= a.G;
     const int hc = bid % n_hc; bid /= n_hc;
-    const int b = bid % a.B; bid /= a.B;
+    const int bi = bid % a.B; bid /= a.B;
+    const int b = rotated_batch_row(bi, bid, a.B);
     const int n_qt = (a.Sq + BM - 1) / BM;
     const int qt = n_qt - 1 - bid;
 

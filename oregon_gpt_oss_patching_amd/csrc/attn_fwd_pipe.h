@@ -60,7 +60,8 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_pipe_kernel(const KArgs a) {
     int bid = blockIdx.x;
     const int g = bid % a.G; bid /= a.G;
     const int hc = bid % n_hc; bid /= n_hc;
-    const int b = bid % a.B; bid /= a.B;
+    const int bi = bid % a.B; bid /= a.B;
+    const int b = rotated_batch_row(bi, bid, a.B);
     const int qt = a.Sq / kTile - 1 - bid;
     const int head = g * a.r + hc * 4 + w;
     const int qw0 = qt * kTile;                    // the four wavefronts hold the same 64 rows of four heads

@@ -102,18 +102,26 @@ constexpr int kDkdvKeys = 32 * kDkdvNB * kDkdvWaves; // keys per dK/dV workgroup
 // Workgroups per key block in the dK/dV kernel.  One workgroup per (batch, KV head, 128 keys) fills
 // the 256 CUs (two workgroups each) only from S = 16384 on, and the causal triangle makes the first
 // key blocks many times longer than the last; shorter problems cut each key block's query tiles into
-// slices so that there are about a thousand workgroups, and sum the slices' fp32 partials afterwards.
-// A slice keeps at least four query tiles (sliding-window layers are never cut).
+// slices so that there are about a thousand workgroups, and sum the slices' fp32 partials afterwards
+// (sliding-window layers are never cut).  Up to 512 blocks the count is rounded up, and a slice keeps at least eight
+// (query tile, head) steps (B = 2, S = 383: 78 us uncut, 25 + 5 us in six slices).  Between 512 and 1024 blocks the first
+// key block of a long row (4096 rows and more) is still longer than the average compute unit's share: two slices; a
+// right-padded batch counts half, because its shorter rows leave the longest one alone (dK/dV of B = 4, S = 4096,
+// lengths 3309 / 1968 / 1554 / 4079: 715 us uncut, 589 in two slices; B = 2, S = 8192 / 4000: 1437 and 1216; but B = 8,
+// S <= 2048: 359 and 370).
 int dkdv_parts_for(const gptoss_attn_params *p) {
     if (p->dtype != GPTOSS_ATTN_BF16) return 1;
     const int64_t blocks = (int64_t)p->G * p->B * ((p->Skv + kDkdvKeys - 1) / kDkdvKeys);
-    int parts = (int)(1024 / (blocks > 0 ? blocks : 1));
     const int window = effective_window(p);
     const int64_t rows_seen = window > 0 ? (int64_t)kDkdvKeys + window - 1 : (int64_t)p->Sq;
-    const int tiles = (int)((rows_seen < p->Sq ? rows_seen : p->Sq) + 63) / 64;
-    if (parts > tiles / 4) parts = tiles / 4;
+    const int64_t tiles = ((rows_seen < p->Sq ? rows_seen : p->Sq) + 63) / 64;
+    int64_t parts = (1024 + blocks - 1) / blocks;
+    if (blocks > 512) parts = p->Sq >= 4096 && (p->seqlens && p->B > 1 ? blocks / 2 : blocks) < 1024 ? 2 : 1;
+    const int64_t steps = window > 0 ? tiles / 4 : tiles * (p->H / p->G) / 8;
+    if (parts > steps) parts = steps;
+    if (parts > tiles) parts = tiles;
     if (parts > 8) parts = 8;
-    return parts < 1 ? 1 : parts;
+    return parts < 1 ? 1 : (int)parts;
 }
 
 // Full-causal self-attention goes to attn_bwd_dkdv64_kernel (64 keys per wavefront, one wavefront per SIMD)
