@@ -1,14 +1,22 @@
 // float32 kernels (dtype GPTOSS_ATTN_FP32): the same forward / backward as the bf16 kernels
 // for callers that keep the model in float32 (the reference runs such tensors natively,
-// attention_kernel.py:11-217 are dtype-generic).  They exist for exactness, not speed: every
-// product runs on the fp32 matrix instruction v_mfma_f32_32x32x2_f32 with fp32 operands
-// straight from global memory (the L1/L2 caches do the sharing; there is no LDS staging), and
-// every element evaluates the full visibility predicate.
+// attention_kernel.py:11-217 are dtype-generic).  Every product runs on the fp32 matrix instruction
+// v_mfma_f32_32x32x2_f32 with fp32 operands and fp32 accumulation.
 //
-// One wavefront is independent of every other (no LDS, no barrier):
-//   forward, dQ : a wavefront owns 32 query rows of one head and walks 32-key tiles;
-//   dK/dV       : a wavefront owns 32 keys of one KV head and walks the query heads of the
-//                 group and their 32-row blocks.
+// What bounds them: that instruction takes 64 cycles for 4096 FLOP (157 TFLOP/s on the chip), sixteen times the bf16
+// instruction's price, so LDS traffic, L2 traffic and vector work are small beside it, and what matters is that every SIMD
+// always has a wavefront with its operands at hand.  A wavefront stages its tiles (32 rows of two tensors, 16 KB) in LDS of
+// its own, without a barrier in the loop; each tensor's half is requested again as soon as its last product has read it, so a
+// request has the time of at least one product to arrive.  A workgroup is four wavefronts, two workgroups share a
+// compute unit, and wavefronts that work on the same rows (KS of them in the forward and dQ, all four in dK/dV) take
+// the tiles these rows meet in turn and add their partial results at the end: a row block of S = 1024 is then 8 or 16
+// steps long instead of 32, and the chip fills from a few hundred rows on.
+//
+// Measured (64 query heads on 8 KV heads, S = 1024, full causal; before, with operands straight from global memory, one
+// wavefront per row block and none sharing it): forward 200 -> 101 us (85 TFLOP/s), dQ with the row statistics 306 -> 131
+// us, dK/dV 2227 -> 190 us (its 256 key blocks were 256 wavefronts).  At S = 4096 the matrix pipes are busy 73 to 81 % of
+// the cycles (2.2 GHz).
+//
 // Register layouts of v_mfma_f32_32x32x2_f32 (lane = 0..63, half = lane/32, l32 = lane%32):
 //   A (32 x 2): lane holds A[l32][half]      B (2 x 32): lane holds B[half][l32]
 //   C (32 x 32): register i holds C[crow(i, half)][l32]   (as for the bf16 instruction)
@@ -18,6 +26,7 @@
 // by the matching row of the other operand -- C registers are fed back as the B operand
 // without any data movement.
 #pragma once
+#include "attn_bwd.h"
 #include "attn_common.h"
 
 namespace gptoss {
@@ -27,7 +36,7 @@ __device__ __forceinline__ f32x16 mfma_f32(float a, float b, const f32x16 c) {
 }
 
 struct F32Ptrs {
-    const float *q, *k, *v, *d_o;
+    const float *q, *k, *v, *d_o, *o_in;
     float *o, *dq, *dk, *dv;
 };
 __device__ __forceinline__ F32Ptrs f32_ptrs(const KArgs &a) {
@@ -36,6 +45,7 @@ __device__ __forceinline__ F32Ptrs f32_ptrs(const KArgs &a) {
     p.k = reinterpret_cast<const float *>(a.k);
     p.v = reinterpret_cast<const float *>(a.v);
     p.d_o = reinterpret_cast<const float *>(a.d_o);
+    p.o_in = reinterpret_cast<const float *>(a.o);
     p.o = reinterpret_cast<float *>(a.o);
     p.dq = reinterpret_cast<float *>(a.dq);
     p.dk = reinterpret_cast<float *>(a.dk);
@@ -54,117 +64,256 @@ __device__ __forceinline__ void load_row32(float (&r)[32], const float *p, bool 
     }
 }
 
-// Per-lane description of one query row.
-struct RowInfo {
-    int pos;        // absolute position, hugely negative for a row that does not exist / is padding
-    unsigned win;   // visible keys are pos - win < key <= pos
+// ---- LDS tiles of 32 rows x 64 floats ---------------------------------------------------------------------
+// Rows are 256 bytes (all banks once), so the sixteen 16-byte chunks of a row are XOR-swizzled with the row number:
+// physical chunk p of row r holds logical chunk p ^ (r & 15).  Sixteen rows reading one logical chunk (natural 128-bit
+// fragment reads) then hit sixteen different bank groups.
+struct F32Tile {
+    static constexpr int kRows = 32, kRowBytes = 256, kBytes = kRows * kRowBytes, kCopies = 8;
 };
-__device__ __forceinline__ RowInfo row_info(const KArgs &a, int q_offset, int b, int row, int q_len) {
-    RowInfo r;
-    const int p = q_offset + row;
-    const bool live = row < a.Sq && p < q_len;
-    r.pos = live ? p : -0x40000000;
-    int w = a.window ? a.window : 0x3fffffff;
-    if (a.doc_start && row < a.Sq) w = min(w, p - a.doc_start[(int64_t)b * a.Sq + row] + 1);
-    r.win = (unsigned)w;
-    return r;
+// requests the tile whose first row is `tile` (kCopies instructions of this wavefront); rows past `last` re-read that one
+__device__ __forceinline__ void f32_copy_tile(uint32_t lds_tile, const float *tile, int stride, int last, int lane) {
+#pragma unroll
+    for (int i = 0; i < F32Tile::kCopies; ++i) {
+        const int r = 4 * i + (lane >> 4), ch = (lane & 15) ^ (r & 15);
+        lds_dma16(lds_tile + i * 1024, tile, (uint32_t)(min(r, last) * stride) * 4u + ch * 16);
+    }
 }
-__device__ __forceinline__ bool visible(const RowInfo &r, int key, int kv_len) {
-    return ((unsigned)(r.pos - key) < r.win) & (key < kv_len);
+// at most n of this wavefront's copies outstanding, and no LDS access moved across
+#define GPTOSS_F32_WAIT(n) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(n) : "memory")
+// every LDS read issued so far has its data: the tile it came from may be overwritten
+#define GPTOSS_F32_READS_DONE() asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory")
+struct F32Offsets {
+    uint32_t nat;      // natural fragment: row l32, logical chunk 8 * half; chunk j of it is at nat ^ (j << 4)
+    uint32_t tr[4];    // [e]: element (row 4 * half + e, column l32); (row + 8 a4, column + 32 dblk) by immediates
+};
+__device__ __forceinline__ F32Offsets make_f32_offsets(int lane) {
+    F32Offsets o;
+    const int l32 = lane & 31, half = lane >> 5;
+    o.nat = l32 * F32Tile::kRowBytes + (((8 * half) ^ (l32 & 15)) << 4);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o.tr[e] = (4 * half + e) * F32Tile::kRowBytes + (((l32 >> 2) ^ (4 * half + e)) << 4) + (l32 & 3) * 4;
+    return o;
+}
+__device__ __forceinline__ f32x4 f32_nat(uint32_t tile, const F32Offsets &o, int j) { return lds_load128f(tile + (o.nat ^ (j << 4)), 0); }
+// (bit 3 of the chunk index is 0 in tr[e]: XOR with 8 adds 128 bytes)
+__device__ __forceinline__ float f32_tr(uint32_t tile, const F32Offsets &o, int a4, int e, int dblk) {
+    typedef __attribute__((address_space(3))) float lds_f32;
+    return *reinterpret_cast<const lds_f32 *>((uintptr_t)(tile + o.tr[e] + 8 * a4 * F32Tile::kRowBytes + ((dblk ^ (a4 & 1)) << 7)));
+}
+// The operands of the next few MFMAs are read from LDS while the current ones run (an MFMA takes 64 cycles; read, wait,
+// multiply one by one, which is what the compiler makes of the plain loops, doubles a tile's time).
+#define GPTOSS_F32_FENCE() __builtin_amdgcn_sched_barrier(0)
+// s += X Y^T over head_dim: X's rows from the tile (result rows), y[] the lane's row of Y (result columns)
+__device__ __forceinline__ void f32_rows_product(f32x16 &s, uint32_t tile, const F32Offsets &o, const float (&y)[32]) {
+    f32x4 x = f32_nat(tile, o, 0);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        f32x4 next = x;
+        if (j < 7) next = f32_nat(tile, o, j + 1);
+        GPTOSS_F32_FENCE();
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s = mfma_f32(x[e], y[4 * j + e], s);
+        GPTOSS_F32_FENCE();
+        x = next;
+    }
+}
+// acc^T[d][col] += tile^T[d][row] p[row][col] over the tile's 32 rows (p in C registers)
+__device__ __forceinline__ void f32_cols_product(f32x16 (&acc)[2], uint32_t tile, const F32Offsets &o, const f32x16 &p) {
+    float x[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = f32_tr(tile, o, 0, e >> 1, e & 1);
+#pragma unroll
+    for (int a4 = 0; a4 < 4; ++a4) {
+        float next[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) next[e] = a4 < 3 ? f32_tr(tile, o, a4 + 1, e >> 1, e & 1) : 0.0f;
+        GPTOSS_F32_FENCE();
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[e & 1] = mfma_f32(x[e], p[4 * a4 + (e >> 1)], acc[e & 1]);
+        GPTOSS_F32_FENCE();
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = next[e];
+    }
 }
 
-// wavefront index -> (batch, head-like index, 32-row block); false when out of range
-__device__ __forceinline__ bool wave_work(int n_blk, int n_head, int n_batch, int &b, int &h, int &blk) {
-    const int64_t wid = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (wid >= (int64_t)n_blk * n_head * n_batch) return false;
-    blk = (int)(wid % n_blk);
-    h = (int)((wid / n_blk) % n_head);
-    b = (int)(wid / ((int64_t)n_blk * n_head));
-    return true;
+// Where a wavefront of the forward / dQ kernels stands: 32 query rows of one head (a unit; 4 / KS units per workgroup) and
+// every KS-th of the 32-key tiles they see.
+struct F32Unit { int head, b, q0; bool live; };
+template <int KS>
+struct F32QueryWork {
+    int g, b, head, q0, q_len, kv_len, weff, pos0, pos1, ds1, t0, n_it, w, lane;
+    const float *kbase, *vbase;
+    uint32_t ksm, vsm;         // this wavefront's K and V tile in LDS
+    // unit i of the workgroup: KV head fastest (its K / V stay in one XCD's L2), then the heads of the group, longest key loops first
+    static __device__ __forceinline__ F32Unit unit(const KArgs &a, int i) {
+        F32Unit u;
+        const int g = (int)(blockIdx.x % a.G);
+        int n = (int)(blockIdx.x / a.G) * (4 / KS) + i;
+        u.head = g * a.r + n % a.r; n /= a.r;
+        const int bi = n % a.B, z = n / a.B, n_q = (a.Sq + 31) / 32;
+        u.b = rotated_batch_row(bi, z, a.B);
+        u.live = z < n_q;
+        u.q0 = 32 * max(n_q - 1 - z, 0);
+        return u;
+    }
+    __device__ __forceinline__ F32QueryWork(const KArgs &a, const F32Ptrs &t, int q_offset, char *lds) {
+        lane = threadIdx.x & 63;
+        w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        ksm = lds_addr(lds) + w * (2 * F32Tile::kBytes);
+        vsm = ksm + F32Tile::kBytes;
+        const F32Unit u = unit(a, w / KS);
+        b = u.b; head = u.head; q0 = u.q0; g = head / a.r;
+        kv_len = a.seqlens ? min(a.Skv, a.seqlens[b]) : a.Skv;
+        q_len = a.seqlens ? a.seqlens[b] : 0x7fffffff;
+        weff = a.window ? a.window : 0x3fffffff;
+        pos0 = q_offset + q0;
+        pos1 = min(q_offset + min(a.Sq, q0 + 32) - 1, q_len - 1);
+        const int32_t *dsrow = a.doc_start ? a.doc_start + (int64_t)b * a.Sq : nullptr;
+        const int ds0 = dsrow ? dsrow[min(q0, a.Sq - 1)] : 0;
+        ds1 = dsrow ? dsrow[min(q0 + 31, a.Sq - 1)] : 0;
+        const int hi = pos1 >= pos0 && u.live ? max(0, min(kv_len, pos1 + 1)) : 0;
+        const int t_lo = max(max(0, pos0 - weff + 1), ds0) / F32Tile::kRows;
+        const int n = max(0, (hi + F32Tile::kRows - 1) / F32Tile::kRows - t_lo);
+        t0 = t_lo + w % KS;
+        n_it = (n - w % KS + KS - 1) / KS;               // tiles t0 + KS it  (0 if n <= w % KS)
+        kbase = t.k + (int64_t)b * a.ks.b + (int64_t)g * a.ks.h;
+        vbase = t.v + (int64_t)b * a.vs.b + (int64_t)g * a.vs.h;
+    }
+    __device__ __forceinline__ int first_key(int it) const { return (t0 + KS * it) * F32Tile::kRows; }
+    __device__ __forceinline__ void request_k(const KArgs &a, int it) const {
+        const int n0 = first_key(it);
+        f32_copy_tile(ksm, kbase + (int64_t)n0 * a.ks.s, (int)a.ks.s, a.Skv - 1 - n0, lane);
+    }
+    __device__ __forceinline__ void request_v(const KArgs &a, int it) const {
+        const int n0 = first_key(it);
+        f32_copy_tile(vsm, vbase + (int64_t)n0 * a.vs.s, (int)a.vs.s, a.Skv - 1 - n0, lane);
+    }
+    __device__ __forceinline__ bool interior(const KArgs &a, int n0) const {
+        return n0 + 31 <= pos0 && n0 > pos1 - weff && n0 + 32 <= kv_len && pos0 + 31 <= pos1 && n0 >= ds1;
+    }
+    // the lane's query position (hugely negative: no such row) and its own window (packed rows: back to its document's start)
+    __device__ __forceinline__ void row_info(const KArgs &a, int q_offset, int row, int &pos, unsigned &win) const {
+        const int p = q_offset + row;
+        pos = row < a.Sq && p < q_len ? p : -0x40000000;
+        win = (unsigned)weff;
+        if (a.doc_start && row < a.Sq) win = (unsigned)min(weff, p - a.doc_start[(int64_t)b * a.Sq + row] + 1);
+    }
+};
+
+// Partial results of the four wavefronts through LDS: a wavefront leaves its transposed 64 x 32 accumulators as 32 rows of 64
+// floats, chunks swizzled like a tile's ...
+__device__ __forceinline__ void f32_leave_partial(char *mine, const f32x16 (&acc)[2], int lane) {
+    const int l32 = lane & 31, half = lane >> 5;
+#pragma unroll
+    for (int dblk = 0; dblk < 2; ++dblk)
+#pragma unroll
+        for (int a4 = 0; a4 < 4; ++a4)
+            *reinterpret_cast<f32x4 *>(mine + l32 * F32Tile::kRowBytes + (((8 * dblk + 2 * a4 + half) ^ (l32 & 15)) << 4)) =
+                f32x4{acc[dblk][4 * a4], acc[dblk][4 * a4 + 1], acc[dblk][4 * a4 + 2], acc[dblk][4 * a4 + 3]};
+}
+// ... and a thread picks up its 16-byte chunk `ch` of row r of wavefront k's
+__device__ __forceinline__ f32x4 f32_partial(const char *smem, int wave_bytes, int k, int r, int ch) {
+    return *reinterpret_cast<const f32x4 *>(smem + k * wave_bytes + r * F32Tile::kRowBytes + ((ch ^ (r & 15)) << 4));
 }
 
 // ---- forward ------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void attn_f32_fwd_kernel(const KArgs a) {
+template <int KS>
+__global__ __launch_bounds__(256, 2) void attn_f32_fwd_kernel(const KArgs a) {
+    __shared__ __attribute__((aligned(1024))) char smem[8 * F32Tile::kBytes];
     const int q_offset = query_offset(a);
     const F32Ptrs t = f32_ptrs(a);
-    const int lane = threadIdx.x & 63, l32 = lane & 31, half = lane >> 5;
-    int b, head, qblk;
-    if (!wave_work((a.Sq + 31) / 32, a.H, a.B, b, head, qblk)) return;
-    const int g = head / a.r;
-    const int kv_len = a.seqlens ? min(a.Skv, a.seqlens[b]) : a.Skv;
-    const int q_len = a.seqlens ? a.seqlens[b] : 0x7fffffff;
-    const int q0 = 32 * qblk, row = q0 + l32;
-    const RowInfo ri = row_info(a, q_offset, b, row, q_len);
-
+    using W = F32QueryWork<KS>;
+    const W wk(a, t, q_offset, smem);
+    const int lane = wk.lane, l32 = lane & 31, half = lane >> 5, row = wk.q0 + l32;
+    int pos;
+    unsigned win;
+    wk.row_info(a, q_offset, row, pos, win);
+    if (wk.n_it > 0) { wk.request_k(a, 0); wk.request_v(a, 0); }
     float qr[32];    // Q[row][32*half + ks]
-    load_row32(qr, t.q + (int64_t)b * a.qs.b + (int64_t)head * a.qs.h + (int64_t)min(row, a.Sq - 1) * a.qs.s + 32 * half, row < a.Sq);
-    const float *kb = t.k + (int64_t)b * a.ks.b + (int64_t)g * a.ks.h;
-    const float *vb = t.v + (int64_t)b * a.vs.b + (int64_t)g * a.vs.h;
-
+    load_row32(qr, t.q + (int64_t)wk.b * a.qs.b + (int64_t)wk.head * a.qs.h + (int64_t)min(row, a.Sq - 1) * a.qs.s + 32 * half, row < a.Sq);
+    const F32Offsets lo = make_f32_offsets(lane);
     const float c = a.scale_log2;
-    const float sink2 = (a.sinks ? a.sinks[head] : 0.0f) * kLog2e;
+    const float sink2 = (a.sinks ? a.sinks[wk.head] : 0.0f) * kLog2e;
     float m = sink2, l = 0.0f;
     f32x16 o[2];
 #pragma unroll
     for (int i = 0; i < 16; ++i) { o[0][i] = 0.0f; o[1][i] = 0.0f; }
 
-    // keys any row of this block can see: [key_lo, key_hi)
-    const int weff = a.window ? a.window : 0x3fffffff;
-    const int pos_hi = min(q_offset + min(a.Sq, q0 + 32) - 1, q_len - 1);
-    const int key_hi = pos_hi >= q_offset + q0 ? min(kv_len, pos_hi + 1) : 0;
-    const int key_lo = max(0, q_offset + q0 - weff + 1);
-    for (int n0 = (key_lo / 32) * 32; n0 < key_hi; n0 += 32) {
-        float kr[32];    // K[n0 + l32][32*half + ks]
-        load_row32(kr, kb + (int64_t)min(n0 + l32, a.Skv - 1) * a.ks.s + 32 * half, true);
+    wait_vmcnt<0>();       // the compiler's own loads have arrived: it puts no vmcnt wait (which would also drain the copies) into the loop
+    for (int it = 0; it < wk.n_it; ++it) {
+        const int n0 = wk.first_key(it);
+        const bool more = it + 1 < wk.n_it;
+        GPTOSS_F32_WAIT(F32Tile::kCopies);         // K is here; V may be on its way
         f32x16 s;
 #pragma unroll
         for (int i = 0; i < 16; ++i) s[i] = 0.0f;
+        f32_rows_product(s, wk.ksm, lo, qr);       // S^T: rows = keys, lane = query row
+        GPTOSS_F32_READS_DONE();
+        if (more) wk.request_k(a, it + 1);
+        if (!wk.interior(a, n0)) {
+            const KeyMask km = make_key_mask(pos - n0, win, wk.kv_len - n0, half);
 #pragma unroll
-        for (int ks = 0; ks < 32; ++ks) s = mfma_f32(kr[ks], qr[ks], s);      // S^T: rows = keys, lane = query row
-        float mx = -INFINITY;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            s[i] = visible(ri, n0 + crow(i, half), kv_len) ? s[i] * c : -INFINITY;
-            mx = fmaxf(mx, s[i]);
+            for (int i = 0; i < 16; ++i) s[i] = key_visible(km, 8 * (i >> 2) + (i & 3)) ? s[i] : -INFINITY;
         }
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
-        const float m_new = fmaxf(m, mx);
-        const float alpha = exp2f(m - m_new);
-        m = m_new;
-        l *= alpha;
+        float mx0 = s[0], mx1 = s[1];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) { o[0][i] *= alpha; o[1][i] *= alpha; }
+        for (int i = 2; i < 16; i += 2) { mx0 = fast_max(mx0, s[i]); mx1 = fast_max(mx1, s[i + 1]); }
+        const float m_new = fast_max(m, xhalf_max(fast_max(mx0, mx1)) * c);
+        if (__builtin_amdgcn_ballot_w64(m_new != m) != 0ull) {
+            const float alpha = fast_exp2(m - m_new);
+            m = m_new;
+            l *= alpha;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            s[i] = exp2f(s[i] - m);
-            l += s[i];
+            for (int i = 0; i < 16; ++i) { o[0][i] *= alpha; o[1][i] *= alpha; }
         }
-        // O^T[d][row] += V^T[d][key] P^T[key][row]
+        float rs0 = 0.0f, rs1 = 0.0f;
 #pragma unroll
-        for (int a4 = 0; a4 < 4; ++a4)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float *vrow = vb + (int64_t)min(n0 + 8 * a4 + 4 * half + e, a.Skv - 1) * a.vs.s;
-#pragma unroll
-                for (int dblk = 0; dblk < 2; ++dblk) o[dblk] = mfma_f32(vrow[32 * dblk + l32], s[4 * a4 + e], o[dblk]);
-            }
+        for (int i = 0; i < 16; i += 2) {
+            s[i] = fast_exp2(fmaf(s[i], c, -m));
+            s[i + 1] = fast_exp2(fmaf(s[i + 1], c, -m));
+            rs0 += s[i];
+            rs1 += s[i + 1];
+        }
+        l += rs0 + rs1;
+        if (more) GPTOSS_F32_WAIT(F32Tile::kCopies); else GPTOSS_F32_WAIT(0);
+        f32_cols_product(o, wk.vsm, lo, s);        // O^T[d][row] += V^T[d][key] P^T[key][row]
+        GPTOSS_F32_READS_DONE();
+        if (more) wk.request_v(a, it + 1);
     }
 
-    const float l_tot = l + __shfl_xor(l, 32);
-    const float z = l_tot + exp2f(sink2 - m);
-    const float inv = 1.0f / z;
-    if (row < a.Sq) {
-        float *orow = t.o + (int64_t)b * a.os.b + (int64_t)head * a.os.h + (int64_t)row * a.os.s;
+    // merge: the row's reference is the largest of the KS wavefronts', z and O are scaled to it
+    float *const ml = reinterpret_cast<float *>(smem + 4 * F32Tile::kBytes);       // [wavefront][m, l][row]
+    const float l_tot = xhalf_sum(l);
+    __syncthreads();
+    f32_leave_partial(smem + wk.w * F32Tile::kBytes, o, lane);
+    if (half == 0) { ml[(2 * wk.w) * 32 + l32] = m; ml[(2 * wk.w + 1) * 32 + l32] = l_tot; }
+    __syncthreads();
 #pragma unroll
-        for (int dblk = 0; dblk < 2; ++dblk)
+    for (int pass = 0; pass < 8 / KS; ++pass) {
+        const int i = pass >> 1, r = (threadIdx.x >> 4) + 16 * (pass & 1), ch = threadIdx.x & 15;
+        const F32Unit u = W::unit(a, i);
+        const float sink = (a.sinks ? a.sinks[u.head] : 0.0f) * kLog2e;
+        float mm = sink;
 #pragma unroll
-            for (int a4 = 0; a4 < 4; ++a4) {
-                f32x4 w4;
+        for (int k = 0; k < KS; ++k) mm = fast_max(mm, ml[2 * (KS * i + k) * 32 + r]);
+        float z = fast_exp2(sink - mm);
+        f32x4 x = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-                for (int e = 0; e < 4; ++e) w4[e] = o[dblk][4 * a4 + e] * inv;
-                *reinterpret_cast<f32x4 *>(orow + 32 * dblk + 8 * a4 + 4 * half) = w4;
-            }
-        if (half == 0) a.lse[((int64_t)b * a.H + head) * a.Sq + row] = (m + log2f(z)) * kLn2;
+        for (int k = 0; k < KS; ++k) {
+            const float f = fast_exp2(ml[2 * (KS * i + k) * 32 + r] - mm);
+            z += f * ml[(2 * (KS * i + k) + 1) * 32 + r];
+            const f32x4 y = f32_partial(smem, F32Tile::kBytes, KS * i + k, r, ch);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[e] = fmaf(f, y[e], x[e]);
+        }
+        const float inv = 1.0f / z;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[e] *= inv;
+        if (u.live && u.q0 + r < a.Sq) {
+            *reinterpret_cast<f32x4 *>(t.o + (int64_t)u.b * a.os.b + (int64_t)u.head * a.os.h + (int64_t)(u.q0 + r) * a.os.s + 4 * ch) = x;
+            if (ch == 0) a.lse[((int64_t)u.b * a.H + u.head) * a.Sq + u.q0 + r] = (mm + log2f(z)) * kLn2;
+        }
     }
 }
 
@@ -195,16 +344,29 @@ __global__ __launch_bounds__(256) void attn_f32_delta_kernel(const KArgs a) {
 }
 
 // ---- backward step 2: dK, dV ------------------------------------------------------------
-__global__ __launch_bounds__(256) void attn_f32_dkdv_kernel(const KArgs a) {
+// Problems with few key blocks are cut into slices of the query tiles besides (fp32 partials in the scratch, as in the
+// bf16 path).
+struct F32Dkdv {
+    static constexpr int kStatBytes = 2 * 32 * 4;                      // 32 x -delta, 32 x lse * log2(e)
+    static constexpr int kStatOff = 8 * F32Tile::kBytes;
+    static constexpr int kLdsBytes = kStatOff + 4 * kStatBytes;
+};
+__global__ __launch_bounds__(256, 2) void attn_f32_dkdv_kernel(const KArgs a) {
+    using C = F32Dkdv;
+    __shared__ __attribute__((aligned(1024))) char smem[C::kLdsBytes];
     const int q_offset = query_offset(a);
     const F32Ptrs t = f32_ptrs(a);
-    const int lane = threadIdx.x & 63, l32 = lane & 31, half = lane >> 5;
-    int b, g, kblk;
-    if (!wave_work((a.Skv + 31) / 32, a.G, a.B, b, g, kblk)) return;
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, half = lane >> 5;
+    int bid = blockIdx.x;
+    const int g = bid % a.G; bid /= a.G;
+    const int bi = bid % a.B; bid /= a.B;
+    const int part = bid % a.dkdv_parts, kblk = bid / a.dkdv_parts;       // ascending: most work first
+    const int b = rotated_batch_row(bi, kblk, a.B);
     const int kv_len = a.seqlens ? min(a.Skv, a.seqlens[b]) : a.Skv;
     const int q_len = a.seqlens ? a.seqlens[b] : 0x7fffffff;
-    const int j0 = 32 * kblk, key = j0 + l32;
+    const int j0 = 32 * kblk, key = j0 + l32, j1 = min(j0 + 32, kv_len) - 1;
     const int64_t total = (int64_t)a.B * a.H * a.Sq;
+    const int32_t *dsrow = a.doc_start ? a.doc_start + (int64_t)b * a.Sq : nullptr;
 
     float kr[32], vr[32];    // K / V[key][32*half + ks]  (B operands of S and dP)
     load_row32(kr, t.k + (int64_t)b * a.ks.b + (int64_t)g * a.ks.h + (int64_t)min(key, a.Skv - 1) * a.ks.s + 32 * half, key < a.Skv);
@@ -213,144 +375,219 @@ __global__ __launch_bounds__(256) void attn_f32_dkdv_kernel(const KArgs a) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) { dk[0][i] = dk[1][i] = 0.0f; dv[0][i] = dv[1][i] = 0.0f; }
 
-    // query rows that can see any key of the block: positions [j0, j0 + 31 + window)
+    // query rows that can see any key of the block: positions [j0, j1 + window), within the documents of the keys
     const int weff = a.window ? a.window : 0x3fffffff;
+    const int row_lim = (int)min((int64_t)a.Sq, max((int64_t)0, (int64_t)q_len - q_offset));
     const int row_lo = max(0, j0 - q_offset);
-    const int64_t row_hi64 = min((int64_t)min(a.Sq, max(0, q_len - q_offset)), (int64_t)j0 + 31 + weff - q_offset);
-    const int row_hi = j0 < kv_len ? (int)row_hi64 : 0;
+    int row_hi = j1 >= j0 ? (int)min((int64_t)row_lim, max((int64_t)0, (int64_t)j1 + weff - q_offset)) : 0;
+    if (dsrow && row_hi > row_lo) row_hi = min(row_hi, document_end(dsrow, a.Sq, j1, lane));
+    const int t_lo = row_lo / 32, n_tiles = max(0, (row_hi + 31) / 32 - t_lo);
+    const int slice = (n_tiles + a.dkdv_parts - 1) / a.dkdv_parts;
+    const int t0 = t_lo + part * slice, n_it = max(0, min(slice, n_tiles - part * slice)) * a.r;
+
+    const uint32_t qsm = lds_addr(smem) + w * (2 * F32Tile::kBytes), gsm = qsm + F32Tile::kBytes;
+    const uint32_t ssm = lds_addr(smem) + C::kStatOff + w * C::kStatBytes;
+    const F32Offsets lo = make_f32_offsets(lane);
     const float c = a.scale_log2;
-    for (int hh = 0; hh < a.r; ++hh) {
-        const int head = g * a.r + hh;
-        const float *qb = t.q + (int64_t)b * a.qs.b + (int64_t)head * a.qs.h;
-        const float *gb = t.d_o + (int64_t)b * a.dos.b + (int64_t)head * a.dos.h;
-        const float *nd = a.delta + ((int64_t)b * a.H + head) * a.Sq;     // -delta
-        const float *l2 = nd + total;                                      // lse * log2(e)
-        for (int q0 = (row_lo / 32) * 32; q0 < row_hi; q0 += 32) {
-            const int qrow = min(q0 + l32, a.Sq - 1);
-            float qr[32], gr[32];   // Q / dO[q0 + l32][32*half + ks]  (A operands)
-            load_row32(qr, qb + (int64_t)qrow * a.qs.s + 32 * half, true);
-            load_row32(gr, gb + (int64_t)qrow * a.dos.s + 32 * half, true);
-            f32x16 s, dp;
+    // requests for step `it` (query tile t0 + it / r, head it % r): the Q tile; the dO tile and the row statistics
+    auto request_q = [&](int it) __attribute__((always_inline)) {
+        const int q0 = 32 * (t0 + it / a.r), head = g * a.r + it % a.r;
+        f32_copy_tile(qsm, t.q + (int64_t)b * a.qs.b + (int64_t)head * a.qs.h + (int64_t)q0 * a.qs.s, (int)a.qs.s, a.Sq - 1 - q0, lane);
+    };
+    auto request_g = [&](int it) __attribute__((always_inline)) {
+        const int q0 = 32 * (t0 + it / a.r), head = g * a.r + it % a.r;
+        f32_copy_tile(gsm, t.d_o + (int64_t)b * a.dos.b + (int64_t)head * a.dos.h + (int64_t)q0 * a.dos.s, (int)a.dos.s, a.Sq - 1 - q0, lane);
+        lds_dma4(ssm, a.delta + ((int64_t)b * a.H + head) * a.Sq, ((half ? (uint32_t)total : 0u) + (uint32_t)min(q0 + l32, a.Sq - 1)) * 4u);
+    };
+    if (w < n_it) { request_g(w); request_q(w); }
+    wait_vmcnt<0>();         // the compiler's own loads have arrived: no vmcnt wait of its own in the loop
+    for (int it = w; it < n_it; it += 4) {
+        const int q0 = 32 * (t0 + it / a.r);
+        const bool more = it + 4 < n_it;
+        GPTOSS_F32_WAIT(F32Tile::kCopies);                             // dO and the statistics are here; Q may be on its way
+        f32x16 s, dp;
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                s[i] = 0.0f;
-                dp[i] = nd[min(q0 + crow(i, half), a.Sq - 1)];          // seeds dP with -delta of its row
-            }
+        for (int a4 = 0; a4 < 4; ++a4) {
+            const f32x4 nd = lds_load128f(ssm + 16 * half, 32 * a4);
 #pragma unroll
-            for (int ks = 0; ks < 32; ++ks) {
-                s = mfma_f32(qr[ks], kr[ks], s);                          // rows = queries, lane = key
-                dp = mfma_f32(gr[ks], vr[ks], dp);
-            }
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const int row = q0 + crow(i, half);
-                RowInfo ri = row_info(a, q_offset, b, row, q_len);
-                const float p = visible(ri, key, kv_len) ? exp2f(fmaf(s[i], c, -l2[min(row, a.Sq - 1)])) : 0.0f;
-                s[i] = p;
-                dp[i] = p * dp[i];                                        // dS (without the softmax scale)
-            }
-            // dV^T[d][key] += dO^T[d][row] P[row][key];  dK^T[d][key] += Q^T[d][row] dS[row][key]
-#pragma unroll
-            for (int a4 = 0; a4 < 4; ++a4)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int r = min(q0 + 8 * a4 + 4 * half + e, a.Sq - 1);
-                    const float *grow = gb + (int64_t)r * a.dos.s;
-                    const float *qrow2 = qb + (int64_t)r * a.qs.s;
-#pragma unroll
-                    for (int dblk = 0; dblk < 2; ++dblk) {
-                        dv[dblk] = mfma_f32(grow[32 * dblk + l32], s[4 * a4 + e], dv[dblk]);
-                        dk[dblk] = mfma_f32(qrow2[32 * dblk + l32], dp[4 * a4 + e], dk[dblk]);
-                    }
-                }
+            for (int e = 0; e < 4; ++e) { s[4 * a4 + e] = 0.0f; dp[4 * a4 + e] = nd[e]; }     // dP starts at -delta of its row
         }
-    }
-    if (key < a.Skv) {
-        float *dkrow = t.dk + (int64_t)b * a.dks.b + (int64_t)g * a.dks.h + (int64_t)key * a.dks.s;
-        float *dvrow = t.dv + (int64_t)b * a.dvs.b + (int64_t)g * a.dvs.h + (int64_t)key * a.dvs.s;
+        f32_rows_product(dp, gsm, lo, vr);                             // rows = queries, lane = key
+        GPTOSS_F32_WAIT(0);
+        f32_rows_product(s, qsm, lo, kr);
+        const bool interior = j0 + 31 <= q_offset + q0 && q_offset + q0 + 31 - weff < j0 && j0 + 32 <= kv_len && q0 + 32 <= row_lim && !dsrow;
 #pragma unroll
-        for (int dblk = 0; dblk < 2; ++dblk)
+        for (int a4 = 0; a4 < 4; ++a4) {
+            const f32x4 l2 = lds_load128f(ssm + 128 + 16 * half, 32 * a4);
 #pragma unroll
-            for (int a4 = 0; a4 < 4; ++a4) {
-                f32x4 wk, wv;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) { wk[e] = dk[dblk][4 * a4 + e] * a.scale; wv[e] = dv[dblk][4 * a4 + e]; }
-                *reinterpret_cast<f32x4 *>(dkrow + 32 * dblk + 8 * a4 + 4 * half) = wk;
-                *reinterpret_cast<f32x4 *>(dvrow + 32 * dblk + 8 * a4 + 4 * half) = wv;
+            for (int e = 0; e < 4; ++e) {
+                const int i = 4 * a4 + e;
+                float p = fast_exp2(fmaf(s[i], c, -l2[e]));
+                if (!interior) {
+                    const int row = q0 + 8 * a4 + 4 * half + e;
+                    bool vis = (unsigned)(q_offset + row - key) < (unsigned)weff && key < kv_len && row < row_lim;
+                    if (dsrow) vis = vis && key >= dsrow[min(row, a.Sq - 1)];
+                    p = vis ? p : 0.0f;
+                }
+                s[i] = p;
+                dp[i] = p * dp[i];                                     // dS (without the softmax scale)
             }
+        }
+        // dV^T[d][key] += dO^T[d][row] P[row][key];  dK^T[d][key] += Q^T[d][row] dS[row][key]
+        f32_cols_product(dv, gsm, lo, s);
+        GPTOSS_F32_READS_DONE();
+        if (more) request_g(it + 4);
+        f32_cols_product(dk, qsm, lo, dp);
+        GPTOSS_F32_READS_DONE();
+        if (more) request_q(it + 4);
+    }
+
+    // the four wavefronts' sums, added in wavefront order
+    const int64_t tensor = (int64_t)a.B * a.G * a.Skv * kD;
+    __syncthreads();
+    f32_leave_partial(smem + w * (2 * F32Tile::kBytes), dk, lane);
+    f32_leave_partial(smem + w * (2 * F32Tile::kBytes) + F32Tile::kBytes, dv, lane);
+    __syncthreads();
+#pragma unroll
+    for (int pass = 0; pass < 4; ++pass) {
+        const int which = pass >> 1, r = (tid >> 4) + 16 * (pass & 1), ch = tid & 15, j = j0 + r;
+        f32x4 x = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const f32x4 y = f32_partial(smem + which * F32Tile::kBytes, 2 * F32Tile::kBytes, k, r, ch);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[e] += y[e];
+        }
+        if (j < a.Skv) {
+            if (a.dkdv_parts > 1) {
+                *reinterpret_cast<f32x4 *>(a.dkdv_partial + (int64_t)(2 * part + which) * tensor + (((int64_t)b * a.G + g) * a.Skv + j) * kD + 4 * ch) = x;
+            } else {
+                const Strides &st = which == 0 ? a.dks : a.dvs;
+                const float mul = which == 0 ? a.scale : 1.0f;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[e] *= mul;
+                *reinterpret_cast<f32x4 *>((which == 0 ? t.dk : t.dv) + (int64_t)b * st.b + (int64_t)g * st.h + (int64_t)j * st.s + 4 * ch) = x;
+            }
+        }
     }
 }
 
+// The slices' partial sums, added in slice order.  One thread per 16-byte output chunk.
+__global__ __launch_bounds__(256) void attn_f32_dkdv_reduce_kernel(const KArgs a) {
+    const F32Ptrs t = f32_ptrs(a);
+    const int64_t rows = (int64_t)a.B * a.G * a.Skv, tensor = rows * kD;
+    const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (idx >= 2 * rows * 16) return;
+    const int which = idx >= rows * 16;
+    const int64_t rem = idx - (int64_t)which * rows * 16, row = rem >> 4;
+    const float *src = a.dkdv_partial + (int64_t)which * tensor + rem * 4;
+    f32x4 x = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int part = 0; part < a.dkdv_parts; ++part) {
+        const f32x4 y = *reinterpret_cast<const f32x4 *>(src + (int64_t)part * 2 * tensor);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[e] += y[e];
+    }
+    const float mul = which == 0 ? a.scale : 1.0f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x[e] *= mul;
+    const int key = (int)(row % a.Skv), bg = (int)(row / a.Skv), g = bg % a.G, b = bg / a.G;
+    const Strides &st = which == 0 ? a.dks : a.dvs;
+    *reinterpret_cast<f32x4 *>((which == 0 ? t.dk : t.dv) + (int64_t)b * st.b + (int64_t)g * st.h + (int64_t)key * st.s + 4 * (rem & 15)) = x;
+}
+
 // ---- backward step 3: dQ ----------------------------------------------------------------
-__global__ __launch_bounds__(256) void attn_f32_dq_kernel(const KArgs a) {
+// FUSE_DELTA: the kernel also forms -delta and lse * log2(e) of its rows, in the summation order of
+// attn_f32_delta_kernel, and leaves them in the scratch for the kernels that follow.
+template <int KS, bool FUSE_DELTA>
+__global__ __launch_bounds__(256, 2) void attn_f32_dq_kernel(const KArgs a) {
+    __shared__ __attribute__((aligned(1024))) char smem[8 * F32Tile::kBytes];
     const int q_offset = query_offset(a);
     const F32Ptrs t = f32_ptrs(a);
-    const int lane = threadIdx.x & 63, l32 = lane & 31, half = lane >> 5;
-    int b, head, qblk;
-    if (!wave_work((a.Sq + 31) / 32, a.H, a.B, b, head, qblk)) return;
-    const int g = head / a.r;
-    const int kv_len = a.seqlens ? min(a.Skv, a.seqlens[b]) : a.Skv;
-    const int q_len = a.seqlens ? a.seqlens[b] : 0x7fffffff;
-    const int q0 = 32 * qblk, row = q0 + l32;
-    const RowInfo ri = row_info(a, q_offset, b, row, q_len);
+    using W = F32QueryWork<KS>;
+    const W wk(a, t, q_offset, smem);
+    const int lane = wk.lane, l32 = lane & 31, half = lane >> 5, row = wk.q0 + l32;
+    const bool row_ok = row < a.Sq;
+    int pos;
+    unsigned win;
+    wk.row_info(a, q_offset, row, pos, win);
     const int64_t total = (int64_t)a.B * a.H * a.Sq;
     const int rowc = min(row, a.Sq - 1);
+    const int64_t rid = ((int64_t)wk.b * a.H + wk.head) * a.Sq + rowc;
 
+    if (wk.n_it > 0) { wk.request_v(a, 0); wk.request_k(a, 0); }
     float qr[32], gr[32];
-    load_row32(qr, t.q + (int64_t)b * a.qs.b + (int64_t)head * a.qs.h + (int64_t)rowc * a.qs.s + 32 * half, row < a.Sq);
-    load_row32(gr, t.d_o + (int64_t)b * a.dos.b + (int64_t)head * a.dos.h + (int64_t)rowc * a.dos.s + 32 * half, row < a.Sq);
-    const float ndelta = a.delta[((int64_t)b * a.H + head) * a.Sq + rowc];
-    const float lse2 = a.delta[total + ((int64_t)b * a.H + head) * a.Sq + rowc];
-    const float *kb = t.k + (int64_t)b * a.ks.b + (int64_t)g * a.ks.h;
-    const float *vb = t.v + (int64_t)b * a.vs.b + (int64_t)g * a.vs.h;
+    load_row32(qr, t.q + (int64_t)wk.b * a.qs.b + (int64_t)wk.head * a.qs.h + (int64_t)rowc * a.qs.s + 32 * half, row_ok);
+    load_row32(gr, t.d_o + (int64_t)wk.b * a.dos.b + (int64_t)wk.head * a.dos.h + (int64_t)rowc * a.dos.s + 32 * half, row_ok);
+    float ndelta, lse2;
+    if constexpr (FUSE_DELTA) {
+        const float *orow = t.o_in + (int64_t)wk.b * a.os.b + (int64_t)wk.head * a.os.h + (int64_t)rowc * a.os.s + 32 * half;
+        float x[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const f32x4 ov = *reinterpret_cast<const f32x4 *>(orow + 4 * j);
+            x[j] = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[j] = fmaf(ov[e], gr[4 * j + e], x[j]);
+        }
+        ndelta = -xhalf_sum(((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7])));
+        lse2 = a.lse[rid] * kLog2e;
+        if (row_ok && half == 0 && wk.w % KS == 0) {       // (a unit past the end holds rows of the first block again: the same values)
+            a.delta[rid] = ndelta;
+            a.delta[total + rid] = lse2;
+        }
+    } else {
+        ndelta = a.delta[rid];
+        lse2 = a.delta[total + rid];
+    }
+    const F32Offsets lo = make_f32_offsets(lane);
     const float c = a.scale_log2;
     f32x16 dq[2];
 #pragma unroll
     for (int i = 0; i < 16; ++i) { dq[0][i] = 0.0f; dq[1][i] = 0.0f; }
 
-    const int weff = a.window ? a.window : 0x3fffffff;
-    const int pos_hi = min(q_offset + min(a.Sq, q0 + 32) - 1, q_len - 1);
-    const int key_hi = pos_hi >= q_offset + q0 ? min(kv_len, pos_hi + 1) : 0;
-    const int key_lo = max(0, q_offset + q0 - weff + 1);
-    for (int n0 = (key_lo / 32) * 32; n0 < key_hi; n0 += 32) {
-        const int krow = min(n0 + l32, a.Skv - 1);
-        float kr[32], vr[32];
-        load_row32(kr, kb + (int64_t)krow * a.ks.s + 32 * half, true);
-        load_row32(vr, vb + (int64_t)krow * a.vs.s + 32 * half, true);
+    wait_vmcnt<0>();         // the compiler's own loads have arrived: no vmcnt wait of its own in the loop
+    for (int it = 0; it < wk.n_it; ++it) {
+        const int n0 = wk.first_key(it);
+        const bool more = it + 1 < wk.n_it;
         f32x16 s, dp;
 #pragma unroll
         for (int i = 0; i < 16; ++i) { s[i] = 0.0f; dp[i] = ndelta; }
-#pragma unroll
-        for (int ks = 0; ks < 32; ++ks) {
-            s = mfma_f32(kr[ks], qr[ks], s);          // S^T
-            dp = mfma_f32(vr[ks], gr[ks], dp);        // dP^T - delta
-        }
+        GPTOSS_F32_WAIT(F32Tile::kCopies);         // V is here; K may be on its way
+        f32_rows_product(dp, wk.vsm, lo, gr);      // dP^T - delta
+        GPTOSS_F32_WAIT(0);
+        GPTOSS_F32_READS_DONE();
+        if (more) wk.request_v(a, it + 1);
+        f32_rows_product(s, wk.ksm, lo, qr);       // S^T
+        const bool interior = wk.interior(a, n0);
+        const KeyMask km = make_key_mask(pos - n0, win, wk.kv_len - n0, half);
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-            const float p = visible(ri, n0 + crow(i, half), kv_len) ? exp2f(fmaf(s[i], c, -lse2)) : 0.0f;
+            float p = fast_exp2(fmaf(s[i], c, -lse2));
+            if (!interior) p = key_visible(km, 8 * (i >> 2) + (i & 3)) ? p : 0.0f;
             dp[i] = p * dp[i];
         }
-        // dQ^T[d][row] += K^T[d][key] dS^T[key][row]
-#pragma unroll
-        for (int a4 = 0; a4 < 4; ++a4)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float *krow2 = kb + (int64_t)min(n0 + 8 * a4 + 4 * half + e, a.Skv - 1) * a.ks.s;
-#pragma unroll
-                for (int dblk = 0; dblk < 2; ++dblk) dq[dblk] = mfma_f32(krow2[32 * dblk + l32], dp[4 * a4 + e], dq[dblk]);
-            }
+        f32_cols_product(dq, wk.ksm, lo, dp);      // dQ^T[d][row] += K^T[d][key] dS^T[key][row]
+        GPTOSS_F32_READS_DONE();
+        if (more) wk.request_k(a, it + 1);
     }
-    if (row < a.Sq) {
-        float *dqrow = t.dq + (int64_t)b * a.dqs.b + (int64_t)head * a.dqs.h + (int64_t)row * a.dqs.s;
+    __syncthreads();
+    f32_leave_partial(smem + wk.w * F32Tile::kBytes, dq, lane);
+    __syncthreads();
 #pragma unroll
-        for (int dblk = 0; dblk < 2; ++dblk)
+    for (int pass = 0; pass < 8 / KS; ++pass) {
+        const int i = pass >> 1, r = (threadIdx.x >> 4) + 16 * (pass & 1), ch = threadIdx.x & 15;
+        const F32Unit u = W::unit(a, i);
+        f32x4 x = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (int a4 = 0; a4 < 4; ++a4) {
-                f32x4 w4;
+        for (int k = 0; k < KS; ++k) {
+            const f32x4 y = f32_partial(smem, F32Tile::kBytes, KS * i + k, r, ch);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) w4[e] = dq[dblk][4 * a4 + e] * a.scale;
-                *reinterpret_cast<f32x4 *>(dqrow + 32 * dblk + 8 * a4 + 4 * half) = w4;
-            }
+            for (int e = 0; e < 4; ++e) x[e] += y[e];
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[e] *= a.scale;
+        if (u.live && u.q0 + r < a.Sq)
+            *reinterpret_cast<f32x4 *>(t.dq + (int64_t)u.b * a.dqs.b + (int64_t)u.head * a.dqs.h + (int64_t)(u.q0 + r) * a.dqs.s + 4 * ch) = x;
     }
 }
 

@@ -110,6 +110,16 @@ constexpr int kDkdvKeys = 32 * kDkdvNB * kDkdvWaves; // keys per dK/dV workgroup
 // lengths 3309 / 1968 / 1554 / 4079: 715 us uncut, 589 in two slices; B = 2, S = 8192 / 4000: 1437 and 1216; but B = 8,
 // S <= 2048: 359 and 370).
 int dkdv_parts_for(const gptoss_attn_params *p) {
+    if (p->dtype == GPTOSS_ATTN_FP32) {
+        // a workgroup per 32 keys, two per compute unit: about four workgroups per unit of a 256-CU part, so that the long
+        // first key blocks of a row do not decide the time
+        const int64_t blocks = (int64_t)p->G * p->B * ((p->Skv + 31) / 32), tiles = (p->Sq + 31) / 32;
+        int64_t parts = effective_window(p) > 0 ? 1 : 1024 / blocks;
+        if (parts > tiles * (p->H / p->G) / 8) parts = tiles * (p->H / p->G) / 8;
+        if (parts > tiles) parts = tiles;
+        if (parts > 4) parts = 4;
+        return parts < 1 ? 1 : (int)parts;
+    }
     if (p->dtype != GPTOSS_ATTN_BF16) return 1;
     const int64_t blocks = (int64_t)p->G * p->B * ((p->Skv + kDkdvKeys - 1) / kDkdvKeys);
     const int window = effective_window(p);
@@ -181,8 +191,18 @@ int decode_splits(const gptoss_attn_params *p) {
     return (int)(n < 1 ? 1 : n);
 }
 
-// workgroups of four independent wavefronts for the float32 kernels
-int64_t f32_grid(int64_t waves) { return (waves + 3) / 4; }
+// float32 forward and dQ: wavefronts that share a unit (32 query rows of one head).  Few units: four, so that the chip fills and
+// a row's keys are walked four at a time (64 heads, S = 256: forward 16 us; 19 with two, 30 with one); more than 1024: two (S = 1024: 101 us
+// forward, 131 dQ; 100 and 132 with four, 119 and 160 with one), and for a window's handful of tiles one (window 128, S =
+// 1024: 36 and 46 us; 40 and 51 with two, 48 and 62 with four).
+int f32_key_splits(const KArgs &a) {
+    const int64_t units = (int64_t)a.B * a.H * ((a.Sq + 31) / 32);
+    return units <= 1024 ? 4 : (a.window > 0 && a.window <= 512 ? 1 : 2);
+}
+int64_t f32_grid(const KArgs &a, int ks) {
+    const int64_t units = (int64_t)a.r * a.B * ((a.Sq + 31) / 32);      // per KV head; 4 / ks of them per workgroup
+    return (int64_t)a.G * ((units + 4 / ks - 1) / (4 / ks));
+}
 
 // One launch.  hipLaunchKernel reports this launch's own status, so an error some earlier call of the
 // thread left in the runtime's sticky state is neither reported here nor cleared.  A grid beyond the
@@ -415,8 +435,11 @@ int gptoss_attn_fwd(const gptoss_attn_params *p, void *stream) {
         if (s || a.kv_splits == 1) return s;
         return launch(attn_decode_combine_kernel, ((int64_t)a.B * a.G * pairs + 3) / 4, 256, st, a);
     }
-    if (p->dtype == GPTOSS_ATTN_FP32)
-        return launch(attn_f32_fwd_kernel, f32_grid((int64_t)a.B * a.H * ((a.Sq + 31) / 32)), 256, st, a);
+    if (p->dtype == GPTOSS_ATTN_FP32) {
+        const int ks = f32_key_splits(a);
+        const int64_t grid32 = f32_grid(a, ks);
+        return ks == 4 ? launch(attn_f32_fwd_kernel<4>, grid32, 256, st, a) : ks == 2 ? launch(attn_f32_fwd_kernel<2>, grid32, 256, st, a) : launch(attn_f32_fwd_kernel<1>, grid32, 256, st, a);
+    }
     const int hpb = hpb_for(a.r), qb = query_blocks_for(a.window);
     const int64_t grid = q_outer_grid(a, hpb, qb);
     if (fwd_window_route(p)) {
@@ -458,10 +481,13 @@ static int launch_dkdv(const gptoss_attn_params *p, void *stream, bool whole_blo
     if (rc) return rc;
     KArgs a = make_args(p);
     hipStream_t st = static_cast<hipStream_t>(stream);
-    if (p->dtype == GPTOSS_ATTN_FP32)
-        return launch(attn_f32_dkdv_kernel, f32_grid((int64_t)a.B * a.G * ((a.Skv + 31) / 32)), 256, st, a);
     a.dkdv_parts = whole_blocks ? 1 : dkdv_parts_for(p);
     a.dkdv_partial = reinterpret_cast<float *>(reinterpret_cast<char *>(p->delta) + stats_bytes(p));
+    if (p->dtype == GPTOSS_ATTN_FP32) {
+        const int s = launch(attn_f32_dkdv_kernel, (int64_t)a.B * a.G * a.dkdv_parts * ((a.Skv + 31) / 32), 256, st, a);
+        if (s || a.dkdv_parts == 1) return s;
+        return launch(attn_f32_dkdv_reduce_kernel, ((int64_t)2 * a.B * a.G * a.Skv * 16 + 255) / 256, 256, st, a);
+    }
     if (dkdv64_route(p, a.dkdv_parts)) {
         const int64_t grid64 = (int64_t)a.G * a.B * a.dkdv_parts * ((a.Skv + Dkdv64::BN - 1) / Dkdv64::BN);
         const int s = a.seqlens ? launch(attn_bwd_dkdv64_kernel<true>, grid64, 256, st, a) : launch(attn_bwd_dkdv64_kernel<false>, grid64, 256, st, a);
@@ -484,8 +510,13 @@ static int launch_dq(const gptoss_attn_params *p, void *stream, int fuse_delta) 
     if (rc) return rc;
     const KArgs a = make_args(p);
     hipStream_t st = static_cast<hipStream_t>(stream);
-    if (p->dtype == GPTOSS_ATTN_FP32)
-        return launch(attn_f32_dq_kernel, f32_grid((int64_t)a.B * a.H * ((a.Sq + 31) / 32)), 256, st, a);
+    if (p->dtype == GPTOSS_ATTN_FP32) {
+        const int ks = f32_key_splits(a);
+        const int64_t grid32 = f32_grid(a, ks);
+#define GPTOSS_LAUNCH_DQ(KS) (fuse_delta ? launch(attn_f32_dq_kernel<KS, true>, grid32, 256, st, a) : launch(attn_f32_dq_kernel<KS, false>, grid32, 256, st, a))
+        return ks == 4 ? GPTOSS_LAUNCH_DQ(4) : ks == 2 ? GPTOSS_LAUNCH_DQ(2) : GPTOSS_LAUNCH_DQ(1);
+#undef GPTOSS_LAUNCH_DQ
+    }
     const int hpb = hpb_for(a.r);
     int qb = query_blocks_for(a.window);
     // short problems: 64-row workgroups (two per compute unit) would be few and uneven (the key loops grow with the row
@@ -502,19 +533,12 @@ static int launch_dq(const gptoss_attn_params *p, void *stream, int fuse_delta) 
 
 int gptoss_attn_bwd_dq(const gptoss_attn_params *p, void *stream) { return launch_dq(p, stream, 0); }
 
-// The whole backward.  bf16: the dQ kernel computes the row statistics on the way (no separate
+// The whole backward: the dQ kernel computes the row statistics on the way (no separate
 // pass over O and dO), then dSinks and dK/dV read them from the scratch buffer.  The results are
 // bit-identical to gptoss_attn_bwd_preprocess + gptoss_attn_bwd_dkdv + gptoss_attn_bwd_dq.
 static int bwd_all(const gptoss_attn_params *p, void *stream, bool whole_blocks) {
     int rc = gptoss_attn_validate(p, 1);
     if (rc) return rc;
-    if (p->dtype == GPTOSS_ATTN_FP32) {
-        rc = gptoss_attn_bwd_preprocess(p, stream);
-        if (rc) return rc;
-        rc = launch_dkdv(p, stream, whole_blocks);
-        if (rc) return rc;
-        return gptoss_attn_bwd_dq(p, stream);
-    }
     if (window_single_pass(p)) return launch_window_bwd(p, static_cast<hipStream_t>(stream), !whole_blocks);
     rc = launch_dq(p, stream, 1);
     if (rc) return rc;
