@@ -7,10 +7,12 @@ from __future__ import annotations
 
 import ctypes
 import os
+import re
 from typing import Optional
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIBRARY = os.path.join(_HERE, "libgptoss_attn.so")
+TORCH_LIBRARY = os.path.join(_HERE, "libgptoss_torch.so")    # the PyTorch operators over it (csrc/torch_ops.cpp)
 
 ABI_VERSION = 4
 DTYPE_BF16 = 0
@@ -111,6 +113,26 @@ def load() -> ctypes.CDLL:
             raise RuntimeError("libgptoss_attn.so ABI version mismatch; rebuild the library")
         _lib = lib
     return _lib
+
+
+def load_torch_ops() -> None:
+    """Registers the `gptoss_attn` operators.  Raises if libgptoss_torch.so has not been built."""
+    if not os.path.exists(TORCH_LIBRARY):
+        raise RuntimeError(
+            f"{TORCH_LIBRARY} is missing: build it with `python -m oregon_gpt_oss_patching_amd.build`. "
+            "There is no fallback attention path.")
+    load()          # the operators link to it
+    import torch
+    torch.ops.load_library(TORCH_LIBRARY)
+
+
+_OP_FAILURE = re.compile(r"(gptoss_attn_\w+) failed with status (-?\d+): ")
+
+
+def as_library_error(e: RuntimeError) -> RuntimeError:
+    """The GptossAttnError for an operator's report of a failed library call; any other error as it is."""
+    m = _OP_FAILURE.match(str(e))
+    return GptossAttnError(m.group(1), int(m.group(2)), status_string(int(m.group(2)))) if m else e
 
 
 def status_string(status: int) -> str:

@@ -21,7 +21,8 @@ an optional `seqlens` (right-padding lengths) is accepted.
 """
 from __future__ import annotations
 
-from typing import Optional, Tuple
+import os
+from typing import Optional
 
 import torch
 
@@ -234,95 +235,65 @@ def attention_backward(q, k, v, sinks, o, lse, d_o, sm_scale, window=None, q_off
     return dq, dk, dv, dsinks
 
 
-# ---- torch custom ops --------------------------------------------------------------------
-# The two library calls are registered as opaque PyTorch operators, `gptoss_attn::fwd` and
-# `gptoss_attn::bwd`, with shape-only ("fake") implementations, so that tracing tools
-# (torch.compile, FakeTensorMode, activation-checkpoint replay) see one node per call and never
-# look inside.  The autograd.Function below calls through them.
+# ---- torch operators ---------------------------------------------------------------------
+# The two library calls are opaque PyTorch operators, `gptoss_attn::fwd` and `gptoss_attn::bwd`, and the differentiable
+# call is a third one made of them, `gptoss_attn::attention`, all in native code (csrc/torch_ops.cpp).  The shape-only
+# ("fake") implementations below let tracing tools (torch.compile, FakeTensorMode, activation-checkpoint replay) see one
+# node per library call and never look inside.
 OP_NAMESPACE = "gptoss_attn"
+_ops_ready = False
 
 
-@torch.library.custom_op(f"{OP_NAMESPACE}::fwd", mutates_args=(), device_types="cuda")
-def _op_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, sinks: Optional[torch.Tensor], sm_scale: float,
-            window: int, q_offset: int, seqlens: Optional[torch.Tensor],
-            doc_start: Optional[torch.Tensor],
-            q_offset_dev: Optional[torch.Tensor] = None) -> Tuple[torch.Tensor, torch.Tensor]:
-    return attention_forward(q, k, v, sinks, sm_scale, window, q_offset, seqlens, doc_start, q_offset_dev)
+def _register_ops() -> None:
+    global _ops_ready
+    _lib.load_torch_ops()
+
+    @torch.library.register_fake(f"{OP_NAMESPACE}::fwd")
+    def _fwd_fake(q, k, v, sinks, sm_scale, window, q_offset, seqlens, doc_start, q_offset_dev=None):
+        b, h, sq, d = q.shape
+        return q.new_empty((b, sq, h, d)), q.new_empty((b, h, sq), dtype=torch.float32)
+
+    @torch.library.register_fake(f"{OP_NAMESPACE}::bwd")
+    def _bwd_fake(q, k, v, sinks, o, lse, d_o, sm_scale, window, q_offset, seqlens, doc_start, need_dsinks,
+                  q_offset_dev=None):
+        return (torch.empty_like(q, memory_format=torch.contiguous_format),
+                torch.empty_like(k, memory_format=torch.contiguous_format),
+                torch.empty_like(v, memory_format=torch.contiguous_format),
+                q.new_empty((q.shape[1] if need_dsinks else 0,), dtype=torch.float32))
+
+    _ops_ready = True
 
 
-@_op_fwd.register_fake
-def _op_fwd_fake(q, k, v, sinks, sm_scale, window, q_offset, seqlens, doc_start, q_offset_dev=None):
-    b, h, sq, d = q.shape
-    return q.new_empty((b, sq, h, d)), q.new_empty((b, h, sq), dtype=torch.float32)
+if os.path.exists(_lib.TORCH_LIBRARY):      # (not while it is being built for the first time)
+    _register_ops()
 
 
-@torch.library.custom_op(f"{OP_NAMESPACE}::bwd", mutates_args=(), device_types="cuda")
-def _op_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, sinks: Optional[torch.Tensor], o: torch.Tensor,
-            lse: torch.Tensor, d_o: torch.Tensor, sm_scale: float, window: int, q_offset: int,
-            seqlens: Optional[torch.Tensor], doc_start: Optional[torch.Tensor],
-            need_dsinks: bool,
-            q_offset_dev: Optional[torch.Tensor] = None) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
-    dq, dk, dv, dsinks = attention_backward(q, k, v, sinks, o, lse, d_o, sm_scale, window, q_offset, seqlens,
-                                            need_dsinks=need_dsinks, doc_start=doc_start, q_offset_dev=q_offset_dev)
-    if dsinks is None:      # an operator cannot return None: an empty tensor stands for "not requested"
-        dsinks = torch.empty((0,), dtype=torch.float32, device=q.device)
-    return dq, dk, dv, dsinks
+def attention(q, k, v, sinks, sm_scale, bandwidth, start_q, seqlens=None, doc_start=None):
+    """Same argument list and gradients as the reference's `_attention.apply` (attention_kernel.py:220-344), plus optional
+    trailing `seqlens` and `doc_start`.
 
-
-@_op_bwd.register_fake
-def _op_bwd_fake(q, k, v, sinks, o, lse, d_o, sm_scale, window, q_offset, seqlens, doc_start, need_dsinks,
-                 q_offset_dev=None):
-    return (torch.empty_like(q, memory_format=torch.contiguous_format),
-            torch.empty_like(k, memory_format=torch.contiguous_format),
-            torch.empty_like(v, memory_format=torch.contiguous_format),
-            q.new_empty((q.shape[1] if need_dsinks else 0,), dtype=torch.float32))
-
-
-class _attention(torch.autograd.Function):
-    """Same argument list and gradient tuple as the reference's `_attention`
-    (attention_kernel.py:220-344), plus optional trailing `seqlens` and `doc_start`.
-
-    bfloat16 tensors take the tuned bf16-MFMA kernels and float32 tensors the float32 kernels
-    (exact to float32 rounding, not tuned for speed).  float16 tensors are accepted for
-    convenience: they are rounded to bfloat16 on the way in and the results cast back."""
-
-    @staticmethod
-    def forward(ctx, q, k, v, sinks, sm_scale, bandwidth, start_q, seqlens=None, doc_start=None):
-        _check_inputs(q, k, v, sinks, allow_cast=True)
-        ctx.in_dtypes = (q.dtype, k.dtype, v.dtype)
-        if q.dtype == torch.float16:
-            q, k, v = (t.to(torch.bfloat16) for t in (q, k, v))
-        # a start_q tensor that lives on the device stays there: the kernels read it (as the
-        # reference's do, attention_kernel.py:44-47), the host does not wait for it
-        q_offset, q_offset_dev = 0, None
-        if torch.is_tensor(start_q) and start_q.is_cuda:
-            q_offset_dev = _prep_q_offset_dev(start_q, q)
-        elif start_q is not None:
-            q_offset = int(start_q.item()) if torch.is_tensor(start_q) else int(start_q)
-        seqlens = _prep_seqlens(seqlens, q.device, q.shape[0])
-        doc_start = _prep_doc_start(doc_start, q)
-        window = int(bandwidth or 0)
-        sinks_in = None if sinks is None else sinks.detach()
-        o, lse = _op_fwd(q, k, v, sinks_in, float(sm_scale), window, q_offset, seqlens, doc_start, q_offset_dev)
-        ctx.save_for_backward(q, k, v, sinks, o, lse, seqlens, doc_start, q_offset_dev)
-        ctx.sm_scale = float(sm_scale)
-        ctx.window = window
-        ctx.q_offset = q_offset
-        return o.to(ctx.in_dtypes[0])
-
-    @staticmethod
-    def backward(ctx, do):
-        q, k, v, sinks, o, lse, seqlens, doc_start, q_offset_dev = ctx.saved_tensors
-        need_ds = sinks is not None and ctx.needs_input_grad[3]
-        sinks_in = None if sinks is None else sinks.detach()
-        dq, dk, dv, dsinks = _op_bwd(q, k, v, sinks_in, o, lse, do.to(q.dtype), ctx.sm_scale, ctx.window,
-                                     ctx.q_offset, seqlens, doc_start, need_ds, q_offset_dev)
-        dsinks = dsinks.to(sinks.dtype).view_as(sinks) if need_ds else None
-        qd, kd, vd = ctx.in_dtypes
-        return dq.to(qd), dk.to(kd), dv.to(vd), dsinks, None, None, None, None, None
-
-
-attention = _attention.apply
+    bfloat16 tensors take the tuned bf16-MFMA kernels and float32 tensors the float32 kernels.  float16 tensors are accepted
+    for convenience: they are rounded to bfloat16 on the way in and the results cast back."""
+    if not _ops_ready:
+        _register_ops()
+    # a start_q tensor that lives on the device stays there: the kernels read it (as the
+    # reference's do, attention_kernel.py:44-47), the host does not wait for it
+    q_offset, q_offset_dev = 0, None
+    if torch.is_tensor(start_q) and start_q.is_cuda:
+        q_offset_dev = start_q
+    elif start_q is not None:
+        q_offset = int(start_q.item()) if torch.is_tensor(start_q) else int(start_q)
+    if seqlens is not None and not torch.is_tensor(seqlens):
+        seqlens = torch.as_tensor(seqlens, dtype=torch.int32)
+    if doc_start is not None and not torch.is_tensor(doc_start):
+        doc_start = torch.as_tensor(doc_start, dtype=torch.int32)
+    call = torch.ops.gptoss_attn.attention.default
+    if torch.compiler.is_compiling():
+        return call(q, k, v, sinks, float(sm_scale), int(bandwidth or 0), q_offset, seqlens, doc_start, q_offset_dev)
+    try:
+        return call(q, k, v, sinks, float(sm_scale), int(bandwidth or 0), q_offset, seqlens, doc_start, q_offset_dev)
+    except RuntimeError as e:
+        raise _lib.as_library_error(e) from None
 
 
 def hip_flash_attention(
