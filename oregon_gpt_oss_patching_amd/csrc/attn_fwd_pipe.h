@@ -1,5 +1,4 @@
-// Forward kernel for the plain full-causal case (bf16, no window, no packed rows, no query offset, right-padded
-// batch rows allowed, Sq == Skv a multiple of 64, query heads per KV head a multiple of 4): the formulas of
+// Forward kernel for full-causal rows (bf16, no window, query heads per KV head a multiple of 4): the formulas of
 // attn_fwd_kernel<4, 2> (attn_fwd.h; the reference's `_attn_fwd`, attention_kernel.py:11-100) with the
 // interior key tiles software-pipelined by hand.  Against that kernel only the order of the row sums of a
 // row's first tile differs: lse agrees to a few units of its last place, O to one bf16 rounding.
@@ -37,12 +36,20 @@ struct FwdPipe {
     static constexpr int kStageBytes = 2 * kStageTileBytes;       // K tile, V tile
 };
 
-// PADDED: right-padded batch rows (seqlens): a row of the batch is a shorter row.  Workgroups past its end write
-// O = 0 and lse = sink and do nothing else; in the workgroup that holds its end the rows past it run along
-// unmasked through the interior tiles (their logits are garbage but finite or at worst NaN, and stay in their own
-// lanes) and are set to that same result before the epilogue; keys past the end exist only in the diagonal
-// tile, whose tile function masks them.
-template <bool PADDED>
+// The plain instantiation is for self-attention of whole tiles (Sq == Skv a multiple of 64, nothing else): key tiles
+// 0 .. qt - 1 are interior, tile qt is the diagonal.  GENERAL takes any lengths, a query offset, right-padded batch rows and
+// packed documents (64 keys at least).  A workgroup's key tiles are then [t_lo, t_hi): first the tile in front of t_a, where a
+// packed row's document starts inside a tile (an exact masked step, which also gives the softmax reference); the interior
+// tiles [t_a, t_b) through the pipeline; the tiles from t_b on (the diagonal, which an offset spreads over two tiles, and
+// the end of the keys) with masked steps.  Where a document ends inside the workgroup's rows, only the rows of
+// the first one see the tiles in front of the diagonal: the others run along unmasked (like rows that do not exist, past
+// the tensor or the padding: their values are garbage but finite or at worst NaN, and stay in their own lanes) and start
+// afresh at the diagonal tile.  Workgroups without any row that exists write O = 0 and lse = sink and do nothing else.
+// Measured against attn_fwd_kernel, which took these cases before (64 query heads on 8 KV heads): 1024 queries behind 7168
+// keys 181 -> 135 us; 2 x 3001 tokens 164 -> 160 us, 1 x 1000 33.6 -> 25.2, 2 x 383 16.1 -> 14.8; seven documents in 8192 tokens
+// 185 -> 180 (without letting the other documents' rows run along, every tile of such a workgroup being an exact
+// step: 230).
+template <bool GENERAL, bool DOCS = false>       // DOCS: packed documents (needs GENERAL)
 __global__ __launch_bounds__(256, 2) void attn_fwd_pipe_kernel(const KArgs a) {
     constexpr int NS = FwdPipe::NS;
     constexpr int SB = FwdPipe::kStageBytes;
@@ -62,12 +69,33 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_pipe_kernel(const KArgs a) {
     const int hc = bid % n_hc; bid /= n_hc;
     const int bi = bid % a.B; bid /= a.B;
     const int b = rotated_batch_row(bi, bid, a.B);
-    const int qt = a.Sq / kTile - 1 - bid;
+    const int q_offset = GENERAL ? query_offset(a) : 0;
+    const int qt = (GENERAL ? (a.Sq + kTile - 1) / kTile : a.Sq / kTile) - 1 - bid;
     const int head = g * a.r + hc * 4 + w;
     const int qw0 = qt * kTile;                    // the four wavefronts hold the same 64 rows of four heads
-    const int n_it = qt + 1;                       // key tiles 0 .. qt, the last one on the diagonal
-    const int len = PADDED ? max(0, min(a.Sq, a.seqlens[b])) : a.Sq;      // rows and keys from len on do not exist
-    const bool wg_dead = PADDED && qw0 >= len;
+    int t_lo = 0, t_a = 0, t_b = qt, t_hi = qt + 1;                       // see above
+    int kv_len = a.Skv, q_len = 0x7fffffff;                               // keys / query positions from here on do not exist
+    const int32_t *dsrow = nullptr;
+    if constexpr (GENERAL) {
+        if (a.seqlens) { q_len = a.seqlens[b]; kv_len = max(0, min(a.Skv, q_len)); }
+        const int pos0 = q_offset + qw0, pos1 = min(q_offset + min(a.Sq, qw0 + kTile) - 1, q_len - 1);
+        int ds0 = 0;
+        bool later = false;
+        if constexpr (DOCS) {
+            dsrow = a.doc_start + (int64_t)b * a.Sq;
+            ds0 = max(dsrow[qw0], 0);
+            // (starts that are not the first row of their document, so that a later document reaches in front of these rows,
+            // leave no interior tile)
+            const int ds = dsrow[min(qw0 + lane, a.Sq - 1)];
+            later = ds > ds0 && ds < qw0;
+        }
+        const int hi = pos1 >= pos0 ? min(kv_len, pos1 + 1) : 0;
+        t_lo = DOCS ? __builtin_amdgcn_readfirstlane(ds0 / kTile) : 0;
+        t_hi = __builtin_amdgcn_readfirstlane(max(t_lo, (hi + kTile - 1) / kTile));
+        if constexpr (DOCS) t_a = __builtin_amdgcn_ballot_w64(later) != 0ull ? t_hi : __builtin_amdgcn_readfirstlane((ds0 + kTile - 1) / kTile);
+        t_b = __builtin_amdgcn_readfirstlane(min(pos0 + 1, kv_len) / kTile);
+    }
+    const int n_it = t_hi - t_lo;
 
     const bf16 *kbase = a.k + (int64_t)b * a.ks.b + (int64_t)g * a.ks.h;
     const bf16 *vbase = a.v + (int64_t)b * a.vs.b + (int64_t)g * a.vs.h;
@@ -75,7 +103,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_pipe_kernel(const KArgs a) {
     bf16x8 qf[2][4];
 #pragma unroll
     for (int qb = 0; qb < 2; ++qb) {
-        const int row = qw0 + 32 * qb + l32;
+        const int row = GENERAL ? min(qw0 + 32 * qb + l32, a.Sq - 1) : qw0 + 32 * qb + l32;
         const bf16 *qrow = a.q + (int64_t)b * a.qs.b + (int64_t)head * a.qs.h + (int64_t)row * a.qs.s;
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) qf[qb][ks] = as_bf16x8(*reinterpret_cast<const u32x4 *>(qrow + 16 * ks + 8 * half));
@@ -95,7 +123,9 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_pipe_kernel(const KArgs a) {
     // tiles are exhausted a request copies the last tile again, into the stage that is free by then, so that
     // "at most one request outstanding" keeps meaning "the tile before it has landed".
     const bf16 *ktile = kbase, *vtile = vbase;
-    int iss_stage = 0, iss_left = n_it;
+    // (a tile that sticks out of the tensor is not requested here: see fetch_end)
+    const int t_req = GENERAL ? min(t_lo, a.Skv / kTile - 1) : 0, n_req = GENERAL ? max(1, min(t_hi, a.Skv / kTile) - t_req) : n_it;
+    int iss_stage = 0, iss_left = n_req;
     auto issue = [&]() __attribute__((always_inline)) {       // the next tile in order, into the next stage in rotation
         // (through the inline-assembly copy: the compiler's own bookkeeping would make every LDS read that
         // follows a copy wait for all outstanding copies, i.e. for the tile just requested)
@@ -112,10 +142,10 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_pipe_kernel(const KArgs a) {
     };
     constexpr int kLoadsPerIt = 4;
     auto reset = [&]() __attribute__((always_inline)) {
-        ktile = kbase;
-        vtile = vbase;
+        ktile = kbase + (GENERAL ? (int64_t)t_req * kTile * a.ks.s : 0);
+        vtile = vbase + (GENERAL ? (int64_t)t_req * kTile * a.vs.s : 0);
         iss_stage = 0;
-        iss_left = n_it;
+        iss_left = n_req;
 #pragma unroll
         for (int qb = 0; qb < 2; ++qb) {
             m[qb] = sink2;
@@ -132,8 +162,38 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_pipe_kernel(const KArgs a) {
         __syncthreads();
         issue();
     };
-    // Rows of a single key tile (the diagonal one) have no interior tile: they go straight to the exact pass below.
-    const bool pipelined = !wg_dead && n_it >= 2;
+    // Tile k of the walk if it sticks out of the tensor, into its stage, rows past the end re-reading the last one; everybody
+    // waits for it.  It can only be the walk's last tile, of the few workgroups that see the last keys at all, and keeping
+    // its lane offsets out of the loop is worth the wait.
+    auto fetch_end = [&](int k) __attribute__((always_inline)) {
+        if (!GENERAL || (t_lo + k + 1) * kTile <= a.Skv) return;
+        const int n0 = (t_lo + k) * kTile, last = a.Skv - 1 - n0, ln = fresh_lane();
+        wait_vmcnt<0>();
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int r = 16 * w + 8 * j + (ln >> 3), ch = ((ln & 7) ^ swz(r)) * 16, rr = min(r, last);
+            const uint32_t dst = copy_base + (k & (NS - 1)) * SB + j * 8 * kRowBytes;
+            lds_dma16(dst, kbase + (int64_t)n0 * a.ks.s, (uint32_t)(rr * (int)a.ks.s) * 2u + ch);
+            lds_dma16(dst + kStageTileBytes, vbase + (int64_t)n0 * a.vs.s, (uint32_t)(rr * (int)a.vs.s) * 2u + ch);
+        }
+        wait_vmcnt<0>();
+        __syncthreads();
+    };
+    // A row description for the masked tile functions, from scratch (see fresh_lane): lane's position (hugely negative for a
+    // row that does not exist) and how far back it sees.
+    auto describe_rows = [&](int l32_, int (&pq)[2], unsigned (&wl)[2]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int qb = 0; qb < 2; ++qb) {
+            const int row = qw0 + 32 * qb + l32_, p = q_offset + row;
+            pq[qb] = row < a.Sq && p < q_len ? p : -0x40000000;
+            wl[qb] = 0x3fffffffu;
+            if (DOCS) wl[qb] = (unsigned)(p - dsrow[min(row, a.Sq - 1)] + 1);
+        }
+    };
+    // Workgroups without an interior tile (rows of a single key tile) go straight to the exact pass below.
+    const bool pipelined = n_it > 0 && t_a < t_b && t_b > t_lo;
+    const int k_a = t_a - t_lo;            // tiles of the walk in front of the first interior one
     if (!pipelined) {
         // (also the state a workgroup without rows ends with: nothing requested, nothing attended)
 #pragma unroll
@@ -145,31 +205,46 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_pipe_kernel(const KArgs a) {
         }
     } else {
         reset();
+        if (DOCS && k_a > 0) {
+            int pq[2], dbase[2];
+            unsigned wl[2];
+            describe_rows(l32, pq, wl);
+            for (int k = 0; k < k_a; ++k) {
+                arrive();
+                const int n0 = (t_lo + k) * kTile;
+                const uint32_t ksm = smem_base + (k & (NS - 1)) * SB;
+#pragma unroll
+                for (int qb = 0; qb < 2; ++qb) dbase[qb] = pq[qb] - n0;
+                fwd_tile<true, 2>(ksm, ksm + kStageTileBytes, lo, qf, o, m, l, c, lane, dbase, wl, 0x3fffffffu, kv_len - n0, q_offset + qw0 - n0);
+            }
+        }
         arrive();
         // The softmax reference of a row: the sink logit or the largest logit of the row's first tile
         // (ref :53, :79-81 after one tile), from a pass over that tile that forms the logits and nothing else
         // (16 MFMAs per row block, against 32 for each of its tiles).  The tile then goes through the pipelined
         // loop like every other interior tile.
-        f32x16 s[2][2];
+        if (!DOCS || k_a == 0) {
+            f32x16 s[2][2];
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
+            for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-            for (int ks = 0; ks < 4; ++ks) {
-                const bf16x8 akf = ofrag_nat(smem_base, lo, kb, ks);
+                for (int ks = 0; ks < 4; ++ks) {
+                    const bf16x8 akf = ofrag_nat(smem_base, lo, kb, ks);
 #pragma unroll
-                for (int qb = 0; qb < 2; ++qb) {
-                    f32x16 z;
+                    for (int qb = 0; qb < 2; ++qb) {
+                        f32x16 z;
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) z[i] = 0.0f;
-                    s[kb][qb] = mfma_bf16(akf, qf[qb][ks], ks == 0 ? z : s[kb][qb]);
+                        for (int i = 0; i < 16; ++i) z[i] = 0.0f;
+                        s[kb][qb] = mfma_bf16(akf, qf[qb][ks], ks == 0 ? z : s[kb][qb]);
+                    }
                 }
+#pragma unroll
+            for (int qb = 0; qb < 2; ++qb) {
+                float mx0 = s[0][qb][0], mx1 = s[1][qb][0];
+#pragma unroll
+                for (int i = 1; i < 16; ++i) { mx0 = fast_max(mx0, s[0][qb][i]); mx1 = fast_max(mx1, s[1][qb][i]); }
+                m[qb] = fast_max(m[qb], xhalf_max(fast_max(mx0, mx1)) * c);
             }
-#pragma unroll
-        for (int qb = 0; qb < 2; ++qb) {
-            float mx0 = s[0][qb][0], mx1 = s[1][qb][0];
-#pragma unroll
-            for (int i = 1; i < 16; ++i) { mx0 = fast_max(mx0, s[0][qb][i]); mx1 = fast_max(mx1, s[1][qb][i]); }
-            m[qb] = fast_max(m[qb], xhalf_max(fast_max(mx0, mx1)) * c);
         }
     }
     float nm[2] = {-m[0], -m[1]};
@@ -187,12 +262,12 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_pipe_kernel(const KArgs a) {
         bf16x8 av[2][2];                    // [u16][dblk] V fragments of the key block being multiplied into O
         uint32_t kadr[4], vadr[2][2];       // per-lane LDS addresses: K of the stage the next K fragments come from, V of this tile's
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks) kadr[ks] = smem_base + lo.nat[ks];                      // tile 0 is in stage 0
+        for (int ks = 0; ks < 4; ++ks) kadr[ks] = smem_base + (DOCS ? (k_a & (NS - 1)) * SB : 0) + lo.nat[ks];    // tile 0 of the walk is in stage 0
 #pragma unroll
         for (int dblk = 0; dblk < 2; ++dblk)
 #pragma unroll
-            for (int t2 = 0; t2 < 2; ++t2) vadr[dblk][t2] = smem_base + kStageTileBytes + lo.tr[dblk][t2];
-        // fill: S of unit 0 of tile 0; the first slot's O MFMAs multiply zeros (O is zero there anyway)
+            for (int t2 = 0; t2 < 2; ++t2) vadr[dblk][t2] = smem_base + (DOCS ? (k_a & (NS - 1)) * SB : 0) + kStageTileBytes + lo.tr[dblk][t2];
+        // fill: S of unit 0 of the first tile; the first slot's O MFMAs multiply zeros (exact: O keeps its bits)
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) ak[ks] = as_bf16x8(lds_load128(kadr[ks], 0));
 #pragma unroll
@@ -260,7 +335,8 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_pipe_kernel(const KArgs a) {
 #pragma unroll
             for (int ks = 0; ks < 4; ++ks) asm volatile("" ::"v"(qf[qb][ks]));
         wait_vmcnt<0>();
-        for (int t = 0; t <= n_it - 2; ++t) {
+        const int k_end = GENERAL ? t_b - t_lo : n_it - 1;
+        for (int t = DOCS ? k_a : 0; t < k_end; ++t) {
             GPTOSS_FP_FENCE();
             slot(I0{}, sa, sb, pb, pa);
             slot(I1{}, sb, sa, pa, pb);
@@ -293,61 +369,117 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_pipe_kernel(const KArgs a) {
     const TileLaneOffsets lo_b = make_tile_offsets(lane_b);
     int pq_b[2];
     unsigned wl_b[2];
-#pragma unroll
-    for (int qb = 0; qb < 2; ++qb) { pq_b[qb] = qw0 + 32 * qb + l32_b < len ? qw0 + 32 * qb + l32_b : -0x40000000; wl_b[qb] = 0x3fffffffu; }   // (hugely negative: nothing is visible to a row that does not exist)
+    describe_rows(l32_b, pq_b, wl_b);
     auto masked_args_b = [&](int n0, int (&dbase)[2]) __attribute__((always_inline)) {
 #pragma unroll
         for (int qb = 0; qb < 2; ++qb) dbase[qb] = pq_b[qb] - n0;
     };
-    if (pipelined) {
-        const int n0 = qt * kTile;
-        const uint32_t ksm = smem_base + (qt & (NS - 1)) * SB;
-        int dbase[2];
-        masked_args_b(n0, dbase);
-        fwd_tile_lean<true, 2>(ksm, ksm + kStageTileBytes, lo_b, qf, o, nm, l, c, lane_b, dbase, wl_b, 0x3fffffffu, len - n0, 0);
-    }
-
-    // A sum beyond 2^96 (or not finite): some logit stood 95 or more above its row's frozen reference; the
-    // workgroup repeats its key loop with the exact online-softmax step on every tile (see attn_fwd_kernel).
     // rows that do not exist: nothing attended, whatever the interior tiles made of them
-    auto clear_dead_rows = [&]() __attribute__((always_inline)) {
-        if constexpr (PADDED) {
+    auto clear_rows = [&](int qb, bool dead_row) __attribute__((always_inline)) {
+        m[qb] = dead_row ? sink2 : m[qb];
+        l[qb] = dead_row ? 0.0f : l[qb];
 #pragma unroll
-            for (int qb = 0; qb < 2; ++qb) {
-                const bool dead_row = pq_b[qb] < 0;
-                m[qb] = dead_row ? sink2 : m[qb];
-                l[qb] = dead_row ? 0.0f : l[qb];
-#pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    o[qb][0][i] = dead_row ? 0.0f : o[qb][0][i];
-                    o[qb][1][i] = dead_row ? 0.0f : o[qb][1][i];
-                }
-            }
+        for (int i = 0; i < 16; ++i) {
+            o[qb][0][i] = dead_row ? 0.0f : o[qb][0][i];
+            o[qb][1][i] = dead_row ? 0.0f : o[qb][1][i];
         }
     };
-    clear_dead_rows();
     // A sum beyond 2^96 (or not finite): some logit stood 95 or more above its row's frozen reference; the
     // workgroup repeats its key loop with the exact online-softmax step on every tile (see attn_fwd_kernel; the
-    // masked form of the step for every tile: this pass is rare and the kernel stays small).  Rows of a single
-    // tile take this pass as their only one.
-    bool unsafe = false;
+    // masked form of the step for every tile: this pass is rare and the kernel stays small).
+    auto frozen_too_low = [&]() __attribute__((always_inline)) {
+        bool unsafe = false;
 #pragma unroll
-    for (int qb = 0; qb < 2; ++qb) unsafe = unsafe || !(l[qb] < 0x1p96f);
-    const bool second_pass = pipelined && __syncthreads_or(unsafe);
-    if (second_pass || (!pipelined && !wg_dead)) {
-        if (second_pass) {
-            wait_vmcnt<0>();      // the repeated copies of the last requests
+        for (int qb = 0; qb < 2; ++qb) unsafe = unsafe || !(l[qb] < 0x1p96f);
+        return __syncthreads_or(unsafe);
+    };
+    auto exact_tile = [&](int it) __attribute__((always_inline)) {
+        const uint32_t ksm = smem_base + (it & (NS - 1)) * SB;
+        int dbase[2];
+        const int n0 = (t_lo + it) * kTile;
+        masked_args_b(n0, dbase);
+        fwd_tile<true, 2>(ksm, ksm + kStageTileBytes, lo_b, qf, o, m, l, c, lane_b, dbase, wl_b, 0x3fffffffu, kv_len - n0, q_offset + qw0 - n0);
+    };
+    auto lean_tile = [&](int it) __attribute__((always_inline)) {
+        const uint32_t ksm = smem_base + (it & (NS - 1)) * SB;
+        int dbase[2];
+        const int n0 = (t_lo + it) * kTile;
+        masked_args_b(n0, dbase);
+        fwd_tile_lean<true, 2>(ksm, ksm + kStageTileBytes, lo_b, qf, o, nm, l, c, lane_b, dbase, wl_b, 0x3fffffffu, kv_len - n0, GENERAL ? q_offset + qw0 - n0 : 0);
+    };
+    if constexpr (!DOCS) {
+        if (pipelined) {
+            // (the first of these tiles has landed: the pipeline's last pass waited for it)
+            if constexpr (GENERAL) {
+#pragma unroll 1
+                for (int it = t_b - t_lo; it < n_it; ++it) {
+                    if (it > t_b - t_lo) arrive();
+                    fetch_end(it);
+                    lean_tile(it);
+                }
+#pragma unroll
+                for (int qb = 0; qb < 2; ++qb) clear_rows(qb, pq_b[qb] < 0);
+            } else {
+                lean_tile(qt);
+            }
+        }
+        // (rows of a single tile take this pass as their only one)
+        const bool second_pass = pipelined && frozen_too_low();
+        if (second_pass || (!pipelined && n_it > 0)) {
+            if (second_pass) {
+                wait_vmcnt<0>();      // the repeated copies of the last requests
+                __syncthreads();
+            }
+            reset();
+            for (int it = 0; it < n_it; ++it) {
+                arrive();
+                fetch_end(it);
+                exact_tile(it);
+            }
+            if (GENERAL)
+#pragma unroll
+                for (int qb = 0; qb < 2; ++qb) clear_rows(qb, pq_b[qb] < 0);
+        }
+    } else {
+        // With an interior tile in front, a row that cannot see tile t_a sees nothing in front of the diagonal tile: it starts
+        // afresh here, and needs a reference of its own, so the workgroup's last tiles take the exact step.  Otherwise the
+        // reference stays frozen.
+        bool fresh = false;
+        if (pipelined) {
+#pragma unroll
+            for (int qb = 0; qb < 2; ++qb) {
+                const bool late = pq_b[qb] - (int)wl_b[qb] + 1 > t_a * kTile;
+                fresh = fresh || late;
+                clear_rows(qb, pq_b[qb] < 0 || late);
+            }
+        }
+        bool lean = pipelined && __builtin_amdgcn_ballot_w64(fresh) == 0ull;
+        int k_exact = pipelined ? t_b - t_lo : 0;
+        bool landed = pipelined;      // the pipeline's last pass waited for the tile that comes next
+        bool repeat = pipelined;      // the reference was frozen: the sums have to be looked at
+        if (!pipelined && n_it > 0) reset();
+#pragma unroll 1
+        for (;;) {
+#pragma unroll 1
+            for (int it = k_exact; it < n_it; ++it) {
+                if (!landed) arrive();
+                landed = false;
+                fetch_end(it);
+                if (lean) lean_tile(it); else exact_tile(it);
+            }
+            if (!repeat) break;
+            repeat = false;
+            lean = false;
+#pragma unroll
+            for (int qb = 0; qb < 2; ++qb) clear_rows(qb, pq_b[qb] < 0);
+            if (!frozen_too_low()) break;
+            wait_vmcnt<0>();          // the repeated copies of the last requests
             __syncthreads();
+            reset();
+            k_exact = 0;
+            landed = false;
         }
-        reset();
-        for (int it = 0; it < n_it; ++it) {
-            arrive();
-            const uint32_t ksm = smem_base + (it & (NS - 1)) * SB;
-            int dbase[2];
-            masked_args_b(it * kTile, dbase);
-            fwd_tile<true, 2>(ksm, ksm + kStageTileBytes, lo_b, qf, o, m, l, c, lane_b, dbase, wl_b, 0x3fffffffu, len - it * kTile, qw0 - it * kTile);
-        }
-        clear_dead_rows();
+        // (rows that do not exist and met only masked tiles end as they began: nothing attended)
     }
 
     // epilogue: z = l + exp(sink - m); O = acc / z; M = m + log z   (ref :93-98)
@@ -363,7 +495,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_pipe_kernel(const KArgs a) {
         bf16 *orow0 = a.o + (int64_t)b * a.os.b + (int64_t)head * a.os.h + (int64_t)r0 * a.os.s;
         store_rows32(stage, o[qb], inv, orow0, a.os.s, a.Sq - r0, lane_b);
         __builtin_amdgcn_wave_barrier();
-        if (half_b == 0) a.lse[((int64_t)b * a.H + head) * a.Sq + r0 + l32_b] = (m[qb] + fast_log2(z)) * kLn2;
+        if (half_b == 0 && (!GENERAL || r0 + l32_b < a.Sq)) a.lse[((int64_t)b * a.H + head) * a.Sq + r0 + l32_b] = (m[qb] + fast_log2(z)) * kLn2;
     }
 }
 

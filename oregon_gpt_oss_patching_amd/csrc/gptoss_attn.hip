@@ -156,11 +156,13 @@ bool dkdv64_route(const gptoss_attn_params *p, int parts) {
            !p->q_offset_dev && p->Sq == p->Skv && p->Sq % kTile == 0 && (blocks > 512 || (parts > 1 && p->Skv >= 2048));
 }
 
-// The hand-pipelined forward kernel (attn_fwd_pipe.h) takes the plain full-causal case (right-padded batch rows
-// included): every key tile but the last of a row is interior, all four wavefronts have a head.
+// The hand-pipelined forward kernel (attn_fwd_pipe.h) takes full-causal rows whose groups of query heads fill its four
+// wavefronts; self-attention of whole tiles without padding or packing has an instantiation of its own.
 bool fwd_pipe_route(const gptoss_attn_params *p) {
-    return p->dtype == GPTOSS_ATTN_BF16 && effective_window(p) == 0 && !p->doc_start && p->q_offset == 0 &&
-           !p->q_offset_dev && p->Sq == p->Skv && p->Sq % kTile == 0 && (p->H / p->G) % 4 == 0;
+    return p->dtype == GPTOSS_ATTN_BF16 && effective_window(p) == 0 && (p->H / p->G) % 4 == 0 && p->Skv >= kTile;
+}
+bool fwd_pipe_plain(const gptoss_attn_params *p) {
+    return p->Sq == p->Skv && p->Sq % kTile == 0 && !p->seqlens && !p->doc_start && p->q_offset == 0 && !p->q_offset_dev;
 }
 
 // The one-pass forward of sliding-window layers (attn_fwd_window.h): a window of 32, 64, 96 or 128 keys on plain
@@ -455,7 +457,10 @@ int gptoss_attn_fwd(const gptoss_attn_params *p, void *stream) {
             default: return launch3(attn_fwd_window_kernel<4>, wgrid, st, a);
         }
     }
-    if (fwd_pipe_route(p)) return a.seqlens ? launch(attn_fwd_pipe_kernel<true>, grid, 256, st, a) : launch(attn_fwd_pipe_kernel<false>, grid, 256, st, a);
+    if (fwd_pipe_route(p)) 
+        return fwd_pipe_plain(p) ? launch(attn_fwd_pipe_kernel<false, false>, grid, 256, st, a)
+               : a.doc_start     ? launch(attn_fwd_pipe_kernel<true, true>, grid, 256, st, a)
+                                 : launch(attn_fwd_pipe_kernel<true, false>, grid, 256, st, a);
 #define GPTOSS_LAUNCH_FWD(HPB, QB) launch(attn_fwd_kernel<HPB, QB>, grid, 256, st, a)
     if (qb == 2) return hpb == 4 ? GPTOSS_LAUNCH_FWD(4, 2) : hpb == 2 ? GPTOSS_LAUNCH_FWD(2, 2) : GPTOSS_LAUNCH_FWD(1, 2);
     return hpb == 4 ? GPTOSS_LAUNCH_FWD(4, 1) : hpb == 2 ? GPTOSS_LAUNCH_FWD(2, 1) : GPTOSS_LAUNCH_FWD(1, 1);

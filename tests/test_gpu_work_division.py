@@ -9,6 +9,7 @@ import test_gpu_parity as TP
 
 pytestmark = pytest.mark.gpu
 A = TP.A
+SCALE = TP.SCALE
 
 
 @pytest.mark.parametrize("b,h,g,docs", [
@@ -40,3 +41,48 @@ def test_sliced_and_rotated_batches_vs_eager_oracle(A, b, h, g, s, lens):
     if lens:
         inp = inp[:4] + (TP.mask_dout(inp[4], lens),)
     TP.compare_all(TP.run_hip(A, *inp, None, 0, lens), TP.oracle_eager(*inp, None, 0, lens))
+
+
+@pytest.mark.parametrize("b,h,g,sq,skv,start,lens", [
+    (1, 8, 2, 64, 64, 0, None),             # one tile
+    (1, 8, 2, 65, 65, 0, None),             # a last tile of one row and one key
+    (2, 16, 4, 127, 127, 0, None),
+    (1, 8, 2, 300, 1000, 700, None),        # an offset inside a tile: the diagonal lies across two tiles
+    (1, 8, 2, 129, 449, 320, None),         # ... on a tile boundary, with a last tile of one key
+    (1, 8, 2, 200, 1000, 300, None),        # a cache longer than what the queries see
+    (1, 4, 1, 100, 90, 10, None),           # fewer keys than positions
+    (3, 8, 2, 333, 333, 0, [333, 64, 1]),   # padded rows of a ragged batch
+    (2, 8, 2, 100, 600, 500, [600, 520]),   # padded rows behind an offset: queries past the row's length
+])
+@pytest.mark.parametrize("lift", [0.0, 40.0])
+def test_full_causal_forward_of_any_length_vs_eager_oracle(A, b, h, g, sq, skv, start, lens, lift):
+    """The pipelined forward off whole tiles.  lift: the second half of the keys is scaled so that a row's later logits stand
+    far above its first tile's (the frozen softmax reference is found too low and the workgroup repeats its walk)."""
+    print(f"case B={b} H={h} G={g} Sq={sq} Skv={skv} start={start} lens={lens} lift={lift}", flush=True)
+    q, k, v, sinks, _ = E.make_inputs(5200 + sq + skv, b, h, g, sq, 64, torch.bfloat16, skv=skv)
+    if lift:
+        k[:, :, skv // 2:] *= lift
+    args = (SCALE, None, start, lens)
+    o, lse = A.attention_forward(*(t.to("cuda") for t in (q, k, v, sinks)), *args)
+    f = [t.float() for t in (q, k, v, sinks)]
+    TP.check("o", o, E.eager_attention(*f, *args))
+    ref = E.logsumexp_rows(f[0], f[1], f[3], *args).float()
+    assert float((lse.cpu() - ref).abs().max()) <= TP.LSE_TOL * (1 if not lift else 1 + float(ref.abs().max()) / 64)   # (fp32 logits of order 300)
+    if lens:
+        for i, n in enumerate(lens):
+            assert (o[i, max(n - start, 0):] == 0).all()
+
+
+@pytest.mark.parametrize("docs", [[100, 28, 200], [1, 63, 64, 65, 190], [300, 10, 10, 10, 500], [129, 700]])
+def test_packed_forward_with_sharply_peaked_rows(A, docs):
+    """Documents that end inside a workgroup's rows, logits of order 40: the rows that start afresh at the diagonal tile take a
+    softmax reference of their own."""
+    s = sum(docs)
+    print(f"case docs={docs}", flush=True)
+    q, k, v, sinks, _ = E.make_inputs(5300 + s, 2, 8, 2, s, 64, torch.bfloat16)
+    q, k = q * 3, k * 3
+    ds = E.doc_start_from_lengths([docs] * 2, s)
+    o, lse = A.attention_forward(*(t.to("cuda") for t in (q, k, v, sinks)), SCALE, None, doc_start=ds)
+    f = [t.float() for t in (q, k, v, sinks)]
+    TP.check("o", o, E.eager_attention(*f, SCALE, None, 0, None, ds))
+    assert float((lse.cpu() - E.logsumexp_rows(f[0], f[1], f[3], SCALE, None, 0, None, ds).float()).abs().max()) <= TP.LSE_TOL
