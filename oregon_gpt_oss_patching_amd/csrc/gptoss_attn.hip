@@ -109,7 +109,7 @@ constexpr int kDkdvKeys = 32 * kDkdvNB * kDkdvWaves; // keys per dK/dV workgroup
 // right-padded batch counts half, because its shorter rows leave the longest one alone (dK/dV of B = 4, S = 4096,
 // lengths 3309 / 1968 / 1554 / 4079: 715 us uncut, 589 in two slices; B = 2, S = 8192 / 4000: 1437 and 1216; but B = 8,
 // S <= 2048: 359 and 370).
-int dkdv_parts_for(const gptoss_attn_params *p) {
+int dkdv_parts_for(const gptoss_attn_params *p, bool padded) {
     if (p->dtype == GPTOSS_ATTN_FP32) {
         // a workgroup per 32 keys, two per compute unit: about four workgroups per unit of a 256-CU part, so that the long
         // first key blocks of a row do not decide the time
@@ -126,7 +126,7 @@ int dkdv_parts_for(const gptoss_attn_params *p) {
     const int64_t rows_seen = window > 0 ? (int64_t)kDkdvKeys + window - 1 : (int64_t)p->Sq;
     const int64_t tiles = ((rows_seen < p->Sq ? rows_seen : p->Sq) + 63) / 64;
     int64_t parts = (1024 + blocks - 1) / blocks;
-    if (blocks > 512) parts = p->Sq >= 4096 && (p->seqlens && p->B > 1 ? blocks / 2 : blocks) < 1024 ? 2 : 1;
+    if (blocks > 512) parts = p->Sq >= 4096 && (padded && p->B > 1 ? blocks / 2 : blocks) < 1024 ? 2 : 1;
     const int64_t steps = window > 0 ? tiles / 4 : tiles * (p->H / p->G) / 8;
     if (parts > steps) parts = steps;
     if (parts > tiles) parts = tiles;
@@ -135,11 +135,11 @@ int dkdv_parts_for(const gptoss_attn_params *p) {
 }
 
 // Full-causal self-attention goes to attn_bwd_dkdv64_kernel (64 keys per wavefront, one wavefront per SIMD)
-// when the shape is the one it is written for (bf16, no window, no packed rows, no offset, Sq == Skv a
-// multiple of 64; right-padded batch rows are fine) and there is enough of it: more than 512 key blocks of 128 (then key blocks are
-// whole: at least 257 workgroups of 256 keys, and the same bits as the 32-key kernel), or rows of 2048 keys
-// or more that the host cuts into `parts` slices anyway (the same number of slices as the 32-key kernel
-// would get, so the scratch is the same; -15 % at S = 2048 ... 8192).
+// when the shape is the one it is written for (bf16, no window, no offset, Sq == Skv; right-padded batch rows and packed
+// documents are fine) and there is enough of it: more than
+// 512 key blocks of 128 (then key blocks are whole: at least 257 workgroups of 256 keys, and the same bits as the 32-key
+// kernel), or rows of 2048 keys or more that the host cuts into `parts` slices anyway (the same number of slices as the
+// 32-key kernel would get, so the scratch is the same; -15 % at S = 2048 ... 8192).
 // (The kernel walks Q, dO and the row statistics of one KV head's group of query heads with 32-bit byte
 // offsets from the group's first row: head strides must not be negative and the group's span must stay
 // below 2^31 bytes; anything else takes the 32-key kernel.)
@@ -152,8 +152,8 @@ bool dkdv64_route(const gptoss_attn_params *p, int parts) {
     if (!walk_fits_32_bits(p->q_stride, heads, p->Sq) || !walk_fits_32_bits(p->do_stride, heads, p->Sq) ||
         heads * p->Sq * 16 >= ((int64_t)1 << 31))
         return false;
-    return p->dtype == GPTOSS_ATTN_BF16 && effective_window(p) == 0 && !p->doc_start && p->q_offset == 0 &&
-           !p->q_offset_dev && p->Sq == p->Skv && p->Sq % kTile == 0 && (blocks > 512 || (parts > 1 && p->Skv >= 2048));
+    return p->dtype == GPTOSS_ATTN_BF16 && effective_window(p) == 0 && p->q_offset == 0 && !p->q_offset_dev && p->Sq == p->Skv &&
+           p->Sq >= kTile && (blocks > 512 || (parts > 1 && p->Skv >= 2048));
 }
 
 // The hand-pipelined forward kernel (attn_fwd_pipe.h) takes full-causal rows whose groups of query heads fill its four
@@ -396,6 +396,12 @@ static size_t stats_bytes(const gptoss_attn_params *p) {
     return fp32_stats_bytes(p) + (size_t)16 * (size_t)p->B * (size_t)p->H * (size_t)p->Sq;
 }
 
+// dK/dV partial sums, for a call with or without lengths of padded rows (the size depends on the shapes only)
+static size_t partials_bytes(const gptoss_attn_params *p) {
+    const int plain = dkdv_parts_for(p, false), padded = dkdv_parts_for(p, true), parts = plain > padded ? plain : padded;
+    return parts > 1 ? (size_t)parts * 2 * sizeof(float) * (size_t)p->B * (size_t)p->G * (size_t)p->Skv * kD : 0;
+}
+
 size_t gptoss_attn_fwd_workspace_bytes(const gptoss_attn_params *p) {
     if (!p || p->B <= 0 || p->H <= 0 || p->G <= 0 || p->Sq <= 0 || p->Skv <= 0) return 0;
     if (decode_route(p)) {
@@ -410,8 +416,7 @@ size_t gptoss_attn_workspace_bytes(const gptoss_attn_params *p) {
     size_t n = stats_bytes(p);
     if (gptoss_attn_fwd_workspace_bytes(p) > n) n = gptoss_attn_fwd_workspace_bytes(p);
     if (p->G > 0 && p->Skv > 0) {
-        const int parts = dkdv_parts_for(p);
-        if (parts > 1) n += (size_t)parts * 2 * sizeof(float) * (size_t)p->B * (size_t)p->G * (size_t)p->Skv * kD;
+        n += partials_bytes(p);
         if (window_single_pass(p)) {
             // gptoss_attn_bwd takes this route and lays its own scratch over the same bytes.  The layout
             // follows the compute-unit count of the device that is current at launch time; the size
@@ -486,7 +491,7 @@ static int launch_dkdv(const gptoss_attn_params *p, void *stream, bool whole_blo
     if (rc) return rc;
     KArgs a = make_args(p);
     hipStream_t st = static_cast<hipStream_t>(stream);
-    a.dkdv_parts = whole_blocks ? 1 : dkdv_parts_for(p);
+    a.dkdv_parts = whole_blocks ? 1 : dkdv_parts_for(p, p->seqlens != nullptr);
     a.dkdv_partial = reinterpret_cast<float *>(reinterpret_cast<char *>(p->delta) + stats_bytes(p));
     if (p->dtype == GPTOSS_ATTN_FP32) {
         const int s = launch(attn_f32_dkdv_kernel, (int64_t)a.B * a.G * a.dkdv_parts * ((a.Skv + 31) / 32), 256, st, a);
@@ -495,7 +500,8 @@ static int launch_dkdv(const gptoss_attn_params *p, void *stream, bool whole_blo
     }
     if (dkdv64_route(p, a.dkdv_parts)) {
         const int64_t grid64 = (int64_t)a.G * a.B * a.dkdv_parts * ((a.Skv + Dkdv64::BN - 1) / Dkdv64::BN);
-        const int s = a.seqlens ? launch(attn_bwd_dkdv64_kernel<true>, grid64, 256, st, a) : launch(attn_bwd_dkdv64_kernel<false>, grid64, 256, st, a);
+        const bool plain = !a.seqlens && !a.doc_start && a.Sq % kTile == 0;
+        const int s = plain ? launch(attn_bwd_dkdv64_kernel<false>, grid64, 256, st, a) : launch(attn_bwd_dkdv64_kernel<true>, grid64, 256, st, a);
         if (s || a.dkdv_parts == 1) return s;
         return launch(attn_bwd_dkdv_reduce_kernel, ((int64_t)2 * a.B * a.G * a.Skv * 8 + 255) / 256, 256, st, a);
     }

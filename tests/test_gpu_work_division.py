@@ -86,3 +86,40 @@ def test_packed_forward_with_sharply_peaked_rows(A, docs):
     f = [t.float() for t in (q, k, v, sinks)]
     TP.check("o", o, E.eager_attention(*f, SCALE, None, 0, None, ds))
     assert float((lse.cpu() - E.logsumexp_rows(f[0], f[1], f[3], SCALE, None, 0, None, ds).float()).abs().max()) <= TP.LSE_TOL
+
+
+@pytest.mark.parametrize("b,h,g,s,lens,docs", [
+    (1, 16, 2, 2049, None, None),                    # a query tile of one row on top of the walk, cut into slices
+    (1, 8, 1, 2303, [2303], None),                   # ... of 63 rows; a single KV head
+    (3, 8, 2, 2111, [2111, 2048, 700], None),        # padded rows that end below the tile that sticks out, and in it
+    (33, 8, 8, 449, None, None),                     # more than 512 key blocks: whole blocks
+    (1, 16, 2, 2100, None, [64, 192, 1, 63, 257, 700, 823]),    # documents inside wavefronts, on their edges, across workgroups
+    (1, 8, 2, 2048, None, [2048]),
+    (2, 8, 2, 2300, None, [1, 2299]),
+    (1, 8, 2, 2500, None, [5] * 500),                # many documents in one wavefront's keys
+    (2, 8, 2, 2200, [2200, 1500], [900, 700, 600]),  # packed and padded
+])
+def test_64_key_backward_of_any_length_vs_eager_oracle(A, b, h, g, s, lens, docs):
+    """attn_bwd_dkdv64_kernel off whole tiles and with packed documents, every gradient, and the same bits on a second run."""
+    print(f"case B={b} H={h} G={g} S={s} lens={lens} docs={docs}", flush=True)
+    inp = E.make_inputs(5400 + s + b, b, h, g, s, 64, torch.bfloat16)
+    if lens:
+        inp = inp[:4] + (TP.mask_dout(inp[4], lens),)
+    ds = E.doc_start_from_lengths([docs] * b, s) if docs else None
+    got = TP.run_hip(A, *inp, None, 0, lens, ds)
+    o, lse, dq, dk, dv, dsinks = (t.detach().cpu() for t in got)
+    rds = torch.zeros(h, dtype=torch.float64)
+    for i in range(b):
+        one = [t[i:i + 1] for t in inp[:3]] + [inp[3], inp[4][i:i + 1]]
+        ro, rlse, rdq, rdk, rdv, rds_i = TP.oracle_eager(*one, None, 0, [lens[i]] if lens else None, ds[i:i + 1] if docs else None)
+        # Documents of five tokens: a dK element is scale * sum of dS q over 5 rows x 4 heads, with |dS| up to p (1 - p) |dP - delta| ~
+        # 4 (dP is a sum of 64 products of N(0, 1) values) and |q| ~ 2, so rounding dS to bf16 (2^-9 relative) moves it by up to
+        # 2^-9 * 20 * 4 * 2 / 8 = 4e-2; everywhere else the bound of 2e-2 holds.
+        atol = 4e-2 if docs and max(docs) <= 5 else 2e-2
+        for name, x, y in (("o", o, ro), ("dq", dq, rdq), ("dk", dk, rdk), ("dv", dv, rdv)):
+            TP.check(name, x[i:i + 1], y, atol=atol)
+        assert float((lse[i:i + 1] - rlse.float()).abs().max()) <= TP.LSE_TOL
+        rds += rds_i.double()
+    TP.check("dsinks", dsinks, rds.float(), atol=None)
+    again = TP.run_hip(A, *inp, None, 0, lens, ds)
+    assert all(torch.equal(x, y) for x, y in zip(got, again))
