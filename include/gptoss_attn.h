@@ -234,6 +234,14 @@ int gptoss_attn_bwd_static(const gptoss_attn_params *params, void *stream);
 size_t gptoss_attn_static_scratch_bytes(void);
 
 /*
+ * The `doc_start` array of packed rows from their position ids: doc_start[b][i] = index of the last token at or before i
+ * whose position id does not follow its predecessor's by one (transformers masking_utils.py:728-757 finds packed documents
+ * that way; the reference ignores position ids).  position_ids: B rows of S integers of `id_bytes` (4 or 8) bytes,
+ * `row_stride` elements apart (0 repeats one row); doc_start: (B, S) int32 contiguous.  B at most 65535.
+ */
+int gptoss_attn_doc_start(const void *position_ids, int id_bytes, int B, int S, int64_t row_stride, int32_t *doc_start, void *stream);
+
+/*
  * Measurement aid with no counterpart in the reference and no part in the attention path: launches a
  * loop of nothing but bf16 MFMAs (v_mfma_f32_32x32x16_bf16, two wavefronts per SIMD on every compute
  * unit, `iters` passes of 16 MFMAs per wavefront) whose operands are read once from `operands`

@@ -21,7 +21,6 @@ an optional `seqlens` (right-padding lengths) is accepted.
 """
 from __future__ import annotations
 
-import os
 from typing import Optional
 
 import torch
@@ -163,6 +162,10 @@ def doc_start_from_position_ids(position_ids: torch.Tensor) -> torch.Tensor:
     a new document begins wherever the position does not follow its predecessor by one."""
     pos = position_ids
     b, s = pos.shape
+    if pos.is_cuda and pos.dtype in (torch.int64, torch.int32):
+        if not _ops_ready:
+            _register_ops()
+        return torch.ops.gptoss_attn.doc_start.default(pos)
     idx = torch.arange(s, device=pos.device).view(1, s).expand(b, s)
     new_doc = torch.ones_like(pos, dtype=torch.bool)
     new_doc[:, 1:] = (pos[:, 1:] - pos[:, :-1]) != 1
@@ -261,11 +264,17 @@ def _register_ops() -> None:
                 torch.empty_like(v, memory_format=torch.contiguous_format),
                 q.new_empty((q.shape[1] if need_dsinks else 0,), dtype=torch.float32))
 
+    @torch.library.register_fake(f"{OP_NAMESPACE}::doc_start")
+    def _doc_start_fake(position_ids):
+        return torch.empty_like(position_ids, dtype=torch.int32, memory_format=torch.contiguous_format)
+
     _ops_ready = True
 
 
-if os.path.exists(_lib.TORCH_LIBRARY):      # (not while it is being built for the first time)
+try:
     _register_ops()
+except Exception:       # not built yet, or built from other sources: importing has to work for the build itself; the first call tries again and raises
+    pass
 
 
 def attention(q, k, v, sinks, sm_scale, bandwidth, start_q, seqlens=None, doc_start=None):

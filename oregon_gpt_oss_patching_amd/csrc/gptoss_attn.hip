@@ -16,6 +16,7 @@
 #include "attn_fwd.h"
 #include "attn_fwd_pipe.h"
 #include "attn_fwd_window.h"
+#include "doc_start.h"
 #include "mfma_rate.h"
 
 using namespace gptoss;
@@ -604,6 +605,19 @@ int gptoss_attn_bwd_static(const gptoss_attn_params *p, void *stream) {
     rc = static_scratch(&q.delta);
     if (rc) return rc;
     return bwd_all(&q, stream, true);
+}
+
+// ---- packed rows (doc_start.h) ----------------------------------------------------------------
+int gptoss_attn_doc_start(const void *position_ids, int id_bytes, int B, int S, int64_t row_stride, int32_t *doc_start, void *stream) {
+    if (!position_ids || !doc_start) return GPTOSS_ATTN_ERR_NULL_TENSOR;
+    if (id_bytes != 4 && id_bytes != 8) return GPTOSS_ATTN_ERR_DTYPE;
+    if (B <= 0 || B > 65535 || S <= 0 || S > (1 << 30)) return GPTOSS_ATTN_ERR_SHAPE;
+    if ((reinterpret_cast<uintptr_t>(position_ids) & (id_bytes - 1)) || (reinterpret_cast<uintptr_t>(doc_start) & 3)) return GPTOSS_ATTN_ERR_ALIGNMENT;
+    const dim3 grid((unsigned)((S + kDocTokens - 1) / kDocTokens), (unsigned)B);
+    void *args[] = {&position_ids, &row_stride, &S, &doc_start};
+    const void *kernel = id_bytes == 8 ? reinterpret_cast<const void *>(doc_start_kernel<int64_t>) : reinterpret_cast<const void *>(doc_start_kernel<int32_t>);
+    const hipError_t e = hipLaunchKernel(kernel, grid, dim3(256), args, 0, static_cast<hipStream_t>(stream));
+    return e == hipSuccess ? GPTOSS_ATTN_OK : static_cast<int>(e);
 }
 
 // ---- measurement aid (mfma_rate.h) -----------------------------------------------------------

@@ -248,6 +248,21 @@ Tensor attention(const Tensor &q, const Tensor &k, const Tensor &v, const OptTen
     return AttentionFunction::apply(q, k, v, sinks, sm_scale, window, q_offset, seqlens, doc_start, q_offset_dev);
 }
 
+// (B, S) int32 document starts of packed rows, see gptoss_attn_doc_start.
+Tensor doc_start(const Tensor &position_ids_) {
+    TORCH_CHECK(position_ids_.dim() == 2 && (position_ids_.scalar_type() == at::kLong || position_ids_.scalar_type() == at::kInt),
+                "position_ids must be (B, S) of int64 or int32");
+    const c10::OptionalDeviceGuard guard(position_ids_.device());
+    const Tensor pos = position_ids_.size(1) > 1 && position_ids_.stride(1) != 1 ? position_ids_.contiguous() : position_ids_;
+    Tensor out = at::empty(pos.sizes(), pos.options().dtype(at::kInt));
+    if (pos.numel() == 0) return out;
+    const int rc = gptoss_attn_doc_start(pos.const_data_ptr(), static_cast<int>(pos.element_size()), static_cast<int>(pos.size(0)),
+                                         static_cast<int>(pos.size(1)), pos.stride(0), out.data_ptr<int32_t>(),
+                                         c10::hip::getCurrentHIPStream(pos.device().index()).stream());
+    TORCH_CHECK(rc == 0, "gptoss_attn_doc_start failed with status ", rc, ": ", gptoss_attn_status_string(rc));
+    return out;
+}
+
 }  // namespace
 
 TORCH_LIBRARY(gptoss_attn, m) {
@@ -255,12 +270,14 @@ TORCH_LIBRARY(gptoss_attn, m) {
           "Tensor? q_offset_dev=None) -> (Tensor, Tensor)");
     m.def("bwd(Tensor q, Tensor k, Tensor v, Tensor? sinks, Tensor o, Tensor lse, Tensor d_o, float sm_scale, int window, int q_offset, "
           "Tensor? seqlens, Tensor? doc_start, bool need_dsinks, Tensor? q_offset_dev=None) -> (Tensor, Tensor, Tensor, Tensor)");
+    m.def("doc_start(Tensor position_ids) -> Tensor");
     m.def("attention(Tensor q, Tensor k, Tensor v, Tensor? sinks, float sm_scale, int window, int q_offset, Tensor? seqlens, Tensor? doc_start, "
           "Tensor? q_offset_dev=None) -> Tensor", &attention);
 }
 TORCH_LIBRARY_IMPL(gptoss_attn, CUDA, m) {
     m.impl("fwd", &fwd);
     m.impl("bwd", &bwd);
+    m.impl("doc_start", &doc_start);
 }
 TORCH_LIBRARY_IMPL(gptoss_attn, Autograd, m) {
     m.impl("fwd", torch::autograd::autogradNotImplementedFallback());
