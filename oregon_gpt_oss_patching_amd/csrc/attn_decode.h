@@ -28,6 +28,10 @@ struct Decode {
 // scratch per (batch, KV head, split): the unnormalised output rows, then (m, l) per row
 __host__ __device__ inline int64_t decode_partial_floats(int pairs) { return (int64_t)pairs * (kD + 2); }
 
+// The softmax reference starts at the sink logit.  A sink of -inf (none at all) must not start it at -inf: a slice or wavefront may hold
+// no key that a row sees, and -inf - (-inf) would make its share NaN.
+constexpr float kNoLogit = -1e30f;
+
 template <int NQB>
 __global__ __launch_bounds__(256, 2) void attn_decode_kernel(const KArgs a) {
     using C = Decode;
@@ -70,7 +74,7 @@ __global__ __launch_bounds__(256, 2) void attn_decode_kernel(const KArgs a) {
         for (int ks = 0; ks < 4; ++ks) qf[qb][ks] = as_bf16x8(*reinterpret_cast<const u32x4 *>(qrow + 16 * ks + 8 * half));
         pq[qb] = ok && q_offset + row < q_len ? q_offset + row : -0x40000000;
         sink2[qb] = (a.sinks ? a.sinks[head] : 0.0f) * kLog2e;
-        m[qb] = sink2[qb];
+        m[qb] = fast_max(sink2[qb], kNoLogit);
         l[qb] = 0.0f;
 #pragma unroll
         for (int i = 0; i < 16; ++i) { o[qb][0][i] = 0.0f; o[qb][1][i] = 0.0f; }
@@ -222,7 +226,7 @@ __global__ __launch_bounds__(256) void attn_decode_combine_kernel(const KArgs a)
     const int64_t step = decode_partial_floats(pairs);
     const float *part = a.fwd_partial + (int64_t)bg * a.kv_splits * step;
     const float sink2 = (a.sinks ? a.sinks[head] : 0.0f) * kLog2e;
-    float mm = sink2, z = 0.0f, acc[8];         // mm: the largest reference among this lane's splits so far
+    float mm = fast_max(sink2, kNoLogit), z = 0.0f, acc[8];         // mm: the largest reference among this lane's splits so far
 #pragma unroll
     for (int e = 0; e < 8; ++e) acc[e] = 0.0f;
     for (int s = sg; s < a.kv_splits; s += 8) {

@@ -80,3 +80,17 @@ def test_decode_without_scratch_and_under_graph_replay(A):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(og, o) and torch.equal(lg, lse)
+
+
+@pytest.mark.parametrize("b,sq,skv,start,lens", [(1, 8, 129, 121, None), (1, 1, 2049, 2048, None), (2, 3, 600, 597, [600, 40])])
+def test_decode_without_sink(A, b, sq, skv, start, lens):
+    """Sink logits of -inf: the plain softmax, also for rows that see nothing of some slice's or wavefront's keys."""
+    print(f"case B={b} Sq={sq} Skv={skv} start={start} lens={lens}", flush=True)
+    q, k, v, sinks, _ = E.make_inputs(4200 + skv, b, 8, 1, sq, 64, torch.bfloat16, skv=skv)
+    none = torch.full_like(sinks, float("-inf"))
+    o, _ = A.attention_forward(q.to(DEV), k.to(DEV), v.to(DEV), none.to(DEV), SCALE, None, start, lens)
+    ref = E.eager_attention(q.float(), k.float(), v.float(), torch.full_like(sinks.float(), -1e4), SCALE, None, start, lens)
+    o = o.float().cpu()
+    live = torch.ones(b, sq, dtype=torch.bool) if lens is None else torch.arange(start, start + sq)[None] < torch.tensor(lens)[:, None]
+    # the bf16 path's bound, as above
+    assert bool(((o - ref).abs() <= 2e-2 + 2.0 ** -8 * ref.abs())[live].all())
