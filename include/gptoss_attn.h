@@ -164,6 +164,12 @@ size_t gptoss_attn_fwd_workspace_bytes(const gptoss_attn_params *params);
 int gptoss_attn_fwd(const gptoss_attn_params *params, void *stream);
 
 /*
+ * The same with the sink logits in `sinks_dtype` (GPTOSS_ATTN_FP32 or GPTOSS_ATTN_BF16; params->sinks points at H of them), the
+ * type a model's parameter has: bf16 logits widen exactly, no converted copy is needed.
+ */
+int gptoss_attn_fwd_sinks(const gptoss_attn_params *params, int sinks_dtype, void *stream);
+
+/*
  * Backward step 1: the row statistics.  The first B*H*Sq floats of `delta` receive
  * -rowsum(dO * O) (the NEGATED row dot: it seeds the dP accumulators of the kernels that
  * follow), the next B*H*Sq floats lse * log2(e); behind them (from the next 16-byte boundary) 16
@@ -208,6 +214,12 @@ int gptoss_attn_bwd_dq(const gptoss_attn_params *params, void *stream);
  * Reads q,k,v,sinks,o,d_o,lse,seqlens,doc_start; writes dq,dk,dv,dsinks,delta.
  */
 int gptoss_attn_bwd(const gptoss_attn_params *params, void *stream);
+
+/*
+ * The same with the sink logits in `sinks_dtype` and their gradient in `dsinks_dtype` (GPTOSS_ATTN_FP32 or GPTOSS_ATTN_BF16;
+ * params->sinks and params->dsinks point at H of them); a bf16 gradient is the fp32 sum rounded once.
+ */
+int gptoss_attn_bwd_sinks(const gptoss_attn_params *params, int sinks_dtype, int dsinks_dtype, void *stream);
 
 /*
  * The whole backward without any workspace from the caller and without any allocation: a variant

@@ -25,10 +25,12 @@ EXPORTS = (
     "gptoss_attn_workspace_bytes",
     "gptoss_attn_fwd_workspace_bytes",
     "gptoss_attn_fwd",
+    "gptoss_attn_fwd_sinks",
     "gptoss_attn_bwd_preprocess",
     "gptoss_attn_bwd_dkdv",
     "gptoss_attn_bwd_dq",
     "gptoss_attn_bwd",
+    "gptoss_attn_bwd_sinks",
     "gptoss_attn_bwd_static",
     "gptoss_attn_static_scratch_bytes",
     "gptoss_attn_doc_start",
@@ -113,6 +115,10 @@ def load() -> ctypes.CDLL:
             fn = getattr(lib, name)
             fn.restype = ctypes.c_int
             fn.argtypes = [ctypes.POINTER(Params), ctypes.c_void_p]
+        lib.gptoss_attn_fwd_sinks.restype = ctypes.c_int
+        lib.gptoss_attn_fwd_sinks.argtypes = [ctypes.POINTER(Params), ctypes.c_int, ctypes.c_void_p]
+        lib.gptoss_attn_bwd_sinks.restype = ctypes.c_int
+        lib.gptoss_attn_bwd_sinks.argtypes = [ctypes.POINTER(Params), ctypes.c_int, ctypes.c_int, ctypes.c_void_p]
         if lib.gptoss_attn_version() != ABI_VERSION:
             raise RuntimeError("libgptoss_attn.so ABI version mismatch; rebuild the library")
         _lib = lib

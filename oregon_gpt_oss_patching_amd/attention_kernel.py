@@ -258,11 +258,12 @@ def _register_ops() -> None:
 
     @torch.library.register_fake(f"{OP_NAMESPACE}::bwd")
     def _bwd_fake(q, k, v, sinks, o, lse, d_o, sm_scale, window, q_offset, seqlens, doc_start, need_dsinks,
-                  q_offset_dev=None):
+                  q_offset_dev=None, dsinks_as_sinks=False):
+        bf16_dsinks = dsinks_as_sinks and sinks is not None and sinks.dtype == torch.bfloat16
         return (torch.empty_like(q, memory_format=torch.contiguous_format),
                 torch.empty_like(k, memory_format=torch.contiguous_format),
                 torch.empty_like(v, memory_format=torch.contiguous_format),
-                q.new_empty((q.shape[1] if need_dsinks else 0,), dtype=torch.float32))
+                q.new_empty((q.shape[1] if need_dsinks else 0,), dtype=torch.bfloat16 if bf16_dsinks else torch.float32))
 
     @torch.library.register_fake(f"{OP_NAMESPACE}::doc_start")
     def _doc_start_fake(position_ids):

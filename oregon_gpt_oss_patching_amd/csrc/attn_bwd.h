@@ -61,24 +61,37 @@ __global__ __launch_bounds__(256) void attn_bwd_delta_kernel(const KArgs a) {
 // ---------------------------------------------------------------------------------
 // One workgroup per query head; fixed summation order, so the result is
 // bit-reproducible (the reference accumulates it with relaxed atomics).
-__global__ __launch_bounds__(1024) void attn_bwd_dsinks_kernel(const KArgs a) {
-    __shared__ float red[1024];
-    const int h = blockIdx.x;
-    const float sink2 = (a.sinks ? a.sinks[h] : 0.0f) * kLog2e;
+// (1024 partial sums and a tree over them whatever the block size, so that every launch that ends here gives the same bits)
+template <int THREADS>
+__device__ __forceinline__ void dsinks_of_head(const KArgs &a, int h, float (&red)[1024]) {
+    constexpr int N = 1024 / THREADS;
+    const float sink2 = sink_logit(a, h) * kLog2e;
     const int64_t total = (int64_t)a.B * a.H * a.Sq;
-    float acc = 0.0f;
+    float acc[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) acc[k] = 0.0f;
     for (int b = 0; b < a.B; ++b) {
         const float *ndl = a.delta + ((int64_t)b * a.H + h) * a.Sq;        // -delta
         const float *lse2 = ndl + total;                                    // lse * log2(e)
-        for (int s = threadIdx.x; s < a.Sq; s += 1024) acc += fast_exp2(sink2 - lse2[s]) * ndl[s];
+        for (int s0 = threadIdx.x; s0 < a.Sq; s0 += 1024)
+#pragma unroll
+            for (int k = 0; k < N; ++k) {
+                const int s = s0 + k * THREADS;
+                if (s < a.Sq) acc[k] = fmaf(fast_exp2(sink2 - lse2[s]), ndl[s], acc[k]);
+            }
     }
-    red[threadIdx.x] = acc;
+#pragma unroll
+    for (int k = 0; k < N; ++k) red[threadIdx.x + k * THREADS] = acc[k];
     __syncthreads();
     for (int off = 512; off > 0; off >>= 1) {
-        if ((int)threadIdx.x < off) red[threadIdx.x] += red[threadIdx.x + off];
+        for (int i = threadIdx.x; i < off; i += THREADS) red[i] += red[i + off];
         __syncthreads();
     }
-    if (threadIdx.x == 0) a.dsinks[h] = red[0];
+    if (threadIdx.x == 0) store_dsink(a, h, red[0]);
+}
+__global__ __launch_bounds__(1024) void attn_bwd_dsinks_kernel(const KArgs a) {
+    __shared__ float red[1024];
+    dsinks_of_head<1024>(a, blockIdx.x, red);
 }
 
 // ---------------------------------------------------------------------------------
@@ -527,10 +540,13 @@ __global__ __launch_bounds__(NW * 64, (NB == 1 ? 2 : 1)) void attn_bwd_dkdv_kern
 // ---------------------------------------------------------------------------------
 // Sum of the dK / dV partials of a split key block, in part order (bit-reproducible), scaled and
 // rounded to the output type.  One thread per 16-byte output chunk: (tensor, b, g, key, 8 columns).
-__global__ __launch_bounds__(256) void attn_bwd_dkdv_reduce_kernel(const KArgs a) {
+// The first `heads` blocks produce dSinks (a launch of their own took 4.5 to 11 us; here they run beside the sums).
+__global__ __launch_bounds__(256) void attn_bwd_dkdv_reduce_kernel(const KArgs a, int heads) {
+    __shared__ float red[1024];
+    if ((int)blockIdx.x < heads) { dsinks_of_head<256>(a, blockIdx.x, red); return; }
     const int64_t rows = (int64_t)a.B * a.G * a.Skv;
     const int64_t tensor = rows * kD;
-    const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;        // chunk index over both tensors
+    const int64_t idx = (int64_t)(blockIdx.x - heads) * 256 + threadIdx.x;   // chunk index over both tensors
     if (idx >= 2 * rows * 8) return;
     const int which = (int)(idx / (rows * 8));                            // 0 = dK, 1 = dV
     const int64_t rem = idx - (int64_t)which * rows * 8;

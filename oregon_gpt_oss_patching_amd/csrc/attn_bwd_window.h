@@ -134,7 +134,6 @@ __global__ __launch_bounds__(WinCfg::NWAVES * 64, 1) void attn_bwd_window_kernel
         // dSinks terms are summed per lane (own LDS slot per head, no cross-lane traffic in the loop)
         float *const my_sink = ssink + (hh * C::kMaxGroup) * 64 + lane;
         for (int h = 0; h < a.r; ++h) my_sink[h * 64] = 0.0f;
-        const float *sinks = a.sinks;
 
         // O and dO half rows + lse of this lane's row of walk position `pos`.  The row pointers
         // follow the walk (heads inner, then the next query tile); the last tile's rows past the
@@ -185,7 +184,7 @@ __global__ __launch_bounds__(WinCfg::NWAVES * 64, 1) void attn_bwd_window_kernel
                 sstat[(stage * 2 + 1) * kTile + srow] = -acc;
             }
             if (a.dsinks && pos.t < t1) {                       // rows of the chunk itself, each counted once
-                const float sink2 = (sinks ? sinks[g * a.r + pos.h] : 0.0f) * kLog2e;
+                const float sink2 = sink_logit(a, g * a.r + pos.h) * kLog2e;
                 const float term = (hr == 0 && pos.t * kTile + srow < a.Sq) ? fast_exp2(sink2 - lse2) * -acc : 0.0f;
                 my_sink[pos.h * 64] += term;
             }
@@ -493,7 +492,7 @@ __global__ __launch_bounds__(256) void attn_bwd_window_finish_kernel(const KArgs
             if ((int)threadIdx.x < off) red[threadIdx.x] += red[threadIdx.x + off];
             __syncthreads();
         }
-        if (threadIdx.x == 0) a.dsinks[h] = red[0];
+        if (threadIdx.x == 0) store_dsink(a, h, red[0]);
         return;
     }
     // chunk index over (b, g, seam, tile, tensor, key, 8 columns)

@@ -35,14 +35,14 @@ struct Strides { int64_t b, h, s; };
 
 struct KArgs {
     const bf16 *q, *k, *v;
-    const float *sinks;
+    const void *sinks;          // optional (H): fp32, or bf16 where sinks_bf16 is set
     const int32_t *seqlens;
     const int32_t *doc_start;   // optional (B, Sq): first key of each query's document
     bf16 *o;
     float *lse;
     const bf16 *d_o;
     bf16 *dq, *dk, *dv;
-    float *dsinks;
+    void *dsinks;               // optional (H): fp32, or bf16 where dsinks_bf16 is set
     float *delta;        // row statistics in fp32: -delta[B][H][Sq], then lse * log2(e) [B][H][Sq]
     u32x4 *split;        // the same statistics as bf16 triples, 16 bytes per row (see split_row_stats)
     Strides qs, ks, vs, os, dos, dqs, dks, dvs;
@@ -60,7 +60,19 @@ struct KArgs {
     int chunk_tiles;     // single-pass window backward: 64-row query tiles per workgroup
     float *dsink_partial; // single-pass window backward: dSinks partial sums, [B][chunk][H][2]
     float *boundary_partial; // single-pass window backward: fp32 dK / dV shares of the tiles on chunk seams, or NULL
+    bool sinks_bf16, dsinks_bf16;
 };
+
+// The sink logits and their gradient in the type the caller's parameter has: a conversion of 64 numbers was a launch of its own
+// (2 to 4.5 us on the GPU and as much host time, three per training call: a sliding-window layer of 4096 tokens 107 -> 95 us, a decoding step on 2049 keys 19.0 -> 13.8).
+__device__ __forceinline__ float sink_logit(const KArgs &a, int head) {
+    if (!a.sinks) return 0.0f;
+    return a.sinks_bf16 ? (float)static_cast<const bf16 *>(a.sinks)[head] : static_cast<const float *>(a.sinks)[head];
+}
+__device__ __forceinline__ void store_dsink(const KArgs &a, int head, float x) {
+    if (a.dsinks_bf16) static_cast<bf16 *>(a.dsinks)[head] = (bf16)x;
+    else static_cast<float *>(a.dsinks)[head] = x;
+}
 
 // Absolute position of query row 0: by value, or (for callers that must not synchronise with the
 // device to learn it) from device memory, one scalar load per workgroup.

@@ -73,7 +73,7 @@ __global__ __launch_bounds__(256, 2) void attn_decode_kernel(const KArgs a) {
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) qf[qb][ks] = as_bf16x8(*reinterpret_cast<const u32x4 *>(qrow + 16 * ks + 8 * half));
         pq[qb] = ok && q_offset + row < q_len ? q_offset + row : -0x40000000;
-        sink2[qb] = (a.sinks ? a.sinks[head] : 0.0f) * kLog2e;
+        sink2[qb] = sink_logit(a, head) * kLog2e;
         m[qb] = fast_max(sink2[qb], kNoLogit);
         l[qb] = 0.0f;
 #pragma unroll
@@ -203,7 +203,7 @@ __global__ __launch_bounds__(256, 2) void attn_decode_kernel(const KArgs a) {
             if (c8 == 0) { part[pairs * kD + 2 * pair] = mm; part[pairs * kD + 2 * pair + 1] = lw; }
         } else {
             const int row = pair / a.r, head = g * a.r + pair % a.r;
-            const float z = lw + fast_exp2((a.sinks ? a.sinks[head] : 0.0f) * kLog2e - mm), inv = 1.0f / z;
+            const float z = lw + fast_exp2(sink_logit(a, head) * kLog2e - mm), inv = 1.0f / z;
             union { bf16x8 v; u32x4 u; } out;
 #pragma unroll
             for (int e = 0; e < 8; ++e) out.v[e] = (bf16)(acc[e] * inv);
@@ -225,7 +225,7 @@ __global__ __launch_bounds__(256) void attn_decode_combine_kernel(const KArgs a)
     const int row = pair / a.r, head = g * a.r + pair % a.r;
     const int64_t step = decode_partial_floats(pairs);
     const float *part = a.fwd_partial + (int64_t)bg * a.kv_splits * step;
-    const float sink2 = (a.sinks ? a.sinks[head] : 0.0f) * kLog2e;
+    const float sink2 = sink_logit(a, head) * kLog2e;
     float mm = fast_max(sink2, kNoLogit), z = 0.0f, acc[8];         // mm: the largest reference among this lane's splits so far
 #pragma unroll
     for (int e = 0; e < 8; ++e) acc[e] = 0.0f;

@@ -234,7 +234,7 @@ __global__ __launch_bounds__(256, 2) void attn_f32_fwd_kernel(const KArgs a) {
     load_row32(qr, t.q + (int64_t)wk.b * a.qs.b + (int64_t)wk.head * a.qs.h + (int64_t)min(row, a.Sq - 1) * a.qs.s + 32 * half, row < a.Sq);
     const F32Offsets lo = make_f32_offsets(lane);
     const float c = a.scale_log2;
-    const float sink2 = (a.sinks ? a.sinks[wk.head] : 0.0f) * kLog2e;
+    const float sink2 = sink_logit(a, wk.head) * kLog2e;
     float m = sink2, l = 0.0f;
     f32x16 o[2];
 #pragma unroll
@@ -293,7 +293,7 @@ __global__ __launch_bounds__(256, 2) void attn_f32_fwd_kernel(const KArgs a) {
     for (int pass = 0; pass < 8 / KS; ++pass) {
         const int i = pass >> 1, r = (threadIdx.x >> 4) + 16 * (pass & 1), ch = threadIdx.x & 15;
         const F32Unit u = W::unit(a, i);
-        const float sink = (a.sinks ? a.sinks[u.head] : 0.0f) * kLog2e;
+        const float sink = sink_logit(a, u.head) * kLog2e;
         float mm = sink;
 #pragma unroll
         for (int k = 0; k < KS; ++k) mm = fast_max(mm, ml[2 * (KS * i + k) * 32 + r]);
@@ -473,10 +473,12 @@ __global__ __launch_bounds__(256, 2) void attn_f32_dkdv_kernel(const KArgs a) {
 }
 
 // The slices' partial sums, added in slice order.  One thread per 16-byte output chunk.
-__global__ __launch_bounds__(256) void attn_f32_dkdv_reduce_kernel(const KArgs a) {
+__global__ __launch_bounds__(256) void attn_f32_dkdv_reduce_kernel(const KArgs a, int heads) {
+    __shared__ float red[1024];
+    if ((int)blockIdx.x < heads) { dsinks_of_head<256>(a, blockIdx.x, red); return; }
     const F32Ptrs t = f32_ptrs(a);
     const int64_t rows = (int64_t)a.B * a.G * a.Skv, tensor = rows * kD;
-    const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t idx = (int64_t)(blockIdx.x - heads) * 256 + threadIdx.x;
     if (idx >= 2 * rows * 16) return;
     const int which = idx >= rows * 16;
     const int64_t rem = idx - (int64_t)which * rows * 16, row = rem >> 4;

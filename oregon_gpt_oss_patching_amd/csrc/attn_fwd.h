@@ -258,7 +258,7 @@ __global__ __launch_bounds__(256, (NQB == 1 ? 3 : 2)) void attn_fwd_kernel(const
     }
 
     const float c = a.scale_log2;
-    const float sink2 = (a.sinks ? a.sinks[head] : 0.0f) * kLog2e;
+    const float sink2 = sink_logit(a, head) * kLog2e;
     float m[NQB], l[NQB];  // softmax reference (log2 domain, starts at the sink logit, ref :53) and
                            // this lane's share of the running sum (own keys only)
     f32x16 o[NQB][2];

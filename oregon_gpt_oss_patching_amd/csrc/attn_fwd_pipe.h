@@ -110,7 +110,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_pipe_kernel(const KArgs a) {
     }
 
     const float c = a.scale_log2;
-    const float sink2 = (a.sinks ? a.sinks[head] : 0.0f) * kLog2e;
+    const float sink2 = sink_logit(a, head) * kLog2e;
     float m[2], l[2];
     f32x16 o[2][2];
 

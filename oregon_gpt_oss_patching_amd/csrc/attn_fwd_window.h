@@ -73,7 +73,7 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_window_kernel(const KArgs a) 
     // right-padded batch rows: query rows at or beyond the row's length have no keys (O = 0, lse = the sink logit); the
     // rows that exist never see a key beyond it
     const int len = a.seqlens ? min(max(a.seqlens[b], 0), a.Sq) : a.Sq;
-    const float sink2 = (a.sinks ? a.sinks[head] : 0.0f) * kLog2e;
+    const float sink2 = sink_logit(a, head) * kLog2e;
 
     char *const oblk0 = reinterpret_cast<char *>(a.o + (int64_t)b * a.os.b + (int64_t)head * a.os.h + (int64_t)r0 * a.os.s);
     float *const lse0 = a.lse + ((int64_t)b * a.H + head) * a.Sq + r0;

@@ -52,8 +52,13 @@ size_t fp32_stats_bytes(const gptoss_attn_params *p) {
     return (n + 15) & ~(size_t)15;
 }
 
-KArgs make_args(const gptoss_attn_params *p) {
+// Element types of the sink logits and of their gradient (the parameter block has fp32 for both).
+struct SinkTypes { bool sinks_bf16 = false, dsinks_bf16 = false; };
+
+KArgs make_args(const gptoss_attn_params *p, SinkTypes ty) {
     KArgs a{};
+    a.sinks_bf16 = ty.sinks_bf16;
+    a.dsinks_bf16 = ty.dsinks_bf16;
     a.q = static_cast<const bf16 *>(p->q);
     a.k = static_cast<const bf16 *>(p->k);
     a.v = static_cast<const bf16 *>(p->v);
@@ -228,6 +233,17 @@ int launch3(Kernel kernel, dim3 grid, hipStream_t st, const KArgs &a) {
     return e == hipSuccess ? GPTOSS_ATTN_OK : static_cast<int>(e);
 }
 
+// The sum of the partials of cut key blocks; dSinks, where it is still to be done, in the first blocks of the same launch.
+template <typename Kernel>
+int launch_reduce(Kernel kernel, int64_t chunks, hipStream_t st, KArgs a, bool with_dsinks) {
+    int heads = with_dsinks ? a.H : 0;
+    const int64_t blocks = (chunks + 255) / 256 + heads;
+    if (blocks > 0x7fffffff) return GPTOSS_ATTN_ERR_SHAPE;
+    void *args[] = {&a, &heads};
+    const hipError_t e = hipLaunchKernel(reinterpret_cast<const void *>(kernel), dim3((unsigned)blocks), dim3(256), args, 0, st);
+    return e == hipSuccess ? GPTOSS_ATTN_OK : static_cast<int>(e);
+}
+
 // ---- single-pass backward of sliding-window layers (attn_bwd_window.h) ------------------------
 // Taken for bf16 self-attention (Sq == Skv, no offset, no packed rows) with a window of at most
 // 128 and 2..16 query heads per KV head (WinCfg::kMaxGroup: the kernel's LDS holds dSinks slots for
@@ -296,10 +312,10 @@ WindowScratch window_scratch(const gptoss_attn_params *p, int cus) { return wind
 
 // seam_sums: neighbouring chunks exchange fp32 shares through the scratch (needs window_scratch bytes);
 // otherwise each chunk walks two query tiles past its end and nothing but the dSinks sums is kept.
-int launch_window_bwd(const gptoss_attn_params *p, hipStream_t st, bool seam_sums) {
+int launch_window_bwd(const gptoss_attn_params *p, hipStream_t st, bool seam_sums, SinkTypes ty) {
     int rc = window_lds_attribute();
     if (rc) return rc;
-    KArgs a = make_args(p);
+    KArgs a = make_args(p, ty);
     const WindowScratch ws = window_scratch(p, compute_units());
     a.chunk_tiles = ws.chunk_tiles;
     a.dsink_partial = p->delta;
@@ -429,10 +445,10 @@ size_t gptoss_attn_workspace_bytes(const gptoss_attn_params *p) {
     return n;
 }
 
-int gptoss_attn_fwd(const gptoss_attn_params *p, void *stream) {
+static int forward(const gptoss_attn_params *p, void *stream, SinkTypes ty) {
     const int rc = gptoss_attn_validate(p, 0);
     if (rc) return rc;
-    KArgs a = make_args(p);
+    KArgs a = make_args(p, ty);
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (p->delta && !aligned16(p->delta)) return GPTOSS_ATTN_ERR_ALIGNMENT;
     if (decode_route(p)) {
@@ -473,10 +489,19 @@ int gptoss_attn_fwd(const gptoss_attn_params *p, void *stream) {
 #undef GPTOSS_LAUNCH_FWD
 }
 
+int gptoss_attn_fwd(const gptoss_attn_params *p, void *stream) { return forward(p, stream, {}); }
+
+static bool sink_dtype_ok(int dtype) { return dtype == GPTOSS_ATTN_FP32 || dtype == GPTOSS_ATTN_BF16; }
+
+int gptoss_attn_fwd_sinks(const gptoss_attn_params *p, int sinks_dtype, void *stream) {
+    if (!sink_dtype_ok(sinks_dtype)) return GPTOSS_ATTN_ERR_DTYPE;
+    return forward(p, stream, {sinks_dtype == GPTOSS_ATTN_BF16, false});
+}
+
 int gptoss_attn_bwd_preprocess(const gptoss_attn_params *p, void *stream) {
     const int rc = gptoss_attn_validate(p, 1);
     if (rc) return rc;
-    const KArgs a = make_args(p);
+    const KArgs a = make_args(p, {});
     hipStream_t st = static_cast<hipStream_t>(stream);
     const int64_t rows = (int64_t)a.B * a.H * a.Sq;
     int s = p->dtype == GPTOSS_ATTN_FP32 ? launch(attn_f32_delta_kernel, (rows + 15) / 16, 256, st, a)
@@ -486,41 +511,44 @@ int gptoss_attn_bwd_preprocess(const gptoss_attn_params *p, void *stream) {
 }
 
 // The dK/dV launch (and the sum of the partials when key blocks are cut).  whole_blocks: never cut a
-// key block, so that nothing beyond the row statistics is kept in the scratch.
-static int launch_dkdv(const gptoss_attn_params *p, void *stream, bool whole_blocks) {
+// key block, so that nothing beyond the row statistics is kept in the scratch.  with_dsinks: dSinks too, from the row statistics.
+static int launch_dkdv(const gptoss_attn_params *p, void *stream, bool whole_blocks, bool with_dsinks, SinkTypes ty) {
     const int rc = gptoss_attn_validate(p, 1);
     if (rc) return rc;
-    KArgs a = make_args(p);
+    KArgs a = make_args(p, ty);
     hipStream_t st = static_cast<hipStream_t>(stream);
     a.dkdv_parts = whole_blocks ? 1 : dkdv_parts_for(p, p->seqlens != nullptr);
     a.dkdv_partial = reinterpret_cast<float *>(reinterpret_cast<char *>(p->delta) + stats_bytes(p));
+    if (with_dsinks && a.dkdv_parts == 1) {
+        const int s = launch(attn_bwd_dsinks_kernel, a.H, 1024, st, a);
+        if (s) return s;
+    }
     if (p->dtype == GPTOSS_ATTN_FP32) {
         const int s = launch(attn_f32_dkdv_kernel, (int64_t)a.B * a.G * a.dkdv_parts * ((a.Skv + 31) / 32), 256, st, a);
         if (s || a.dkdv_parts == 1) return s;
-        return launch(attn_f32_dkdv_reduce_kernel, ((int64_t)2 * a.B * a.G * a.Skv * 16 + 255) / 256, 256, st, a);
+        return launch_reduce(attn_f32_dkdv_reduce_kernel, (int64_t)2 * a.B * a.G * a.Skv * 16, st, a, with_dsinks);
     }
     if (dkdv64_route(p, a.dkdv_parts)) {
         const int64_t grid64 = (int64_t)a.G * a.B * a.dkdv_parts * ((a.Skv + Dkdv64::BN - 1) / Dkdv64::BN);
         const bool plain = !a.seqlens && !a.doc_start && a.Sq % kTile == 0;
         const int s = plain ? launch(attn_bwd_dkdv64_kernel<false>, grid64, 256, st, a) : launch(attn_bwd_dkdv64_kernel<true>, grid64, 256, st, a);
         if (s || a.dkdv_parts == 1) return s;
-        return launch(attn_bwd_dkdv_reduce_kernel, ((int64_t)2 * a.B * a.G * a.Skv * 8 + 255) / 256, 256, st, a);
+        return launch_reduce(attn_bwd_dkdv_reduce_kernel, (int64_t)2 * a.B * a.G * a.Skv * 8, st, a, with_dsinks);
     }
     const int64_t grid = (int64_t)a.G * a.B * a.dkdv_parts * ((a.Skv + kDkdvKeys - 1) / kDkdvKeys);
     const int s = a.doc_start ? launch(attn_bwd_dkdv_kernel<kDkdvWaves, kDkdvNB, true>, grid, 64 * kDkdvWaves, st, a)
                               : launch(attn_bwd_dkdv_kernel<kDkdvWaves, kDkdvNB, false>, grid, 64 * kDkdvWaves, st, a);
     if (s || a.dkdv_parts == 1) return s;
-    const int64_t chunks = (int64_t)2 * a.B * a.G * a.Skv * 8;
-    return launch(attn_bwd_dkdv_reduce_kernel, (chunks + 255) / 256, 256, st, a);
+    return launch_reduce(attn_bwd_dkdv_reduce_kernel, (int64_t)2 * a.B * a.G * a.Skv * 8, st, a, with_dsinks);
 }
 
-int gptoss_attn_bwd_dkdv(const gptoss_attn_params *p, void *stream) { return launch_dkdv(p, stream, false); }
+int gptoss_attn_bwd_dkdv(const gptoss_attn_params *p, void *stream) { return launch_dkdv(p, stream, false, false, {}); }
 
 // The dQ launch; fuse_delta: the kernel also produces the row statistics (see attn_bwd_dq_kernel).
 static int launch_dq(const gptoss_attn_params *p, void *stream, int fuse_delta) {
     const int rc = gptoss_attn_validate(p, 1);
     if (rc) return rc;
-    const KArgs a = make_args(p);
+    const KArgs a = make_args(p, {});
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (p->dtype == GPTOSS_ATTN_FP32) {
         const int ks = f32_key_splits(a);
@@ -546,23 +574,23 @@ static int launch_dq(const gptoss_attn_params *p, void *stream, int fuse_delta) 
 int gptoss_attn_bwd_dq(const gptoss_attn_params *p, void *stream) { return launch_dq(p, stream, 0); }
 
 // The whole backward: the dQ kernel computes the row statistics on the way (no separate
-// pass over O and dO), then dSinks and dK/dV read them from the scratch buffer.  The results are
+// pass over O and dO), then dK/dV and dSinks read them from the scratch buffer.  The results are
 // bit-identical to gptoss_attn_bwd_preprocess + gptoss_attn_bwd_dkdv + gptoss_attn_bwd_dq.
-static int bwd_all(const gptoss_attn_params *p, void *stream, bool whole_blocks) {
+static int bwd_all(const gptoss_attn_params *p, void *stream, bool whole_blocks, SinkTypes ty) {
     int rc = gptoss_attn_validate(p, 1);
     if (rc) return rc;
-    if (window_single_pass(p)) return launch_window_bwd(p, static_cast<hipStream_t>(stream), !whole_blocks);
+    if (window_single_pass(p)) return launch_window_bwd(p, static_cast<hipStream_t>(stream), !whole_blocks, ty);
     rc = launch_dq(p, stream, 1);
     if (rc) return rc;
-    if (p->dsinks) {
-        const KArgs a = make_args(p);
-        rc = launch(attn_bwd_dsinks_kernel, a.H, 1024, static_cast<hipStream_t>(stream), a);
-        if (rc) return rc;
-    }
-    return launch_dkdv(p, stream, whole_blocks);
+    return launch_dkdv(p, stream, whole_blocks, p->dsinks != nullptr, ty);
 }
 
-int gptoss_attn_bwd(const gptoss_attn_params *p, void *stream) { return bwd_all(p, stream, false); }
+int gptoss_attn_bwd(const gptoss_attn_params *p, void *stream) { return bwd_all(p, stream, false, {}); }
+
+int gptoss_attn_bwd_sinks(const gptoss_attn_params *p, int sinks_dtype, int dsinks_dtype, void *stream) {
+    if (!sink_dtype_ok(sinks_dtype) || !sink_dtype_ok(dsinks_dtype)) return GPTOSS_ATTN_ERR_DTYPE;
+    return bwd_all(p, stream, false, {sinks_dtype == GPTOSS_ATTN_BF16, dsinks_dtype == GPTOSS_ATTN_BF16});
+}
 
 // ---- the backward for callers that cannot allocate ------------------------------------------
 // Same kernels as gptoss_attn_bwd; the row statistics live in a device array that is part of the
@@ -604,7 +632,7 @@ int gptoss_attn_bwd_static(const gptoss_attn_params *p, void *stream) {
     if (stats_bytes(&q) > kStaticScratchBytes) return GPTOSS_ATTN_ERR_WORKSPACE;
     rc = static_scratch(&q.delta);
     if (rc) return rc;
-    return bwd_all(&q, stream, true);
+    return bwd_all(&q, stream, true, {});
 }
 
 // ---- packed rows (doc_start.h) ----------------------------------------------------------------

@@ -66,6 +66,7 @@ void set(gptoss_attn_strides &s, const Tensor &t, bool bshd) {
 struct Call {
     gptoss_attn_params p{};
     Tensor q, k, v, sinks, seqlens, doc_start, q_offset_dev;
+    int sinks_dtype = GPTOSS_ATTN_FP32;
 };
 
 void fill(Call &c, const Tensor &q, const Tensor &k, const Tensor &v, const OptTensor &sinks, double sm_scale, int64_t window, int64_t q_offset,
@@ -93,8 +94,10 @@ void fill(Call &c, const Tensor &q, const Tensor &k, const Tensor &v, const OptT
     set(p.k_stride, c.k, false);
     set(p.v_stride, c.v, false);
     if (sinks) {
-        c.sinks = sinks->to(at::kFloat).contiguous();
-        p.sinks = c.sinks.const_data_ptr<float>();
+        const bool bf16 = sinks->scalar_type() == at::kBFloat16;      // read as they are: no converted copy
+        c.sinks = (bf16 ? *sinks : sinks->to(at::kFloat)).contiguous();
+        c.sinks_dtype = bf16 ? GPTOSS_ATTN_BF16 : GPTOSS_ATTN_FP32;
+        p.sinks = static_cast<const float *>(c.sinks.const_data_ptr());
     }
     if (seqlens) {
         c.seqlens = seqlens->to(q.device(), at::kInt).contiguous();
@@ -115,8 +118,9 @@ void fill(Call &c, const Tensor &q, const Tensor &k, const Tensor &v, const OptT
     }
 }
 
-void launch(const char *name, int (*fn)(const gptoss_attn_params *, void *), const Call &c) {
-    const int rc = fn(&c.p, c10::hip::getCurrentHIPStream(c.q.device().index()).stream());
+void *stream_of(const Call &c) { return c10::hip::getCurrentHIPStream(c.q.device().index()).stream(); }
+
+void check(const char *name, int rc) {
     TORCH_CHECK(rc == 0, name, " failed with status ", rc, ": ", gptoss_attn_status_string(rc));
 }
 
@@ -135,14 +139,15 @@ std::tuple<Tensor, Tensor> fwd(const Tensor &q, const Tensor &k, const Tensor &v
         scratch = at::empty({static_cast<int64_t>(need / sizeof(float))}, lse.options());
         c.p.delta = scratch.data_ptr<float>();
     }
-    launch("gptoss_attn_fwd", gptoss_attn_fwd, c);
+    check("gptoss_attn_fwd", gptoss_attn_fwd_sinks(&c.p, c.sinks_dtype, stream_of(c)));
     return {o, lse};
 }
 
-// (an operator cannot return None: an empty dsinks stands for "not requested")
+// (an operator cannot return None: an empty dsinks stands for "not requested"; dsinks_as_sinks: in bf16 where the logits are)
 std::tuple<Tensor, Tensor, Tensor, Tensor> bwd(const Tensor &q, const Tensor &k, const Tensor &v, const OptTensor &sinks, const Tensor &o_,
                                                const Tensor &lse_, const Tensor &d_o_, double sm_scale, int64_t window, int64_t q_offset,
-                                               const OptTensor &seqlens, const OptTensor &doc_start, bool need_dsinks, const OptTensor &q_offset_dev) {
+                                               const OptTensor &seqlens, const OptTensor &doc_start, bool need_dsinks, const OptTensor &q_offset_dev,
+                                               bool dsinks_as_sinks) {
     const c10::OptionalDeviceGuard guard(q.device());
     Call c;
     fill(c, q, k, v, sinks, sm_scale, window, q_offset, seqlens, doc_start, q_offset_dev);
@@ -158,7 +163,8 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> bwd(const Tensor &q, const Tensor &k,
     const Tensor o = row_contiguous(o_, 1), d_o = row_contiguous(d_o_, 1), lse = lse_.contiguous();
 
     Tensor dq = at::empty({b, h, s, d}, q.options()), dk = at::empty(k.sizes(), k.options()), dv = at::empty(v.sizes(), v.options());
-    Tensor dsinks = at::empty({need_dsinks ? h : 0}, lse.options());
+    const bool bf16_dsinks = dsinks_as_sinks && c.sinks_dtype == GPTOSS_ATTN_BF16;
+    Tensor dsinks = at::empty({need_dsinks ? h : 0}, lse.options().dtype(bf16_dsinks ? at::kBFloat16 : at::kFloat));
     // scratch: the row statistics, then the dK/dV partial sums of split key blocks or the window kernel's shares
     Tensor scratch = at::empty({static_cast<int64_t>(gptoss_attn_workspace_bytes(&c.p) / sizeof(float))}, lse.options());
     gptoss_attn_params &p = c.p;
@@ -168,14 +174,14 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> bwd(const Tensor &q, const Tensor &k,
     p.dq = dq.data_ptr();
     p.dk = dk.data_ptr();
     p.dv = dv.data_ptr();
-    p.dsinks = need_dsinks ? dsinks.data_ptr<float>() : nullptr;
+    p.dsinks = need_dsinks ? static_cast<float *>(dsinks.data_ptr()) : nullptr;
     p.delta = scratch.data_ptr<float>();
     set(p.o_stride, o, true);
     set(p.do_stride, d_o, true);
     set(p.dq_stride, dq, false);
     set(p.dk_stride, dk, false);
     set(p.dv_stride, dv, false);
-    launch("gptoss_attn_bwd", gptoss_attn_bwd, c);
+    check("gptoss_attn_bwd", gptoss_attn_bwd_sinks(&c.p, c.sinks_dtype, bf16_dsinks ? GPTOSS_ATTN_BF16 : GPTOSS_ATTN_FP32, stream_of(c)));
     return {dq, dk, dv, dsinks};
 }
 
@@ -188,9 +194,9 @@ std::tuple<Tensor, Tensor> call_fwd(const Tensor &q, const Tensor &k, const Tens
 std::tuple<Tensor, Tensor, Tensor, Tensor> call_bwd(const Tensor &q, const Tensor &k, const Tensor &v, const OptTensor &sinks, const Tensor &o,
                                                     const Tensor &lse, const Tensor &d_o, double sm_scale, int64_t window, int64_t q_offset,
                                                     const OptTensor &seqlens, const OptTensor &doc_start, bool need_dsinks,
-                                                    const OptTensor &q_offset_dev) {
+                                                    const OptTensor &q_offset_dev, bool dsinks_as_sinks) {
     static const auto op = c10::Dispatcher::singleton().findSchemaOrThrow("gptoss_attn::bwd", "").typed<decltype(bwd)>();
-    return op.call(q, k, v, sinks, o, lse, d_o, sm_scale, window, q_offset, seqlens, doc_start, need_dsinks, q_offset_dev);
+    return op.call(q, k, v, sinks, o, lse, d_o, sm_scale, window, q_offset, seqlens, doc_start, need_dsinks, q_offset_dev, dsinks_as_sinks);
 }
 
 OptTensor optional_of(const Tensor &t) { return t.defined() ? OptTensor(t) : OptTensor(); }
@@ -232,7 +238,7 @@ struct AttentionFunction : public torch::autograd::Function<AttentionFunction> {
         auto [dq, dk, dv, dsinks] = call_bwd(q, saved[1], saved[2], optional_of(sinks), saved[4], saved[5], grads[0].to(q.scalar_type()),
                                              ctx->saved_data["sm_scale"].toDouble(), ctx->saved_data["window"].toInt(),
                                              ctx->saved_data["q_offset"].toInt(), optional_of(saved[6]), optional_of(saved[7]), need_dsinks,
-                                             optional_of(saved[8]));
+                                             optional_of(saved[8]), true);
         if (half) {
             dq = dq.to(at::kHalf);
             dk = dk.to(at::kHalf);
@@ -269,7 +275,7 @@ TORCH_LIBRARY(gptoss_attn, m) {
     m.def("fwd(Tensor q, Tensor k, Tensor v, Tensor? sinks, float sm_scale, int window, int q_offset, Tensor? seqlens, Tensor? doc_start, "
           "Tensor? q_offset_dev=None) -> (Tensor, Tensor)");
     m.def("bwd(Tensor q, Tensor k, Tensor v, Tensor? sinks, Tensor o, Tensor lse, Tensor d_o, float sm_scale, int window, int q_offset, "
-          "Tensor? seqlens, Tensor? doc_start, bool need_dsinks, Tensor? q_offset_dev=None) -> (Tensor, Tensor, Tensor, Tensor)");
+          "Tensor? seqlens, Tensor? doc_start, bool need_dsinks, Tensor? q_offset_dev=None, bool dsinks_as_sinks=False) -> (Tensor, Tensor, Tensor, Tensor)");
     m.def("doc_start(Tensor position_ids) -> Tensor");
     m.def("attention(Tensor q, Tensor k, Tensor v, Tensor? sinks, float sm_scale, int window, int q_offset, Tensor? seqlens, Tensor? doc_start, "
           "Tensor? q_offset_dev=None) -> Tensor", &attention);
