@@ -123,3 +123,17 @@ def test_64_key_backward_of_any_length_vs_eager_oracle(A, b, h, g, s, lens, docs
     TP.check("dsinks", dsinks, rds.float(), atol=None)
     again = TP.run_hip(A, *inp, None, 0, lens, ds)
     assert all(torch.equal(x, y) for x, y in zip(got, again))
+
+
+@pytest.mark.parametrize("b,h,g,s,lens", [
+    (2, 8, 4, 64 * 5 + 1, None),                    # a last chunk of less than two tiles
+    (1, 16, 8, 64 * 97, None),                      # 97 tiles x 8 heads: chunks of four on 256 compute units, a last one of a single tile
+    (3, 16, 8, 1999, [1999, 700, 65]),              # chunks of three
+])
+def test_window_backward_chunks_vs_eager_oracle(A, b, h, g, s, lens):
+    """The single-pass window backward where the chunk length follows the rounds of workgroups."""
+    print(f"case B={b} H={h} G={g} S={s} lens={lens}", flush=True)
+    inp = E.make_inputs(5500 + s, b, h, g, s, 64, torch.bfloat16)
+    if lens:
+        inp = inp[:4] + (TP.mask_dout(inp[4], lens),)
+    TP.compare_all(TP.run_hip(A, *inp, 128, 0, lens), TP.oracle_tiled(*inp, 128, 0, lens))
