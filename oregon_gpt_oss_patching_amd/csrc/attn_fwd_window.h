@@ -45,7 +45,11 @@ struct FwdWindow {
 // into assembly text.
 __device__ __forceinline__ float max3_f32(float a, float b, float c) { return __builtin_fmaxf(__builtin_fmaxf(a, b), c); }
 
-template <int WH>
+// The plain instantiation is for self-attention (Sq == Skv a multiple of 32, right padding allowed).  GENERAL takes any
+// lengths, a query offset and packed documents: rows and keys past the end re-read the last one and are not stored or
+// masked, and a query block in which some row sees fewer than W keys for another reason than the start of the row (its document
+// starts inside the window, or the keys end before the queries do) takes the general test.
+template <int WH, bool GENERAL = false>
 __global__ __launch_bounds__(256, 3) void attn_fwd_window_kernel(const KArgs a) {
     using C = FwdWindow<WH>;
     constexpr int W = C::W, NH = C::NH;
@@ -68,25 +72,27 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_window_kernel(const KArgs a) 
     const bool pairs = 32 * (int)gridDim.z < a.Sq;
     const int r0 = (pairs ? 64 : 32) * blockIdx.z; // first query row of the workgroup
     const int head = g * a.r + 4 * hc + w;
-    const int k0 = r0 - W;                         // first staged key; negative for the first blocks of a row
+    const int off = GENERAL ? query_offset(a) : 0; // absolute position of query row 0
+    const int k0 = off + r0 - W;                   // first staged key; negative for the first blocks of a row
     const bool two = pairs && r0 + 32 < a.Sq;      // (a row may end with a single block)
     // right-padded batch rows: query rows at or beyond the row's length have no keys (O = 0, lse = the sink logit); the
     // rows that exist never see a key beyond it
-    const int len = a.seqlens ? min(max(a.seqlens[b], 0), a.Sq) : a.Sq;
+    const int len = GENERAL ? (a.seqlens ? min(max(a.seqlens[b] - off, 0), a.Sq) : a.Sq) : a.seqlens ? min(max(a.seqlens[b], 0), a.Sq) : a.Sq;
     const float sink2 = sink_logit(a, head) * kLog2e;
 
     char *const oblk0 = reinterpret_cast<char *>(a.o + (int64_t)b * a.os.b + (int64_t)head * a.os.h + (int64_t)r0 * a.os.s);
     float *const lse0 = a.lse + ((int64_t)b * a.H + head) * a.Sq + r0;
     // lane's 16 bytes of an 8-row group of output rows: row lane / 8, piece lane % 8
     auto out_offset = [&](int ln) __attribute__((always_inline)) { return (uint32_t)((ln >> 3) * (int)a.os.s + (ln & 7) * 8) * 2u; };
+    auto row_exists = [&](int X, int row) __attribute__((always_inline)) { return !GENERAL || r0 + 32 * X + row < a.Sq; };
     // a query block of nothing but padding: zeros, and the lse the arithmetic below gives a row without keys
     auto padding_block = [&](int X) __attribute__((always_inline)) {
         const int ln = fresh_lane();
         const uint32_t ooff = out_offset(ln);
 #pragma unroll
         for (int pass = 0; pass < 4; ++pass)
-            *reinterpret_cast<u32x4 *>(oblk0 + (int64_t)(32 * X + 8 * pass) * a.os.s * 2 + ooff) = u32x4{0u, 0u, 0u, 0u};
-        if (ln < 32) lse0[32 * X + ln] = (sink2 + fast_log2(1.0f)) * kLn2;
+            if (row_exists(X, 8 * pass + (ln >> 3))) *reinterpret_cast<u32x4 *>(oblk0 + (int64_t)(32 * X + 8 * pass) * a.os.s * 2 + ooff) = u32x4{0u, 0u, 0u, 0u};
+        if (ln < 32 && row_exists(X, ln)) lse0[32 * X + ln] = (sink2 + fast_log2(1.0f)) * kLn2;
     };
     if (r0 >= len) {
         padding_block(0);
@@ -99,7 +105,8 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_window_kernel(const KArgs a) 
     const char *const qblk0 = reinterpret_cast<const char *>(a.q + (int64_t)b * a.qs.b + (int64_t)head * a.qs.h + (int64_t)r0 * a.qs.s);
     auto load_q = [&](int X) __attribute__((always_inline)) {
         const int ln = fresh_lane();
-        const uint32_t qoff = (uint32_t)((ln & 31) * (int)a.qs.s + 8 * (ln >> 5)) * 2u;
+        const int row = GENERAL ? min(ln & 31, a.Sq - 1 - r0 - 32 * X) : ln & 31;
+        const uint32_t qoff = (uint32_t)(row * (int)a.qs.s + 8 * (ln >> 5)) * 2u;
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks)
             qf[ks] = as_bf16x8(*reinterpret_cast<const u32x4 *>(qblk0 + (int64_t)(32 * X) * a.qs.s * 2 + qoff + 32 * ks));
@@ -117,7 +124,7 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_window_kernel(const KArgs a) 
         // addresses are (scalar pointer) + (32-bit lane offset): the row of copy j is a scalar step away from copy 0's,
         // except where rows are held at key 0
         auto copy_all = [&](const bf16 *base, int stride, char *dst) __attribute__((always_inline)) {
-            if (k0 >= 0) {
+            if (k0 >= 0 && (!GENERAL || k0 + 32 * (NH + 1) <= a.Skv)) {
                 const uint32_t voff = (uint32_t)(rloc * stride + ch * 8) * 2u;
 #pragma unroll
                 for (int j = 0; j <= NH; ++j)
@@ -128,8 +135,9 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_window_kernel(const KArgs a) 
 #pragma unroll
                 for (int j = 0; j <= NH; ++j)
                     if (j < NH || live1) {
-                        const uint32_t voff = (uint32_t)(max(k0 + rloc + 32 * j, 0) * stride + ch * 8) * 2u;
-                        __builtin_amdgcn_global_load_lds((glb_void_t *)(reinterpret_cast<const char *>(base) + voff),
+                        const int first = GENERAL ? min(max(k0, 0), a.Skv - 1) : 0, row = max(k0 + rloc + 32 * j, first);
+                        const uint32_t voff = (uint32_t)((GENERAL ? min(row, a.Skv - 1) - first : row) * stride + ch * 8) * 2u;
+                        __builtin_amdgcn_global_load_lds((glb_void_t *)(reinterpret_cast<const char *>(base + (GENERAL ? (int64_t)first * stride : 0)) + voff),
                                                          (lds_void_t *)(dst + j * 32 * kRowBytes), 16, 0, 0);
                     }
             }
@@ -152,8 +160,17 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_window_kernel(const KArgs a) 
     float m, l;
     auto block = [&](auto x_tag) __attribute__((always_inline)) {
         constexpr int X = decltype(x_tag)::value;
-        const bool edge = k0 + 32 * X < 0;
-        const bool no_keys = r0 + 32 * X + l32 >= len;          // this lane's row is padding
+        bool edge = k0 + 32 * X < 0;
+        int doc = 0;                                            // first key of the row's document
+        if constexpr (GENERAL) {
+            const int row0 = r0 + 32 * X;
+            edge = edge || off + min(row0 + 32, a.Sq) > a.Skv;
+            if (a.doc_start) {
+                doc = a.doc_start[(int64_t)b * a.Sq + min(row0 + l32, a.Sq - 1)];
+                edge = edge || __builtin_amdgcn_ballot_w64(doc > off + row0 + l32 - W + 1) != 0ull;
+            }
+        }
+        bool no_keys = r0 + 32 * X + l32 >= len;                // this lane's row is padding
         // S^T = K Q^T for all NH blocks: lane = query row l32, register i of block h = key 32 h + rc(i) + 4 half
         f32x16 s[NH];
 #pragma unroll
@@ -220,8 +237,12 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_window_kernel(const KArgs a) 
         } else {
             // general test: key k0 + 32 (X + h) + rc + 4 half is visible to row r0 + 32 X + l32 iff it is not in front of
             // key 0, not after the row and less than W behind it: lo_l <= 32 h + rc <= x + W
-            const int lo_l = max(x + 1, -(k0 + 32 * X) - 4 * half);
-            const unsigned width = (unsigned)(x + W - lo_l);
+            // (GENERAL: nor in front of its document, nor past the last key)
+            const int kx = k0 + 32 * X + 4 * half;
+            const int lo_l = max(x + 1, (GENERAL ? max(doc, 0) : 0) - kx);
+            const int hi_l = GENERAL ? min(x + W, a.Skv - 1 - kx) : x + W;
+            if (GENERAL) no_keys = no_keys || hi_l < lo_l;
+            const unsigned width = (unsigned)(hi_l - lo_l);     // (of a row without keys: anything, its weights are zeroed below)
             float mx0 = -INFINITY, mx1 = -INFINITY;
 #pragma unroll
             for (int h = 0; h < NH; ++h)
@@ -281,9 +302,10 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_window_kernel(const KArgs a) 
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
         for (int pass = 0; pass < 4; ++pass)
-            *reinterpret_cast<u32x4 *>(oblk0 + (int64_t)(32 * X + 8 * pass) * a.os.s * 2 + ooff) =
-                *reinterpret_cast<const u32x4 *>(stage + (rr + 8 * pass) * kLS + cc * 8);
-        if (hf == 0) lse0[32 * X + row] = (m + fast_log2(z)) * kLn2;
+            if (row_exists(X, rr + 8 * pass))
+                *reinterpret_cast<u32x4 *>(oblk0 + (int64_t)(32 * X + 8 * pass) * a.os.s * 2 + ooff) =
+                    *reinterpret_cast<const u32x4 *>(stage + (rr + 8 * pass) * kLS + cc * 8);
+        if (hf == 0 && row_exists(X, row)) lse0[32 * X + row] = (m + fast_log2(z)) * kLn2;
     };
     // The first block while the second still needs the staged rows: only the first 32 rows of K and of V are free (the
     // second block starts one 32-key block later), 2 KB per wavefront, so the rows go in two halves of 16, unpadded,

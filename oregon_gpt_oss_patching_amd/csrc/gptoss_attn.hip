@@ -171,17 +171,18 @@ bool fwd_pipe_plain(const gptoss_attn_params *p) {
     return p->Sq == p->Skv && p->Sq % kTile == 0 && !p->seqlens && !p->doc_start && p->q_offset == 0 && !p->q_offset_dev;
 }
 
-// The one-pass forward of sliding-window layers (attn_fwd_window.h): a window of 32, 64, 96 or 128 keys on plain
-// self-attention rows (no offset, no packed rows; right-padded batch rows are fine) whose padded length is a
-// multiple of 32, all four wavefronts of a workgroup with a head of their own.
+// The one-pass forward of sliding-window layers (attn_fwd_window.h): a window of 32, 64, 96 or 128 keys, all four wavefronts of
+// a workgroup with a head of their own.  Self-attention of whole 32-row blocks without packing has an instantiation of its own.
 bool fwd_window_route(const gptoss_attn_params *p) {
     const int w = effective_window(p);
     // lane offsets are 32-bit: up to 160 rows of K / V, 32 of Q and O; the grid's y and z dimensions end at 65535
     const int64_t row_limit = (int64_t)1 << 22;
     if (p->k_stride.s >= row_limit || p->v_stride.s >= row_limit || p->q_stride.s >= row_limit || p->o_stride.s >= row_limit) return false;
-    if ((int64_t)(p->H / p->G / 4) * p->B > 65535 || p->Sq / 32 > 65535) return false;
-    return p->dtype == GPTOSS_ATTN_BF16 && w >= 32 && w <= 128 && w % 32 == 0 && !p->doc_start &&
-           p->q_offset == 0 && !p->q_offset_dev && p->Sq == p->Skv && p->Sq % 32 == 0 && (p->H / p->G) % 4 == 0;
+    if ((int64_t)(p->H / p->G / 4) * p->B > 65535 || (p->Sq + 31) / 32 > 65535) return false;
+    return p->dtype == GPTOSS_ATTN_BF16 && w >= 32 && w <= 128 && w % 32 == 0 && (p->H / p->G) % 4 == 0;
+}
+bool fwd_window_plain(const gptoss_attn_params *p) {
+    return !p->doc_start && p->q_offset == 0 && !p->q_offset_dev && p->Sq == p->Skv && p->Sq % 32 == 0;
 }
 
 // A few queries on a long cache (attn_decode.h): all (query, head) pairs of a KV head fit two 32-column blocks.
@@ -480,13 +481,16 @@ static int forward(const gptoss_attn_params *p, void *stream, SinkTypes ty) {
         // unit several rounds of workgroups, else one
         const int64_t pairs = (int64_t)a.G * (a.r / 4) * a.B * ((a.Sq + 63) / 64);
         const bool by_pairs = a.Sq > 32 && pairs >= 8 * (int64_t)compute_units();
-        const dim3 wgrid((unsigned)a.G, (unsigned)((a.r / 4) * a.B), (unsigned)(by_pairs ? (a.Sq + 63) / 64 : a.Sq / 32));
+        const dim3 wgrid((unsigned)a.G, (unsigned)((a.r / 4) * a.B), (unsigned)(by_pairs ? (a.Sq + 63) / 64 : (a.Sq + 31) / 32));
+        const bool plain = fwd_window_plain(p);
+#define GPTOSS_LAUNCH_WIN(WH) (plain ? launch3(attn_fwd_window_kernel<WH, false>, wgrid, st, a) : launch3(attn_fwd_window_kernel<WH, true>, wgrid, st, a))
         switch (a.window / 32) {
-            case 1: return launch3(attn_fwd_window_kernel<1>, wgrid, st, a);
-            case 2: return launch3(attn_fwd_window_kernel<2>, wgrid, st, a);
-            case 3: return launch3(attn_fwd_window_kernel<3>, wgrid, st, a);
-            default: return launch3(attn_fwd_window_kernel<4>, wgrid, st, a);
+            case 1: return GPTOSS_LAUNCH_WIN(1);
+            case 2: return GPTOSS_LAUNCH_WIN(2);
+            case 3: return GPTOSS_LAUNCH_WIN(3);
+            default: return GPTOSS_LAUNCH_WIN(4);
         }
+#undef GPTOSS_LAUNCH_WIN
     }
     if (fwd_pipe_route(p)) 
         return fwd_pipe_plain(p) ? launch(attn_fwd_pipe_kernel<false, false>, grid, 256, st, a)
