@@ -114,8 +114,10 @@ constexpr int kDkdvKeys = 32 * kDkdvNB * kDkdvWaves; // keys per dK/dV workgroup
 // key block of a long row (4096 rows and more) is still longer than the average compute unit's share: two slices; a
 // right-padded batch counts half, because its shorter rows leave the longest one alone (dK/dV of B = 4, S = 4096,
 // lengths 3309 / 1968 / 1554 / 4079: 715 us uncut, 589 in two slices; B = 2, S = 8192 / 4000: 1437 and 1216; but B = 8,
-// S <= 2048: 359 and 370).
-int dkdv_parts_for(const gptoss_attn_params *p, bool padded) {
+// S <= 2048: 359 and 370).  Packed rows: a walk ends with its document, so the longest document's first blocks stand out more, and
+// the host does not see the documents: up to four slices (layer, seven documents in 8192 tokens: 801 us in two, 759 in four; six in 12000:
+// 1411 and 1385; 8192 tokens in ONE document: 2174 and 2192).
+int dkdv_parts_for(const gptoss_attn_params *p, bool padded, bool packed) {
     if (p->dtype == GPTOSS_ATTN_FP32) {
         // a workgroup per 32 keys, two per compute unit: about four workgroups per unit of a 256-CU part, so that the long
         // first key blocks of a row do not decide the time
@@ -133,6 +135,7 @@ int dkdv_parts_for(const gptoss_attn_params *p, bool padded) {
     const int64_t tiles = ((rows_seen < p->Sq ? rows_seen : p->Sq) + 63) / 64;
     int64_t parts = (1024 + blocks - 1) / blocks;
     if (blocks > 512) parts = p->Sq >= 4096 && (padded && p->B > 1 ? blocks / 2 : blocks) < 1024 ? 2 : 1;
+    if (packed && window == 0 && blocks >= 256 && blocks <= 1024 && parts < 4) parts = 3072 / blocks < 4 ? 3072 / blocks : 4;
     const int64_t steps = window > 0 ? tiles / 4 : tiles * (p->H / p->G) / 8;
     if (parts > steps) parts = steps;
     if (parts > tiles) parts = tiles;
@@ -423,9 +426,13 @@ static size_t stats_bytes(const gptoss_attn_params *p) {
     return fp32_stats_bytes(p) + (size_t)16 * (size_t)p->B * (size_t)p->H * (size_t)p->Sq;
 }
 
-// dK/dV partial sums, for a call with or without lengths of padded rows (the size depends on the shapes only)
+// dK/dV partial sums, for a call with or without lengths of padded rows and documents (the size depends on the shapes only)
 static size_t partials_bytes(const gptoss_attn_params *p) {
-    const int plain = dkdv_parts_for(p, false), padded = dkdv_parts_for(p, true), parts = plain > padded ? plain : padded;
+    int parts = 1;
+    for (int kind = 0; kind < 4; ++kind) {
+        const int n = dkdv_parts_for(p, kind & 1, kind & 2);
+        if (n > parts) parts = n;
+    }
     return parts > 1 ? (size_t)parts * 2 * sizeof(float) * (size_t)p->B * (size_t)p->G * (size_t)p->Skv * kD : 0;
 }
 
@@ -530,7 +537,7 @@ static int launch_dkdv(const gptoss_attn_params *p, void *stream, bool whole_blo
     if (rc) return rc;
     KArgs a = make_args(p, ty);
     hipStream_t st = static_cast<hipStream_t>(stream);
-    a.dkdv_parts = whole_blocks ? 1 : dkdv_parts_for(p, p->seqlens != nullptr);
+    a.dkdv_parts = whole_blocks ? 1 : dkdv_parts_for(p, p->seqlens != nullptr, p->doc_start != nullptr);
     a.dkdv_partial = reinterpret_cast<float *>(reinterpret_cast<char *>(p->delta) + stats_bytes(p));
     if (with_dsinks && a.dkdv_parts == 1) {
         const int s = launch(attn_bwd_dsinks_kernel, a.H, 1024, st, a);
