@@ -65,6 +65,8 @@ __global__ __launch_bounds__(256) void attn_bwd_delta_kernel(const KArgs a) {
 template <int THREADS>
 __device__ __forceinline__ void dsinks_of_head(const KArgs &a, int h, float (&red)[1024]) {
     constexpr int N = 1024 / THREADS;
+    constexpr int U = 16 / N;          // rounds of 1024 rows in flight: the loads' latency is all there is (one round at a time, B = 4,
+                                       // S = 4096: 45 us for the launch whose other blocks take 26)
     const float sink2 = sink_logit(a, h) * kLog2e;
     const int64_t total = (int64_t)a.B * a.H * a.Sq;
     float acc[N];
@@ -73,12 +75,22 @@ __device__ __forceinline__ void dsinks_of_head(const KArgs &a, int h, float (&re
     for (int b = 0; b < a.B; ++b) {
         const float *ndl = a.delta + ((int64_t)b * a.H + h) * a.Sq;        // -delta
         const float *lse2 = ndl + total;                                    // lse * log2(e)
-        for (int s0 = threadIdx.x; s0 < a.Sq; s0 += 1024)
+        for (int s0 = threadIdx.x; s0 < a.Sq; s0 += 1024 * U) {
+            float x[U][N], y[U][N];
 #pragma unroll
-            for (int k = 0; k < N; ++k) {
-                const int s = s0 + k * THREADS;
-                if (s < a.Sq) acc[k] = fmaf(fast_exp2(sink2 - lse2[s]), ndl[s], acc[k]);
-            }
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int k = 0; k < N; ++k) {
+                    const int s = min(s0 + 1024 * u + k * THREADS, a.Sq - 1);
+                    x[u][k] = lse2[s];
+                    y[u][k] = ndl[s];
+                }
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int k = 0; k < N; ++k)
+                    if (s0 + 1024 * u + k * THREADS < a.Sq) acc[k] = fmaf(fast_exp2(sink2 - x[u][k]), y[u][k], acc[k]);
+        }
     }
 #pragma unroll
     for (int k = 0; k < N; ++k) red[threadIdx.x + k * THREADS] = acc[k];
