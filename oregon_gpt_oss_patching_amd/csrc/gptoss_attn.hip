@@ -135,7 +135,7 @@ int dkdv_parts_for(const gptoss_attn_params *p, bool padded, bool packed) {
     const int64_t tiles = ((rows_seen < p->Sq ? rows_seen : p->Sq) + 63) / 64;
     int64_t parts = (1024 + blocks - 1) / blocks;
     if (blocks > 512) parts = p->Sq >= 4096 && (padded && p->B > 1 ? blocks / 2 : blocks) < 1024 ? 2 : 1;
-    if (packed && window == 0 && blocks >= 256 && blocks <= 1024 && parts < 4) parts = 3072 / blocks < 4 ? 3072 / blocks : 4;
+    if (packed && window == 0 && p->Sq >= 4096 && blocks >= 256 && blocks <= 1024 && parts < 4) parts = 3072 / blocks < 4 ? 3072 / blocks : 4;
     const int64_t steps = window > 0 ? tiles / 4 : tiles * (p->H / p->G) / 8;
     if (parts > steps) parts = steps;
     if (parts > tiles) parts = tiles;
