@@ -115,7 +115,7 @@ constexpr int kDkdvKeys = 32 * kDkdvNB * kDkdvWaves; // keys per dK/dV workgroup
 // right-padded batch counts half, because its shorter rows leave the longest one alone (dK/dV of B = 4, S = 4096,
 // lengths 3309 / 1968 / 1554 / 4079: 715 us uncut, 589 in two slices; B = 2, S = 8192 / 4000: 1437 and 1216; but B = 8,
 // S <= 2048: 359 and 370).  Packed rows: a walk ends with its document, so the longest document's first blocks stand out more, and
-// the host does not see the documents: up to four slices (layer, seven documents in 8192 tokens: 801 us in two, 759 in four; six in 12000:
+// the host does not see the documents: four slices up to 768 blocks of rows of 4096 keys and more (layer, seven documents in 8192 tokens: 801 us in two, 759 in four; six in 12000:
 // 1411 and 1385; 8192 tokens in ONE document: 2174 and 2192).
 int dkdv_parts_for(const gptoss_attn_params *p, bool padded, bool packed) {
     if (p->dtype == GPTOSS_ATTN_FP32) {
@@ -135,7 +135,7 @@ int dkdv_parts_for(const gptoss_attn_params *p, bool padded, bool packed) {
     const int64_t tiles = ((rows_seen < p->Sq ? rows_seen : p->Sq) + 63) / 64;
     int64_t parts = (1024 + blocks - 1) / blocks;
     if (blocks > 512) parts = p->Sq >= 4096 && (padded && p->B > 1 ? blocks / 2 : blocks) < 1024 ? 2 : 1;
-    if (packed && window == 0 && p->Sq >= 4096 && blocks >= 256 && blocks <= 1024 && parts < 4) parts = 3072 / blocks < 4 ? 3072 / blocks : 4;
+    if (packed && window == 0 && p->Sq >= 4096 && blocks >= 256 && blocks <= 768 && parts < 4) parts = 4;
     const int64_t steps = window > 0 ? tiles / 4 : tiles * (p->H / p->G) / 8;
     if (parts > steps) parts = steps;
     if (parts > tiles) parts = tiles;
