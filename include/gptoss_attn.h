@@ -148,8 +148,8 @@ const char *gptoss_attn_status_string(int status);
 size_t gptoss_attn_workspace_bytes(const gptoss_attn_params *params);
 
 /*
- * Bytes of scratch gptoss_attn_fwd can use for these shapes (0 for most): a few queries on a long key / value cache are
- * cut over the keys, and the slices leave fp32 partial results there.  Given through `delta` (16-byte aligned);
+ * Bytes of scratch gptoss_attn_fwd can use for these shapes (0 for most): few queries on a long key / value cache (a decoding step, a
+ * short piece of a prompt) are cut over the keys, and the slices leave fp32 partial results there.  Given through `delta` (16-byte aligned);
  * with delta == NULL the same kernel runs uncut.  Never more than gptoss_attn_workspace_bytes.  Host-only.
  */
 size_t gptoss_attn_fwd_workspace_bytes(const gptoss_attn_params *params);

@@ -69,6 +69,10 @@ __device__ __forceinline__ float sink_logit(const KArgs &a, int head) {
     if (!a.sinks) return 0.0f;
     return a.sinks_bf16 ? (float)static_cast<const bf16 *>(a.sinks)[head] : static_cast<const float *>(a.sinks)[head];
 }
+// The softmax reference starts at the sink logit.  A sink of -inf (none at all) must not start it at -inf: a slice or wavefront may hold
+// no key that a row sees, and -inf - (-inf) would make its share NaN.
+constexpr float kNoLogit = -1e30f;
+
 __device__ __forceinline__ void store_dsink(const KArgs &a, int head, float x) {
     if (a.dsinks_bf16) static_cast<bf16 *>(a.dsinks)[head] = (bf16)x;
     else static_cast<float *>(a.dsinks)[head] = x;

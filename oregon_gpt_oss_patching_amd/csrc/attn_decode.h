@@ -25,12 +25,8 @@ struct Decode {
     static constexpr int kCopies = 8;                              // copy instructions per tile
     static constexpr int kMaxPairs = 64;                           // (query, head) pairs per KV head
 };
-// scratch per (batch, KV head, split): the unnormalised output rows, then (m, l) per row
-__host__ __device__ inline int64_t decode_partial_floats(int pairs) { return (int64_t)pairs * (kD + 2); }
-
-// The softmax reference starts at the sink logit.  A sink of -inf (none at all) must not start it at -inf: a slice or wavefront may hold
-// no key that a row sees, and -inf - (-inf) would make its share NaN.
-constexpr float kNoLogit = -1e30f;
+// scratch per (batch, KV head, split): the unnormalised output rows, then (m, l) per row (a multiple of 16 bytes)
+__host__ __device__ inline int64_t decode_partial_floats(int pairs) { return ((int64_t)pairs * (kD + 2) + 3) & ~(int64_t)3; }
 
 template <int NQB>
 __global__ __launch_bounds__(256, 2) void attn_decode_kernel(const KArgs a) {

@@ -49,6 +49,10 @@ struct FwdPipe {
 // keys 181 -> 135 us; 2 x 3001 tokens 164 -> 160 us, 1 x 1000 33.6 -> 25.2, 2 x 383 16.1 -> 14.8; seven documents in 8192 tokens
 // 185 -> 180 (without letting the other documents' rows run along, every tile of such a workgroup being an exact
 // step: 230).
+// Few queries on a long cache leave most of the chip idle (100 queries on 4096 keys: 32 workgroups).  With kv_splits > 1 a query block's
+// key tiles are cut into that many consecutive shares, one workgroup each, which leave their unnormalised rows with (reference,
+// sum) in the scratch; attn_fwd_combine_kernel adds them in share order.  Each share freezes a reference of its own (100 queries on 4096 keys
+// of 64 heads: 62 -> 30 us, the sum included).
 template <bool GENERAL, bool DOCS = false>       // DOCS: packed documents (needs GENERAL)
 __global__ __launch_bounds__(256, 2) void attn_fwd_pipe_kernel(const KArgs a) {
     constexpr int NS = FwdPipe::NS;
@@ -67,6 +71,8 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_pipe_kernel(const KArgs a) {
     int bid = blockIdx.x;
     const int g = bid % a.G; bid /= a.G;
     const int hc = bid % n_hc; bid /= n_hc;
+    int split = 0;                                 // few query blocks: a share of the key tiles each (see attn_fwd_combine_kernel)
+    if constexpr (GENERAL && !DOCS) { split = bid % a.kv_splits; bid /= a.kv_splits; }
     const int bi = bid % a.B; bid /= a.B;
     const int b = rotated_batch_row(bi, bid, a.B);
     const int q_offset = GENERAL ? query_offset(a) : 0;
@@ -94,6 +100,14 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_pipe_kernel(const KArgs a) {
         t_hi = __builtin_amdgcn_readfirstlane(max(t_lo, (hi + kTile - 1) / kTile));
         if constexpr (DOCS) t_a = __builtin_amdgcn_ballot_w64(later) != 0ull ? t_hi : __builtin_amdgcn_readfirstlane((ds0 + kTile - 1) / kTile);
         t_b = __builtin_amdgcn_readfirstlane(min(pos0 + 1, kv_len) / kTile);
+        if constexpr (!DOCS) {
+            if (a.kv_splits > 1) {
+                const int n = t_hi;
+                t_lo = t_a = (int)((int64_t)n * split / a.kv_splits);
+                t_hi = (int)((int64_t)n * (split + 1) / a.kv_splits);
+                t_b = min(max(t_b, t_lo), t_hi);
+            }
+        }
     }
     const int n_it = t_hi - t_lo;
 
@@ -111,6 +125,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_pipe_kernel(const KArgs a) {
 
     const float c = a.scale_log2;
     const float sink2 = sink_logit(a, head) * kLog2e;
+    const float m_first = fast_max(sink2, kNoLogit);
     float m[2], l[2];
     f32x16 o[2][2];
 
@@ -148,7 +163,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_pipe_kernel(const KArgs a) {
         iss_left = n_req;
 #pragma unroll
         for (int qb = 0; qb < 2; ++qb) {
-            m[qb] = sink2;
+            m[qb] = m_first;
             l[qb] = 0.0f;
 #pragma unroll
             for (int i = 0; i < 16; ++i) { o[qb][0][i] = 0.0f; o[qb][1][i] = 0.0f; }
@@ -198,7 +213,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_pipe_kernel(const KArgs a) {
         // (also the state a workgroup without rows ends with: nothing requested, nothing attended)
 #pragma unroll
         for (int qb = 0; qb < 2; ++qb) {
-            m[qb] = sink2;
+            m[qb] = m_first;
             l[qb] = 0.0f;
 #pragma unroll
             for (int i = 0; i < 16; ++i) { o[qb][0][i] = 0.0f; o[qb][1][i] = 0.0f; }
@@ -376,7 +391,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_pipe_kernel(const KArgs a) {
     };
     // rows that do not exist: nothing attended, whatever the interior tiles made of them
     auto clear_rows = [&](int qb, bool dead_row) __attribute__((always_inline)) {
-        m[qb] = dead_row ? sink2 : m[qb];
+        m[qb] = dead_row ? m_first : m[qb];
         l[qb] = dead_row ? 0.0f : l[qb];
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
@@ -489,6 +504,28 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_pipe_kernel(const KArgs a) {
 #pragma unroll
     for (int qb = 0; qb < 2; ++qb) {
         const float l_tot = l[qb] + __shfl_xor(l[qb], 32);
+        if constexpr (GENERAL && !DOCS) {
+            if (a.kv_splits > 1) {
+                // this share's unnormalised rows and their (reference, sum); lane = row, four consecutive columns per store
+                const int row = qw0 + 32 * qb + l32_b;
+                if (row < a.Sq) {
+                    const int64_t rows = (int64_t)a.B * a.H * a.Sq, rid = ((int64_t)b * a.H + head) * a.Sq + row;
+                    float *part = a.fwd_partial + ((int64_t)split * rows + rid) * kD;
+#pragma unroll
+                    for (int dblk = 0; dblk < 2; ++dblk)
+#pragma unroll
+                        for (int a4 = 0; a4 < 4; ++a4)
+                            *reinterpret_cast<f32x4 *>(part + 32 * dblk + 8 * a4 + 4 * half_b) =
+                                f32x4{o[qb][dblk][4 * a4], o[qb][dblk][4 * a4 + 1], o[qb][dblk][4 * a4 + 2], o[qb][dblk][4 * a4 + 3]};
+                    if (half_b == 0) {
+                        float *ml = a.fwd_partial + (int64_t)a.kv_splits * rows * kD + 2 * ((int64_t)split * rows + rid);
+                        ml[0] = m[qb];
+                        ml[1] = l_tot;
+                    }
+                }
+                continue;
+            }
+        }
         const float z = l_tot + fast_exp2(sink2 - m[qb]);
         const float inv = 1.0f / z;
         const int r0 = qw0 + 32 * qb;
@@ -497,6 +534,36 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_pipe_kernel(const KArgs a) {
         __builtin_amdgcn_wave_barrier();
         if (half_b == 0 && (!GENERAL || r0 + l32_b < a.Sq)) a.lse[((int64_t)b * a.H + head) * a.Sq + r0 + l32_b] = (m[qb] + fast_log2(z)) * kLn2;
     }
+}
+
+// The shares of a row's keys, added in their order: eight lanes per row, eight columns each.
+__global__ __launch_bounds__(256) void attn_fwd_combine_kernel(const KArgs a) {
+    const int64_t rows = (int64_t)a.B * a.H * a.Sq, rid = (int64_t)blockIdx.x * 32 + (threadIdx.x >> 3);
+    if (rid >= rows) return;
+    const int c8 = (threadIdx.x & 7) * 8;
+    const int s_ = (int)(rid % a.Sq);
+    const int bh = (int)(rid / a.Sq), h = bh % a.H, b = bh / a.H;
+    const float sink2 = sink_logit(a, h) * kLog2e;
+    const float *ml = a.fwd_partial + (int64_t)a.kv_splits * rows * kD + 2 * rid;
+    float mm = fast_max(sink2, kNoLogit);
+    for (int i = 0; i < a.kv_splits; ++i) mm = fast_max(mm, ml[2 * rows * i]);
+    float z = fast_exp2(sink2 - mm), acc[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[e] = 0.0f;
+    for (int i = 0; i < a.kv_splits; ++i) {
+        const float f = fast_exp2(ml[2 * rows * i] - mm);
+        z = fmaf(f, ml[2 * rows * i + 1], z);
+        const float *p = a.fwd_partial + ((int64_t)i * rows + rid) * kD + c8;
+        const f32x4 x = *reinterpret_cast<const f32x4 *>(p), y = *reinterpret_cast<const f32x4 *>(p + 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { acc[e] = fmaf(f, x[e], acc[e]); acc[4 + e] = fmaf(f, y[e], acc[4 + e]); }
+    }
+    const float inv = 1.0f / z;
+    union { bf16x8 v; u32x4 u; } out;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) out.v[e] = (bf16)(acc[e] * inv);
+    *reinterpret_cast<u32x4 *>(a.o + (int64_t)b * a.os.b + (int64_t)h * a.os.h + (int64_t)s_ * a.os.s + c8) = out.u;
+    if (c8 == 0) a.lse[rid] = (mm + fast_log2(z)) * kLn2;
 }
 
 }  // namespace gptoss

@@ -174,6 +174,21 @@ bool fwd_pipe_plain(const gptoss_attn_params *p) {
     return p->Sq == p->Skv && p->Sq % kTile == 0 && !p->seqlens && !p->doc_start && p->q_offset == 0 && !p->q_offset_dev;
 }
 
+// Shares of the keys per query block where new queries on a cache (fewer queries than keys, no packing) are too few to fill the chip: two
+// workgroups per compute unit of a 256-CU part, at least eight tiles each.  From the shapes alone, so that the scratch does not
+// depend on where the queries stand.  64 query heads on 8 KV heads: 100 queries on 4096 keys 62 -> 30 us, 300 on 12000 167 -> 82
+// (four tiles each: 37 us and 83); 8 heads on one KV head: 300 on 12000 164 -> 34 (more than sixteen shares: 36), 1000 on 17000 231 -> 57.
+// Two shares are not worth the sum: 1024 on 8192 134 -> 137.
+int fwd_pipe_splits(const gptoss_attn_params *p) {
+    if (p->Skv <= p->Sq) return 1;
+    const int64_t wgs = (int64_t)p->G * (p->H / p->G / 4) * p->B * ((p->Sq + kTile - 1) / kTile);
+    const int64_t tiles = (p->Skv + kTile - 1) / kTile;
+    int64_t n = 512 / wgs;
+    if (n > tiles / 8) n = tiles / 8;
+    if (n > 16) n = 16;
+    return n < 3 ? 1 : (int)n;
+}
+
 // The one-pass forward of sliding-window layers (attn_fwd_window.h): a window of 32, 64, 96 or 128 keys, all four wavefronts of
 // a workgroup with a head of their own.  Self-attention of whole 32-row blocks without packing has an instantiation of its own.
 bool fwd_window_route(const gptoss_attn_params *p) {
@@ -441,6 +456,10 @@ size_t gptoss_attn_fwd_workspace_bytes(const gptoss_attn_params *p) {
     if (decode_route(p)) {
         const int splits = decode_splits(p);
         if (splits > 1) return (size_t)p->B * p->G * splits * decode_partial_floats(p->Sq * (p->H / p->G)) * sizeof(float);
+    } else if (p->dtype == GPTOSS_ATTN_BF16 && (p->window <= 0 || p->window >= p->Sq) && (p->H / p->G) % 4 == 0 && p->Skv >= kTile) {
+        // (a window that covers the whole row is none; where the queries stand may not be known yet)
+        const int splits = fwd_pipe_splits(p);
+        if (splits > 1) return (size_t)splits * p->B * p->H * p->Sq * (kD + 2) * sizeof(float);
     }
     return 0;
 }
@@ -499,10 +518,18 @@ static int forward(const gptoss_attn_params *p, void *stream, SinkTypes ty) {
         }
 #undef GPTOSS_LAUNCH_WIN
     }
-    if (fwd_pipe_route(p)) 
+    if (fwd_pipe_route(p)) {
+        const int splits = p->delta && !a.doc_start ? fwd_pipe_splits(p) : 1;
+        if (splits > 1) {
+            a.kv_splits = splits;
+            a.fwd_partial = p->delta;
+            const int s = launch(attn_fwd_pipe_kernel<true, false>, grid * splits, 256, st, a);
+            return s ? s : launch(attn_fwd_combine_kernel, ((int64_t)a.B * a.H * a.Sq + 31) / 32, 256, st, a);
+        }
         return fwd_pipe_plain(p) ? launch(attn_fwd_pipe_kernel<false, false>, grid, 256, st, a)
                : a.doc_start     ? launch(attn_fwd_pipe_kernel<true, true>, grid, 256, st, a)
                                  : launch(attn_fwd_pipe_kernel<true, false>, grid, 256, st, a);
+    }
 #define GPTOSS_LAUNCH_FWD(HPB, QB) launch(attn_fwd_kernel<HPB, QB>, grid, 256, st, a)
     if (qb == 2) return hpb == 4 ? GPTOSS_LAUNCH_FWD(4, 2) : hpb == 2 ? GPTOSS_LAUNCH_FWD(2, 2) : GPTOSS_LAUNCH_FWD(1, 2);
     return hpb == 4 ? GPTOSS_LAUNCH_FWD(4, 1) : hpb == 2 ? GPTOSS_LAUNCH_FWD(2, 1) : GPTOSS_LAUNCH_FWD(1, 1);
