@@ -5,14 +5,16 @@
 // a decoding step is 2 G B workgroups, each walking the whole cache tile by tile, and every K / V row is staged twice.
 //
 // Work split.  The Sq * r (query, head of the group) pairs of a KV head are the columns of one S^T block (two for up to 64
-// pairs), so K and V are read once.  The keys are cut over `kv_splits` workgroups of four wavefronts; inside a workgroup
+// pairs), so K and V are read once.  The keys are cut over `kv_splits` workgroups of four wavefronts, or walked by one of eight (NW) where
+// they are so few that the second launch costs more; inside a workgroup
 // the wavefronts take 32-key tiles in turn, each through LDS stages of its own (no barrier in the loop, NS tiles in
 // flight per wavefront), and merge their (m, l, O) at the end.  With one split the workgroup writes O and lse;
 // otherwise it leaves fp32 partials in the scratch and attn_decode_combine_kernel adds them in an order that depends on
 // their number only.
 //
 // Measured (64 query heads on 8 KV heads, one query, MI355X): B = 16 on 8192 keys 246 us with attn_fwd_kernel, 42 + 4 us
-// here (268 MB: 6.3 TB/s, a plain 4 GiB copy moves 4.7); B = 1 on 2049 keys 57 us, 5.4 + 4.2 us here (launch latencies).
+// here (268 MB: 6.3 TB/s, a plain 4 GiB copy moves 4.7); B = 1 on 2049 keys 57 us,
+// 5.4 + 4.2 us here (launch latencies); on 1024 keys a call takes 12.4 us in slices and 11.1 in one launch.
 #pragma once
 #include "attn_common.h"
 
@@ -28,12 +30,17 @@ struct Decode {
 // scratch per (batch, KV head, split): the unnormalised output rows, then (m, l) per row (a multiple of 16 bytes)
 __host__ __device__ inline int64_t decode_partial_floats(int pairs) { return ((int64_t)pairs * (kD + 2) + 3) & ~(int64_t)3; }
 
-template <int NQB>
-__global__ __launch_bounds__(256, 2) void attn_decode_kernel(const KArgs a) {
+// Bytes of LDS of a workgroup of NW wavefronts: their stages, later their results.
+template <int NQB, int NW>
+constexpr int decode_lds_bytes() {
+    constexpr int merge = NW * 32 * NQB * (kD + 2) * 4, stages = NW * Decode::NS * Decode::kTileBytes;
+    return stages > merge ? stages : merge;
+}
+
+template <int NQB, int NW>
+__global__ __launch_bounds__(64 * NW, 2) void attn_decode_kernel(const KArgs a) {
     using C = Decode;
-    constexpr int kMergeBytes = 4 * 32 * NQB * (kD + 2) * 4;
-    constexpr int kLds = 4 * C::NS * C::kTileBytes > kMergeBytes ? 4 * C::NS * C::kTileBytes : kMergeBytes;
-    __shared__ __attribute__((aligned(16))) char smem[kLds];
+    extern __shared__ __attribute__((aligned(1024))) char smem[];
 
     const int q_offset = query_offset(a);
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -53,7 +60,7 @@ __global__ __launch_bounds__(256, 2) void attn_decode_kernel(const KArgs a) {
     const int n_all = max(0, (hi + C::kKeys - 1) / C::kKeys - t_first);
     const int t_lo = t_first + (int)((int64_t)n_all * split / a.kv_splits);
     const int n_wg = t_first + (int)((int64_t)n_all * (split + 1) / a.kv_splits) - t_lo;
-    const int n_it = (n_wg - w + 3) >> 2;                          // this wavefront's tiles: t_lo + w + 4 j  (0 if n_wg <= w)
+    const int n_it = n_wg > w ? (n_wg - w + NW - 1) / NW : 0;      // this wavefront's tiles: t_lo + w + NW j
 
     // columns: pair 32 qb + l32 = (query row, head of the group)
     bf16x8 qf[NQB][4];
@@ -81,7 +88,7 @@ __global__ __launch_bounds__(256, 2) void attn_decode_kernel(const KArgs a) {
     const uint32_t stage0 = lds_addr(smem) + w * (C::NS * C::kTileBytes);
     const bf16 *kbase = a.k + (int64_t)b * a.ks.b + (int64_t)g * a.ks.h, *vbase = a.v + (int64_t)b * a.vs.b + (int64_t)g * a.vs.h;
     auto issue = [&](int j) __attribute__((always_inline)) {
-        const int n0 = (t_lo + w + 4 * j) * C::kKeys;
+        const int n0 = (t_lo + w + NW * j) * C::kKeys;
         const uint32_t dst = stage0 + (j % C::NS) * C::kTileBytes;
         const bf16 *kt = kbase + (int64_t)n0 * a.ks.s, *vt = vbase + (int64_t)n0 * a.vs.s;
         const int last = a.Skv - 1 - n0;
@@ -105,7 +112,7 @@ __global__ __launch_bounds__(256, 2) void attn_decode_kernel(const KArgs a) {
         } else {
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         }
-        const int n0 = (t_lo + w + 4 * j) * C::kKeys;
+        const int n0 = (t_lo + w + NW * j) * C::kKeys;
         const uint32_t ksm = stage0 + (j % C::NS) * C::kTileBytes, vsm = ksm + C::kKeys * kRowBytes;
         const bool interior = n0 + C::kKeys - 1 <= pos0 && n0 > pos1 - weff && n0 + C::kKeys <= kv_len && pos1 < q_len;
         f32x16 s[NQB];
@@ -159,7 +166,7 @@ __global__ __launch_bounds__(256, 2) void attn_decode_kernel(const KArgs a) {
             }
     }
 
-    // ---- merge the four wavefronts: rows [wavefront][pair][64 + (m, l)] in LDS ----
+    // ---- merge the wavefronts: rows [wavefront][pair][64 + (m, l)] in LDS ----
     __syncthreads();
     constexpr int kRow = kD + 2, kWave = 32 * NQB * kRow;
     float *red = reinterpret_cast<float *>(smem);
@@ -176,15 +183,17 @@ __global__ __launch_bounds__(256, 2) void attn_decode_kernel(const KArgs a) {
     __syncthreads();
     // eight lanes per row, eight columns each
     const int c8 = (tid & 7) * 8;
-    for (int pair = tid >> 3; pair < pairs; pair += 32) {
-        float mw[4], lw = 0.0f, acc[8], mm;
+    for (int pair = tid >> 3; pair < pairs; pair += 8 * NW) {
+        float mw[NW], lw = 0.0f, acc[8], mm;
 #pragma unroll
-        for (int k = 0; k < 4; ++k) mw[k] = red[k * kWave + pair * kRow + kD];
-        mm = fast_max(fast_max(mw[0], mw[1]), fast_max(mw[2], mw[3]));
+        for (int k = 0; k < NW; ++k) mw[k] = red[k * kWave + pair * kRow + kD];
+        mm = mw[0];
+#pragma unroll
+        for (int k = 1; k < NW; ++k) mm = fast_max(mm, mw[k]);
 #pragma unroll
         for (int e = 0; e < 8; ++e) acc[e] = 0.0f;
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
+        for (int k = 0; k < NW; ++k) {
             const float f = fast_exp2(mw[k] - mm);
             const float *row = red + k * kWave + pair * kRow;
             lw += f * row[kD + 1];

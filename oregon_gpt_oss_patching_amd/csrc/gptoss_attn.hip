@@ -207,10 +207,23 @@ bool fwd_window_plain(const gptoss_attn_params *p) {
 bool decode_route(const gptoss_attn_params *p) {
     return p->dtype == GPTOSS_ATTN_BF16 && !p->doc_start && (int64_t)p->Sq * (p->H / p->G) <= Decode::kMaxPairs;
 }
+int64_t decode_keys(const gptoss_attn_params *p) {
+    return p->window > 0 && (int64_t)p->window + p->Sq < p->Skv ? (int64_t)p->window + p->Sq : p->Skv;
+}
+// The keys of a KV head walked by one workgroup of eight wavefronts, no slices to add and one launch less.  Where the cache comes from HBM
+// (us a call, sliced / whole, 8 query heads per KV head), B G = 8: 257 keys 12.5 / 10.6, 1024 12.4 / 11.1, 1500 12.4 / 13.6, 2049 12.4 / 16.7;
+// B G = 128: 1024 14.1 / 13.0, 2049 20.9 / 20.1, 4096 32.8 / 34.3, 8192 55.7 / 65.5; B G = 256: 1000 20.1 / 17.1; two column blocks, B G = 8: 600 12.6 / 11.7, 1000
+// 12.6 / 14.6.  (A cache that is still in the last-level cache moves the line up to 3000 keys, but a decoding step reads all layers'
+// weights between two calls on one cache.)  512 groups fill the chip unsliced.
+bool decode_whole(const gptoss_attn_params *p) {
+    const int64_t groups = (int64_t)p->B * p->G, pairs = (int64_t)p->Sq * (p->H / p->G);
+    return groups < 512 && decode_keys(p) <= (pairs > 32 ? 640 : 1024);
+}
 // Slices of the keys: about two workgroups per compute unit of a 256-CU part (so that the scratch does not depend on the
 // device), each wavefront of a slice with a tile of its own at least.
 int decode_splits(const gptoss_attn_params *p) {
-    const int64_t keys = p->window > 0 && (int64_t)p->window + p->Sq < p->Skv ? (int64_t)p->window + p->Sq : p->Skv;
+    if (decode_whole(p)) return 1;
+    const int64_t keys = decode_keys(p);
     const int64_t groups = (int64_t)p->B * p->G;
     int64_t n = (512 + groups - 1) / groups;
     const int64_t most = keys / (4 * Decode::kKeys);
@@ -307,15 +320,15 @@ int window_chunk_tiles(const gptoss_attn_params *p, int cus) {
 }
 
 // A kernel that uses more than 64 KB of LDS has to be told so once per device.
-int window_lds_attribute() {
+template <auto Kernel>
+int lds_attribute(int bytes) {
     static std::atomic<bool> done[kMaxDevices];
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return static_cast<int>(e);
     const bool tracked = dev >= 0 && dev < kMaxDevices;
     if (!tracked || !done[dev].load(std::memory_order_acquire)) {
-        e = hipFuncSetAttribute(reinterpret_cast<const void *>(attn_bwd_window_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                WinCfg::kLdsBytes);
+        e = hipFuncSetAttribute(reinterpret_cast<const void *>(Kernel), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
         if (e != hipSuccess) return static_cast<int>(e);
         if (tracked) done[dev].store(true, std::memory_order_release);
     }
@@ -341,7 +354,7 @@ WindowScratch window_scratch(const gptoss_attn_params *p, int cus) { return wind
 // seam_sums: neighbouring chunks exchange fp32 shares through the scratch (needs window_scratch bytes);
 // otherwise each chunk walks two query tiles past its end and nothing but the dSinks sums is kept.
 int launch_window_bwd(const gptoss_attn_params *p, hipStream_t st, bool seam_sums, SinkTypes ty) {
-    int rc = window_lds_attribute();
+    int rc = lds_attribute<&attn_bwd_window_kernel>(WinCfg::kLdsBytes);
     if (rc) return rc;
     KArgs a = make_args(p, ty);
     const WindowScratch ws = window_scratch(p, compute_units());
@@ -361,6 +374,13 @@ int launch_window_bwd(const gptoss_attn_params *p, hipStream_t st, bool seam_sum
     const hipError_t e = hipLaunchKernel(reinterpret_cast<const void *>(attn_bwd_window_finish_kernel),
                                          dim3((unsigned)(seam_blocks + sink_blocks)), dim3(256), args, 0, st);
     return e == hipSuccess ? GPTOSS_ATTN_OK : static_cast<int>(e);
+}
+
+template <int NQB, int NW>
+int launch_decode(int64_t workgroups, hipStream_t st, const KArgs &a) {
+    constexpr int lds = decode_lds_bytes<NQB, NW>();
+    const int rc = lds > 64 * 1024 ? lds_attribute<&attn_decode_kernel<NQB, NW>>(lds) : GPTOSS_ATTN_OK;
+    return rc ? rc : launch(attn_decode_kernel<NQB, NW>, workgroups, 64 * NW, st, a, lds);
 }
 
 // workgroups of the forward / dQ launch: (KV head, chunk of HPB query heads, batch, query tile)
@@ -491,7 +511,8 @@ static int forward(const gptoss_attn_params *p, void *stream, SinkTypes ty) {
         if (p->delta) { a.kv_splits = decode_splits(p); a.fwd_partial = p->delta; }
         const int pairs = a.Sq * a.r;
         const int64_t wgs = (int64_t)a.G * a.B * a.kv_splits;
-        const int s = pairs <= 32 ? launch(attn_decode_kernel<1>, wgs, 256, st, a) : launch(attn_decode_kernel<2>, wgs, 256, st, a);
+        if (decode_whole(p)) return pairs <= 32 ? launch_decode<1, 8>(wgs, st, a) : launch_decode<2, 8>(wgs, st, a);
+        const int s = pairs <= 32 ? launch_decode<1, 4>(wgs, st, a) : launch_decode<2, 4>(wgs, st, a);
         if (s || a.kv_splits == 1) return s;
         return launch(attn_decode_combine_kernel, ((int64_t)a.B * a.G * pairs + 3) / 4, 256, st, a);
     }

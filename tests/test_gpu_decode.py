@@ -32,6 +32,13 @@ def A():
     (2, 8, 2, 2, 640, 126, None, None),
     (3, 8, 2, 2, 900, 700, None, [900, 701, 5]),   # padded rows: whole, a dead second query, dead altogether
     (1, 8, 2, 8, 8, 0, None, None),                # self-attention of eight tokens
+    (1, 8, 1, 1, 1024, 1023, None, None),          # the most keys one workgroup walks alone, and one more
+    (1, 8, 1, 1, 1025, 1024, None, None),
+    (1, 8, 1, 1, 257, 256, None, None),            # nine tiles of eight wavefronts, the last of one key
+    (1, 8, 1, 8, 640, 632, None, None),            # 64 pairs, unsliced and sliced
+    (1, 8, 1, 8, 641, 633, None, None),
+    (130, 8, 4, 1, 300, 299, None, None),          # 520 KV heads: four wavefronts, unsliced
+    (4, 8, 1, 1, 40000, 39999, 128, None),         # a window at the end of a long cache, unsliced
 ])
 @pytest.mark.parametrize("on_device", [False, True])
 def test_decode_vs_eager_oracle(A, b, h, g, sq, skv, start, w, lens, on_device):
