@@ -162,7 +162,7 @@ def doc_start_from_position_ids(position_ids: torch.Tensor) -> torch.Tensor:
     a new document begins wherever the position does not follow its predecessor by one."""
     pos = position_ids
     b, s = pos.shape
-    if pos.is_cuda and pos.dtype in (torch.int64, torch.int32):
+    if pos.is_cuda and pos.dtype in (torch.int64, torch.int32) and b <= 65535:      # (one grid row per batch row)
         if not _ops_ready:
             _register_ops()
         return torch.ops.gptoss_attn.doc_start.default(pos)
