@@ -235,7 +235,7 @@ __global__ __launch_bounds__(256, 2) void attn_f32_fwd_kernel(const KArgs a) {
     const F32Offsets lo = make_f32_offsets(lane);
     const float c = a.scale_log2;
     const float sink2 = sink_logit(a, wk.head) * kLog2e;
-    float m = sink2, l = 0.0f;
+    float m = fast_max(sink2, kNoLogit), l = 0.0f;
     f32x16 o[2];
 #pragma unroll
     for (int i = 0; i < 16; ++i) { o[0][i] = 0.0f; o[1][i] = 0.0f; }
@@ -294,7 +294,7 @@ __global__ __launch_bounds__(256, 2) void attn_f32_fwd_kernel(const KArgs a) {
         const int i = pass >> 1, r = (threadIdx.x >> 4) + 16 * (pass & 1), ch = threadIdx.x & 15;
         const F32Unit u = W::unit(a, i);
         const float sink = sink_logit(a, u.head) * kLog2e;
-        float mm = sink;
+        float mm = fast_max(sink, kNoLogit);
 #pragma unroll
         for (int k = 0; k < KS; ++k) mm = fast_max(mm, ml[2 * (KS * i + k) * 32 + r]);
         float z = fast_exp2(sink - mm);
