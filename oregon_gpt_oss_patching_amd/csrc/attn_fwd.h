@@ -294,7 +294,7 @@ __global__ __launch_bounds__(256, (NQB == 1 ? 3 : 2)) void attn_fwd_kernel(const
         next_row0 = t_lo * kTile;
 #pragma unroll
         for (int qb = 0; qb < NQB; ++qb) {
-            m[qb] = sink2;
+            m[qb] = fast_max(sink2, kNoLogit);
             l[qb] = 0.0f;
 #pragma unroll
             for (int i = 0; i < 16; ++i) { o[qb][0][i] = 0.0f; o[qb][1][i] = 0.0f; }

@@ -1,4 +1,5 @@
-"""GPU tests of sink logits of -inf (no sink: the plain softmax) where a wavefront or a row's first tile holds no key that the row sees."""
+"""GPU tests of sink logits of -inf (no sink: the plain softmax) where a wavefront or a row's first tile holds no key that the row sees:
+float32 rows shared by several wavefronts, and the general bf16 forward."""
 import pytest
 import torch
 
@@ -39,3 +40,15 @@ def test_float32_without_sink(A, h, g, sq, skv, start, w, docs):
     assert torch.isfinite(o).all()
     assert float((o.cpu().double() - ref).norm()) <= 2e-5 * float(ref.norm())
     assert float((lse.cpu().double() - ref_lse).abs().max()) <= 2e-5
+
+
+@pytest.mark.parametrize("h,g,sq,skv,start,w,docs", [
+    (8, 2, 300, 300, 0, 100, None),             # a window that is no multiple of 32
+    (8, 2, 300, 300, 0, 200, None),
+    (6, 2, 200, 200, 0, None, [70, 1, 100, 29]),
+    (6, 2, 90, 400, 310, 2000, None),
+])
+def test_general_forward_without_sink(A, h, g, sq, skv, start, w, docs):
+    o, lse, ref, ref_lse = _no_sink(A, torch.bfloat16, h, g, sq, skv, start, w, docs)
+    TP.check("o", o, ref.float())
+    assert float((lse.cpu().double() - ref_lse).abs().max()) <= TP.LSE_TOL
