@@ -472,7 +472,8 @@ static size_t partials_bytes(const gptoss_attn_params *p) {
 }
 
 size_t gptoss_attn_fwd_workspace_bytes(const gptoss_attn_params *p) {
-    if (!p || p->B <= 0 || p->H <= 0 || p->G <= 0 || p->Sq <= 0 || p->Skv <= 0) return 0;
+    // (asked before anything has looked at the shapes: heads the forward will refuse would divide by zero below)
+    if (!p || p->B <= 0 || p->H <= 0 || p->G <= 0 || p->H % p->G || p->Sq <= 0 || p->Skv <= 0) return 0;
     if (decode_route(p)) {
         const int splits = decode_splits(p);
         if (splits > 1) return (size_t)p->B * p->G * splits * decode_partial_floats(p->Sq * (p->H / p->G)) * sizeof(float);
