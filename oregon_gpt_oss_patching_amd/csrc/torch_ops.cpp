@@ -22,6 +22,7 @@ namespace {
 
 using at::Tensor;
 using OptTensor = std::optional<Tensor>;
+using c10::SymInt;
 
 constexpr int64_t kMaxSeqStride = int64_t(1) << 24;   // elements; the library refuses larger sequence strides (ERR_STRIDE)
 
@@ -39,13 +40,19 @@ void require_on(const Tensor &q, const char *name, const Tensor &t) {
     TORCH_CHECK(t.device() == q.device(), name, " is on ", t.device(), " but q is on ", q.device(), ": every tensor must be on q's GPU");
 }
 
-void check_inputs(const Tensor &q, const Tensor &k, const Tensor &v, const OptTensor &sinks, bool allow_cast) {
+// What can be looked at without a size (a traced call's sizes are symbols, and reading one as a number would tie the traced
+// program to it).
+void check_kinds(const Tensor &q, const Tensor &k, const Tensor &v, bool allow_cast) {
     TORCH_CHECK(q.is_cuda() && k.is_cuda() && v.is_cuda(), "gptoss attention runs on the GPU only (HIP kernels); got a CPU tensor");
     const auto dt = q.scalar_type();
     const bool ok = dt == at::kBFloat16 || dt == at::kFloat || (allow_cast && dt == at::kHalf);
     TORCH_CHECK(ok && k.scalar_type() == dt && v.scalar_type() == dt, "unsupported dtypes ", dt, "/", k.scalar_type(), "/", v.scalar_type(),
                 ": q, k, v must all be bfloat16 or all be float32");
     TORCH_CHECK(q.dim() == 4 && k.dim() == 4 && v.dim() == 4, "q must be (B,H,S,D) and k, v (B,G,S_kv,D)");
+}
+
+void check_inputs(const Tensor &q, const Tensor &k, const Tensor &v, const OptTensor &sinks) {
+    check_kinds(q, k, v, false);
     TORCH_CHECK(k.sizes() == v.sizes() && q.size(0) == k.size(0) && q.size(3) == k.size(3), "shape mismatch: q ", q.sizes(), ", k ", k.sizes(),
                 ", v ", v.sizes());
     if (sinks) {
@@ -71,7 +78,7 @@ struct Call {
 
 void fill(Call &c, const Tensor &q, const Tensor &k, const Tensor &v, const OptTensor &sinks, double sm_scale, int64_t window, int64_t q_offset,
           const OptTensor &seqlens, const OptTensor &doc_start, const OptTensor &q_offset_dev) {
-    check_inputs(q, k, v, sinks, false);
+    check_inputs(q, k, v, sinks);
     c.q = row_contiguous(q, 2);
     c.k = row_contiguous(k, 2);
     c.v = row_contiguous(v, 2);
@@ -186,16 +193,16 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> bwd(const Tensor &q, const Tensor &k,
 }
 
 // The two operators through the dispatcher (tracing modes see them).
-std::tuple<Tensor, Tensor> call_fwd(const Tensor &q, const Tensor &k, const Tensor &v, const OptTensor &sinks, double sm_scale, int64_t window,
-                                    int64_t q_offset, const OptTensor &seqlens, const OptTensor &doc_start, const OptTensor &q_offset_dev) {
-    static const auto op = c10::Dispatcher::singleton().findSchemaOrThrow("gptoss_attn::fwd", "").typed<decltype(fwd)>();
+std::tuple<Tensor, Tensor> call_fwd(const Tensor &q, const Tensor &k, const Tensor &v, const OptTensor &sinks, double sm_scale, SymInt window,
+                                    SymInt q_offset, const OptTensor &seqlens, const OptTensor &doc_start, const OptTensor &q_offset_dev) {
+    static const auto op = c10::Dispatcher::singleton().findSchemaOrThrow("gptoss_attn::fwd", "").typed<decltype(call_fwd)>();
     return op.call(q, k, v, sinks, sm_scale, window, q_offset, seqlens, doc_start, q_offset_dev);
 }
 std::tuple<Tensor, Tensor, Tensor, Tensor> call_bwd(const Tensor &q, const Tensor &k, const Tensor &v, const OptTensor &sinks, const Tensor &o,
-                                                    const Tensor &lse, const Tensor &d_o, double sm_scale, int64_t window, int64_t q_offset,
+                                                    const Tensor &lse, const Tensor &d_o, double sm_scale, SymInt window, SymInt q_offset,
                                                     const OptTensor &seqlens, const OptTensor &doc_start, bool need_dsinks,
                                                     const OptTensor &q_offset_dev, bool dsinks_as_sinks) {
-    static const auto op = c10::Dispatcher::singleton().findSchemaOrThrow("gptoss_attn::bwd", "").typed<decltype(bwd)>();
+    static const auto op = c10::Dispatcher::singleton().findSchemaOrThrow("gptoss_attn::bwd", "").typed<decltype(call_bwd)>();
     return op.call(q, k, v, sinks, o, lse, d_o, sm_scale, window, q_offset, seqlens, doc_start, need_dsinks, q_offset_dev, dsinks_as_sinks);
 }
 
@@ -205,7 +212,7 @@ Tensor tensor_of(const OptTensor &t) { return t ? *t : Tensor(); }
 // float16 tensors are rounded to bfloat16 on the way in and the results cast back.
 struct AttentionFunction : public torch::autograd::Function<AttentionFunction> {
     static Tensor forward(torch::autograd::AutogradContext *ctx, const Tensor &q_, const Tensor &k_, const Tensor &v_, const OptTensor &sinks,
-                          double sm_scale, int64_t window, int64_t q_offset, const OptTensor &seqlens, const OptTensor &doc_start,
+                          double sm_scale, SymInt window, SymInt q_offset, const OptTensor &seqlens, const OptTensor &doc_start,
                           const OptTensor &q_offset_dev) {
         const at::AutoDispatchBelowADInplaceOrView below;
         const auto dtype = q_.scalar_type();
@@ -236,8 +243,8 @@ struct AttentionFunction : public torch::autograd::Function<AttentionFunction> {
         std::optional<at::AutoDispatchBelowADInplaceOrView> below;
         if (!at::GradMode::is_enabled()) below.emplace();
         auto [dq, dk, dv, dsinks] = call_bwd(q, saved[1], saved[2], optional_of(sinks), saved[4], saved[5], grads[0].to(q.scalar_type()),
-                                             ctx->saved_data["sm_scale"].toDouble(), ctx->saved_data["window"].toInt(),
-                                             ctx->saved_data["q_offset"].toInt(), optional_of(saved[6]), optional_of(saved[7]), need_dsinks,
+                                             ctx->saved_data["sm_scale"].toDouble(), ctx->saved_data["window"].toSymInt(),
+                                             ctx->saved_data["q_offset"].toSymInt(), optional_of(saved[6]), optional_of(saved[7]), need_dsinks,
                                              optional_of(saved[8]), true);
         if (half) {
             dq = dq.to(at::kHalf);
@@ -248,9 +255,9 @@ struct AttentionFunction : public torch::autograd::Function<AttentionFunction> {
     }
 };
 
-Tensor attention(const Tensor &q, const Tensor &k, const Tensor &v, const OptTensor &sinks, double sm_scale, int64_t window, int64_t q_offset,
+Tensor attention(const Tensor &q, const Tensor &k, const Tensor &v, const OptTensor &sinks, double sm_scale, SymInt window, SymInt q_offset,
                  const OptTensor &seqlens, const OptTensor &doc_start, const OptTensor &q_offset_dev) {
-    check_inputs(q, k, v, sinks, true);
+    check_kinds(q, k, v, true);        // (the shapes: gptoss_attn::fwd)
     return AttentionFunction::apply(q, k, v, sinks, sm_scale, window, q_offset, seqlens, doc_start, q_offset_dev);
 }
 
@@ -272,12 +279,12 @@ Tensor doc_start(const Tensor &position_ids_) {
 }  // namespace
 
 TORCH_LIBRARY(gptoss_attn, m) {
-    m.def("fwd(Tensor q, Tensor k, Tensor v, Tensor? sinks, float sm_scale, int window, int q_offset, Tensor? seqlens, Tensor? doc_start, "
+    m.def("fwd(Tensor q, Tensor k, Tensor v, Tensor? sinks, float sm_scale, SymInt window, SymInt q_offset, Tensor? seqlens, Tensor? doc_start, "
           "Tensor? q_offset_dev=None) -> (Tensor, Tensor)");
-    m.def("bwd(Tensor q, Tensor k, Tensor v, Tensor? sinks, Tensor o, Tensor lse, Tensor d_o, float sm_scale, int window, int q_offset, "
+    m.def("bwd(Tensor q, Tensor k, Tensor v, Tensor? sinks, Tensor o, Tensor lse, Tensor d_o, float sm_scale, SymInt window, SymInt q_offset, "
           "Tensor? seqlens, Tensor? doc_start, bool need_dsinks, Tensor? q_offset_dev=None, bool dsinks_as_sinks=False) -> (Tensor, Tensor, Tensor, Tensor)");
     m.def("doc_start(Tensor position_ids) -> Tensor");
-    m.def("attention(Tensor q, Tensor k, Tensor v, Tensor? sinks, float sm_scale, int window, int q_offset, Tensor? seqlens, Tensor? doc_start, "
+    m.def("attention(Tensor q, Tensor k, Tensor v, Tensor? sinks, float sm_scale, SymInt window, SymInt q_offset, Tensor? seqlens, Tensor? doc_start, "
           "Tensor? q_offset_dev=None) -> Tensor", &attention);
 }
 TORCH_LIBRARY_IMPL(gptoss_attn, CUDA, m) {
