@@ -222,11 +222,13 @@ struct AttentionFunction : public torch::autograd::Function<AttentionFunction> {
             k = k.to(at::kBFloat16);
             v = v.to(at::kBFloat16);
         }
-        // (converted once for both directions)
+        // converted once for both directions (and what is converted is a copy: the caller may move its int64 position on before
+        // the backward); what is no offset at all is refused by the forward operator
+        const OptTensor start = q_offset_dev && !q_offset_dev->is_floating_point() ? OptTensor(q_offset_dev->to(at::kInt)) : q_offset_dev;
         const OptTensor lens = seqlens ? OptTensor(seqlens->to(q.device(), at::kInt).contiguous()) : OptTensor();
         const OptTensor docs = doc_start ? OptTensor(doc_start->to(q.device(), at::kInt).contiguous()) : OptTensor();
-        auto [o, lse] = call_fwd(q, k, v, sinks, sm_scale, window, q_offset, lens, docs, q_offset_dev);
-        ctx->save_for_backward({q, k, v, tensor_of(sinks), o, lse, tensor_of(lens), tensor_of(docs), tensor_of(q_offset_dev)});
+        auto [o, lse] = call_fwd(q, k, v, sinks, sm_scale, window, q_offset, lens, docs, start);
+        ctx->save_for_backward({q, k, v, tensor_of(sinks), o, lse, tensor_of(lens), tensor_of(docs), tensor_of(start)});
         ctx->saved_data["sm_scale"] = sm_scale;
         ctx->saved_data["window"] = window;
         ctx->saved_data["q_offset"] = q_offset;
