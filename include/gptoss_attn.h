@@ -108,7 +108,7 @@ typedef struct gptoss_attn_params {
     const void *d_o;
     void *dq, *dk, *dv;
     float *dsinks;          /* optional: NULL skips the sink gradient */
-    float *delta;           /* fp32 scratch of gptoss_attn_workspace_bytes() bytes (forward: optional) */
+    float *delta;           /* fp32 scratch of gptoss_attn_workspace_bytes() bytes */
 
     gptoss_attn_strides q_stride, k_stride, v_stride, o_stride;
     gptoss_attn_strides do_stride, dq_stride, dk_stride, dv_stride;
@@ -148,9 +148,9 @@ const char *gptoss_attn_status_string(int status);
 size_t gptoss_attn_workspace_bytes(const gptoss_attn_params *params);
 
 /*
- * Bytes of scratch gptoss_attn_fwd can use for these shapes (0 for most): few queries on a long key / value cache (a decoding step, a
- * short piece of a prompt) are cut over the keys, and the slices leave fp32 partial results there.  Given through `delta` (16-byte aligned);
- * with delta == NULL the same kernel runs uncut.  Never more than gptoss_attn_workspace_bytes.  Host-only.
+ * Bytes of scratch gptoss_attn_fwd_scratch can use for this call (0 for most): few queries on a long key / value cache (a decoding
+ * step, a short piece of a prompt) are cut over the keys, and the slices leave fp32 partial results there.  Never more than
+ * gptoss_attn_workspace_bytes.  Host-only.
  */
 size_t gptoss_attn_fwd_workspace_bytes(const gptoss_attn_params *params);
 
@@ -158,8 +158,7 @@ size_t gptoss_attn_fwd_workspace_bytes(const gptoss_attn_params *params);
  * Forward: O and logsumexp.  Replaces the `_attn_fwd` launch in
  * `_attention.forward` (attention_kernel.py:11-100, 241-262) including the
  * output transpose copy at :272 (O is written directly in the caller's layout).
- * Reads q,k,v,sinks,seqlens,doc_start; writes o,lse (and delta, where
- * gptoss_attn_fwd_workspace_bytes asks for it).
+ * Reads q,k,v,sinks,seqlens,doc_start; writes o,lse.
  */
 int gptoss_attn_fwd(const gptoss_attn_params *params, void *stream);
 
@@ -168,6 +167,13 @@ int gptoss_attn_fwd(const gptoss_attn_params *params, void *stream);
  * type a model's parameter has: bf16 logits widen exactly, no converted copy is needed.
  */
 int gptoss_attn_fwd_sinks(const gptoss_attn_params *params, int sinks_dtype, void *stream);
+
+/*
+ * The same with scratch of the caller's for few queries on a long cache: `scratch` (16-byte aligned) holds `scratch_bytes` bytes, which
+ * no other call may use until this one has run.  With NULL, or with fewer bytes than gptoss_attn_fwd_workspace_bytes gives
+ * for the same block, the same kernel walks each row's keys uncut, as the two calls above do (O then agrees to one bf16 rounding).
+ */
+int gptoss_attn_fwd_scratch(const gptoss_attn_params *params, int sinks_dtype, void *scratch, size_t scratch_bytes, void *stream);
 
 /*
  * Backward step 1: the row statistics.  The first B*H*Sq floats of `delta` receive

@@ -26,6 +26,7 @@ EXPORTS = (
     "gptoss_attn_fwd_workspace_bytes",
     "gptoss_attn_fwd",
     "gptoss_attn_fwd_sinks",
+    "gptoss_attn_fwd_scratch",
     "gptoss_attn_bwd_preprocess",
     "gptoss_attn_bwd_dkdv",
     "gptoss_attn_bwd_dq",
@@ -117,6 +118,8 @@ def load() -> ctypes.CDLL:
             fn.argtypes = [ctypes.POINTER(Params), ctypes.c_void_p]
         lib.gptoss_attn_fwd_sinks.restype = ctypes.c_int
         lib.gptoss_attn_fwd_sinks.argtypes = [ctypes.POINTER(Params), ctypes.c_int, ctypes.c_void_p]
+        lib.gptoss_attn_fwd_scratch.restype = ctypes.c_int
+        lib.gptoss_attn_fwd_scratch.argtypes = [ctypes.POINTER(Params), ctypes.c_int, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]
         lib.gptoss_attn_bwd_sinks.restype = ctypes.c_int
         lib.gptoss_attn_bwd_sinks.argtypes = [ctypes.POINTER(Params), ctypes.c_int, ctypes.c_int, ctypes.c_void_p]
         if lib.gptoss_attn_version() != ABI_VERSION:
@@ -149,9 +152,9 @@ def status_string(status: int) -> str:
     return load().gptoss_attn_status_string(int(status)).decode()
 
 
-def call(name: str, params: Params, stream: int = 0) -> None:
-    """Calls an entry point and raises GptossAttnError on a non-zero status."""
-    rc = getattr(load(), name)(ctypes.byref(params), ctypes.c_void_p(stream))
+def call(name: str, params: Params, stream: int = 0, *between) -> None:
+    """Calls an entry point (`between`: its arguments between the block and the stream) and raises GptossAttnError on a non-zero status."""
+    rc = getattr(load(), name)(ctypes.byref(params), *between, ctypes.c_void_p(stream))
     if rc != 0:
         raise GptossAttnError(name, rc, status_string(rc))
 

@@ -191,11 +191,9 @@ def attention_forward(q, k, v, sinks, sm_scale, window=None, q_offset=0, seqlens
         p = _base_params(q, k, v, sinks32, sl, sm_scale, window, q_offset, ds, qod)
         p.o, p.lse = o.data_ptr(), lse.data_ptr()
         _set(p.o_stride, _strides_bhs(o, "bshd"))
-        need = _lib.load().gptoss_attn_fwd_workspace_bytes(p)      # partial results of a decoding call cut over its keys
-        if need:
-            scratch = torch.empty((need // 4,), dtype=torch.float32, device=q.device)
-            p.delta = scratch.data_ptr()
-        _lib.call("gptoss_attn_fwd", p, _stream(q))
+        need = _lib.load().gptoss_attn_fwd_workspace_bytes(p)      # partial results of few queries' rows, cut over their keys
+        scratch = torch.empty((need // 4,), dtype=torch.float32, device=q.device) if need else None
+        _lib.call("gptoss_attn_fwd_scratch", p, _stream(q), _lib.DTYPE_FP32, scratch.data_ptr() if need else None, need)
     return o, lse
 
 

@@ -502,14 +502,16 @@ size_t gptoss_attn_workspace_bytes(const gptoss_attn_params *p) {
     return n;
 }
 
-static int forward(const gptoss_attn_params *p, void *stream, SinkTypes ty) {
+// scratch: see gptoss_attn_fwd_scratch (NULL or too little: the keys are not cut)
+static int forward(const gptoss_attn_params *p, void *stream, SinkTypes ty, void *scratch, size_t scratch_bytes) {
     const int rc = gptoss_attn_validate(p, 0);
     if (rc) return rc;
+    if (!aligned16(scratch)) return GPTOSS_ATTN_ERR_ALIGNMENT;
+    const bool cut = scratch && scratch_bytes >= gptoss_attn_fwd_workspace_bytes(p);
     KArgs a = make_args(p, ty);
     hipStream_t st = static_cast<hipStream_t>(stream);
-    if (p->delta && !aligned16(p->delta)) return GPTOSS_ATTN_ERR_ALIGNMENT;
     if (decode_route(p)) {
-        if (p->delta) { a.kv_splits = decode_splits(p); a.fwd_partial = p->delta; }
+        if (cut) { a.kv_splits = decode_splits(p); a.fwd_partial = static_cast<float *>(scratch); }
         const int pairs = a.Sq * a.r;
         const int64_t wgs = (int64_t)a.G * a.B * a.kv_splits;
         if (decode_whole(p)) return pairs <= 32 ? launch_decode<1, 8>(wgs, st, a) : launch_decode<2, 8>(wgs, st, a);
@@ -541,10 +543,10 @@ static int forward(const gptoss_attn_params *p, void *stream, SinkTypes ty) {
 #undef GPTOSS_LAUNCH_WIN
     }
     if (fwd_pipe_route(p)) {
-        const int splits = p->delta && !a.doc_start ? fwd_pipe_splits(p) : 1;
+        const int splits = cut && !a.doc_start ? fwd_pipe_splits(p) : 1;
         if (splits > 1) {
             a.kv_splits = splits;
-            a.fwd_partial = p->delta;
+            a.fwd_partial = static_cast<float *>(scratch);
             const int s = launch(attn_fwd_pipe_kernel<true, false>, grid * splits, 256, st, a);
             return s ? s : launch(attn_fwd_combine_kernel, ((int64_t)a.B * a.H * a.Sq + 31) / 32, 256, st, a);
         }
@@ -558,13 +560,18 @@ static int forward(const gptoss_attn_params *p, void *stream, SinkTypes ty) {
 #undef GPTOSS_LAUNCH_FWD
 }
 
-int gptoss_attn_fwd(const gptoss_attn_params *p, void *stream) { return forward(p, stream, {}); }
+int gptoss_attn_fwd(const gptoss_attn_params *p, void *stream) { return forward(p, stream, {}, nullptr, 0); }
 
 static bool sink_dtype_ok(int dtype) { return dtype == GPTOSS_ATTN_FP32 || dtype == GPTOSS_ATTN_BF16; }
 
 int gptoss_attn_fwd_sinks(const gptoss_attn_params *p, int sinks_dtype, void *stream) {
     if (!sink_dtype_ok(sinks_dtype)) return GPTOSS_ATTN_ERR_DTYPE;
-    return forward(p, stream, {sinks_dtype == GPTOSS_ATTN_BF16, false});
+    return forward(p, stream, {sinks_dtype == GPTOSS_ATTN_BF16, false}, nullptr, 0);
+}
+
+int gptoss_attn_fwd_scratch(const gptoss_attn_params *p, int sinks_dtype, void *scratch, size_t scratch_bytes, void *stream) {
+    if (!sink_dtype_ok(sinks_dtype)) return GPTOSS_ATTN_ERR_DTYPE;
+    return forward(p, stream, {sinks_dtype == GPTOSS_ATTN_BF16, false}, scratch, scratch_bytes);
 }
 
 int gptoss_attn_bwd_preprocess(const gptoss_attn_params *p, void *stream) {

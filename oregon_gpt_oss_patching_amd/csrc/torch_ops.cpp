@@ -141,12 +141,9 @@ std::tuple<Tensor, Tensor> fwd(const Tensor &q, const Tensor &k, const Tensor &v
     c.p.o = o.data_ptr();
     c.p.lse = lse.data_ptr<float>();
     set(c.p.o_stride, o, true);
-    Tensor scratch;                    // partial results of a decoding call cut over its keys
-    if (const size_t need = gptoss_attn_fwd_workspace_bytes(&c.p)) {
-        scratch = at::empty({static_cast<int64_t>(need / sizeof(float))}, lse.options());
-        c.p.delta = scratch.data_ptr<float>();
-    }
-    check("gptoss_attn_fwd", gptoss_attn_fwd_sinks(&c.p, c.sinks_dtype, stream_of(c)));
+    const size_t need = gptoss_attn_fwd_workspace_bytes(&c.p);      // partial results of few queries' rows, cut over their keys
+    const Tensor scratch = need ? at::empty({static_cast<int64_t>(need / sizeof(float))}, lse.options()) : Tensor();
+    check("gptoss_attn_fwd", gptoss_attn_fwd_scratch(&c.p, c.sinks_dtype, need ? scratch.data_ptr() : nullptr, need, stream_of(c)));
     return {o, lse};
 }
 
