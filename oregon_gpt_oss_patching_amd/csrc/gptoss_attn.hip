@@ -477,8 +477,7 @@ size_t gptoss_attn_fwd_workspace_bytes(const gptoss_attn_params *p) {
     if (decode_route(p)) {
         const int splits = decode_splits(p);
         if (splits > 1) return (size_t)p->B * p->G * splits * decode_partial_floats(p->Sq * (p->H / p->G)) * sizeof(float);
-    } else if (p->dtype == GPTOSS_ATTN_BF16 && (p->window <= 0 || p->window >= p->Sq) && (p->H / p->G) % 4 == 0 && p->Skv >= kTile) {
-        // (a window that covers the whole row is none; where the queries stand may not be known yet)
+    } else if (fwd_pipe_route(p) && !p->doc_start) {
         const int splits = fwd_pipe_splits(p);
         if (splits > 1) return (size_t)splits * p->B * p->H * p->Sq * (kD + 2) * sizeof(float);
     }

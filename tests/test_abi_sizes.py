@@ -24,3 +24,19 @@ def test_sizes_of_head_counts_that_the_calls_refuse(h, g):
         assert lib.gptoss_attn_fwd_workspace_bytes(ctypes.byref(p)) == 0
         lib.gptoss_attn_workspace_bytes(ctypes.byref(p))
         assert lib.gptoss_attn_validate(ctypes.byref(p), 0) == -4
+
+
+@pytest.mark.parametrize("sq,skv,window,start,shares", [
+    (100, 8192, 128, 8092, 0),       # a window layer takes the window kernel, which cuts nothing
+    (100, 8192, 0, 8092, 16),
+    (100, 8192, 8192, 8092, 16),     # a window that reaches back past the first key is none
+    (100, 8192, 8191, 8092, 0),
+    (1024, 8192, 1024, 7168, 0),
+])
+def test_forward_scratch_follows_the_kernel_that_runs(sq, skv, window, start, shares):
+    p = _params(sq=sq, skv=skv, window=window, q_offset=start)
+    rows = 64 * sq
+    assert _lib.load().gptoss_attn_fwd_workspace_bytes(ctypes.byref(p)) == shares * rows * (64 + 2) * 4
+    if window > skv - 1:             # (where the position is on the device, the host does not know that)
+        p.q_offset_dev = 256
+        assert _lib.load().gptoss_attn_fwd_workspace_bytes(ctypes.byref(p)) == 0
