@@ -143,9 +143,16 @@ const char *gptoss_attn_status_string(int status);
  * sliding-window layers that gptoss_attn_bwd runs as one kernel the same bytes hold that kernel's
  * dSinks partial sums and the fp32 dK / dV shares of the key tiles on the seams between workgroups;
  * how many seams there are depends on the compute-unit count of the device the launch runs on, and
- * the size returned covers the largest number any device can ask for.  Host-only: no HIP call.
+ * the size returned covers the largest number any device can ask for.  It also covers calls with and without seqlens and
+ * doc_start, which cut key blocks into different numbers of slices.  Host-only: no HIP call.
  */
 size_t gptoss_attn_workspace_bytes(const gptoss_attn_params *params);
+
+/*
+ * The same for the backward of exactly this block, seqlens and doc_start as they are set (the pointers' presence; nothing is read
+ * through them): often less (64 query heads on 8 KV heads, two plain rows of 8192 tokens: 25 MB, the call above 159).
+ */
+size_t gptoss_attn_bwd_workspace_bytes(const gptoss_attn_params *params);
 
 /*
  * Bytes of scratch gptoss_attn_fwd_scratch can use for this call (0 for most): few queries on a long key / value cache (a decoding

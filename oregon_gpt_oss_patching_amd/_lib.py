@@ -23,6 +23,7 @@ EXPORTS = (
     "gptoss_attn_status_string",
     "gptoss_attn_validate",
     "gptoss_attn_workspace_bytes",
+    "gptoss_attn_bwd_workspace_bytes",
     "gptoss_attn_fwd_workspace_bytes",
     "gptoss_attn_fwd",
     "gptoss_attn_fwd_sinks",
@@ -98,6 +99,8 @@ def load() -> ctypes.CDLL:
         lib.gptoss_attn_validate.argtypes = [ctypes.POINTER(Params), ctypes.c_int]
         lib.gptoss_attn_workspace_bytes.restype = ctypes.c_size_t
         lib.gptoss_attn_workspace_bytes.argtypes = [ctypes.POINTER(Params)]
+        lib.gptoss_attn_bwd_workspace_bytes.restype = ctypes.c_size_t
+        lib.gptoss_attn_bwd_workspace_bytes.argtypes = [ctypes.POINTER(Params)]
         lib.gptoss_attn_fwd_workspace_bytes.restype = ctypes.c_size_t
         lib.gptoss_attn_fwd_workspace_bytes.argtypes = [ctypes.POINTER(Params)]
         lib.gptoss_attn_static_scratch_bytes.restype = ctypes.c_size_t

@@ -219,7 +219,7 @@ def attention_backward(q, k, v, sinks, o, lse, d_o, sm_scale, window=None, q_off
     with torch.cuda.device(q.device):
         p = _base_params(q, k, v, sinks32, sl, sm_scale, window, q_offset, ds, qod)
         # scratch: [-delta; lse*log2e], then the dK/dV partial sums of split key blocks (short sequences)
-        delta = torch.empty((_lib.load().gptoss_attn_workspace_bytes(p) // 4,), dtype=torch.float32, device=q.device)
+        delta = torch.empty((_lib.load().gptoss_attn_bwd_workspace_bytes(p) // 4,), dtype=torch.float32, device=q.device)
         p.o, p.lse = o.data_ptr(), lse.data_ptr()
         _set(p.o_stride, _strides_bhs(o, "bshd"))
         p.d_o = d_o.data_ptr()

@@ -461,13 +461,8 @@ static size_t stats_bytes(const gptoss_attn_params *p) {
     return fp32_stats_bytes(p) + (size_t)16 * (size_t)p->B * (size_t)p->H * (size_t)p->Sq;
 }
 
-// dK/dV partial sums, for a call with or without lengths of padded rows and documents (the size depends on the shapes only)
-static size_t partials_bytes(const gptoss_attn_params *p) {
-    int parts = 1;
-    for (int kind = 0; kind < 4; ++kind) {
-        const int n = dkdv_parts_for(p, kind & 1, kind & 2);
-        if (n > parts) parts = n;
-    }
+// dK/dV partial sums of `parts` slices
+static size_t partials_bytes(const gptoss_attn_params *p, int parts) {
     return parts > 1 ? (size_t)parts * 2 * sizeof(float) * (size_t)p->B * (size_t)p->G * (size_t)p->Skv * kD : 0;
 }
 
@@ -484,12 +479,11 @@ size_t gptoss_attn_fwd_workspace_bytes(const gptoss_attn_params *p) {
     return 0;
 }
 
-size_t gptoss_attn_workspace_bytes(const gptoss_attn_params *p) {
-    if (!p || p->B <= 0 || p->H <= 0 || p->Sq <= 0) return 0;
+// The backward's scratch with `parts` slices of the key blocks.
+static size_t bwd_bytes(const gptoss_attn_params *p, int parts) {
     size_t n = stats_bytes(p);
-    if (gptoss_attn_fwd_workspace_bytes(p) > n) n = gptoss_attn_fwd_workspace_bytes(p);
     if (p->G > 0 && p->Skv > 0) {
-        n += partials_bytes(p);
+        n += partials_bytes(p, parts);
         if (window_single_pass(p)) {
             // gptoss_attn_bwd takes this route and lays its own scratch over the same bytes.  The layout
             // follows the compute-unit count of the device that is current at launch time; the size
@@ -499,6 +493,23 @@ size_t gptoss_attn_workspace_bytes(const gptoss_attn_params *p) {
         }
     }
     return n;
+}
+
+size_t gptoss_attn_bwd_workspace_bytes(const gptoss_attn_params *p) {
+    if (!p || p->B <= 0 || p->H <= 0 || p->Sq <= 0) return 0;
+    return bwd_bytes(p, p->G > 0 && p->Skv > 0 ? dkdv_parts_for(p, p->seqlens != nullptr, p->doc_start != nullptr) : 1);
+}
+
+size_t gptoss_attn_workspace_bytes(const gptoss_attn_params *p) {
+    if (!p || p->B <= 0 || p->H <= 0 || p->Sq <= 0) return 0;
+    // with or without lengths of padded rows and documents: who asks may not have filled these in yet
+    int parts = 1;
+    for (int kind = 0; kind < 4 && p->G > 0 && p->Skv > 0; ++kind) {
+        const int n = dkdv_parts_for(p, kind & 1, kind & 2);
+        if (n > parts) parts = n;
+    }
+    const size_t n = bwd_bytes(p, parts), fwd = gptoss_attn_fwd_workspace_bytes(p);
+    return fwd > n ? fwd : n;
 }
 
 // scratch: see gptoss_attn_fwd_scratch (NULL or too little: the keys are not cut)

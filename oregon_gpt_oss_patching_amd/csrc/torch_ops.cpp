@@ -170,7 +170,7 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> bwd(const Tensor &q, const Tensor &k,
     const bool bf16_dsinks = dsinks_as_sinks && c.sinks_dtype == GPTOSS_ATTN_BF16;
     Tensor dsinks = at::empty({need_dsinks ? h : 0}, lse.options().dtype(bf16_dsinks ? at::kBFloat16 : at::kFloat));
     // scratch: the row statistics, then the dK/dV partial sums of split key blocks or the window kernel's shares
-    Tensor scratch = at::empty({static_cast<int64_t>(gptoss_attn_workspace_bytes(&c.p) / sizeof(float))}, lse.options());
+    Tensor scratch = at::empty({static_cast<int64_t>(gptoss_attn_bwd_workspace_bytes(&c.p) / sizeof(float))}, lse.options());
     gptoss_attn_params &p = c.p;
     p.o = const_cast<void *>(o.const_data_ptr());             // (read only here)
     p.lse = const_cast<float *>(lse.const_data_ptr<float>());

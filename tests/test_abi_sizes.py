@@ -40,3 +40,24 @@ def test_forward_scratch_follows_the_kernel_that_runs(sq, skv, window, start, sh
     if window > skv - 1:             # (where the position is on the device, the host does not know that)
         p.q_offset_dev = 256
         assert _lib.load().gptoss_attn_fwd_workspace_bytes(ctypes.byref(p)) == 0
+
+
+def test_backward_scratch_of_the_call_itself():
+    """gptoss_attn_bwd_workspace_bytes counts the slices this call is cut into; gptoss_attn_workspace_bytes, which may be asked before lengths
+    and documents are filled in, covers every one of them."""
+    lib = _lib.load()
+    exact, bound = (lambda p: lib.gptoss_attn_bwd_workspace_bytes(ctypes.byref(p))), (lambda p: lib.gptoss_attn_workspace_bytes(ctypes.byref(p)))
+    for b, s, plain, padded, packed in ((2, 8192, 1, 2, 1), (1, 8192, 2, 2, 4), (2, 4096, 2, 2, 4), (4, 4096, 1, 2, 1), (1, 16384, 1, 1, 1), (2, 383, 6, 6, 6)):
+        stats, part = 24 * b * 64 * s, 2 * 4 * b * 8 * s * 64
+        sizes = []
+        for ptrs, parts in (({}, plain), ({"seqlens": 256}, padded), ({"doc_start": 256}, packed)):
+            p = _params(b=b, sq=s, skv=s, **ptrs)
+            assert exact(p) == stats + (parts * part if parts > 1 else 0), (b, s, ptrs)
+            sizes.append(bound(p))
+        assert sizes == [sizes[0]] * 3 and sizes[0] >= stats + max(plain, padded, packed) * part * (max(plain, padded, packed) > 1)
+    for dtype, window in itertools.product((0, 1), (0, 128, 512)):
+        for ptrs in ({}, {"seqlens": 256}, {"doc_start": 256}):
+            for sq in (1, 65, 1000, 4096):
+                p = _params(dtype, 2, 64, 8, sq, sq, window, **ptrs)
+                assert 24 * 2 * 64 * sq <= exact(p) <= bound(p)
+    assert exact(_params(sq=0)) == 0 and lib.gptoss_attn_bwd_workspace_bytes(None) == 0
