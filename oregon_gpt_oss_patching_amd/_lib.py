@@ -7,7 +7,6 @@ from __future__ import annotations
 
 import ctypes
 import os
-import re
 from typing import Optional
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -140,15 +139,6 @@ def load_torch_ops() -> None:
     load()          # the operators link to it
     import torch
     torch.ops.load_library(TORCH_LIBRARY)
-
-
-_OP_FAILURE = re.compile(r"(gptoss_attn_\w+) failed with status (-?\d+): ")
-
-
-def as_library_error(e: RuntimeError) -> RuntimeError:
-    """The GptossAttnError for an operator's report of a failed library call; any other error as it is."""
-    m = _OP_FAILURE.match(str(e))
-    return GptossAttnError(m.group(1), int(m.group(2)), status_string(int(m.group(2)))) if m else e
 
 
 def status_string(status: int) -> str:

@@ -295,13 +295,8 @@ def attention(q, k, v, sinks, sm_scale, bandwidth, start_q, seqlens=None, doc_st
         seqlens = torch.as_tensor(seqlens, dtype=torch.int32)
     if doc_start is not None and not torch.is_tensor(doc_start):
         doc_start = torch.as_tensor(doc_start, dtype=torch.int32)
-    call = torch.ops.gptoss_attn.attention.default
-    if torch.compiler.is_compiling():
-        return call(q, k, v, sinks, float(sm_scale), int(bandwidth or 0), q_offset, seqlens, doc_start, q_offset_dev)
-    try:
-        return call(q, k, v, sinks, float(sm_scale), int(bandwidth or 0), q_offset, seqlens, doc_start, q_offset_dev)
-    except RuntimeError as e:
-        raise _lib.as_library_error(e) from None
+    return torch.ops.gptoss_attn.attention.default(q, k, v, sinks, float(sm_scale), int(bandwidth or 0), q_offset, seqlens, doc_start,
+                                                   q_offset_dev)
 
 
 def hip_flash_attention(

@@ -8,6 +8,7 @@ from __future__ import annotations
 import os
 import shutil
 import subprocess
+import sysconfig
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 SOURCE = os.path.join(_HERE, "csrc", "gptoss_attn.hip")
@@ -57,7 +58,7 @@ def build_torch_ops(verbose: bool = False) -> str:
     _run([shutil.which("g++") or "c++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM",
           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
           "-isystem", os.path.join(root, "include"), "-isystem", os.path.join(root, "include", "torch", "csrc", "api", "include"),
-          "-isystem", os.path.join(rocm, "include"), "-o", TORCH_LIBRARY, TORCH_SOURCE,
+          "-isystem", os.path.join(rocm, "include"), "-isystem", sysconfig.get_paths()["include"], "-o", TORCH_LIBRARY, TORCH_SOURCE,
           "-L" + os.path.join(root, "lib"), "-lc10", "-ltorch_cpu", "-lc10_hip", "-L" + _HERE, "-lgptoss_attn", "-Wl,-rpath,$ORIGIN"], verbose)
     return TORCH_LIBRARY
 

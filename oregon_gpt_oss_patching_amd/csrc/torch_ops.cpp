@@ -12,6 +12,7 @@
 #include <ATen/ATen.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
+#include <pybind11/pybind11.h>
 #include <torch/csrc/autograd/autograd_not_implemented_fallback.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/library.h>
@@ -127,8 +128,13 @@ void fill(Call &c, const Tensor &q, const Tensor &k, const Tensor &v, const OptT
 
 void *stream_of(const Call &c) { return c10::hip::getCurrentHIPStream(c.q.device().index()).stream(); }
 
+// A failed library call is the package's GptossAttnError wherever it happens: in a call, a backward or a traced program.
 void check(const char *name, int rc) {
-    TORCH_CHECK(rc == 0, name, " failed with status ", rc, ": ", gptoss_attn_status_string(rc));
+    if (rc == 0) return;
+    const pybind11::gil_scoped_acquire gil;
+    const pybind11::object type = pybind11::module_::import("oregon_gpt_oss_patching_amd._lib").attr("GptossAttnError");
+    PyErr_SetObject(type.ptr(), type(name, rc, gptoss_attn_status_string(rc)).ptr());
+    throw pybind11::error_already_set();
 }
 
 std::tuple<Tensor, Tensor> fwd(const Tensor &q, const Tensor &k, const Tensor &v, const OptTensor &sinks, double sm_scale, int64_t window,
@@ -268,10 +274,9 @@ Tensor doc_start(const Tensor &position_ids_) {
     const Tensor pos = position_ids_.size(1) > 1 && position_ids_.stride(1) != 1 ? position_ids_.contiguous() : position_ids_;
     Tensor out = at::empty(pos.sizes(), pos.options().dtype(at::kInt));
     if (pos.numel() == 0) return out;
-    const int rc = gptoss_attn_doc_start(pos.const_data_ptr(), static_cast<int>(pos.element_size()), static_cast<int>(pos.size(0)),
-                                         static_cast<int>(pos.size(1)), pos.stride(0), out.data_ptr<int32_t>(),
-                                         c10::hip::getCurrentHIPStream(pos.device().index()).stream());
-    TORCH_CHECK(rc == 0, "gptoss_attn_doc_start failed with status ", rc, ": ", gptoss_attn_status_string(rc));
+    check("gptoss_attn_doc_start", gptoss_attn_doc_start(pos.const_data_ptr(), static_cast<int>(pos.element_size()), static_cast<int>(pos.size(0)),
+                                                         static_cast<int>(pos.size(1)), pos.stride(0), out.data_ptr<int32_t>(),
+                                                         c10::hip::getCurrentHIPStream(pos.device().index()).stream()));
     return out;
 }
 
