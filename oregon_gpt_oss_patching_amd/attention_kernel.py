@@ -299,6 +299,11 @@ def attention(q, k, v, sinks, sm_scale, bandwidth, start_q, seqlens=None, doc_st
                                                    q_offset_dev)
 
 
+class _attention:
+    """The reference's name for the differentiable call (attention_kernel.py:220-347): `_attention.apply(...)`."""
+    apply = staticmethod(attention)
+
+
 def hip_flash_attention(
     module,
     query: torch.Tensor,
