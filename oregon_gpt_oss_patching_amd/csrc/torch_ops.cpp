@@ -280,6 +280,11 @@ Tensor doc_start(const Tensor &position_ids_) {
     return out;
 }
 
+// Function transforms have no rule for the autograd node; without this vmap would run it slice by slice behind the caller's back.
+void refuse_vmap(const c10::OperatorHandle &, torch::jit::Stack *) {
+    TORCH_CHECK(false, "gptoss attention cannot be vmapped: its tensors have a batch dimension of their own");
+}
+
 }  // namespace
 
 TORCH_LIBRARY(gptoss_attn, m) {
@@ -299,4 +304,7 @@ TORCH_LIBRARY_IMPL(gptoss_attn, CUDA, m) {
 TORCH_LIBRARY_IMPL(gptoss_attn, Autograd, m) {
     m.impl("fwd", torch::autograd::autogradNotImplementedFallback());
     m.impl("bwd", torch::autograd::autogradNotImplementedFallback());
+}
+TORCH_LIBRARY_IMPL(gptoss_attn, FuncTorchBatched, m) {
+    m.impl("attention", torch::CppFunction::makeFromBoxedFunction<&refuse_vmap>());
 }
