@@ -159,6 +159,24 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_window_kernel(const KArgs a) 
     // output in o, the row's reference m and this lane's share l of the row sum.
     f32x16 o[2];
     float m, l;
+    // O += P V of step u (16 keys) of the staged block h.  rest: the weights' rounding to bf16 goes through the matrix pipe as well, for one step
+    // of a block (GENERAL only).  Why: attn_fwd_kernel, which took these calls before, rounds its weights against a running maximum,
+    // and every key that sets a new one has the weight 1, exactly; against the final maximum only one key does.  O's error from
+    // float64 was 0.5 to 1.7 % larger for it.  One step without rounding, of the eight a window of 128 has, brings it below (3001
+    // tokens: 2.143e-3, 2.071e-3 so, 2.109e-3 with a running maximum) and costs 0.6 us of the 115 of B = 2, forward + backward.
+    auto add_values = [&](int h, int u, const f32x16 &p, bool first, bool rest) __attribute__((always_inline)) {
+        const bf16x8 pf = cfrag(p, u);
+        bf16x8 pr;
+        if (rest)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) pr[j] = (bf16)(p[8 * u + j] - (float)pf[j]);
+#pragma unroll
+        for (int dblk = 0; dblk < 2; ++dblk) {
+            const bf16x8 av = ofrag_tr(vsm, lo, h, u, dblk);
+            o[dblk] = mfma_bf16(av, pf, first ? zero16 : o[dblk]);
+            if (rest) o[dblk] = mfma_bf16(av, pr, o[dblk]);
+        }
+    };
     auto block = [&](auto x_tag) __attribute__((always_inline)) {
         constexpr int X = decltype(x_tag)::value;
         bool edge = k0 + 32 * X < 0;
@@ -213,17 +231,12 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_window_kernel(const KArgs a) 
                 pa[i] = last ? 0.0f : t[i];
                 pb[i] = last ? t[i] : 0.0f;
             }
-            auto pv = [&](int h, const f32x16 &p, auto first_tag) __attribute__((always_inline)) {
+            auto pv = [&](int h, const f32x16 &p, auto first_tag, bool rest) __attribute__((always_inline)) {
 #pragma unroll
-                for (int u = 0; u < 2; ++u) {
-                    const bf16x8 pf = cfrag(p, u);
-#pragma unroll
-                    for (int dblk = 0; dblk < 2; ++dblk)
-                        o[dblk] = mfma_bf16(ofrag_tr(vsm, lo, X + h, u, dblk), pf, (decltype(first_tag)::value && u == 0) ? zero16 : o[dblk]);
-                }
+                for (int u = 0; u < 2; ++u) add_values(X + h, u, p, decltype(first_tag)::value && u == 0, GENERAL && rest && u == 0);
             };
-            pv(0, pa, std::true_type{});
-            pv(NH - 1, pb, std::false_type{});
+            pv(0, pa, std::true_type{}, NH == 2);
+            pv(NH - 1, pb, std::false_type{}, NH == 2);
 #pragma unroll
             for (int h = 1; h < NH - 1; ++h) {
 #pragma unroll
@@ -232,7 +245,7 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_window_kernel(const KArgs a) 
                     s[h][i] = e0; s[h][i + 1] = e1;
                     rs0 += e0; rs1 += e1;
                 }
-                pv(h, s[h], std::false_type{});
+                pv(h, s[h], std::false_type{}, h == 1);
             }
             l = rs0 + rs1;
         } else {
@@ -269,12 +282,7 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_window_kernel(const KArgs a) 
                     rs0 += e0; rs1 += e1;
                 }
 #pragma unroll
-                for (int u = 0; u < 2; ++u) {
-                    const bf16x8 pf = cfrag(s[h], u);
-#pragma unroll
-                    for (int dblk = 0; dblk < 2; ++dblk)
-                        o[dblk] = mfma_bf16(ofrag_tr(vsm, lo, X + h, u, dblk), pf, (h == 0 && u == 0) ? zero16 : o[dblk]);
-                }
+                for (int u = 0; u < 2; ++u) add_values(X + h, u, s[h], h == 0 && u == 0, GENERAL && h == NH - 1);
             }
             l = rs0 + rs1;
         }
