@@ -29,7 +29,7 @@
  *   lse          (B, H, Sq) fp32 contiguous
  *   delta        fp32 scratch of gptoss_attn_workspace_bytes() bytes, 16-byte aligned: -rowsum(dO*O), then
  *                lse*log2(e), then both once more as 16 bytes per row of bf16 terms for the dK/dV
- *                kernels, then (short sequences) partial dK/dV sums
+ *                kernels, then (key blocks cut into slices) partial dK/dV sums
  *   sinks, dsinks (H,) fp32;  sinks == NULL means a sink logit of 0, as in the
  *                reference (attention_kernel.py:39-42)
  *   seqlens      (B,) int32 or NULL: right-padding lengths.  Keys at or beyond
@@ -59,7 +59,7 @@ extern "C" {
 enum gptoss_attn_dtype {
     GPTOSS_ATTN_BF16 = 0, /* 2-byte bfloat16 tensors, bf16 MFMA products, fp32 accumulation: the fast path */
     GPTOSS_ATTN_FP32 = 1  /* 4-byte float tensors, fp32 MFMA products (the reference's fp32 mode,
-                             attention_kernel.py is dtype-generic): built for exactness, not tuned */
+                             attention_kernel.py is dtype-generic), at a sixteenth of the bf16 matrix rate */
 };
 
 enum gptoss_attn_status {
@@ -136,8 +136,8 @@ const char *gptoss_attn_status_string(int status);
  * 24 bytes of row statistics per (batch, head, query row): 2 * B * H * Sq floats, and the same numbers
  * (lse / scale and -delta) each split into three bf16 terms, which the dK/dV kernels feed to the matrix
  * pipe as one more step of their S and dP products.  When the problem has too few key blocks to fill the
- * GPU (bf16, full-causal, short sequences), the fp32 partial dK / dV sums of the slices each key
- * block is cut into.  The reference allocates its counterpart itself
+ * GPU (short rows, long ones next to shorter ones, packed ones), the fp32 partial dK / dV sums of the slices
+ * each key block is cut into follow.  The reference allocates its counterpart itself
  * (`delta = torch.empty_like(M)`, attention_kernel.py:303) and accumulates dK / dV with atomics
  * (:204,212); here the caller owns the scratch and the sums are taken in a fixed order.  For the
  * sliding-window layers that gptoss_attn_bwd runs as one kernel the same bytes hold that kernel's

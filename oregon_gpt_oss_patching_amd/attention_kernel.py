@@ -218,7 +218,7 @@ def attention_backward(q, k, v, sinks, o, lse, d_o, sm_scale, window=None, q_off
     dsinks = torch.empty((h,), dtype=torch.float32, device=q.device) if need_dsinks else None
     with torch.cuda.device(q.device):
         p = _base_params(q, k, v, sinks32, sl, sm_scale, window, q_offset, ds, qod)
-        # scratch: [-delta; lse*log2e], then the dK/dV partial sums of split key blocks (short sequences)
+        # scratch: [-delta; lse*log2e], then the dK/dV partial sums of key blocks cut into slices
         delta = torch.empty((_lib.load().gptoss_attn_bwd_workspace_bytes(p) // 4,), dtype=torch.float32, device=q.device)
         p.o, p.lse = o.data_ptr(), lse.data_ptr()
         _set(p.o_stride, _strides_bhs(o, "bshd"))
@@ -278,7 +278,8 @@ except Exception:       # not built yet, or built from other sources: importing 
 
 def attention(q, k, v, sinks, sm_scale, bandwidth, start_q, seqlens=None, doc_start=None):
     """Same argument list and gradients as the reference's `_attention.apply` (attention_kernel.py:220-344), plus optional
-    trailing `seqlens` and `doc_start`.
+    trailing `seqlens` (B valid lengths of right-padded rows) and `doc_start` ((B, S): the first token of each query's document, never
+    decreasing along a row, see `doc_start_from_position_ids`).
 
     bfloat16 tensors take the tuned bf16-MFMA kernels and float32 tensors the float32 kernels.  float16 tensors are accepted
     for convenience: they are rounded to bfloat16 on the way in and the results cast back."""

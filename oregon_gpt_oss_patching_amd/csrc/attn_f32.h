@@ -13,13 +13,13 @@
 // steps long instead of 32, and the chip fills from a few hundred rows on.
 //
 // Measured (64 query heads on 8 KV heads, S = 1024, full causal; before, with operands straight from global memory, one
-// wavefront per row block and none sharing it): forward 200 -> 101 us (85 TFLOP/s), dQ with the row statistics 306 -> 131
-// us, dK/dV 2227 -> 190 us (its 256 key blocks were 256 wavefronts).  At S = 4096 the matrix pipes are busy 73 to 81 % of
-// the cycles (2.2 GHz).
+// wavefront per row block and none sharing it): forward 200 -> 101 us (85 TFLOP/s), dQ with the row statistics 306 -> 134
+// us, dK/dV 2227 -> 176 us (its 256 key blocks were 256 wavefronts).  The matrix pipes are busy 59 % (forward), 65 % (dQ) and 67 %
+// (dK/dV) of the cycles there, 73 to 81 % at S = 4096 (2.2 GHz).
 //
 // Weights come from exp2f, not from the bare exponential instruction (fast_exp2), which flushes what is below 2^-126: a key far down
-// the softmax still counts where the others' values are small or zero.  S = 1024, forward + backward: 411 us a call with the
-// bare instruction, 415 so.
+// the softmax still counts where the others' values are small or zero.  S = 1024, with the bare instruction and so: forward 97 and
+// 101 us, dQ 131 and 134, dK/dV 180 and 176, a whole call 410 and 414.
 //
 // Register layouts of v_mfma_f32_32x32x2_f32 (lane = 0..63, half = lane/32, l32 = lane%32):
 //   A (32 x 2): lane holds A[l32][half]      B (2 x 32): lane holds B[half][l32]

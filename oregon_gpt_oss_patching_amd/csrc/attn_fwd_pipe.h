@@ -46,7 +46,7 @@ struct FwdPipe {
 // the tensor or the padding: their values are garbage but finite or at worst NaN, and stay in their own lanes) and start
 // afresh at the diagonal tile.  Workgroups without any row that exists write O = 0 and lse = sink and do nothing else.
 // Measured against attn_fwd_kernel, which took these cases before (64 query heads on 8 KV heads): 1024 queries behind 7168
-// keys 181 -> 135 us; 2 x 3001 tokens 164 -> 160 us, 1 x 1000 33.6 -> 25.2, 2 x 383 16.1 -> 14.8; seven documents in 8192 tokens
+// keys 181 -> 135 us a call; 2 x 3001 tokens 164 -> 160 us, 1 x 1000 33.6 -> 25.2, 2 x 383 16.1 -> 14.8; seven documents in 8192 tokens
 // 185 -> 180 (without letting the other documents' rows run along, every tile of such a workgroup being an exact
 // step: 230).
 // Few queries on a long cache leave most of the chip idle (100 queries on 4096 keys: 32 workgroups).  With kv_splits > 1 a query block's

@@ -1,7 +1,7 @@
 // C ABI of the gfx950 GPT-OSS attention library (declared in include/gptoss_attn.h):
 // host-side argument validation, launch geometry, and the kernel launches.
-// No torch headers, no allocation; the only process-wide state is three per-device caches that are
-// written once (compute-unit count, the window kernel's LDS attribute, the address of the built-in scratch).
+// No torch headers, no allocation; the only process-wide state is per-device values that are written once
+// (compute-unit count, the LDS attributes of kernels that need more than 64 KB, the address of the built-in scratch).
 #include <hip/hip_runtime.h>
 
 #include <atomic>
@@ -108,15 +108,19 @@ constexpr int kDkdvKeys = 32 * kDkdvNB * kDkdvWaves; // keys per dK/dV workgroup
 // Workgroups per key block in the dK/dV kernel.  One workgroup per (batch, KV head, 128 keys) fills
 // the 256 CUs (two workgroups each) only from S = 16384 on, and the causal triangle makes the first
 // key blocks many times longer than the last; shorter problems cut each key block's query tiles into
-// slices so that there are about a thousand workgroups, and sum the slices' fp32 partials afterwards
-// (sliding-window layers are never cut).  Up to 512 blocks the count is rounded up, and a slice keeps at least eight
-// (query tile, head) steps (B = 2, S = 383: 78 us uncut, 25 + 5 us in six slices).  Between 512 and 1024 blocks the first
+// slices so that there are about a thousand workgroups, and sum the slices' fp32 partials afterwards.  A slice
+// keeps at least four query tiles of a sliding-window layer (windows of up to 321 keys stay whole, wider ones are cut) and at least
+// eight (query tile, head) steps of a full-causal one, which may be a single tile.  Up to 512 blocks the count is rounded
+// up (B = 2, S = 383: 78 us uncut, 25 + 5 us in six slices).  Between 512 and 1024 blocks the first
 // key block of a long row (4096 rows and more) is still longer than the average compute unit's share: two slices; a
 // right-padded batch counts half, because its shorter rows leave the longest one alone (dK/dV of B = 4, S = 4096,
 // lengths 3309 / 1968 / 1554 / 4079: 715 us uncut, 589 in two slices; B = 2, S = 8192 / 4000: 1437 and 1216; but B = 8,
 // S <= 2048: 359 and 370).  Packed rows: a walk ends with its document, so the longest document's first blocks stand out more, and
-// the host does not see the documents: four slices up to 768 blocks of rows of 4096 keys and more (layer, seven documents in 8192 tokens: 801 us in two, 759 in four; six in 12000:
-// 1411 and 1385; 8192 tokens in ONE document: 2174 and 2192).
+// the host does not see the documents: four slices from 256 to 768 blocks of rows of 4096 keys and more.  Whole backward of one row of
+// 64 query heads, two slices / four, documents of up to 1500 tokens, up to 4096, 1500 to 6000, and ONE: 8192 tokens 367 / 373,
+// 602 / 568, 994 / 924, 1683 / 1689 us; 12288 (768 blocks) 554 / 557, 970 / 963, 1296 / 1254, 3826 / 3712; beyond the line 14000 571 / 593,
+// 872 / 866, 1508 / 1501, 4913 / 4875 and 16384 687 / 711, 928 / 941, 1623 / 1631, 6636 / 6690.  (Two rows of 4096, 512 blocks, would
+// rather have two: 340 / 359, 526 / 513, 864 / 902, 904 / 919.)
 int dkdv_parts_for(const gptoss_attn_params *p, bool padded, bool packed) {
     if (p->dtype == GPTOSS_ATTN_FP32) {
         // a workgroup per 32 keys, two per compute unit: about four workgroups per unit of a 256-CU part, so that the long
@@ -232,9 +236,9 @@ int decode_splits(const gptoss_attn_params *p) {
 }
 
 // float32 forward and dQ: wavefronts that share a unit (32 query rows of one head).  Few units: four, so that the chip fills and
-// a row's keys are walked four at a time (64 heads, S = 256: forward 16 us; 19 with two, 30 with one); more than 1024: two (S = 1024: 101 us
-// forward, 131 dQ; 100 and 132 with four, 119 and 160 with one), and for a window's handful of tiles one (window 128, S =
-// 1024: 36 and 46 us; 40 and 51 with two, 48 and 62 with four).
+// a row's keys are walked four at a time (64 heads, S = 256: forward 15 us; 18 with two, 29 with one); more than 1024: two (S = 1024: 101 us
+// forward, 136 dQ; 100 and 136 with four, 121 and 164 with one), and for a window's handful of tiles one (window 128, S =
+// 1024: 36 and 47 us; 40 and 53 with two, 49 and 68 with four).
 int f32_key_splits(const KArgs &a) {
     const int64_t units = (int64_t)a.B * a.H * ((a.Sq + 31) / 32);
     return units <= 1024 ? 4 : (a.window > 0 && a.window <= 512 ? 1 : 2);

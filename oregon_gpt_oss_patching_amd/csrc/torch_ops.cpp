@@ -7,8 +7,8 @@
 //
 // Why native: the calls of a training step on short rows take less time on the GPU than their host side took in Python
 // (an autograd.Function around two Python custom operators and a ctypes call each: 250 us per forward + backward
-// whatever the size; the same calls through this file take 101 us for two rows of 383 tokens or a sliding-window layer of 4096, of
-// which 72 and 90 are kernels, and a decoding step 18 us instead of 44).  This file is built against torch; the kernels are not.
+// whatever the size; the same calls through this file take 60 to 90 us for two rows of 383 tokens, 88 for a sliding-window layer of
+// 4096, of which 64 and 83 are kernels, and a decoding step 13 us instead of 44).  This file is built against torch; the kernels are not.
 #include <ATen/ATen.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
