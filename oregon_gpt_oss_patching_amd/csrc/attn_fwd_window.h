@@ -159,17 +159,17 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_window_kernel(const KArgs a) 
     // output in o, the row's reference m and this lane's share l of the row sum.
     f32x16 o[2];
     float m, l;
-    // O += P V of step u (16 keys) of the staged block h.  rest: the weights' rounding to bf16 goes through the matrix pipe as well, for one step
-    // of a block (GENERAL only).  Why: attn_fwd_kernel, which took these calls before, rounds its weights against a running maximum,
-    // and every key that sets a new one has the weight 1, exactly; against the final maximum only one key does.  O's error from
-    // float64 was 0.5 to 1.7 % larger for it.  One step without rounding, of the eight a window of 128 has, brings it below (3001
-    // tokens: 2.143e-3, 2.071e-3 so, 2.109e-3 with a running maximum) and costs 0.6 us of the 115 of B = 2, forward + backward.
-    auto add_values = [&](int h, int u, const f32x16 &p, bool first, bool rest) __attribute__((always_inline)) {
+    // O += P V of step u (16 keys) of the staged block h.  rest (GENERAL only): those of a lane's eight weights send their rounding
+    // to bf16 through the matrix pipe as well, an eighth of what a row sees.  Why: attn_fwd_kernel, which took these calls before, rounds
+    // its weights against a running maximum, and every key that sets a new one has the weight 1, exactly; against the final
+    // maximum only one key does.  O's error from float64 was 0.5 to 1.7 % larger for it; with an eighth unrounded it is 1 to 2 %
+    // smaller (3001 tokens, window 128: 2.143e-3, 2.090e-3 so, 2.109e-3 with a running maximum).  It costs 0.6 us of the
+    // 115 of B = 2, forward + backward.
+    auto add_values = [&](int h, int u, const f32x16 &p, bool first, unsigned rest) __attribute__((always_inline)) {
         const bf16x8 pf = cfrag(p, u);
         bf16x8 pr;
-        if (rest)
 #pragma unroll
-            for (int j = 0; j < 8; ++j) pr[j] = (bf16)(p[8 * u + j] - (float)pf[j]);
+        for (int j = 0; j < 8; ++j) pr[j] = rest >> j & 1 ? (bf16)(p[8 * u + j] - (float)pf[j]) : (bf16)0.0f;
 #pragma unroll
         for (int dblk = 0; dblk < 2; ++dblk) {
             const bf16x8 av = ofrag_tr(vsm, lo, h, u, dblk);
@@ -233,7 +233,7 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_window_kernel(const KArgs a) 
             }
             auto pv = [&](int h, const f32x16 &p, auto first_tag, bool rest) __attribute__((always_inline)) {
 #pragma unroll
-                for (int u = 0; u < 2; ++u) add_values(X + h, u, p, decltype(first_tag)::value && u == 0, GENERAL && rest && u == 0);
+                for (int u = 0; u < 2; ++u) add_values(X + h, u, p, decltype(first_tag)::value && u == 0, GENERAL && rest && u == 0 ? (1u << W / 16) - 1 : 0u);
             };
             pv(0, pa, std::true_type{}, NH == 2);
             pv(NH - 1, pb, std::false_type{}, NH == 2);
@@ -282,7 +282,7 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_window_kernel(const KArgs a) 
                     rs0 += e0; rs1 += e1;
                 }
 #pragma unroll
-                for (int u = 0; u < 2; ++u) add_values(X + h, u, s[h], h == 0 && u == 0, GENERAL && h == NH - 1);
+                for (int u = 0; u < 2; ++u) add_values(X + h, u, s[h], h == 0 && u == 0, GENERAL && h == NH - 1 ? 1u << 3 : 0u);
             }
             l = rs0 + rs1;
         }
