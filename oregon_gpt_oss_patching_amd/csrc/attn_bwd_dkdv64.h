@@ -177,13 +177,14 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv64_kernel(const KArgs a) 
     // per request: on to the next head, or (after the last head of the group) back to the first head of the tile below
     const uint32_t q_step = (uint32_t)a.qs.h * 2u, q_wrap = 0u - ((uint32_t)(a.r - 1) * (uint32_t)a.qs.h + (uint32_t)kTile * (uint32_t)a.qs.s) * 2u;
     const uint32_t g_step = (uint32_t)a.dos.h * 2u, g_wrap = 0u - ((uint32_t)(a.r - 1) * (uint32_t)a.dos.h + (uint32_t)kTile * (uint32_t)a.dos.s) * 2u;
-    // GENERAL: a tile that sticks out of the tensor is the first one of its walk; while the walk is on it, the lanes whose rows
-    // do not exist stay on the last row that does: their offsets are `over` rows short, which the move to the tile below adds.
+    // GENERAL: a tile that sticks out of the rows that exist (the tensor, or a padded row's length: what padding holds must not
+    // matter, 0 * NaN) is the first one of its walk; while the walk is on it, the lanes whose rows do not exist stay on the last
+    // row that does: their offsets are `over` rows short, which the move to the tile below adds.
     uint32_t cq0 = 0, cq1 = 0, cg0 = 0, cg1 = 0, cs = 0;
     bool on_end = false;
     if constexpr (GENERAL) {
-        on_end = nq > 0 && t_base + t_first == n_tiles;
-        const int last = a.Sq - 1 - n_tiles * kTile;
+        const int n_whole = len / kTile, last = len - 1 - n_whole * kTile;
+        on_end = nq > 0 && t_base + t_first == n_whole;
         const uint32_t over0 = on_end ? max(C::kWaveRows * w + (lane >> 3) - last, 0) : 0, over1 = on_end ? max(C::kWaveRows * w + 8 + (lane >> 3) - last, 0) : 0;
         cq0 = over0 * (uint32_t)a.qs.s * 2u; cq1 = over1 * (uint32_t)a.qs.s * 2u;
         cg0 = over0 * (uint32_t)a.dos.s * 2u; cg1 = over1 * (uint32_t)a.dos.s * 2u;

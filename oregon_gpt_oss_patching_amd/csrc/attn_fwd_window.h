@@ -105,7 +105,7 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_window_kernel(const KArgs a) 
     const char *const qblk0 = reinterpret_cast<const char *>(a.q + (int64_t)b * a.qs.b + (int64_t)head * a.qs.h + (int64_t)r0 * a.qs.s);
     auto load_q = [&](int X) __attribute__((always_inline)) {
         const int ln = fresh_lane();
-        const int row = GENERAL ? min(ln & 31, a.Sq - 1 - r0 - 32 * X) : ln & 31;
+        const int row = GENERAL ? min(ln & 31, len - 1 - r0 - 32 * X) : ln & 31;        // (what padded rows hold must not matter)
         const uint32_t qoff = (uint32_t)(row * (int)a.qs.s + 8 * (ln >> 5)) * 2u;
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks)
