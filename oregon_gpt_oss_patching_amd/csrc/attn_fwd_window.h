@@ -115,17 +115,18 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_window_kernel(const KArgs a) 
     const uint32_t ksm = lds_addr(smem), vsm = ksm + C::kKBytes;
     {
         // copy j of wavefront w fills rows 8 (w + 4 j) .. + 7 of the staged range (the second block's own 32 keys, j = NH,
-        // only where that block exists); rows in front of key 0 re-read key 0 (their logits are masked, they only have
-        // to be finite), rows behind the last query's position re-read its key (nobody may have written them yet: 0 * NaN)
+        // only where that block exists); rows in front of key 0, or of the first row's document, re-read its first key (their logits
+        // are masked, they only have to be finite), rows behind the last query's position re-read its key (nobody may have written them yet: 0 * NaN)
         const int rloc = 8 * w + (lane >> 3);
         const int ch = (lane & 7) ^ swz(rloc);     // swz() of the row: 32 j does not reach the bits it looks at
         const bf16 *kbase = a.k + (int64_t)b * a.ks.b + (int64_t)g * a.ks.h, *vbase = a.v + (int64_t)b * a.vs.b + (int64_t)g * a.vs.h;
         const int key_end = GENERAL ? min(a.Skv, off + len) : a.Skv;
+        const int key_0 = GENERAL && a.doc_start ? max(__builtin_amdgcn_readfirstlane(a.doc_start[(int64_t)b * a.Sq + r0]), 0) : 0;
         char *kdst = smem + w * 8 * kRowBytes, *vdst = smem + C::kKBytes + w * 8 * kRowBytes;
         // addresses are (scalar pointer) + (32-bit lane offset): the row of copy j is a scalar step away from copy 0's,
-        // except where rows are held at key 0
+        // except where rows are held at the first or the last key
         auto copy_all = [&](const bf16 *base, int stride, char *dst) __attribute__((always_inline)) {
-            if (k0 >= 0 && (!GENERAL || k0 + 32 * (NH + 1) <= key_end)) {
+            if (k0 >= key_0 && (!GENERAL || k0 + 32 * (NH + 1) <= key_end)) {
                 const uint32_t voff = (uint32_t)(rloc * stride + ch * 8) * 2u;
 #pragma unroll
                 for (int j = 0; j <= NH; ++j)
@@ -136,7 +137,7 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_window_kernel(const KArgs a) 
 #pragma unroll
                 for (int j = 0; j <= NH; ++j)
                     if (j < NH || live1) {
-                        const int first = GENERAL ? min(max(k0, 0), key_end - 1) : 0, row = max(k0 + rloc + 32 * j, first);
+                        const int first = GENERAL ? min(max(k0, key_0), key_end - 1) : 0, row = max(k0 + rloc + 32 * j, first);
                         const uint32_t voff = (uint32_t)((GENERAL ? min(row, key_end - 1) - first : row) * stride + ch * 8) * 2u;
                         __builtin_amdgcn_global_load_lds((glb_void_t *)(reinterpret_cast<const char *>(base + (GENERAL ? (int64_t)first * stride : 0)) + voff),
                                                          (lds_void_t *)(dst + j * 32 * kRowBytes), 16, 0, 0);
