@@ -162,6 +162,13 @@ size_t gptoss_attn_bwd_workspace_bytes(const gptoss_attn_params *params);
 size_t gptoss_attn_fwd_workspace_bytes(const gptoss_attn_params *params);
 
 /*
+ * Bytes of scratch with which float32 calls run on the bf16 matrix pipes, every operand cut into three bf16 terms (no less precise, about
+ * twice as fast; 0 where the call has no such route): for gptoss_attn_fwd_scratch (backward == 0) or gptoss_attn_bwd_scratch
+ * (backward != 0).  Not part of gptoss_attn_workspace_bytes.  Host-only.
+ */
+size_t gptoss_attn_split_bytes(const gptoss_attn_params *params, int backward);
+
+/*
  * Forward: O and logsumexp.  Replaces the `_attn_fwd` launch in
  * `_attention.forward` (attention_kernel.py:11-100, 241-262) including the
  * output transpose copy at :272 (O is written directly in the caller's layout).
@@ -179,6 +186,7 @@ int gptoss_attn_fwd_sinks(const gptoss_attn_params *params, int sinks_dtype, voi
  * The same with scratch of the caller's for few queries on a long cache: `scratch` (16-byte aligned) holds `scratch_bytes` bytes, which
  * no other call may use until this one has run.  With NULL, or with fewer bytes than gptoss_attn_fwd_workspace_bytes gives
  * for the same block, the same kernel walks each row's keys uncut, as the two calls above do (O then agrees to one bf16 rounding).
+ * float32 calls take gptoss_attn_split_bytes(params, 0) bytes; with less they run on the fp32 matrix instruction, as the two calls above do.
  */
 int gptoss_attn_fwd_scratch(const gptoss_attn_params *params, int sinks_dtype, void *scratch, size_t scratch_bytes, void *stream);
 
@@ -233,6 +241,12 @@ int gptoss_attn_bwd(const gptoss_attn_params *params, void *stream);
  * params->sinks and params->dsinks point at H of them); a bf16 gradient is the fp32 sum rounded once.
  */
 int gptoss_attn_bwd_sinks(const gptoss_attn_params *params, int sinks_dtype, int dsinks_dtype, void *stream);
+
+/*
+ * The same with scratch besides `delta`: `scratch` (16-byte aligned) holds `scratch_bytes` bytes, gptoss_attn_split_bytes(params, 1) for
+ * float32 calls.  With NULL or less it is gptoss_attn_bwd_sinks.
+ */
+int gptoss_attn_bwd_scratch(const gptoss_attn_params *params, int sinks_dtype, int dsinks_dtype, void *scratch, size_t scratch_bytes, void *stream);
 
 /*
  * The whole backward without any workspace from the caller and without any allocation: a variant

@@ -32,6 +32,8 @@ EXPORTS = (
     "gptoss_attn_bwd_dq",
     "gptoss_attn_bwd",
     "gptoss_attn_bwd_sinks",
+    "gptoss_attn_bwd_scratch",
+    "gptoss_attn_split_bytes",
     "gptoss_attn_bwd_static",
     "gptoss_attn_static_scratch_bytes",
     "gptoss_attn_doc_start",
@@ -124,6 +126,11 @@ def load() -> ctypes.CDLL:
         lib.gptoss_attn_fwd_scratch.argtypes = [ctypes.POINTER(Params), ctypes.c_int, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]
         lib.gptoss_attn_bwd_sinks.restype = ctypes.c_int
         lib.gptoss_attn_bwd_sinks.argtypes = [ctypes.POINTER(Params), ctypes.c_int, ctypes.c_int, ctypes.c_void_p]
+        lib.gptoss_attn_bwd_scratch.restype = ctypes.c_int
+        lib.gptoss_attn_bwd_scratch.argtypes = [ctypes.POINTER(Params), ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_size_t,
+                                                ctypes.c_void_p]
+        lib.gptoss_attn_split_bytes.restype = ctypes.c_size_t
+        lib.gptoss_attn_split_bytes.argtypes = [ctypes.POINTER(Params), ctypes.c_int]
         if lib.gptoss_attn_version() != ABI_VERSION:
             raise RuntimeError("libgptoss_attn.so ABI version mismatch; rebuild the library")
         _lib = lib

@@ -191,7 +191,8 @@ def attention_forward(q, k, v, sinks, sm_scale, window=None, q_offset=0, seqlens
         p = _base_params(q, k, v, sinks32, sl, sm_scale, window, q_offset, ds, qod)
         p.o, p.lse = o.data_ptr(), lse.data_ptr()
         _set(p.o_stride, _strides_bhs(o, "bshd"))
-        need = _lib.load().gptoss_attn_fwd_workspace_bytes(p)      # partial results of few queries' rows, cut over their keys
+        # partial results of few queries' rows, cut over their keys; records of float32 operands
+        need = max(_lib.load().gptoss_attn_fwd_workspace_bytes(p), _lib.load().gptoss_attn_split_bytes(p, 0))
         scratch = torch.empty((need // 4,), dtype=torch.float32, device=q.device) if need else None
         _lib.call("gptoss_attn_fwd_scratch", p, _stream(q), _lib.DTYPE_FP32, scratch.data_ptr() if need else None, need)
     return o, lse
@@ -199,8 +200,8 @@ def attention_forward(q, k, v, sinks, sm_scale, window=None, q_offset=0, seqlens
 
 def attention_backward(q, k, v, sinks, o, lse, d_o, sm_scale, window=None, q_offset=0, seqlens=None,
                        need_dsinks=True, doc_start=None, split=False, q_offset_dev=None):
-    """Runs the backward: `gptoss_attn_bwd`, or with `split=True` the three separate entry points
-    (preprocess, dK/dV, dQ), which give the same bits.  o and d_o are (B,S,H,D).
+    """Runs the backward: `gptoss_attn_bwd_scratch`, or with `split=True` the three separate entry points
+    (preprocess, dK/dV, dQ), which give the same bits for bfloat16 tensors.  o and d_o are (B,S,H,D).
     Returns (dq, dk, dv, dsinks_fp32_or_None)."""
     _check_inputs(q, k, v, sinks)
     _check_saved(q, o, lse, d_o)
@@ -230,9 +231,13 @@ def attention_backward(q, k, v, sinks, o, lse, d_o, sm_scale, window=None, q_off
         _set(p.dv_stride, _strides_bhs(dv, "bhsd"))
         p.delta = delta.data_ptr()
         p.dsinks = dsinks.data_ptr() if dsinks is not None else None
-        for name in (("gptoss_attn_bwd_preprocess", "gptoss_attn_bwd_dkdv", "gptoss_attn_bwd_dq") if split
-                     else ("gptoss_attn_bwd",)):
-            _lib.call(name, p, _stream(q))
+        if split:
+            for name in ("gptoss_attn_bwd_preprocess", "gptoss_attn_bwd_dkdv", "gptoss_attn_bwd_dq"):
+                _lib.call(name, p, _stream(q))
+        else:
+            need = _lib.load().gptoss_attn_split_bytes(p, 1)
+            scratch = torch.empty((need // 4,), dtype=torch.float32, device=q.device) if need else None
+            _lib.call("gptoss_attn_bwd_scratch", p, _stream(q), _lib.DTYPE_FP32, _lib.DTYPE_FP32, scratch.data_ptr() if need else None, need)
     return dq, dk, dv, dsinks
 
 

@@ -61,6 +61,12 @@ struct KArgs {
     float *dsink_partial; // single-pass window backward: dSinks partial sums, [B][chunk][H][2]
     float *boundary_partial; // single-pass window backward: fp32 dK / dV shares of the tiles on chunk seams, or NULL
     bool sinks_bf16, dsinks_bf16;
+    // float32 on the bf16 matrix pipes (attn_f32_split.h): records of K / V and of Q / dO, which of them hold numbers the split does
+    // not take, steps per dK/dV workgroup, parts of all key blocks of a row, their partial sums (or NULL)
+    char *split_kv, *split_q;
+    uint32_t *split_kv_bad, *split_q_bad;
+    int split_steps, split_slots;
+    float *split_partial;
 };
 
 // The sink logits and their gradient in the type the caller's parameter has: a conversion of 64 numbers was a launch of its own

@@ -1,6 +1,7 @@
 // float32 kernels (dtype GPTOSS_ATTN_FP32): the same forward / backward as the bf16 kernels
 // for callers that keep the model in float32 (the reference runs such tensors natively,
-// attention_kernel.py:11-217 are dtype-generic).  Every product runs on the fp32 matrix instruction
+// attention_kernel.py:11-217 are dtype-generic).  Larger problems take the kernels of attn_f32_split.h, which come here for the numbers they
+// do not hold; the rest starts here.  Every product runs on the fp32 matrix instruction
 // v_mfma_f32_32x32x2_f32 with fp32 operands and fp32 accumulation.
 //
 // What bounds them: that instruction takes 64 cycles for 4096 FLOP (157 TFLOP/s on the chip), sixteen times the bf16
@@ -144,16 +145,16 @@ __device__ __forceinline__ void f32_cols_product(f32x16 (&acc)[2], uint32_t tile
 // Where a wavefront of the forward / dQ kernels stands: 32 query rows of one head (a unit; 4 / KS units per workgroup) and
 // every KS-th of the 32-key tiles they see.
 struct F32Unit { int head, b, q0; bool live; };
-template <int KS>
+template <int KS, int NW = 4>
 struct F32QueryWork {
-    int g, b, head, q0, q_len, kv_len, weff, pos0, pos1, ds1, t0, n_it, w, lane;
+    int g, b, head, q0, q_len, kv_len, weff, pos0, pos1, ds1, t_lo, n, t0, n_it, w, lane;
     const float *kbase, *vbase;
     uint32_t ksm, vsm;         // this wavefront's K and V tile in LDS
     // unit i of the workgroup: KV head fastest (its K / V stay in one XCD's L2), then the heads of the group, longest key loops first
     static __device__ __forceinline__ F32Unit unit(const KArgs &a, int i) {
         F32Unit u;
         const int g = (int)(blockIdx.x % a.G);
-        int n = (int)(blockIdx.x / a.G) * (4 / KS) + i;
+        int n = (int)(blockIdx.x / a.G) * (NW / KS) + i;
         u.head = g * a.r + n % a.r; n /= a.r;
         const int bi = n % a.B, z = n / a.B, n_q = (a.Sq + 31) / 32;
         u.b = rotated_batch_row(bi, z, a.B);
@@ -177,8 +178,8 @@ struct F32QueryWork {
         const int ds0 = dsrow ? dsrow[min(q0, a.Sq - 1)] : 0;
         ds1 = dsrow ? dsrow[min(q0 + 31, a.Sq - 1)] : 0;
         const int hi = pos1 >= pos0 && u.live ? max(0, min(kv_len, pos1 + 1)) : 0;
-        const int t_lo = max(max(0, pos0 - weff + 1), ds0) / F32Tile::kRows;
-        const int n = max(0, (hi + F32Tile::kRows - 1) / F32Tile::kRows - t_lo);
+        t_lo = max(max(0, pos0 - weff + 1), ds0) / F32Tile::kRows;
+        n = max(0, (hi + F32Tile::kRows - 1) / F32Tile::kRows - t_lo);
         t0 = t_lo + w % KS;
         n_it = (n - w % KS + KS - 1) / KS;               // tiles t0 + KS it  (0 if n <= w % KS)
         kbase = t.k + (int64_t)b * a.ks.b + (int64_t)g * a.ks.h;
@@ -222,12 +223,51 @@ __device__ __forceinline__ f32x4 f32_partial(const char *smem, int wave_bytes, i
 }
 
 // ---- forward ------------------------------------------------------------------------
-template <int KS>
-__global__ __launch_bounds__(256, 2) void attn_f32_fwd_kernel(const KArgs a) {
-    __shared__ __attribute__((aligned(1024))) char smem[8 * F32Tile::kBytes];
+// (the merge of the wavefronts' shares: m, l and O of each in its own registers)
+template <int KS, int NW>
+__device__ __forceinline__ void f32_fwd_merge(const KArgs &a, const F32Ptrs &t, char *smem, int w, int lane, float m, float l, const f32x16 (&o)[2]) {
+    using W = F32QueryWork<KS, NW>;
+    const int l32 = lane & 31, half = lane >> 5;
+    // merge: the row's reference is the largest of the KS wavefronts', z and O are scaled to it
+    float *const ml = reinterpret_cast<float *>(smem + NW * F32Tile::kBytes);       // [wavefront][m, l][row]
+    const float l_tot = xhalf_sum(l);
+    __syncthreads();
+    f32_leave_partial(smem + w * F32Tile::kBytes, o, lane);
+    if (half == 0) { ml[(2 * w) * 32 + l32] = m; ml[(2 * w + 1) * 32 + l32] = l_tot; }
+    __syncthreads();
+#pragma unroll
+    for (int pass = 0; pass < 8 / KS; ++pass) {                     // a pass takes NW / 8 units
+        const int u16 = (threadIdx.x >> 4) + 4 * NW * pass, i = u16 >> 5, r = u16 & 31, ch = threadIdx.x & 15;
+        const F32Unit u = W::unit(a, i);
+        const float sink = sink_logit(a, u.head) * kLog2e;
+        float mm = fast_max(sink, kNoLogit);
+#pragma unroll
+        for (int k = 0; k < KS; ++k) mm = fast_max(mm, ml[2 * (KS * i + k) * 32 + r]);
+        float z = exp2f(sink - mm);
+        f32x4 x = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int k = 0; k < KS; ++k) {
+            const float f = exp2f(ml[2 * (KS * i + k) * 32 + r] - mm);
+            z += f * ml[(2 * (KS * i + k) + 1) * 32 + r];
+            const f32x4 y = f32_partial(smem, F32Tile::kBytes, KS * i + k, r, ch);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[e] = fmaf(f, y[e], x[e]);
+        }
+        const float inv = 1.0f / z;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[e] *= inv;
+        if (u.live && u.q0 + r < a.Sq) {
+            *reinterpret_cast<f32x4 *>(t.o + (int64_t)u.b * a.os.b + (int64_t)u.head * a.os.h + (int64_t)(u.q0 + r) * a.os.s + 4 * ch) = x;
+            if (ch == 0) a.lse[((int64_t)u.b * a.H + u.head) * a.Sq + u.q0 + r] = (mm + log2f(z)) * kLn2;
+        }
+    }
+}
+// The forward of a workgroup of NW wavefronts (16 KB of LDS each).
+template <int KS, int NW>
+__device__ __forceinline__ void f32_fwd_rows(const KArgs &a, char *smem) {
     const int q_offset = query_offset(a);
     const F32Ptrs t = f32_ptrs(a);
-    using W = F32QueryWork<KS>;
+    using W = F32QueryWork<KS, NW>;
     const W wk(a, t, q_offset, smem);
     const int lane = wk.lane, l32 = lane & 31, half = lane >> 5, row = wk.q0 + l32;
     int pos;
@@ -286,39 +326,12 @@ __global__ __launch_bounds__(256, 2) void attn_f32_fwd_kernel(const KArgs a) {
         if (more) wk.request_v(a, it + 1);
     }
 
-    // merge: the row's reference is the largest of the KS wavefronts', z and O are scaled to it
-    float *const ml = reinterpret_cast<float *>(smem + 4 * F32Tile::kBytes);       // [wavefront][m, l][row]
-    const float l_tot = xhalf_sum(l);
-    __syncthreads();
-    f32_leave_partial(smem + wk.w * F32Tile::kBytes, o, lane);
-    if (half == 0) { ml[(2 * wk.w) * 32 + l32] = m; ml[(2 * wk.w + 1) * 32 + l32] = l_tot; }
-    __syncthreads();
-#pragma unroll
-    for (int pass = 0; pass < 8 / KS; ++pass) {
-        const int i = pass >> 1, r = (threadIdx.x >> 4) + 16 * (pass & 1), ch = threadIdx.x & 15;
-        const F32Unit u = W::unit(a, i);
-        const float sink = sink_logit(a, u.head) * kLog2e;
-        float mm = fast_max(sink, kNoLogit);
-#pragma unroll
-        for (int k = 0; k < KS; ++k) mm = fast_max(mm, ml[2 * (KS * i + k) * 32 + r]);
-        float z = exp2f(sink - mm);
-        f32x4 x = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int k = 0; k < KS; ++k) {
-            const float f = exp2f(ml[2 * (KS * i + k) * 32 + r] - mm);
-            z += f * ml[(2 * (KS * i + k) + 1) * 32 + r];
-            const f32x4 y = f32_partial(smem, F32Tile::kBytes, KS * i + k, r, ch);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) x[e] = fmaf(f, y[e], x[e]);
-        }
-        const float inv = 1.0f / z;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) x[e] *= inv;
-        if (u.live && u.q0 + r < a.Sq) {
-            *reinterpret_cast<f32x4 *>(t.o + (int64_t)u.b * a.os.b + (int64_t)u.head * a.os.h + (int64_t)(u.q0 + r) * a.os.s + 4 * ch) = x;
-            if (ch == 0) a.lse[((int64_t)u.b * a.H + u.head) * a.Sq + u.q0 + r] = (mm + log2f(z)) * kLn2;
-        }
-    }
+    f32_fwd_merge<KS, NW>(a, t, smem, wk.w, lane, m, l, o);
+}
+template <int KS>
+__global__ __launch_bounds__(256, 2) void attn_f32_fwd_kernel(const KArgs a) {
+    __shared__ __attribute__((aligned(1024))) char smem[8 * F32Tile::kBytes];
+    f32_fwd_rows<KS, 4>(a, smem);
 }
 
 // ---- backward step 1: -delta and lse*log2(e) into the scratch (same layout as the bf16 path) ----
@@ -355,20 +368,42 @@ struct F32Dkdv {
     static constexpr int kStatOff = 8 * F32Tile::kBytes;
     static constexpr int kLdsBytes = kStatOff + 4 * kStatBytes;
 };
-__global__ __launch_bounds__(256, 2) void attn_f32_dkdv_kernel(const KArgs a) {
+// The 32-row query tiles [t_lo, t_hi) whose rows can see any key of [j0, j0 + keys): positions [j0, last key + window), within the
+// documents of the keys.
+struct F32TileSpan { int t_lo, t_hi, row_lim; };
+__device__ __forceinline__ F32TileSpan f32_tiles_of_keys(const KArgs &a, int q_offset, int b, int j0, int keys, int lane) {
+    const int kv_len = a.seqlens ? min(a.Skv, a.seqlens[b]) : a.Skv;
+    const int q_len = a.seqlens ? a.seqlens[b] : 0x7fffffff;
+    const int j1 = min(j0 + keys, kv_len) - 1;
+    const int32_t *dsrow = a.doc_start ? a.doc_start + (int64_t)b * a.Sq : nullptr;
+    const int weff = a.window ? a.window : 0x3fffffff;
+    F32TileSpan x;
+    x.row_lim = (int)min((int64_t)a.Sq, max((int64_t)0, (int64_t)q_len - q_offset));
+    const int row_lo = max(0, j0 - q_offset);
+    int row_hi = j1 >= j0 ? (int)min((int64_t)x.row_lim, max((int64_t)0, (int64_t)j1 + weff - q_offset)) : 0;
+    if (dsrow && row_hi > row_lo) row_hi = min(row_hi, document_end(dsrow, a.Sq, j1, lane));
+    x.t_lo = row_lo / 32;
+    x.t_hi = max(x.t_lo, (row_hi + 31) / 32);
+    return x;
+}
+// Step `it` of a walk over (query tile, head): `each` consecutive tiles of a head, the heads of the group, the tiles after these.
+// Tiles outside [t_from, t_to) have no row that sees the keys and are passed over.
+struct F32Walk {
+    int t0, t_end, each, first, n_it, t_from, t_to;
+    __device__ __forceinline__ int tile(int it, int r) const { return t0 + each * ((first + it / each) / r) + it % each; }
+    __device__ __forceinline__ int head(int it, int r) const { return (first + it / each) % r; }
+};
+// dK, dV of 32 keys from j0 over a walk (its steps dealt to the NW wavefronts in turn); out: fp32 partial sums, rows of 64 floats, or
+// NULL for the scaled results
+template <int NW>
+__device__ __forceinline__ void f32_dkdv_keys(const KArgs &a, char *smem, int g, int b, int j0, const F32Walk walk, float *out_k, float *out_v) {
     using C = F32Dkdv;
-    __shared__ __attribute__((aligned(1024))) char smem[C::kLdsBytes];
     const int q_offset = query_offset(a);
     const F32Ptrs t = f32_ptrs(a);
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, half = lane >> 5;
-    int bid = blockIdx.x;
-    const int g = bid % a.G; bid /= a.G;
-    const int bi = bid % a.B; bid /= a.B;
-    const int part = bid % a.dkdv_parts, kblk = bid / a.dkdv_parts;       // ascending: most work first
-    const int b = rotated_batch_row(bi, kblk, a.B);
     const int kv_len = a.seqlens ? min(a.Skv, a.seqlens[b]) : a.Skv;
     const int q_len = a.seqlens ? a.seqlens[b] : 0x7fffffff;
-    const int j0 = 32 * kblk, key = j0 + l32, j1 = min(j0 + 32, kv_len) - 1;
+    const int key = j0 + l32;
     const int64_t total = (int64_t)a.B * a.H * a.Sq;
     const int32_t *dsrow = a.doc_start ? a.doc_start + (int64_t)b * a.Sq : nullptr;
 
@@ -379,35 +414,34 @@ __global__ __launch_bounds__(256, 2) void attn_f32_dkdv_kernel(const KArgs a) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) { dk[0][i] = dk[1][i] = 0.0f; dv[0][i] = dv[1][i] = 0.0f; }
 
-    // query rows that can see any key of the block: positions [j0, j1 + window), within the documents of the keys
     const int weff = a.window ? a.window : 0x3fffffff;
     const int row_lim = (int)min((int64_t)a.Sq, max((int64_t)0, (int64_t)q_len - q_offset));
-    const int row_lo = max(0, j0 - q_offset);
-    int row_hi = j1 >= j0 ? (int)min((int64_t)row_lim, max((int64_t)0, (int64_t)j1 + weff - q_offset)) : 0;
-    if (dsrow && row_hi > row_lo) row_hi = min(row_hi, document_end(dsrow, a.Sq, j1, lane));
-    const int t_lo = row_lo / 32, n_tiles = max(0, (row_hi + 31) / 32 - t_lo);
-    const int slice = (n_tiles + a.dkdv_parts - 1) / a.dkdv_parts;
-    const int t0 = t_lo + part * slice, n_it = max(0, min(slice, n_tiles - part * slice)) * a.r;
+    const int n_it = walk.n_it;
 
     const uint32_t qsm = lds_addr(smem) + w * (2 * F32Tile::kBytes), gsm = qsm + F32Tile::kBytes;
-    const uint32_t ssm = lds_addr(smem) + C::kStatOff + w * C::kStatBytes;
+    const uint32_t ssm = lds_addr(smem) + NW * 2 * F32Tile::kBytes + w * C::kStatBytes;
     const F32Offsets lo = make_f32_offsets(lane);
     const float c = a.scale_log2;
-    // requests for step `it` (query tile t0 + it / r, head it % r): the Q tile; the dO tile and the row statistics
+    // requests for step `it`: the Q tile; the dO tile and the row statistics (a tile past the last one re-reads that one)
     auto request_q = [&](int it) __attribute__((always_inline)) {
-        const int q0 = 32 * (t0 + it / a.r), head = g * a.r + it % a.r;
+        const int q0 = 32 * min(walk.tile(it, a.r), walk.t_end - 1), head = g * a.r + walk.head(it, a.r);
         f32_copy_tile(qsm, t.q + (int64_t)b * a.qs.b + (int64_t)head * a.qs.h + (int64_t)q0 * a.qs.s, (int)a.qs.s, a.Sq - 1 - q0, lane);
     };
     auto request_g = [&](int it) __attribute__((always_inline)) {
-        const int q0 = 32 * (t0 + it / a.r), head = g * a.r + it % a.r;
+        const int q0 = 32 * min(walk.tile(it, a.r), walk.t_end - 1), head = g * a.r + walk.head(it, a.r);
         f32_copy_tile(gsm, t.d_o + (int64_t)b * a.dos.b + (int64_t)head * a.dos.h + (int64_t)q0 * a.dos.s, (int)a.dos.s, a.Sq - 1 - q0, lane);
         lds_dma4(ssm, a.delta + ((int64_t)b * a.H + head) * a.Sq, ((half ? (uint32_t)total : 0u) + (uint32_t)min(q0 + l32, a.Sq - 1)) * 4u);
     };
     if (w < n_it) { request_g(w); request_q(w); }
     wait_vmcnt<0>();         // the compiler's own loads have arrived: no vmcnt wait of its own in the loop
-    for (int it = w; it < n_it; it += 4) {
-        const int q0 = 32 * (t0 + it / a.r);
-        const bool more = it + 4 < n_it;
+    for (int it = w; it < n_it; it += NW) {
+        const int tile = walk.tile(it, a.r), q0 = 32 * tile;
+        const bool more = it + NW < n_it;
+        if (tile < walk.t_from || tile >= walk.t_to) {
+            GPTOSS_F32_WAIT(0);
+            if (more) { request_g(it + NW); request_q(it + NW); }
+            continue;
+        }
         GPTOSS_F32_WAIT(F32Tile::kCopies);                             // dO and the statistics are here; Q may be on its way
         f32x16 s, dp;
 #pragma unroll
@@ -440,31 +474,30 @@ __global__ __launch_bounds__(256, 2) void attn_f32_dkdv_kernel(const KArgs a) {
         // dV^T[d][key] += dO^T[d][row] P[row][key];  dK^T[d][key] += Q^T[d][row] dS[row][key]
         f32_cols_product(dv, gsm, lo, s);
         GPTOSS_F32_READS_DONE();
-        if (more) request_g(it + 4);
+        if (more) request_g(it + NW);
         f32_cols_product(dk, qsm, lo, dp);
         GPTOSS_F32_READS_DONE();
-        if (more) request_q(it + 4);
+        if (more) request_q(it + NW);
     }
 
-    // the four wavefronts' sums, added in wavefront order
-    const int64_t tensor = (int64_t)a.B * a.G * a.Skv * kD;
+    // the wavefronts' sums, added in wavefront order
     __syncthreads();
     f32_leave_partial(smem + w * (2 * F32Tile::kBytes), dk, lane);
     f32_leave_partial(smem + w * (2 * F32Tile::kBytes) + F32Tile::kBytes, dv, lane);
     __syncthreads();
 #pragma unroll
-    for (int pass = 0; pass < 4; ++pass) {
-        const int which = pass >> 1, r = (tid >> 4) + 16 * (pass & 1), ch = tid & 15, j = j0 + r;
+    for (int pass = 0; pass < 16 / NW; ++pass) {
+        const int row = (tid >> 4) + 4 * NW * pass, which = row >> 5, r = row & 31, ch = tid & 15, j = j0 + r;
         f32x4 x = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
+        for (int k = 0; k < NW; ++k) {
             const f32x4 y = f32_partial(smem + which * F32Tile::kBytes, 2 * F32Tile::kBytes, k, r, ch);
 #pragma unroll
             for (int e = 0; e < 4; ++e) x[e] += y[e];
         }
         if (j < a.Skv) {
-            if (a.dkdv_parts > 1) {
-                *reinterpret_cast<f32x4 *>(a.dkdv_partial + (int64_t)(2 * part + which) * tensor + (((int64_t)b * a.G + g) * a.Skv + j) * kD + 4 * ch) = x;
+            if (out_k) {
+                *reinterpret_cast<f32x4 *>((which == 0 ? out_k : out_v) + r * kD + 4 * ch) = x;
             } else {
                 const Strides &st = which == 0 ? a.dks : a.dvs;
                 const float mul = which == 0 ? a.scale : 1.0f;
@@ -474,6 +507,20 @@ __global__ __launch_bounds__(256, 2) void attn_f32_dkdv_kernel(const KArgs a) {
             }
         }
     }
+}
+__global__ __launch_bounds__(256, 2) void attn_f32_dkdv_kernel(const KArgs a) {
+    __shared__ __attribute__((aligned(1024))) char smem[F32Dkdv::kLdsBytes];
+    int bid = blockIdx.x;
+    const int g = bid % a.G; bid /= a.G;
+    const int bi = bid % a.B; bid /= a.B;
+    const int part = bid % a.dkdv_parts, kblk = bid / a.dkdv_parts;       // ascending: most work first
+    const int b = rotated_batch_row(bi, kblk, a.B), j0 = 32 * kblk;
+    const F32TileSpan span = f32_tiles_of_keys(a, query_offset(a), b, j0, 32, threadIdx.x & 63);
+    const int n_tiles = span.t_hi - span.t_lo, slice = (n_tiles + a.dkdv_parts - 1) / a.dkdv_parts;
+    const F32Walk walk{span.t_lo + part * slice, span.t_hi, 1, 0, max(0, min(slice, n_tiles - part * slice)) * a.r, span.t_lo, span.t_hi};
+    const int64_t tensor = (int64_t)a.B * a.G * a.Skv * kD;
+    float *out = a.dkdv_parts > 1 ? a.dkdv_partial + 2 * part * tensor + (((int64_t)b * a.G + g) * a.Skv + j0) * kD : nullptr;
+    f32_dkdv_keys<4>(a, smem, g, b, j0, walk, out, out ? out + tensor : nullptr);
 }
 
 // The slices' partial sums, added in slice order.  One thread per 16-byte output chunk.
@@ -504,12 +551,34 @@ __global__ __launch_bounds__(256) void attn_f32_dkdv_reduce_kernel(const KArgs a
 // ---- backward step 3: dQ ----------------------------------------------------------------
 // FUSE_DELTA: the kernel also forms -delta and lse * log2(e) of its rows, in the summation order of
 // attn_f32_delta_kernel, and leaves them in the scratch for the kernels that follow.
-template <int KS, bool FUSE_DELTA>
-__global__ __launch_bounds__(256, 2) void attn_f32_dq_kernel(const KArgs a) {
-    __shared__ __attribute__((aligned(1024))) char smem[8 * F32Tile::kBytes];
+template <int KS, int NW>
+__device__ __forceinline__ void f32_dq_merge(const KArgs &a, const F32Ptrs &t, char *smem, int w, int lane, float mul, const f32x16 (&dq)[2]) {
+    using W = F32QueryWork<KS, NW>;
+    __syncthreads();
+    f32_leave_partial(smem + w * F32Tile::kBytes, dq, lane);
+    __syncthreads();
+#pragma unroll
+    for (int pass = 0; pass < 8 / KS; ++pass) {
+        const int u16 = (threadIdx.x >> 4) + 4 * NW * pass, i = u16 >> 5, r = u16 & 31, ch = threadIdx.x & 15;
+        const F32Unit u = W::unit(a, i);
+        f32x4 x = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int k = 0; k < KS; ++k) {
+            const f32x4 y = f32_partial(smem, F32Tile::kBytes, KS * i + k, r, ch);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[e] += y[e];
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[e] *= mul;
+        if (u.live && u.q0 + r < a.Sq)
+            *reinterpret_cast<f32x4 *>(t.dq + (int64_t)u.b * a.dqs.b + (int64_t)u.head * a.dqs.h + (int64_t)(u.q0 + r) * a.dqs.s + 4 * ch) = x;
+    }
+}
+template <int KS, bool FUSE_DELTA, int NW>
+__device__ __forceinline__ void f32_dq_rows(const KArgs &a, char *smem) {
     const int q_offset = query_offset(a);
     const F32Ptrs t = f32_ptrs(a);
-    using W = F32QueryWork<KS>;
+    using W = F32QueryWork<KS, NW>;
     const W wk(a, t, q_offset, smem);
     const int lane = wk.lane, l32 = lane & 31, half = lane >> 5, row = wk.q0 + l32;
     const bool row_ok = row < a.Sq;
@@ -576,25 +645,12 @@ __global__ __launch_bounds__(256, 2) void attn_f32_dq_kernel(const KArgs a) {
         GPTOSS_F32_READS_DONE();
         if (more) wk.request_k(a, it + 1);
     }
-    __syncthreads();
-    f32_leave_partial(smem + wk.w * F32Tile::kBytes, dq, lane);
-    __syncthreads();
-#pragma unroll
-    for (int pass = 0; pass < 8 / KS; ++pass) {
-        const int i = pass >> 1, r = (threadIdx.x >> 4) + 16 * (pass & 1), ch = threadIdx.x & 15;
-        const F32Unit u = W::unit(a, i);
-        f32x4 x = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int k = 0; k < KS; ++k) {
-            const f32x4 y = f32_partial(smem, F32Tile::kBytes, KS * i + k, r, ch);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) x[e] += y[e];
-        }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) x[e] *= a.scale;
-        if (u.live && u.q0 + r < a.Sq)
-            *reinterpret_cast<f32x4 *>(t.dq + (int64_t)u.b * a.dqs.b + (int64_t)u.head * a.dqs.h + (int64_t)(u.q0 + r) * a.dqs.s + 4 * ch) = x;
-    }
+    f32_dq_merge<KS, NW>(a, t, smem, wk.w, lane, a.scale, dq);
+}
+template <int KS, bool FUSE_DELTA>
+__global__ __launch_bounds__(256, 2) void attn_f32_dq_kernel(const KArgs a) {
+    __shared__ __attribute__((aligned(1024))) char smem[8 * F32Tile::kBytes];
+    f32_dq_rows<KS, FUSE_DELTA, 4>(a, smem);
 }
 
 }  // namespace gptoss

@@ -13,6 +13,7 @@
 #include "attn_common.h"
 #include "attn_decode.h"
 #include "attn_f32.h"
+#include "attn_f32_split.h"
 #include "attn_fwd.h"
 #include "attn_fwd_pipe.h"
 #include "attn_fwd_window.h"
@@ -89,6 +90,10 @@ KArgs make_args(const gptoss_attn_params *p, SinkTypes ty) {
     a.chunk_tiles = 0;
     a.dsink_partial = nullptr;
     a.boundary_partial = nullptr;
+    a.split_kv = a.split_q = nullptr;
+    a.split_kv_bad = a.split_q_bad = nullptr;
+    a.split_steps = a.split_slots = 0;
+    a.split_partial = nullptr;
     return a;
 }
 
@@ -248,6 +253,70 @@ int64_t f32_grid(const KArgs &a, int ks) {
     return (int64_t)a.G * ((units + 4 / ks - 1) / (4 / ks));
 }
 
+// ---- float32 on the bf16 matrix pipes (attn_f32_split.h) -----------------------------------------
+// Taken where the caller has scratch for the records, four consecutive heads share a KV head (the four units of a workgroup then stand
+// at the same rows), the backward for self-attention without an offset, and where it is the faster one: it costs a launch and fills the
+// chip with workgroups of eight wavefronts.  fp32 instruction / this, us a call, 64 query heads on 8 KV heads, forward + backward: 8 x 128
+// rows 121 / 123, 256 95 / 104, 320 101 / 96, 448 139 / 106, 1024 413 / 254, 4096 5350 / 3280; 8 heads on one KV head 1024 (64 workgroups) 150 /
+// 145, 2048 on two (128) 263 / 225; a window of 128 is a handful of tiles per workgroup, whose start and end then decide: 320
+// 111 / 106, 640 132 / 120, 1024 (512 workgroups) 148 / 151, 2048 254 / 268; of 512, 1024 rows 382 / 228.  Queries on a cache: 1 on
+// 2048 47 / 88, 64 x 4 on 4096 158 / 174, 256 on 4096 155 / 139, 1024 on 8192 1119 / 614.
+bool f32_split_route(const gptoss_attn_params *p, bool bwd) {
+    if (p->dtype != GPTOSS_ATTN_FP32 || p->B <= 0 || p->G <= 0 || p->H <= 0 || p->H % p->G || (p->H / p->G) % 4 || p->Skv <= 0) return false;
+    if (bwd && (p->Sq != p->Skv || p->q_offset != 0 || p->q_offset_dev)) return false;
+    const int64_t wgs = (int64_t)(p->H / 4) * p->B * (((int64_t)p->Sq + 31) / 32);
+    const int window = effective_window(p);
+    if (window > 0 && window < 384 && wgs > 400) return false;
+    return p->Sq >= 192 && (wgs >= 160 || (wgs >= 128 && p->Skv >= 2048));
+}
+// Steps per dK/dV workgroup: the count whose rounds of workgroups take the least time on 256 compute units, one workgroup each (so that
+// the scratch does not depend on the device), a workgroup's start and end counted as three steps; more than four rounds even out.
+struct F32SplitParts { int steps, slots; bool cut; };
+F32SplitParts f32_split_parts(const gptoss_attn_params *p) {
+    const int window = effective_window(p), r = p->H / p->G, blocks = (p->Skv + F32Split::kKeys - 1) / F32Split::kKeys;
+    const int64_t rows = (int64_t)p->G * p->B, cus = 256;
+    const int most = split_block_steps(p->Sq, window, r, 0);
+    if (rows * blocks > 8 * cus) return {most, blocks, false};
+    int64_t all = 0;
+    for (int i = 0; i < blocks; ++i) all += split_block_steps(p->Sq, window, r, i);
+    F32SplitParts best{most, blocks, false};
+    int64_t best_cost = 0;
+    for (int steps = most; steps >= 4; steps -= 1 + steps / 32) {
+        int slots = 0;
+        for (int i = 0; i < blocks; ++i) slots += split_block_parts(p->Sq, window, r, i, steps);
+        const int64_t wgs = rows * slots;
+        const int64_t cost = wgs <= 4 * cus ? 4 * ((wgs + cus - 1) / cus) * (steps + 3) : 4 * (rows * all + 3 * wgs) / cus + 3 * steps;
+        if (steps == most || cost < best_cost) { best = {steps, slots, slots > blocks}; best_cost = cost; }
+    }
+    return best;
+}
+// The scratch: which K / V records are bad, these records; for the backward the same of Q / dO, then the parts' sums.
+struct F32SplitScratch { size_t kv_bad, kv, q_bad, q, partial, bytes; F32SplitParts parts; };
+F32SplitScratch f32_split_scratch(const gptoss_attn_params *p, bool bwd) {
+    auto up = [](size_t n) { return (n + 255) & ~(size_t)255; };
+    F32SplitScratch s{};
+    const size_t n_kv = (size_t)p->B * p->G * ((p->Skv + 31) / 32), n_q = (size_t)p->B * p->H * ((p->Sq + 31) / 32);
+    s.kv = up(4 * n_kv);
+    s.bytes = s.kv + n_kv * F32Split::kKvRecord;
+    if (!bwd) return s;
+    s.q_bad = s.bytes;
+    s.q = s.q_bad + up(4 * n_q);
+    s.partial = s.q + n_q * F32Split::kQRecord;
+    s.parts = f32_split_parts(p);
+    s.bytes = s.partial + (s.parts.cut ? (size_t)p->B * p->G * s.parts.slots * (2 * F32Split::kKeys * kD * sizeof(float)) : 0);
+    return s;
+}
+void f32_split_args(KArgs &a, const F32SplitScratch &s, void *scratch) {
+    char *base = static_cast<char *>(scratch);
+    a.split_kv_bad = reinterpret_cast<uint32_t *>(base);
+    a.split_kv = base + s.kv;
+    a.split_q_bad = reinterpret_cast<uint32_t *>(base + s.q_bad);
+    a.split_q = base + s.q;
+    a.split_steps = s.parts.steps;
+    a.split_slots = s.parts.slots;
+    a.split_partial = s.parts.cut ? reinterpret_cast<float *>(base + s.partial) : nullptr;
+}
+
 // One launch.  hipLaunchKernel reports this launch's own status, so an error some earlier call of the
 // thread left in the runtime's sticky state is neither reported here nor cleared.  A grid beyond the
 // x-dimension limit is refused on the host.
@@ -378,6 +447,29 @@ int launch_window_bwd(const gptoss_attn_params *p, hipStream_t st, bool seam_sum
     const hipError_t e = hipLaunchKernel(reinterpret_cast<const void *>(attn_bwd_window_finish_kernel),
                                          dim3((unsigned)(seam_blocks + sink_blocks)), dim3(256), args, 0, st);
     return e == hipSuccess ? GPTOSS_ATTN_OK : static_cast<int>(e);
+}
+
+int launch_f32_split_kv(const KArgs &a, hipStream_t st) { return launch(attn_f32_split_kv_kernel, (int64_t)a.B * a.G * ((a.Skv + 31) / 32), 256, st, a); }
+int64_t f32_split_grid(const KArgs &a) { return (int64_t)a.G * (a.r / 4) * a.B * ((a.Sq + 31) / 32); }
+
+int launch_f32_split_fwd(const gptoss_attn_params *p, hipStream_t st, SinkTypes ty, void *scratch) {
+    KArgs a = make_args(p, ty);
+    f32_split_args(a, f32_split_scratch(p, false), scratch);
+    int rc = lds_attribute<&attn_f32_split_fwd_kernel>(F32Split::kRowsLds);
+    if (rc || (rc = launch_f32_split_kv(a, st))) return rc;
+    return launch(attn_f32_split_fwd_kernel, f32_split_grid(a), 512, st, a, F32Split::kRowsLds);
+}
+
+int launch_f32_split_bwd(const gptoss_attn_params *p, hipStream_t st, SinkTypes ty, void *scratch) {
+    KArgs a = make_args(p, ty);
+    f32_split_args(a, f32_split_scratch(p, true), scratch);
+    int rc = lds_attribute<&attn_f32_split_dq_kernel>(F32Split::kDqLds);
+    if (rc || (rc = lds_attribute<&attn_f32_split_dkdv_kernel>(F32Split::kDkdvLds)) || (rc = launch_f32_split_kv(a, st))) return rc;
+    if ((rc = launch(attn_f32_split_dq_kernel, f32_split_grid(a), 512, st, a, F32Split::kDqLds))) return rc;
+    if (!a.split_partial && a.dsinks && (rc = launch(attn_bwd_dsinks_kernel, a.H, 1024, st, a))) return rc;
+    rc = launch(attn_f32_split_dkdv_kernel, (int64_t)a.G * a.B * a.split_slots, 512, st, a, F32Split::kDkdvLds);
+    if (rc || !a.split_partial) return rc;
+    return launch_reduce(attn_f32_split_reduce_kernel, (int64_t)2 * a.B * a.G * a.Skv * 16, st, a, a.dsinks != nullptr);
 }
 
 template <int NQB, int NW>
@@ -516,6 +608,10 @@ size_t gptoss_attn_workspace_bytes(const gptoss_attn_params *p) {
     return fwd > n ? fwd : n;
 }
 
+size_t gptoss_attn_split_bytes(const gptoss_attn_params *p, int backward) {
+    return p && f32_split_route(p, backward != 0) ? f32_split_scratch(p, backward != 0).bytes : 0;
+}
+
 // scratch: see gptoss_attn_fwd_scratch (NULL or too little: the keys are not cut)
 static int forward(const gptoss_attn_params *p, void *stream, SinkTypes ty, void *scratch, size_t scratch_bytes) {
     const int rc = gptoss_attn_validate(p, 0);
@@ -534,6 +630,8 @@ static int forward(const gptoss_attn_params *p, void *stream, SinkTypes ty, void
         return launch(attn_decode_combine_kernel, ((int64_t)a.B * a.G * pairs + 3) / 4, 256, st, a);
     }
     if (p->dtype == GPTOSS_ATTN_FP32) {
+        const size_t records = gptoss_attn_split_bytes(p, 0);
+        if (records && scratch && scratch_bytes >= records) return launch_f32_split_fwd(p, st, ty, scratch);
         const int ks = f32_key_splits(a);
         const int64_t grid32 = f32_grid(a, ks);
         return ks == 4 ? launch(attn_f32_fwd_kernel<4>, grid32, 256, st, a) : ks == 2 ? launch(attn_f32_fwd_kernel<2>, grid32, 256, st, a) : launch(attn_f32_fwd_kernel<1>, grid32, 256, st, a);
@@ -666,9 +764,12 @@ int gptoss_attn_bwd_dq(const gptoss_attn_params *p, void *stream) { return launc
 // The whole backward: the dQ kernel computes the row statistics on the way (no separate
 // pass over O and dO), then dK/dV and dSinks read them from the scratch buffer.  The results are
 // bit-identical to gptoss_attn_bwd_preprocess + gptoss_attn_bwd_dkdv + gptoss_attn_bwd_dq.
-static int bwd_all(const gptoss_attn_params *p, void *stream, bool whole_blocks, SinkTypes ty) {
+static int bwd_all(const gptoss_attn_params *p, void *stream, bool whole_blocks, SinkTypes ty, void *scratch = nullptr, size_t scratch_bytes = 0) {
     int rc = gptoss_attn_validate(p, 1);
     if (rc) return rc;
+    if (!aligned16(scratch)) return GPTOSS_ATTN_ERR_ALIGNMENT;
+    const size_t records = gptoss_attn_split_bytes(p, 1);
+    if (records && scratch && scratch_bytes >= records) return launch_f32_split_bwd(p, static_cast<hipStream_t>(stream), ty, scratch);
     if (window_single_pass(p)) return launch_window_bwd(p, static_cast<hipStream_t>(stream), !whole_blocks, ty);
     rc = launch_dq(p, stream, 1);
     if (rc) return rc;
@@ -680,6 +781,11 @@ int gptoss_attn_bwd(const gptoss_attn_params *p, void *stream) { return bwd_all(
 int gptoss_attn_bwd_sinks(const gptoss_attn_params *p, int sinks_dtype, int dsinks_dtype, void *stream) {
     if (!sink_dtype_ok(sinks_dtype) || !sink_dtype_ok(dsinks_dtype)) return GPTOSS_ATTN_ERR_DTYPE;
     return bwd_all(p, stream, false, {sinks_dtype == GPTOSS_ATTN_BF16, dsinks_dtype == GPTOSS_ATTN_BF16});
+}
+
+int gptoss_attn_bwd_scratch(const gptoss_attn_params *p, int sinks_dtype, int dsinks_dtype, void *scratch, size_t scratch_bytes, void *stream) {
+    if (!sink_dtype_ok(sinks_dtype) || !sink_dtype_ok(dsinks_dtype)) return GPTOSS_ATTN_ERR_DTYPE;
+    return bwd_all(p, stream, false, {sinks_dtype == GPTOSS_ATTN_BF16, dsinks_dtype == GPTOSS_ATTN_BF16}, scratch, scratch_bytes);
 }
 
 // ---- the backward for callers that cannot allocate ------------------------------------------

@@ -147,7 +147,8 @@ std::tuple<Tensor, Tensor> fwd(const Tensor &q, const Tensor &k, const Tensor &v
     c.p.o = o.data_ptr();
     c.p.lse = lse.data_ptr<float>();
     set(c.p.o_stride, o, true);
-    const size_t need = gptoss_attn_fwd_workspace_bytes(&c.p);      // partial results of few queries' rows, cut over their keys
+    // partial results of few queries' rows, cut over their keys; records of float32 operands
+    const size_t need = c.p.dtype == GPTOSS_ATTN_FP32 ? gptoss_attn_split_bytes(&c.p, 0) : gptoss_attn_fwd_workspace_bytes(&c.p);
     const Tensor scratch = need ? at::empty({static_cast<int64_t>(need / sizeof(float))}, lse.options()) : Tensor();
     check("gptoss_attn_fwd", gptoss_attn_fwd_scratch(&c.p, c.sinks_dtype, need ? scratch.data_ptr() : nullptr, need, stream_of(c)));
     return {o, lse};
@@ -191,7 +192,10 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> bwd(const Tensor &q, const Tensor &k,
     set(p.dq_stride, dq, false);
     set(p.dk_stride, dk, false);
     set(p.dv_stride, dv, false);
-    check("gptoss_attn_bwd", gptoss_attn_bwd_sinks(&c.p, c.sinks_dtype, bf16_dsinks ? GPTOSS_ATTN_BF16 : GPTOSS_ATTN_FP32, stream_of(c)));
+    const size_t records = gptoss_attn_split_bytes(&c.p, 1);        // (float32 operands as bf16 terms)
+    const Tensor split = records ? at::empty({static_cast<int64_t>(records / sizeof(float))}, lse.options()) : Tensor();
+    check("gptoss_attn_bwd", gptoss_attn_bwd_scratch(&c.p, c.sinks_dtype, bf16_dsinks ? GPTOSS_ATTN_BF16 : GPTOSS_ATTN_FP32,
+                                                     records ? split.data_ptr() : nullptr, records, stream_of(c)));
     return {dq, dk, dv, dsinks};
 }
 

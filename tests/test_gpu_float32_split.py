@@ -1,0 +1,98 @@
+"""GPU tests of float32 attention on the bf16 matrix pipes (operands as three bf16 terms): edges of tiles, groups and parts, no further
+from float64 than the fp32 matrix instruction, and the numbers the terms do not hold."""
+import ctypes
+
+import pytest
+import torch
+
+from oracle import eager_ref as E
+import test_gpu_float32 as TF
+import test_gpu_parity as TP
+
+pytestmark = pytest.mark.gpu
+A = TF.A
+SCALE, DEV = TF.SCALE, "cuda"
+
+
+def _both(A, inp, window, seqlens=None, docs=None, start=0, backward=True):
+    """(results, results of the fp32 matrix instruction)"""
+    from oregon_gpt_oss_patching_amd import _lib
+    from oregon_gpt_oss_patching_amd import attention_kernel as ak
+    q, k, v, sinks, d_out = (t.to(DEV) for t in inp)
+    lens = None if seqlens is None else torch.tensor(seqlens, dtype=torch.int32, device=DEV)
+    ds = None if docs is None else E.doc_start_from_lengths([docs] * q.shape[0], q.shape[2]).to(DEV).to(torch.int32)
+    p = ak._base_params(q, k, v, sinks, lens, SCALE, window, start, ds)
+    o, lse = A.attention_forward(q, k, v, sinks, SCALE, window, start, lens, ds)
+    o2, lse2 = torch.empty_like(o), torch.empty_like(lse)
+    p.o, p.lse = o2.data_ptr(), lse2.data_ptr()
+    ak._set(p.o_stride, ak._strides_bhs(o2, "bshd"))
+    assert _lib.load().gptoss_attn_split_bytes(ctypes.byref(p), int(backward)) > 0
+    _lib.call("gptoss_attn_fwd", p, torch.cuda.current_stream().cuda_stream)
+    if not backward:
+        return (o, lse), (o2, lse2)
+    args = (d_out, SCALE, window, 0, lens)
+    return ((o, lse) + A.attention_backward(q, k, v, sinks, o, lse, *args, doc_start=ds),
+            (o2, lse2) + A.attention_backward(q, k, v, sinks, o2, lse2, *args, doc_start=ds, split=True))
+
+
+@pytest.mark.parametrize("b,h,g,s,w,lens,docs", [
+    (1, 64, 8, 320, None, None, None),             # whole tiles, one key block of two and a half
+    (1, 64, 8, 333, None, None, None),             # a last tile of 13 rows
+    (2, 64, 8, 193, 128, None, None),              # one row past a tile, a window
+    (3, 64, 8, 257, None, [257, 1, 130], None),    # padded rows, one of them a single token
+    (1, 96, 8, 417, 33, None, None),               # twelve heads per KV head
+    (2, 32, 8, 640, 500, None, None),              # four heads per KV head, a long window
+    (1, 64, 8, 700, None, None, [5, 300, 32, 363]),
+    (1, 8, 1, 2500, None, None, None),             # key blocks in parts of unequal number
+])
+def test_no_further_from_float64_than_the_fp32_instruction(A, b, h, g, s, w, lens, docs):
+    print(f"case B={b} H={h} G={g} S={s} W={w} lens={lens} docs={docs}", flush=True)
+    inp = list(E.make_inputs(7000 + s, b, h, g, s, 64, torch.float32))
+    if lens:
+        inp[4] = inp[4] * (torch.arange(s).view(1, s) < torch.tensor(lens).view(b, 1)).view(b, s, 1, 1)
+    ds = E.doc_start_from_lengths([docs] * b, s) if docs else None
+    new, old = _both(A, inp, w, lens, docs)
+    f = [t.double().to(DEV) for t in inp]
+    out, *grads = E.eager_attention_grads(*f, SCALE, w, 0, lens, ds)
+    lse = E.logsumexp_rows(f[0], f[1], f[3], SCALE, w, 0, lens, ds)
+    for name, x, y, ref in zip(("o", "lse", "dq", "dk", "dv", "dsinks"), new, old, (out, lse, *grads)):
+        err, was = (float((t.double() - ref).norm() / ref.norm()) for t in (x, y))
+        # dSinks is a cancelling sum over the rows: its error is the rows' common one, either way.  lse: most of its error is the last
+        # rounding, an eighth of 2^-24 more is below what a row's order of additions makes
+        room = {"dsinks": float("inf"), "lse": 1.125}.get(name, 1.05)
+        assert err <= min(2e-5, room * was), (name, err, was)
+    again, _ = _both(A, inp, w, lens, docs)
+    assert all(torch.equal(x, y) for x, y in zip(new, again))
+    if lens:
+        for i, n in enumerate(lens):
+            for t in (new[0][i, n:], new[2][i, :, n:], new[3][i, :, n:], new[4][i, :, n:]):
+                assert t.numel() == 0 or float(t.abs().max()) == 0.0
+
+
+@pytest.mark.parametrize("sq,skv,w", [(256, 2049, None), (330, 1000, None), (330, 777, 100)])
+def test_chunks_behind_a_cache(A, sq, skv, w):
+    inp = E.make_inputs(7600 + sq, 1, 64, 8, sq, 64, torch.float32, skv=skv)
+    new, old = _both(A, inp, w, start=skv - sq, backward=False)
+    q, k, v, sinks, _ = (t.double().to(DEV) for t in inp)
+    ref = E.eager_attention(q, k, v, sinks, SCALE, w, skv - sq)
+    ref = ref[0] if isinstance(ref, tuple) else ref
+    err, was = (float((t[0].double() - ref).norm() / ref.norm()) for t in (new, old))
+    assert err <= min(2e-5, 1.05 * was), (err, was)
+    assert float((new[1] - old[1]).abs().max()) <= 2e-5
+
+
+@pytest.mark.parametrize("which,value", [("k", float("inf")), ("v", float("inf")), ("v", 1e30), ("v", float("nan")), ("q", 1e-35), ("q", 3e7),
+                                         ("d_out", 1e-34), ("d_out", -float("inf")), ("v", 2.0 ** 24), ("v", 2.0 ** -100)])
+def test_numbers_that_three_terms_do_not_hold(A, which, value):
+    """One such number: what it reaches is what it reaches through the fp32 instruction."""
+    inp = dict(zip(("q", "k", "v", "sinks", "d_out"), E.make_inputs(7700, 1, 64, 8, 333, 64, torch.float32)))
+    t = inp[which]
+    (t[0, 200, 5] if which == "d_out" else t[0, 2, 200])[7] = value
+    new, old = _both(A, tuple(inp.values()), None)
+    for name, x, y in zip(("o", "lse", "dq", "dk", "dv", "dsinks"), new, old):
+        same = torch.isfinite(x) == torch.isfinite(y)
+        assert bool(same.all()), (name, int((~same).sum()))
+        assert torch.equal(torch.isnan(x), torch.isnan(y)), name
+        ok = torch.isfinite(y)
+        x, y = x[ok].double(), y[ok].double()
+        assert float((x - y).norm()) <= 2e-5 * float(y.norm()), name
