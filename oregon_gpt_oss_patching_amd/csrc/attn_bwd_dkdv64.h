@@ -48,6 +48,127 @@ struct Dkdv64 {
     static constexpr int kWaveRows = 16;                           // rows of each tile one wavefront copies
 };
 
+// ---- the division of a KV head's work into pieces ---------------------------------------------------------------
+// A key block's walk is as long as its row or document lets it be, and a workgroup has its compute unit to itself, so the time is set by
+// how evenly the walks fill the units.  Where dkdv_parts > 1 (there is scratch for partial sums) every walk is cut into that many equal
+// shares (dkdv_parts_for), one workgroup each; with padded rows or packed documents (dkdv_slots > 0) a KV head's blocks, of all batch
+// rows, are divided by their lengths, which only the device knows: a unit's share is L = (all tiles) / (units
+// of the KV head); walks longer than that are cut into pieces of L tiles from their end down, and the rest of each.  The pieces of L tiles start
+// first (the first ones of all blocks, then the second ones: neighbours walk the same Q and dO tiles), the rests follow, the longest first.  A walk that is not cut writes its result itself; the pieces of one that is leave fp32
+// partial sums, in slots of the scratch (attn_bwd_dkdv64_reduce_kernel adds them).  Every workgroup finds its own piece (the
+// blocks' lengths in LDS, then counting over a wavefront: about 2 us, documents 4).
+// Equal shares leave padded and packed rows' short walks in as many pieces as the long ones', each with a start, an end and 128 KB of
+// partial sums of its own.  Forward + backward, us equal shares / pieces (64 query heads on 8 KV heads): 4 x 4096 padded to 3309 / 1968 / 1554 / 4079
+// 1400 / 1329, 2 x 5438 to 2212 / 2754 634 / 594; documents of 95 to 3067 in 8192 tokens 785 / 768, of 100 to 4000 in 12000 1450 / 1395;
+// ONE document of 8192 2270 / 2300.  Rows of one length stay with equal shares, whose workgroups keep in step on the same tiles: 2 x 3001 690 / 707, 4150
+// 663 / 675, 2500 295 / 307.
+struct Dkdv64Plan {
+    static constexpr int kMaxBlocks = 2048;
+    int nblk, L, full, lane;           // blocks, tiles of a full piece, number of full pieces
+    const int *tiles;                  // [nblk] tiles of the blocks' walks (LDS), block = 256-key block * B + batch row
+    __device__ __forceinline__ int of(int i) const { return i < nblk ? tiles[i] : 0; }
+    __device__ __forceinline__ int cuts(int n) const { return n > 0 ? (n - 1) / L : 0; }       // full pieces of a walk
+    // the walks' lengths, by the whole workgroup; `n` holds nblk numbers
+    static __device__ __forceinline__ void lengths(const KArgs &a, int nblk, int *n, int tid) {
+        for (int i0 = 0; i0 < nblk; i0 += 32) {                        // eight lanes per block
+            const int i = i0 + (tid >> 3), b = i % a.B, j0 = Dkdv64::BN * (i / a.B);
+            int len = a.Sq;
+            if (a.seqlens) len = max(0, min(a.Sq, a.seqlens[b]));
+            int end = len;
+            if (a.doc_start) {                              // the first row of a later document than the block's last key
+                const int32_t *row = a.doc_start + (int64_t)b * a.Sq;
+                const int j = min(j0 + Dkdv64::BN, len) - 1;
+                int lo = max(0, min(j + 1, a.Sq)), hi = j >= j0 && i < nblk ? a.Sq : lo;
+                while (__builtin_amdgcn_ballot_w64(lo < hi) != 0ull) {
+                    const int x = lo + (hi - lo) * ((tid & 7) + 1) / 9;
+                    const uint64_t past = __builtin_amdgcn_ballot_w64(x >= hi || row[min(x, a.Sq - 1)] > j);
+                    const int c = __builtin_ctz((uint32_t)(past >> (tid & 56)) | 0x100u);        // lanes in front of the first one past it
+                    const int new_lo = c > 0 ? lo + (hi - lo) * c / 9 + 1 : lo, new_hi = c < 8 ? lo + (hi - lo) * (c + 1) / 9 : hi;
+                    if (lo < hi) { lo = new_lo; hi = new_hi; }
+                }
+                end = min(len, hi);
+            }
+            if ((tid & 7) == 0 && i < nblk) n[i] = j0 < len ? max(0, (end + kTile - 1) / kTile - j0 / kTile) : 0;
+        }
+        __syncthreads();
+    }
+    __device__ __forceinline__ Dkdv64Plan(const KArgs &a, const int *n, int nblk_, int slots, int lane_) : nblk(nblk_), lane(lane_), tiles(n) {
+        int sum = 0;
+        for (int i0 = 0; i0 < nblk; i0 += 64) sum += of(i0 + lane);
+#pragma unroll
+        for (int d = 1; d < 64; d *= 2) sum += __shfl_xor(sum, d);
+        sum = __builtin_amdgcn_readfirstlane(sum);
+        const int units = max(1, 256 / a.G), room = max(1, slots - nblk);
+        L = max(max((sum + units - 1) / units, (sum + room - 1) / room), (8 + a.r - 1) / a.r);
+        int f = 0;
+        for (int i0 = 0; i0 < nblk; i0 += 64) f += cuts(of(i0 + lane));
+#pragma unroll
+        for (int d = 1; d < 64; d *= 2) f += __shfl_xor(f, d);
+        full = __builtin_amdgcn_readfirstlane(f);
+    }
+    // blocks whose rest has at least v tiles
+    __device__ __forceinline__ int count_rests(int v) const {
+        int c = 0;
+        for (int i0 = 0; i0 < nblk; i0 += 64) {
+            const int n = of(i0 + lane);
+            c += __builtin_popcountll(__builtin_amdgcn_ballot_w64(i0 + lane < nblk && n - cuts(n) * L >= v));
+        }
+        return c;
+    }
+    // blocks with more than k full pieces, those in front of block i of them
+    __device__ __forceinline__ int count_cut(int k, int i) const {
+        int c = 0;
+        for (int i0 = 0; i0 < nblk; i0 += 64) c += __builtin_popcountll(__builtin_amdgcn_ballot_w64(i0 + lane < i && cuts(of(i0 + lane)) > k));
+        return c;
+    }
+    // Piece p: its block, its number among the block's pieces, its slot of the scratch (-1: the whole walk).  False: there is none.
+    __device__ __forceinline__ bool piece(int p, int &block, int &k, int &slot) const {
+        if (p < full) {                        // the first pieces of all blocks, the second ones, ...: neighbours walk the same tiles
+            slot = p;
+            for (k = 0;; ++k) {
+                const int c = count_cut(k, nblk);
+                if (p < c) break;
+                p -= c;
+            }
+            for (int i0 = 0; i0 < nblk; i0 += 64) {
+                uint64_t more = __builtin_amdgcn_ballot_w64(cuts(of(i0 + lane)) > k);
+                const int c = __builtin_popcountll(more);
+                if (p < c) {
+                    for (; p > 0; --p) more &= more - 1;
+                    block = i0 + __builtin_ctzll(more);
+                    break;
+                }
+                p -= c;
+            }
+            return true;
+        }
+        const int q = p - full;                // the q-th longest rest
+        if (q >= nblk) return false;
+        int lo = 0, hi = L;                    // the largest v of which more than q rests have as much
+        while (lo < hi) {
+            const int v = (lo + hi + 1) >> 1;
+            if (count_rests(v) > q) lo = v; else hi = v - 1;
+        }
+        int left = q - count_rests(lo + 1);    // among equals, by number
+        for (int i0 = 0; i0 < nblk; i0 += 64) {
+            const int n = of(i0 + lane);
+            uint64_t same = __builtin_amdgcn_ballot_w64(i0 + lane < nblk && n - cuts(n) * L == lo);
+            const int c = __builtin_popcountll(same);
+            if (left < c) {
+                for (; left > 0; --left) same &= same - 1;
+                block = i0 + __builtin_ctzll(same);
+                k = cuts(tiles[block]);
+                slot = k > 0 ? full + count_cut(0, block) : -1;
+                return true;
+            }
+            left -= c;
+        }
+        return false;
+    }
+};
+// floats of a slot: dK and dV of a key block
+constexpr int64_t kDkdv64Slot = (int64_t)2 * Dkdv64::BN * kD;
+
 template <bool GENERAL>
 __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv64_kernel(const KArgs a) {
     using C = Dkdv64;
@@ -59,27 +180,46 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv64_kernel(const KArgs a) 
 
     int bid = blockIdx.x;
     const int g = bid % a.G; bid /= a.G;
-    const int bi = bid % a.B; bid /= a.B;
-    const int part = bid % a.dkdv_parts; bid /= a.dkdv_parts;
-    const int kt = bid;                                   // ascending: most work first
-    const int b = rotated_batch_row(bi, kt, a.B);
+    // GENERAL: the walk's tiles, those above this piece, the piece's, its slot of the scratch
+    int kt, b, part = 0, n_plan = -1, cut_at = 0, n_piece = 0, sums_slot = -1;
+    const bool by_lengths = GENERAL && a.dkdv_slots > 0;
+    if (by_lengths) {
+        int *const n = reinterpret_cast<int *>(&smem[0]);
+        const int nblk = a.B * ((a.Skv + BN - 1) / BN);
+        Dkdv64Plan::lengths(a, nblk, n, tid);
+        const Dkdv64Plan plan(a, n, nblk, a.dkdv_slots, lane);
+        int block = 0, k = 0;
+        if (!plan.piece(bid, block, k, sums_slot)) return;
+        block = __builtin_amdgcn_readfirstlane(block);
+        k = __builtin_amdgcn_readfirstlane(k);
+        sums_slot = __builtin_amdgcn_readfirstlane(sums_slot);
+        n_plan = __builtin_amdgcn_readfirstlane(n[block]);
+        cut_at = k * plan.L;
+        n_piece = __builtin_amdgcn_readfirstlane(min(plan.L, n_plan - cut_at));
+        kt = block / a.B;
+        b = block % a.B;
+        __syncthreads();                                  // (the lengths are read: the copies take their place)
+    } else {
+        const int bi = bid % a.B; bid /= a.B;
+        part = bid % a.dkdv_parts; bid /= a.dkdv_parts;
+        kt = bid;                                         // ascending: most work first
+        b = rotated_batch_row(bi, kt, a.B);
+    }
     const int j0 = kt * BN;                               // first key of the workgroup
     const int wj0 = j0 + WK * w;                          // first key of the wavefront
 
     // The query tiles that can see the workgroup's keys run from the one that holds its first key to the
-    // last one; with dkdv_parts > 1 they are cut into that many consecutive slices, one per workgroup, each
-    // of which leaves an fp32 partial sum (attn_bwd_dkdv_reduce_kernel adds them in slice order).  The
-    // workgroup walks its slice from the last tile down, all heads of the group per tile.  Wavefront w's
-    // diagonal tile is tile wq; below it none concerns the wavefront.
+    // last one.  The workgroup walks them, or its piece of them, from the last tile down, all heads of the group per tile.
+    // Wavefront w's diagonal tile is tile wq; below it none concerns the wavefront.
     const int len = GENERAL && a.seqlens ? max(0, min(a.Sq, a.seqlens[b])) : a.Sq;     // rows and keys from len on do not exist
     const int32_t *dsrow = GENERAL && a.doc_start ? a.doc_start + (int64_t)b * a.Sq : nullptr;
     auto end_of = [&](int j) __attribute__((always_inline)) { return dsrow ? min(len, document_end(dsrow, a.Sq, j, lane)) : len; };   // (a wave-uniform key that exists)
     const int qt_lo = j0 / kTile;
-    const int qt_all_hi = GENERAL ? (j0 < len ? (end_of(min(j0 + BN, len) - 1) + kTile - 1) / kTile : qt_lo) : a.Sq / kTile;
-    const int nq_all = max(0, qt_all_hi - qt_lo);
+    const int nq_all = n_plan >= 0 ? n_plan : GENERAL ? (j0 < len ? max(0, (end_of(min(j0 + BN, len) - 1) + kTile - 1) / kTile - qt_lo) : 0) : a.Sq / kTile - qt_lo;
     const int slice = (nq_all + a.dkdv_parts - 1) / a.dkdv_parts;
-    const int qt_hi = GENERAL ? __builtin_amdgcn_readfirstlane(qt_all_hi - part * slice) : qt_all_hi - part * slice;     // end of this workgroup's slice
-    const int nq = GENERAL ? __builtin_amdgcn_readfirstlane(max(0, min(slice, nq_all - part * slice))) : max(0, min(slice, nq_all - part * slice));
+    const int above = by_lengths ? cut_at : part * slice, piece = by_lengths ? n_piece : max(0, min(slice, nq_all - part * slice));
+    const int qt_hi = GENERAL ? __builtin_amdgcn_readfirstlane(qt_lo + nq_all - above) : qt_lo + nq_all - above;       // end of this workgroup's piece
+    const int nq = GENERAL ? __builtin_amdgcn_readfirstlane(piece) : piece;
     const int n_it = nq * a.r;
     const int wq = qt_lo + w;                             // the query tile on the wavefront's diagonal
     const bool wave_live = wj0 < len;
@@ -483,11 +623,12 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv64_kernel(const KArgs a) 
 
     wait_vmcnt<0>();          // the repeated copies of the last requests
     agpr_accumulators_settled(dk, dv);
-    if (a.dkdv_parts > 1) {
+    if (by_lengths ? sums_slot >= 0 : a.dkdv_parts > 1) {
         // unscaled fp32 partial sums; lane = key row, register i of block dblk = column 32*dblk + crow(i, half),
         // four consecutive columns per 16-byte store
-        const int64_t tensor = (int64_t)a.B * a.G * a.Skv * kD;
-        float *pk = a.dkdv_partial + (int64_t)part * 2 * tensor + (((int64_t)b * a.G + g) * a.Skv) * kD;
+        const int64_t tensor = by_lengths ? BN * kD : (int64_t)a.B * a.G * a.Skv * kD;
+        float *pk = by_lengths ? a.dkdv_partial + ((int64_t)g * a.dkdv_slots + sums_slot) * kDkdv64Slot - (int64_t)j0 * kD
+                            : a.dkdv_partial + (int64_t)part * 2 * tensor + (((int64_t)b * a.G + g) * a.Skv) * kD;
         float *pv = pk + tensor;
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
@@ -521,6 +662,40 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv64_kernel(const KArgs a) 
                      a.dvs.s, nvalid, lane);
         __builtin_amdgcn_wave_barrier();
     }
+}
+
+// The partial sums of the cut key blocks, in the order of their pieces, scaled and rounded; sixteen workgroups per block, a thread
+// per 16-byte output chunk.  The first `heads` workgroups produce dSinks.
+__global__ __launch_bounds__(256) void attn_bwd_dkdv64_reduce_kernel(const KArgs a, int heads) {
+    __shared__ int lds[Dkdv64Plan::kMaxBlocks];
+    __shared__ float red[1024];
+    if ((int)blockIdx.x < heads) { dsinks_of_head<256>(a, blockIdx.x, red); return; }
+    const int tid = threadIdx.x, lane = tid & 63, nblk = a.B * ((a.Skv + Dkdv64::BN - 1) / Dkdv64::BN);
+    int bid = blockIdx.x - heads;
+    const int g = bid % a.G; bid /= a.G;
+    const int chunk = (bid & 15) * 256 + tid, block = bid >> 4, kt = block / a.B, b = block % a.B;
+    Dkdv64Plan::lengths(a, nblk, lds, tid);
+    const Dkdv64Plan plan(a, lds, nblk, a.dkdv_slots, lane);
+    const int n = plan.cuts(lds[block]);
+    if (n == 0) return;
+    const int which = chunk >> 11, key = (chunk >> 3) & (Dkdv64::BN - 1), c8 = (chunk & 7) * 8, j = kt * Dkdv64::BN + key;
+    const bool live = j < a.Skv;               // (the counting takes whole wavefronts)
+    const float *src = a.dkdv_partial + (int64_t)g * a.dkdv_slots * kDkdv64Slot + (which * Dkdv64::BN + key) * kD + c8;       // (a slot holds all 256 keys)
+    float x[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+    int before = 0;                            // full pieces of smaller number
+    for (int i = 0; i <= n; ++i) {
+        const float *p = src + (int64_t)(i < n ? before + plan.count_cut(i, block) : plan.full + plan.count_cut(0, block)) * kDkdv64Slot;
+        if (i < n) before += plan.count_cut(i, nblk);
+        const f32x4 y = *reinterpret_cast<const f32x4 *>(p), z = *reinterpret_cast<const f32x4 *>(p + 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { x[e] += y[e]; x[4 + e] += z[e]; }
+    }
+    const float mul = which == 0 ? a.scale : 1.0f;
+    union { bf16x8 v; u32x4 u; } out;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) out.v[e] = (bf16)(x[e] * mul);
+    const Strides &st = which == 0 ? a.dks : a.dvs;
+    if (live) *reinterpret_cast<u32x4 *>((which == 0 ? a.dk : a.dv) + (int64_t)b * st.b + (int64_t)g * st.h + (int64_t)j * st.s + c8) = out.u;
 }
 
 }  // namespace gptoss

@@ -85,6 +85,7 @@ KArgs make_args(const gptoss_attn_params *p, SinkTypes ty) {
     a.scale = p->scale;
     a.scale_log2 = p->scale * kLog2e;
     a.dkdv_parts = 1;
+    a.dkdv_slots = 0;
     a.kv_splits = 1;
     a.fwd_partial = nullptr;
     a.chunk_tiles = 0;
@@ -143,7 +144,7 @@ int dkdv_parts_for(const gptoss_attn_params *p, bool padded, bool packed) {
     const int64_t rows_seen = window > 0 ? (int64_t)kDkdvKeys + window - 1 : (int64_t)p->Sq;
     const int64_t tiles = ((rows_seen < p->Sq ? rows_seen : p->Sq) + 63) / 64;
     int64_t parts = (1024 + blocks - 1) / blocks;
-    if (blocks > 512) parts = p->Sq >= 4096 && (padded && p->B > 1 ? blocks / 2 : blocks) < 1024 ? 2 : 1;
+    if (blocks > 512) parts = p->Sq >= (padded && p->B > 1 ? 1024 : 4096) && (padded && p->B > 1 ? blocks / 2 : blocks) < 1024 ? 2 : 1;
     if (packed && window == 0 && p->Sq >= 4096 && blocks >= 256 && blocks <= 768 && parts < 4) parts = 4;
     const int64_t steps = window > 0 ? tiles / 4 : tiles * (p->H / p->G) / 8;
     if (parts > steps) parts = steps;
@@ -717,10 +718,15 @@ static int launch_dkdv(const gptoss_attn_params *p, void *stream, bool whole_blo
         return launch_reduce(attn_f32_dkdv_reduce_kernel, (int64_t)2 * a.B * a.G * a.Skv * 16, st, a, with_dsinks);
     }
     if (dkdv64_route(p, a.dkdv_parts)) {
-        const int64_t grid64 = (int64_t)a.G * a.B * a.dkdv_parts * ((a.Skv + Dkdv64::BN - 1) / Dkdv64::BN);
+        const int64_t blocks = (int64_t)a.B * ((a.Skv + Dkdv64::BN - 1) / Dkdv64::BN);      // of a KV head
+        // padded and packed rows: pieces by the walks' lengths, at most as many as there are slots for partial sums (Dkdv64Plan)
+        const bool by_lengths = a.dkdv_parts > 1 && (a.seqlens || a.doc_start);
+        if (by_lengths) a.dkdv_slots = (int)((int64_t)a.dkdv_parts * a.B * a.Skv / Dkdv64::BN);
+        const int64_t grid64 = a.G * (by_lengths ? a.dkdv_slots : blocks * a.dkdv_parts);
         const bool plain = !a.seqlens && !a.doc_start && a.Sq % kTile == 0;
         const int s = plain ? launch(attn_bwd_dkdv64_kernel<false>, grid64, 256, st, a) : launch(attn_bwd_dkdv64_kernel<true>, grid64, 256, st, a);
         if (s || a.dkdv_parts == 1) return s;
+        if (by_lengths) return launch_reduce(attn_bwd_dkdv64_reduce_kernel, a.G * blocks * 16 * 256, st, a, with_dsinks);
         return launch_reduce(attn_bwd_dkdv_reduce_kernel, (int64_t)2 * a.B * a.G * a.Skv * 8, st, a, with_dsinks);
     }
     const int64_t grid = (int64_t)a.G * a.B * a.dkdv_parts * ((a.Skv + kDkdvKeys - 1) / kDkdvKeys);
