@@ -111,6 +111,9 @@ constexpr int kDkdvNB = 1;
 constexpr int kDkdvWaves = 4;                        // wavefronts per dK/dV workgroup
 constexpr int kDkdvKeys = 32 * kDkdvNB * kDkdvWaves; // keys per dK/dV workgroup
 
+// More key blocks than are cut into equal shares by their number alone.
+bool many_key_blocks(const gptoss_attn_params *p) { return (int64_t)p->G * p->B * ((p->Skv + kDkdvKeys - 1) / kDkdvKeys) > 512; }
+
 // Workgroups per key block in the dK/dV kernel.  One workgroup per (batch, KV head, 128 keys) fills
 // the 256 CUs (two workgroups each) only from S = 16384 on, and the causal triangle makes the first
 // key blocks many times longer than the last; shorter problems cut each key block's query tiles into
@@ -120,8 +123,9 @@ constexpr int kDkdvKeys = 32 * kDkdvNB * kDkdvWaves; // keys per dK/dV workgroup
 // up (B = 2, S = 383: 78 us uncut, 25 + 5 us in six slices).  Between 512 and 1024 blocks the first
 // key block of a long row (4096 rows and more) is still longer than the average compute unit's share: two slices; a
 // right-padded batch counts half, because its shorter rows leave the longest one alone (dK/dV of B = 4, S = 4096,
-// lengths 3309 / 1968 / 1554 / 4079: 715 us uncut, 589 in two slices; B = 2, S = 8192 / 4000: 1437 and 1216; but B = 8,
-// S <= 2048: 359 and 370).  Packed rows: a walk ends with its document, so the longest document's first blocks stand out more, and
+// lengths 3309 / 1968 / 1554 / 4079: 715 us uncut, 589 in two slices; B = 2, S = 8192 / 4000: 1437 and 1216).  Several rows of 1280 tokens and
+// more (padded: 1024) get the same scratch, for pieces by the walks' lengths (Dkdv64Plan), which cut only the longest walks: whole backward and forward of 5 x 1600
+// 564 -> 514 us, 6 x 1500 610 -> 584, 3 x 3000 1074 -> 995, 7 x 1417 645 and 646, 8 x 1300 611 -> 602; but 9 x 1100 536 -> 547.  Packed rows: a walk ends with its document, so the longest document's first blocks stand out more, and
 // the host does not see the documents: four slices from 256 to 768 blocks of rows of 4096 keys and more.  Whole backward of one row of
 // 64 query heads, two slices / four, documents of up to 1500 tokens, up to 4096, 1500 to 6000, and ONE: 8192 tokens 367 / 373,
 // 602 / 568, 994 / 924, 1683 / 1689 us; 12288 (768 blocks) 554 / 557, 970 / 963, 1296 / 1254, 3826 / 3712; beyond the line 14000 571 / 593,
@@ -144,7 +148,9 @@ int dkdv_parts_for(const gptoss_attn_params *p, bool padded, bool packed) {
     const int64_t rows_seen = window > 0 ? (int64_t)kDkdvKeys + window - 1 : (int64_t)p->Sq;
     const int64_t tiles = ((rows_seen < p->Sq ? rows_seen : p->Sq) + 63) / 64;
     int64_t parts = (1024 + blocks - 1) / blocks;
-    if (blocks > 512) parts = p->Sq >= (padded && p->B > 1 ? 1024 : 4096) && (padded && p->B > 1 ? blocks / 2 : blocks) < 1024 ? 2 : 1;
+    // (rows that attn_bwd_dkdv64_kernel takes)
+    const bool by_lengths = p->B > 1 && window == 0 && p->Sq == p->Skv && p->q_offset == 0 && !p->q_offset_dev;
+    if (many_key_blocks(p)) parts = p->Sq >= (!by_lengths ? 4096 : padded ? 1024 : 1280) && (padded && p->B > 1 ? blocks / 2 : blocks) < 1024 ? 2 : 1;
     if (packed && window == 0 && p->Sq >= 4096 && blocks >= 256 && blocks <= 768 && parts < 4) parts = 4;
     const int64_t steps = window > 0 ? tiles / 4 : tiles * (p->H / p->G) / 8;
     if (parts > steps) parts = steps;
@@ -719,11 +725,12 @@ static int launch_dkdv(const gptoss_attn_params *p, void *stream, bool whole_blo
     }
     if (dkdv64_route(p, a.dkdv_parts)) {
         const int64_t blocks = (int64_t)a.B * ((a.Skv + Dkdv64::BN - 1) / Dkdv64::BN);      // of a KV head
-        // padded and packed rows: pieces by the walks' lengths, at most as many as there are slots for partial sums (Dkdv64Plan)
-        const bool by_lengths = a.dkdv_parts > 1 && (a.seqlens || a.doc_start);
+        // padded and packed rows, and several rows of one length whose blocks would stay whole otherwise: pieces by the walks' lengths,
+        // at most as many as there are slots for partial sums (Dkdv64Plan)
+        const bool by_lengths = a.dkdv_parts > 1 && (a.seqlens || a.doc_start || (a.B > 1 && a.Sq < 4096 && many_key_blocks(p)));
         if (by_lengths) a.dkdv_slots = (int)((int64_t)a.dkdv_parts * a.B * a.Skv / Dkdv64::BN);
         const int64_t grid64 = a.G * (by_lengths ? a.dkdv_slots : blocks * a.dkdv_parts);
-        const bool plain = !a.seqlens && !a.doc_start && a.Sq % kTile == 0;
+        const bool plain = !by_lengths && !a.seqlens && !a.doc_start && a.Sq % kTile == 0;
         const int s = plain ? launch(attn_bwd_dkdv64_kernel<false>, grid64, 256, st, a) : launch(attn_bwd_dkdv64_kernel<true>, grid64, 256, st, a);
         if (s || a.dkdv_parts == 1) return s;
         if (by_lengths) return launch_reduce(attn_bwd_dkdv64_reduce_kernel, a.G * blocks * 16 * 256, st, a, with_dsinks);

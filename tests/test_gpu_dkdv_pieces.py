@@ -21,3 +21,8 @@ _check = TWD.test_64_key_backward_of_any_length_vs_eager_oracle
 ])
 def test_pieces_vs_eager_oracle(A, b, h, g, s, lens, docs):
     _check(A, b, h, g, s, lens, docs)
+
+
+@pytest.mark.parametrize("b,h,g,s", [(7, 8, 8, 1283), (33, 4, 2, 1344)])       # off whole tiles and on them
+def test_several_rows_of_one_length(A, b, h, g, s):
+    _check(A, b, h, g, s, None, None)
