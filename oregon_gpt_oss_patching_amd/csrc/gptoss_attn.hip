@@ -147,7 +147,12 @@ int dkdv_parts_for(const gptoss_attn_params *p, bool padded, bool packed) {
     const int window = effective_window(p);
     const int64_t rows_seen = window > 0 ? (int64_t)kDkdvKeys + window - 1 : (int64_t)p->Sq;
     const int64_t tiles = ((rows_seen < p->Sq ? rows_seen : p->Sq) + 63) / 64;
-    int64_t parts = (1024 + blocks - 1) / blocks;
+    // Rows of one length of up to 1024 tokens: fewer shares, each with 64 KB of partial sums that are written and read again (forward + backward, us,
+    // shares for a thousand workgroups / for 768: 8 x 300 tokens 112.6 / 105.5, 6 x 400 118.7 / 112.3, 5 x 621 167.6 / 161.4, 3 x 700 135 / 129, 2 x 900
+    // 135 / 131, 4 x 1000 243 / 232; 1 x 1500 160 / 159, but 3 x 1200 226 / 232; padded 5 x 621 117 / 121, 2 x 1555
+    // 151 / 155; the 64-key kernel's 1 x 2500 303 / 302, but 2 x 3001 would get two shares instead of three).
+    const int64_t workgroups = p->Skv <= 1024 && window == 0 && !padded && !packed ? 768 : 1024;
+    int64_t parts = (workgroups + blocks - 1) / blocks;
     // (rows that attn_bwd_dkdv64_kernel takes)
     const bool by_lengths = p->B > 1 && window == 0 && p->Sq == p->Skv && p->q_offset == 0 && !p->q_offset_dev;
     if (many_key_blocks(p)) parts = p->Sq >= (!by_lengths ? 4096 : padded ? 1024 : 1280) && (padded && p->B > 1 ? blocks / 2 : blocks) < 1024 ? 2 : 1;
