@@ -248,11 +248,13 @@ def attention_backward(q, k, v, sinks, o, lse, d_o, sm_scale, window=None, q_off
 # node per library call and never look inside.
 OP_NAMESPACE = "gptoss_attn"
 _ops_ready = False
+_attention_op = None
 
 
 def _register_ops() -> None:
-    global _ops_ready
+    global _ops_ready, _attention_op
     _lib.load_torch_ops()
+    _attention_op = torch.ops.gptoss_attn.attention.default
 
     @torch.library.register_fake(f"{OP_NAMESPACE}::fwd")
     def _fwd_fake(q, k, v, sinks, sm_scale, window, q_offset, seqlens, doc_start, q_offset_dev=None):
@@ -301,8 +303,7 @@ def attention(q, k, v, sinks, sm_scale, bandwidth, start_q, seqlens=None, doc_st
         seqlens = torch.as_tensor(seqlens, dtype=torch.int32)
     if doc_start is not None and not torch.is_tensor(doc_start):
         doc_start = torch.as_tensor(doc_start, dtype=torch.int32)
-    return torch.ops.gptoss_attn.attention.default(q, k, v, sinks, float(sm_scale), int(bandwidth or 0), q_offset, seqlens, doc_start,
-                                                   q_offset_dev)
+    return _attention_op(q, k, v, sinks, float(sm_scale), int(bandwidth or 0), q_offset, seqlens, doc_start, q_offset_dev)
 
 
 class _attention:

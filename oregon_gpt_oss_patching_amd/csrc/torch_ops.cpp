@@ -267,6 +267,15 @@ struct AttentionFunction : public torch::autograd::Function<AttentionFunction> {
 Tensor attention(const Tensor &q, const Tensor &k, const Tensor &v, const OptTensor &sinks, double sm_scale, SymInt window, SymInt q_offset,
                  const OptTensor &seqlens, const OptTensor &doc_start, const OptTensor &q_offset_dev) {
     check_kinds(q, k, v, true);        // (the shapes: gptoss_attn::fwd)
+    // Nothing to differentiate (inference): no node, nothing saved; a microsecond of a decoding step's twelve.  (Dual tensors take the
+    // node, which refuses them.)
+    bool inference = q.scalar_type() != at::kHalf;
+    for (const Tensor *t : {&q, &k, &v, sinks ? &*sinks : &q})
+        inference = inference && !(at::GradMode::is_enabled() && t->requires_grad()) && !t->_fw_grad(0).defined();
+    if (inference) {
+        const at::AutoDispatchBelowADInplaceOrView below;
+        return std::get<0>(call_fwd(q, k, v, sinks, sm_scale, window, q_offset, seqlens, doc_start, q_offset_dev));
+    }
     return AttentionFunction::apply(q, k, v, sinks, sm_scale, window, q_offset, seqlens, doc_start, q_offset_dev);
 }
 
