@@ -320,7 +320,27 @@ __device__ __forceinline__ int document_end(const int32_t *dsrow, int S, int j, 
     return __builtin_amdgcn_readfirstlane(hi);
 }
 
-template <int NW, int NB, bool DOCS>  // NB = 32-key blocks per wavefront; DOCS = packed rows (doc_start given)
+// Short rows of self-attention without padding: the walks of a row's key blocks (all query tiles x r heads for the first one, two tiles less
+// for each that follows) cut into pieces of dkdv_steps (query tile, head) steps, numbered block by block.  What bounds these launches is their
+// longest workgroup (about 10 us and 1.9 per step); slices of whole tiles are 16 to 32 steps where the share of a compute unit is 8
+// to 20.  A piece's sums are a slot of the scratch: dK, then dV, of 4 wavefronts' 32 keys, each as its eight accumulator quads
+// of 64 lanes (whole cache lines both when they are written and when they are read).
+struct DkdvPieces {
+    static constexpr int kWaveFloats = 32 * kD, kSlot = 2 * 4 * kWaveFloats;
+    static __host__ __device__ int of(int Sq, int r, int steps, int kt) { return ((((Sq + kTile - 1) / kTile - 2 * kt) * r) + steps - 1) / steps; }
+    // block and number within the block of piece p
+    static __device__ __forceinline__ void find(const KArgs &a, int lane, int p, int &kt, int &k) {
+        const int mine = of(a.Sq, a.r, a.dkdv_steps, lane);                // (lane = block; the caller's rows have at most 64)
+        for (kt = 0, k = p;; ++kt) {
+            const int c = __builtin_amdgcn_readlane(mine, kt);
+            if (k < c) break;
+            k -= c;
+        }
+    }
+};
+
+// NB = 32-key blocks per wavefront; DOCS = packed rows (doc_start given); PIECES: DkdvPieces (an instantiation: the slices' one is 4 % slower with both)
+template <int NW, int NB, bool DOCS, bool PIECES = false>
 __global__ __launch_bounds__(NW * 64, (NB == 1 ? 2 : 1)) void attn_bwd_dkdv_kernel(const KArgs a) {
     const int q_offset = query_offset(a);
     static_assert(NW == 4, "the asynchronous tile copy is written for 4 wavefronts");
@@ -337,9 +357,14 @@ __global__ __launch_bounds__(NW * 64, (NB == 1 ? 2 : 1)) void attn_bwd_dkdv_kern
     int bid = blockIdx.x;
     const int g = bid % a.G; bid /= a.G;
     const int bi = bid % a.B; bid /= a.B;
-    const int part = bid % a.dkdv_parts; bid /= a.dkdv_parts;
-    const int kt = bid;                                   // ascending: most work first
-    const int b = rotated_batch_row(bi, kt, a.B);
+    int part, kt;
+    if constexpr (PIECES) {
+        DkdvPieces::find(a, lane, bid, kt, part);
+    } else {
+        part = bid % a.dkdv_parts;
+        kt = bid / a.dkdv_parts;                          // ascending: most work first
+    }
+    const int b = PIECES ? bi : rotated_batch_row(bi, kt, a.B);
     const int j0 = kt * BN;                               // first key of the workgroup
     const int wj0 = j0 + WK * w;                          // first key of the wavefront
 
@@ -365,9 +390,11 @@ __global__ __launch_bounds__(NW * 64, (NB == 1 ? 2 : 1)) void attn_bwd_dkdv_kern
     const int qt_all_hi = (i_hi + kTile - 1) / kTile;
     const int nq_all = max(0, qt_all_hi - qt_lo);
     const int slice = (nq_all + a.dkdv_parts - 1) / a.dkdv_parts;
-    const int qt_hi = qt_all_hi - part * slice;
+    // A piece may start and end inside a tile.
+    const int first = PIECES ? part * a.dkdv_steps : 0, h_first = PIECES ? first % a.r : 0;
+    const int qt_hi = qt_all_hi - (PIECES ? first / a.r : part * slice);
     const int nq = max(0, min(slice, nq_all - part * slice));
-    const int n_it = nq * a.r;
+    const int n_it = PIECES ? max(0, min(a.dkdv_steps, nq_all * a.r - first)) : nq * a.r;
 
     // K, V fragments (B operands): lane = key, slots = head_dim
     bf16x8 kf[NB][4], vf[NB][4];
@@ -412,10 +439,10 @@ __global__ __launch_bounds__(NW * 64, (NB == 1 ? 2 : 1)) void attn_bwd_dkdv_kern
     // them in its XCD's L2.  The walk is kept as running pointers (one step per request):
     // no division or 64-bit multiplication in the loop.
     const AsyncLaneOffsets qlane = make_async_offsets(a.qs.s, lane, w), glane = make_async_offsets(a.dos.s, lane, w);
-    int iss_h = 0, iss_i0 = (qt_hi - 1) * kTile;                      // head within the group, first row of the tile
-    const bf16 *qtile = a.q + (int64_t)b * a.qs.b + (int64_t)(g * a.r) * a.qs.h + (int64_t)iss_i0 * a.qs.s;
-    const bf16 *gtile = a.d_o + (int64_t)b * a.dos.b + (int64_t)(g * a.r) * a.dos.h + (int64_t)iss_i0 * a.dos.s;
-    int64_t stat_off = ((int64_t)b * a.H + (int64_t)g * a.r) * a.Sq + iss_i0;    // (b, head, row) of the tile's first row
+    int iss_h = h_first, iss_i0 = (qt_hi - 1) * kTile;                // head within the group, first row of the tile
+    const bf16 *qtile = a.q + (int64_t)b * a.qs.b + (int64_t)(g * a.r + h_first) * a.qs.h + (int64_t)iss_i0 * a.qs.s;
+    const bf16 *gtile = a.d_o + (int64_t)b * a.dos.b + (int64_t)(g * a.r + h_first) * a.dos.h + (int64_t)iss_i0 * a.dos.s;
+    int64_t stat_off = ((int64_t)b * a.H + (int64_t)g * a.r + h_first) * a.Sq + iss_i0;    // (b, head, row) of the tile's first row
     // wavefront w copies the statistics of 16 rows (16 bytes each) per tile, and 16 document starts
     const u32x4 *stat_lane = a.split + 16 * w + (lane & 15);
     const int32_t *doc_lane = DOCS ? a.doc_start + (int64_t)b * a.Sq + 16 * w + (lane & 15) : nullptr;
@@ -453,7 +480,7 @@ __global__ __launch_bounds__(NW * 64, (NB == 1 ? 2 : 1)) void attn_bwd_dkdv_kern
             stat_off -= (int64_t)a.r * a.Sq + kTile;
         }
     };
-    int cur_h = 0, cur_i0 = (qt_hi - 1) * kTile;                      // the same walk for the tile being consumed
+    int cur_h = h_first, cur_i0 = (qt_hi - 1) * kTile;                // the same walk for the tile being consumed
     // vector-memory instructions one wavefront issues per iteration: 5, or 6 with document starts
 
     // One iteration on a compile-time LDS stage, so that every fragment address is
@@ -509,6 +536,21 @@ __global__ __launch_bounds__(NW * 64, (NB == 1 ? 2 : 1)) void attn_bwd_dkdv_kern
         if (it + 2 < n_it) iterate(it + 2, std::integral_constant<int, 2>{});
     }
 
+    if constexpr (PIECES) {
+        float *out = a.dkdv_partial + (((int64_t)b * a.G + g) * a.dkdv_slots + bid) * DkdvPieces::kSlot + w * DkdvPieces::kWaveFloats + lane * 4;
+        static_assert(NB == 1, "a slot holds 32 keys per wavefront");
+#pragma unroll
+        for (int dblk = 0; dblk < 2; ++dblk)
+#pragma unroll
+            for (int a4 = 0; a4 < 4; ++a4) {
+                f32x4 xk, xv;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) { xk[e] = dk[0][dblk][4 * a4 + e]; xv[e] = dv[0][dblk][4 * a4 + e]; }
+                *reinterpret_cast<f32x4 *>(out + (4 * dblk + a4) * 256) = xk;
+                *reinterpret_cast<f32x4 *>(out + DkdvPieces::kSlot / 2 + (4 * dblk + a4) * 256) = xv;
+            }
+        return;
+    }
     if (a.dkdv_parts > 1) {
         // unscaled fp32 partial sums; lane = key row, register i of block dblk = column 32*dblk + crow(i, half),
         // four consecutive columns per 16-byte store
@@ -584,6 +626,38 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_reduce_kernel(const KArgs a
     union { bf16x8 v; u32x4 u; } cv;
     cv.v = out;
     *reinterpret_cast<u32x4 *>(dst) = cv.u;
+}
+
+// The same for slots of DkdvPieces.  A block of threads: 32 keys of one tensor, eight threads per key.
+__global__ __launch_bounds__(256) void attn_bwd_dkdv_pieces_reduce_kernel(const KArgs a, int heads) {
+    __shared__ float red[1024];
+    if ((int)blockIdx.x < heads) { dsinks_of_head<256>(a, blockIdx.x, red); return; }
+    int bid = blockIdx.x - heads;
+    const int which = bid & 1; bid >>= 1;                                 // 0 = dK, 1 = dV
+    const int key_blocks = (a.Skv + 31) / 32, k32 = bid % key_blocks; bid /= key_blocks;
+    const int g = bid % a.G, b = bid / a.G;
+    const int kt = k32 >> 2, w = k32 & 3, chunk = threadIdx.x & 7, row = threadIdx.x >> 3, key = 32 * k32 + row;
+    const int mine = DkdvPieces::of(a.Sq, a.r, a.dkdv_steps, threadIdx.x & 63);
+    int base = 0;
+    for (int i = 0; i < kt; ++i) base += __builtin_amdgcn_readlane(mine, i);
+    const int n = __builtin_amdgcn_readlane(mine, kt);
+    if (key >= a.Skv) return;
+    const float *src = a.dkdv_partial + (((int64_t)b * a.G + g) * a.dkdv_slots + base) * DkdvPieces::kSlot + which * (DkdvPieces::kSlot / 2) +
+                       w * DkdvPieces::kWaveFloats + chunk * 256 + row * 4;
+    f32x4 lo = {0.0f, 0.0f, 0.0f, 0.0f}, hi = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 4
+    for (int k = 0; k < n; ++k) {
+        const f32x4 x = *reinterpret_cast<const f32x4 *>(src + (int64_t)k * DkdvPieces::kSlot);
+        const f32x4 y = *reinterpret_cast<const f32x4 *>(src + (int64_t)k * DkdvPieces::kSlot + 128);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { lo[e] += x[e]; hi[e] += y[e]; }
+    }
+    const float mul = which == 0 ? a.scale : 1.0f;
+    union { bf16x8 v; u32x4 u; } out;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) { out.v[e] = (bf16)(lo[e] * mul); out.v[4 + e] = (bf16)(hi[e] * mul); }
+    const Strides &st = which == 0 ? a.dks : a.dvs;
+    *reinterpret_cast<u32x4 *>((which == 0 ? a.dk : a.dv) + (int64_t)b * st.b + (int64_t)g * st.h + (int64_t)key * st.s + chunk * 8) = out.u;
 }
 
 // ---------------------------------------------------------------------------------

@@ -56,6 +56,7 @@ struct KArgs {
     int dkdv_parts;      // dK/dV kernel: workgroups that share one key block, each taking a slice of its query tiles
     float *dkdv_partial; // dkdv_parts > 1: fp32 partial sums, [part][dK, dV][B][G][Skv][64] or in slots (dkdv_slots)
     int dkdv_slots;      // > 0: attn_bwd_dkdv64_kernel divides the work by the walks' lengths (Dkdv64Plan); slots per KV head that these bytes hold
+    int dkdv_steps;      // > 0: attn_bwd_dkdv_kernel cuts its walks into pieces of so many (query tile, head) steps (DkdvPieces), dkdv_slots of them per batch row and KV head
     int kv_splits;       // forward: workgroups that share one query block, each taking a slice of its keys
     float *fwd_partial;  // kv_splits > 1: fp32 partial results of the slices
     int chunk_tiles;     // single-pass window backward: 64-row query tiles per workgroup

@@ -86,6 +86,7 @@ KArgs make_args(const gptoss_attn_params *p, SinkTypes ty) {
     a.scale_log2 = p->scale * kLog2e;
     a.dkdv_parts = 1;
     a.dkdv_slots = 0;
+    a.dkdv_steps = 0;
     a.kv_splits = 1;
     a.fwd_partial = nullptr;
     a.chunk_tiles = 0;
@@ -120,7 +121,7 @@ bool many_key_blocks(const gptoss_attn_params *p) { return (int64_t)p->G * p->B 
 // slices so that there are about a thousand workgroups, and sum the slices' fp32 partials afterwards.  A slice
 // keeps at least four query tiles of a sliding-window layer (windows of up to 321 keys stay whole, wider ones are cut) and at least
 // eight (query tile, head) steps of a full-causal one, which may be a single tile.  Up to 512 blocks the count is rounded
-// up (B = 2, S = 383: 78 us uncut, 25 + 5 us in six slices).  Between 512 and 1024 blocks the first
+// up (B = 2, S = 383: 78 us uncut, 25 + 5 us in six slices; unpadded short rows then take pieces of other lengths in the same scratch, dkdv_pieces_for).  Between 512 and 1024 blocks the first
 // key block of a long row (4096 rows and more) is still longer than the average compute unit's share: two slices; a
 // right-padded batch counts half, because its shorter rows leave the longest one alone (dK/dV of B = 4, S = 4096,
 // lengths 3309 / 1968 / 1554 / 4079: 715 us uncut, 589 in two slices; B = 2, S = 8192 / 4000: 1437 and 1216).  Several rows of 1280 tokens and
@@ -162,6 +163,33 @@ int dkdv_parts_for(const gptoss_attn_params *p, bool padded, bool packed) {
     if (parts > tiles) parts = tiles;
     if (parts > 8) parts = 8;
     return parts < 1 ? 1 : (int)parts;
+}
+
+// Pieces of the 32-key kernel's walks (DkdvPieces) instead of equal slices of whole tiles: the shortest ones, of four steps or more, of which
+// there are no more than 512 (two workgroups per compute unit of a 256-CU part: all run at once and end together) and than the
+// scratch has slots for.  Taken for one row where they are no longer than the longest slice, for several (whose tiles a piece that starts elsewhere does
+// not find in L2) where they are shorter.  dK/dV and the sum of its parts, us, slices / pieces: 2 x 383 tokens 29.8 / 26.9, 2 x 621 47.0 / 37.5,
+// 1 x 1024 47.0 / 41.5, 1 x 1900 95 / 83; not taken: 4 x 1000 (pieces as long as the slices) whole call 227 / 234, 3 x 1200 (longer)
+// 234 / 243, 4 x 160 (longer) 47 / 52.  Nor for padded or packed rows, whose slices follow the lengths: 1500 and 700 tokens 194 / 210, documents of
+// 700, 600 and 500 150 / 164.  From 2048 tokens on the 64-key kernel takes over.
+void dkdv_pieces_for(const gptoss_attn_params *p, KArgs &a) {
+    if (a.dkdv_parts == 1 || p->seqlens || p->doc_start || effective_window(p) > 0 || p->Sq != p->Skv || p->q_offset != 0 || p->q_offset_dev ||
+        p->Skv >= 2048)
+        return;
+    const int blocks = (p->Skv + kDkdvKeys - 1) / kDkdvKeys, tiles = (p->Sq + kTile - 1) / kTile;
+    const int64_t rows = (int64_t)p->G * p->B, slots = (int64_t)a.dkdv_parts * p->Skv / kDkdvKeys;       // (of a row)
+    const int64_t most = slots < 512 / rows ? slots : 512 / rows;
+    const int slice = (tiles + a.dkdv_parts - 1) / a.dkdv_parts * a.r;
+    if (most < blocks) return;
+    const int64_t all = (int64_t)blocks * (tiles + 1 - blocks) * a.r;                                    // steps of a row: no shorter pieces than all / most
+    for (int steps = (int)(all > 4 * most ? (all + most - 1) / most : 4); steps < slice + (p->B == 1); ++steps) {
+        int n = 0;
+        for (int i = 0; i < blocks; ++i) n += DkdvPieces::of(a.Sq, a.r, steps, i);
+        if (n > most) continue;
+        a.dkdv_steps = steps;
+        a.dkdv_slots = n;
+        return;
+    }
 }
 
 // Full-causal self-attention goes to attn_bwd_dkdv64_kernel (64 keys per wavefront, one wavefront per SIMD)
@@ -741,10 +769,13 @@ static int launch_dkdv(const gptoss_attn_params *p, void *stream, bool whole_blo
         if (by_lengths) return launch_reduce(attn_bwd_dkdv64_reduce_kernel, a.G * blocks * 16 * 256, st, a, with_dsinks);
         return launch_reduce(attn_bwd_dkdv_reduce_kernel, (int64_t)2 * a.B * a.G * a.Skv * 8, st, a, with_dsinks);
     }
-    const int64_t grid = (int64_t)a.G * a.B * a.dkdv_parts * ((a.Skv + kDkdvKeys - 1) / kDkdvKeys);
+    dkdv_pieces_for(p, a);
+    const int64_t grid = (int64_t)a.G * a.B * (a.dkdv_steps ? a.dkdv_slots : a.dkdv_parts * ((a.Skv + kDkdvKeys - 1) / kDkdvKeys));
     const int s = a.doc_start ? launch(attn_bwd_dkdv_kernel<kDkdvWaves, kDkdvNB, true>, grid, 64 * kDkdvWaves, st, a)
+                 : a.dkdv_steps ? launch(attn_bwd_dkdv_kernel<kDkdvWaves, kDkdvNB, false, true>, grid, 64 * kDkdvWaves, st, a)
                               : launch(attn_bwd_dkdv_kernel<kDkdvWaves, kDkdvNB, false>, grid, 64 * kDkdvWaves, st, a);
     if (s || a.dkdv_parts == 1) return s;
+    if (a.dkdv_steps) return launch_reduce(attn_bwd_dkdv_pieces_reduce_kernel, (int64_t)2 * a.B * a.G * ((a.Skv + 31) / 32) * 256, st, a, with_dsinks);
     return launch_reduce(attn_bwd_dkdv_reduce_kernel, (int64_t)2 * a.B * a.G * a.Skv * 8, st, a, with_dsinks);
 }
 
