@@ -1,12 +1,14 @@
 // float32 attention on the bf16 matrix pipes: every float32 operand as the sum of three bf16 terms.
 //
 // Why.  The fp32 matrix instruction takes sixteen times as long per product as the bf16 one, and the kernels of attn_f32.h are
-// bound by it.  A float32 number IS the sum of three bf16 numbers (its significand cut into 8 + 8 + 8 bits, each term exact), a
-// product of two bf16 numbers is exact in fp32, and the bf16 instruction accumulates in fp32.  Of the nine term products six are
-// kept (hi lo, lo hi, mid mid, hi mid, mid hi, hi hi: added from small to large); the three dropped ones are below 2^-23 of the
-// product together, less than one rounding of the accumulation.  That is 192 cycles of the pipe where the fp32 instruction takes
-// 512, and one rounding per 16 steps of a contraction instead of one per 2: against float64 the error of a contraction over 64
-// is 1.33e-7 (relative 2-norm, N(0, 1); fp32 instruction 1.43e-7), over 1024 4.7e-7 (5.9e-7).
+// bound by it.  A float32 number IS the sum of three bf16 numbers (the number rounded to nearest, what is left rounded to nearest, the
+// rest: 8 + 8 + 8 bits, each term exact), a product of two bf16 numbers is exact in fp32, and the bf16 instruction accumulates in
+// fp32.  Of the nine term products six are kept (hi lo, lo hi, mid mid, hi mid, mid hi, hi hi).  With operands in [1, 2) mid is at most 2^-8 and lo
+// at most 2^-17, so the three dropped ones are at most 2^-24 together, either sign: half a rounding of the product in the last
+// place.  (Terms cut off instead of rounded would lose up to 2^-21 and always towards zero.)  That is 192 cycles of the pipe where the fp32 instruction takes 512.
+// The order of the additions matters as much as the terms: an addition to an accumulator rounds at the accumulator's size (the instruction
+// adds its 16 products in two groups of eight, each sum rounded once).  S and dP therefore take the small products of the whole contraction first and
+// the four hi hi last: eight roundings at full size instead of 48.  And -delta, which is often almost all of dP, is added behind the products.
 //
 // What the split asks of the numbers.  Terms are exact while they stay normal and nothing overflows: inputs that are 0 or of magnitude
 // 2^-100 to 2^24 (SplitCheck); a workgroup that meets any other (infinities and NaN among them) takes the walk of attn_f32.h
@@ -24,7 +26,10 @@
 // What bounds it (S = 1024, 64 query heads on 8 KV heads, full causal; fp32 instruction / this): forward 101 / 61 us, dQ 134 / 85, dK/dV
 // 176 / 95, the whole call 413 / 259; S = 4096 5350 / 3280.  The matrix pipes are busy 43, 46 and 55 % of the cycles: about eight
 // vector instructions per MFMA in the forward (cutting the weights is 88 of a tile's 290), and the two wavefronts of a SIMD start each step together.
-// Error against float64 (relative 2-norm; fp32 instruction / this): O 2.8e-7 / 2.2e-7, lse 5.0e-8 / 5.4e-8 (its last rounding is 4e-8), dQ 4.7e-7 / 3.8e-7, dK 6.4e-7 / 4.1e-7, dV 6.2e-7 / 3.9e-7.
+// Error against float64 (relative 2-norm, S = 1024, fp32 instruction / this), N(0, 1): O 3.0e-7 / 1.3e-7, lse 4.8e-8 / 4.8e-8, dQ 4.4e-7 / 3.4e-7, dK
+// 6.0e-7 / 5.1e-7, dV 5.9e-7 / 5.1e-7; all operands in [1, 1 + 2^-7], where dP - delta cancels: dQ 2.2e-3 / 2.1e-3, dK 1.24e-5 / 1.15e-5; powers of two
+// times 1 + 2^-7 - 2^-23: O 2.6e-7 / 1.4e-7, dK 5.6e-7 / 4.3e-7; one non-zero number per row: O 7.7e-8 / 7.1e-8, dK 2.85e-7 / 2.85e-7, dV 2.86e-7 / 3.06e-7 (a product is six
+// additions to dV, which shows where a sum has few).
 #pragma once
 #include "attn_f32.h"
 
@@ -72,40 +77,45 @@ struct SplitCheck {
     __device__ __forceinline__ bool bad() const { return most > 0x4B800000u || least < 0x0D800000u - 1u; }
 };
 
-// eight numbers as three bf16 vectors whose sum they are: the top 16 bits, the top 16 bits of what is left, the rest (exact)
+// A pair of numbers as bf16, each to nearest even, in one register; and what they leave of it (exact).
+__device__ __forceinline__ uint32_t split_round2(float x, float y) {
+    typedef __attribute__((ext_vector_type(2))) float f32x2;
+    typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{x, y}), bf16x2));
+}
+__device__ __forceinline__ void split_rest2(float &x, float &y, uint32_t p) {
+    x -= __uint_as_float(p << 16);
+    y -= __uint_as_float(p & 0xffff0000u);
+}
+// eight numbers as three bf16 vectors whose sum they are: the number rounded to bf16, what is left rounded to bf16, the rest (exact)
 __device__ __forceinline__ void split8(const float (&x)[8], bf16x8 (&t)[3]) {
     u32x4 w[3];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        uint32_t a[3], b[3];
         float u = x[2 * i], v = x[2 * i + 1];
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
-            a[k] = __float_as_uint(u);
-            b[k] = __float_as_uint(v);
-            if (k < 2) {
-                u -= __uint_as_float(a[k] & 0xffff0000u);
-                v -= __uint_as_float(b[k] & 0xffff0000u);
-            }
-            w[k][i] = __builtin_amdgcn_perm(b[k], a[k], 0x07060302u);
+            w[k][i] = split_round2(u, v);
+            if (k < 2) split_rest2(u, v, w[k][i]);
         }
     }
 #pragma unroll
     for (int k = 0; k < 3; ++k) t[k] = as_bf16x8(w[k]);
 }
 // Registers 8u .. 8u + 7 of a C block, the k slots that a transposed fragment of the same 16-row step holds, cut into terms in twelve
-// steps of four or five instructions (an MFMA leaves room for four), a pair of numbers in three.
+// steps of at most five instructions (an MFMA leaves room for four), a pair of numbers in three.
 struct SplitSteps {
     float r[2];
     u32x4 w[3];
     __device__ __forceinline__ void step(const f32x16 &c, int u, int i) {
         const int pair = i / 3, k = i % 3;
-        const float x = k == 0 ? c[8 * u + 2 * pair] : r[0], y = k == 0 ? c[8 * u + 2 * pair + 1] : r[1];
-        const uint32_t a = __float_as_uint(x), b = __float_as_uint(y);
-        w[k][pair] = __builtin_amdgcn_perm(b, a, 0x07060302u);
+        float x = k == 0 ? c[8 * u + 2 * pair] : r[0], y = k == 0 ? c[8 * u + 2 * pair + 1] : r[1];
+        const uint32_t p = split_round2(x, y);
+        w[k][pair] = p;
         if (k < 2) {
-            r[0] = x - __uint_as_float(a & 0xffff0000u);
-            r[1] = y - __uint_as_float(b & 0xffff0000u);
+            split_rest2(x, y, p);
+            r[0] = x;
+            r[1] = y;
         }
     }
     __device__ __forceinline__ void take(bf16x8 (&t)[3]) const {
@@ -127,42 +137,65 @@ struct SplitKept {
         *reinterpret_cast<__attribute__((address_space(3))) bf16x8 *>((uintptr_t)(at + i * 1024)) = x;
     }
 };
-// A step of a contraction is six MFMAs, the small terms first (the large ones first: O of 1024 keys 2.9e-7 from float64 instead of 2.6e-7).
-// s += X Y^T over head_dim: X's rows from three planes (OFF bytes behind the addresses `at`), y the lane's row of Y.  A fragment's
-// register is loaded with the next step's right behind its last use.  Term p of y in step ks is fragment KEPT(p, ks) of `kept`, or
-// in its register where that is negative.
+// s += X Y^T over head_dim: X's rows from three planes (OFF bytes behind the addresses `at`), y the lane's row of Y.  24 MFMAs: the five
+// small products of the four 16-deep steps, small ones first, then the four products of the first terms, the last step's first
+// (its operands are at hand; the others' are read again).  S of N(0, 1) with the six products of a step together: O 2.0e-7 from float64 instead of 1.3e-7, lse 4.82e-8 instead of
+// 4.79e-8, the whole call 0.2 % faster.  A fragment's register is loaded with the next step's right behind its last use.  Term p of y in step ks is
+// fragment KEPT(p, ks) of `kept`, or in its register where that is negative.
+// FLIP: X and Y have changed places (dK/dV, whose tiles are the rows that dQ holds): each pair of products of equal size is added in the other
+// order, so that S and dP have the bits that the forward and dQ see.
 // work(i) is issued behind MFMA i of the 24.
-template <int OFF, typename Kept, typename Work>
+template <int OFF, bool FLIP, typename Kept, typename Work>
 __device__ __forceinline__ void split_rows_product(f32x16 &s, const TileLaneOffsets &at, const bf16x8 (&y)[4][3], const SplitKept &kept, Kept kept_at, Work work) {
     auto load = [&](int ks, int p) __attribute__((always_inline)) { return as_bf16x8(lds_load128(at.nat[ks], OFF + p * F32Split::kPlane)); };
     auto term = [&](int ks, int p) __attribute__((always_inline)) { return kept_at(p, ks) >= 0 ? kept.get(kept_at(p, ks)) : y[ks][p]; };
+    auto mac = [&](const bf16x8 &x, const bf16x8 &y_, int i) __attribute__((always_inline)) {
+        s = mfma_bf16(x, y_, s);
+        work(i);
+        GPTOSS_F32_FENCE();
+    };
     bf16x8 x2 = load(0, 2), y0 = term(0, 0), x1 = load(0, 1), y1 = term(0, 1), x0 = load(0, 0), y2 = term(0, 2);
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
         const bool more = ks < 3;
-        auto mac = [&](const bf16x8 &x, const bf16x8 &y_, int i) __attribute__((always_inline)) {
-            s = mfma_bf16(x, y_, s);
-            work(6 * ks + i);
-            GPTOSS_F32_FENCE();
-        };
         GPTOSS_F32_FENCE();
-        mac(x2, y0, 0);
-        if (more) x2 = load(ks + 1, 2);
-        mac(x1, y1, 1);
-        mac(x0, y2, 2);
-        if (more) y2 = term(ks + 1, 2);
-        mac(x1, y0, 3);
-        if (more) x1 = load(ks + 1, 1);
-        mac(x0, y1, 4);
-        if (more) y1 = term(ks + 1, 1);
-        mac(x0, y0, 5);
+        if (FLIP) {
+            mac(x0, y2, 5 * ks);
+            if (more) y2 = term(ks + 1, 2);
+            mac(x1, y1, 5 * ks + 1);
+            mac(x2, y0, 5 * ks + 2);
+            if (more) x2 = load(ks + 1, 2);
+            mac(x0, y1, 5 * ks + 3);
+            if (more) y1 = term(ks + 1, 1);
+            mac(x1, y0, 5 * ks + 4);
+            if (more) x1 = load(ks + 1, 1);
+        } else {
+            mac(x2, y0, 5 * ks);
+            if (more) x2 = load(ks + 1, 2);
+            mac(x1, y1, 5 * ks + 1);
+            mac(x0, y2, 5 * ks + 2);
+            if (more) y2 = term(ks + 1, 2);
+            mac(x1, y0, 5 * ks + 3);
+            if (more) x1 = load(ks + 1, 1);
+            mac(x0, y1, 5 * ks + 4);
+            if (more) y1 = term(ks + 1, 1);
+        }
         if (more) { x0 = load(ks + 1, 0); y0 = term(ks + 1, 0); }
+    }
+#pragma unroll
+    for (int ks = 3; ks >= 0; --ks) {
+        bf16x8 next_x = x0, next_y = y0;
+        if (ks > 0) { next_x = load(ks - 1, 0); next_y = term(ks - 1, 0); }
+        GPTOSS_F32_FENCE();
+        mac(x0, y0, 23 - ks);
+        x0 = next_x;
+        y0 = next_y;
     }
 }
 constexpr int kInRegister = -1;
 struct SplitNoneKept { __device__ __forceinline__ constexpr int operator()(int, int) const { return kInRegister; } };
 struct SplitNoWork { __device__ __forceinline__ void operator()(int) const {} };
-// acc^T[d][col] += X^T[d][row] p[row][col] over the 32 rows of three planes, p as terms of C registers: the first half's at hand, the
+// acc^T[d][col] += X^T[d][row] p[row][col] over the 32 rows of three planes, six MFMAs per 16 rows and 32 columns, small ones first; p as terms of C registers: the first half's at hand, the
 // second half's when work(11) has been issued
 template <int OFF, typename Work>
 __device__ __forceinline__ void split_cols_product(f32x16 (&acc)[2], const TileLaneOffsets &at, const bf16x8 (&p)[2][3], Work work) {
@@ -326,7 +359,7 @@ __global__ __launch_bounds__(512, 2) void attn_f32_split_fwd_kernel(const KArgs 
             f32x16 s;
 #pragma unroll
             for (int i = 0; i < 16; ++i) s[i] = 0.0f;
-            split_rows_product<0>(s, at, qf, SplitKept{}, SplitNoneKept{}, SplitNoWork{});      // S^T: rows = keys, lane = query row
+            split_rows_product<0, false>(s, at, qf, SplitKept{}, SplitNoneKept{}, SplitNoWork{});      // S^T: rows = keys, lane = query row
             if (!wk.interior(a, n0)) {
                 const KeyMask km = make_key_mask(pos - n0, win, wk.kv_len - n0, half);
 #pragma unroll
@@ -456,23 +489,23 @@ __global__ __launch_bounds__(512, 2) void attn_f32_split_dq_kernel(const KArgs a
         if (tile < wk.t_lo + wk.n) {
             f32x16 s, dp;
 #pragma unroll
-            for (int i = 0; i < 16; ++i) { s[i] = 0.0f; dp[i] = ndelta; }
-            split_rows_product<0>(s, at, qf, kept, kept_q, SplitNoWork{});               // S^T
+            for (int i = 0; i < 16; ++i) { s[i] = 0.0f; dp[i] = 0.0f; }
+            split_rows_product<0, false>(s, at, qf, kept, kept_q, SplitNoWork{});               // S^T
 #pragma unroll
             for (int i = 0; i < 16; ++i) s[i] = fmaf(s[i], c, -lse2);
-            // dP^T - delta; the weights behind its MFMAs where all are visible and normal
+            // dP^T; the weights behind its MFMAs where all are visible and normal
             constexpr int kV = F32Split::kTerms * F32Split::kPlane;
             if (wk.interior(a, n0) && split_weights_normal(s)) {
-                split_rows_product<kV>(dp, at, gf, kept, kept_g, [&](int i) __attribute__((always_inline)) { if (i < 16) s[i] = split_weight(s[i]); });
+                split_rows_product<kV, false>(dp, at, gf, kept, kept_g, [&](int i) __attribute__((always_inline)) { if (i < 16) s[i] = split_weight(s[i]); });
             } else {
                 split_any_weights(s);
                 const KeyMask km = make_key_mask(pos - n0, win, wk.kv_len - n0, half);
 #pragma unroll
                 for (int i = 0; i < 16; ++i) s[i] = key_visible(km, 8 * (i >> 2) + (i & 3)) ? s[i] : 0.0f;
-                split_rows_product<kV>(dp, at, gf, kept, kept_g, SplitNoWork{});
+                split_rows_product<kV, false>(dp, at, gf, kept, kept_g, SplitNoWork{});
             }
 #pragma unroll
-            for (int i = 0; i < 16; ++i) dp[i] = s[i] * dp[i];
+            for (int i = 0; i < 16; ++i) dp[i] = s[i] * (dp[i] + ndelta);
             split_cols_product<0>(dq, at, dp);                                           // dQ^T[d][row] += K^T[d][key] dS^T[key][row]
         }
         tile_offsets_move(at, (step & 1) ? (uint32_t)(-2 * F32Split::kKvRecord) : (uint32_t)(2 * F32Split::kKvRecord));
@@ -579,24 +612,15 @@ __global__ __launch_bounds__(512, 2) void attn_f32_split_dkdv_kernel(const KArgs
         if (tile < t_hi && q0 + 31 >= j0 && q0 - weff < j0 + 31 && j0 < kv_len) {
             f32x16 s, dp;
 #pragma unroll
-            for (int i = 0; i < 16; ++i) s[i] = 0.0f;
-            split_rows_product<0>(s, at, kf, kept, kept_k, SplitNoWork{});               // rows = queries, lane = key
+            for (int i = 0; i < 16; ++i) s[i] = dp[i] = 0.0f;
+            split_rows_product<0, true>(s, at, kf, kept, kept_k, SplitNoWork{});               // rows = queries, lane = key
 #pragma unroll
             for (int a4 = 0; a4 < 4; ++a4) {
                 const f32x4 l2 = lds_load128f(stat, 128 + 32 * a4);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) s[4 * a4 + e] = fmaf(s[4 * a4 + e], c, -l2[e]);
             }
-            auto start_dp = [&]() __attribute__((always_inline)) {                       // at -delta of its row
-                GPTOSS_F32_FENCE();
-#pragma unroll
-                for (int a4 = 0; a4 < 4; ++a4) {
-                    const f32x4 nd = lds_load128f(stat, 32 * a4);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) dp[4 * a4 + e] = nd[e];
-                }
-            };
-            // dP - delta; behind its MFMAs the weights, where all are visible and normal, and the terms of their first half
+            // dP; behind its MFMAs the weights, where all are visible and normal, and the terms of their first half
             constexpr int kG = C::kTerms * C::kPlane;
             bf16x8 f[2][3];
             SplitSteps cut;
@@ -606,8 +630,7 @@ __global__ __launch_bounds__(512, 2) void attn_f32_split_dkdv_kernel(const KArgs
             };
             const bool interior = j0 + 31 <= q0 && q0 + 31 - weff < j0 && j0 + 32 <= kv_len && q0 + 32 <= span.row_lim && !dsrow;
             if (interior && split_weights_normal(s)) {
-                start_dp();
-                split_rows_product<kG>(dp, at, vf, kept, kept_v, [&](int i) __attribute__((always_inline)) {
+                split_rows_product<kG, true>(dp, at, vf, kept, kept_v, [&](int i) __attribute__((always_inline)) {
                     if (i < 16) s[i] = split_weight(s[i]);
                     cut_first(i);
                 });
@@ -625,12 +648,15 @@ __global__ __launch_bounds__(512, 2) void attn_f32_split_dkdv_kernel(const KArgs
                         for (int i = 0; i < 16; ++i) s[i] = key >= dsrow[min(first + crow(i, 0), a.Sq - 1)] ? s[i] : 0.0f;
                     }
                 }
-                start_dp();
-                split_rows_product<kG>(dp, at, vf, kept, kept_v, cut_first);
+                split_rows_product<kG, true>(dp, at, vf, kept, kept_v, cut_first);
             }
             // dV^T[d][key] += dO^T[d][row] P[row][key]: the second half of P is cut behind the first MFMAs, the first of dS behind the others
 #pragma unroll
-            for (int i = 0; i < 16; ++i) dp[i] = s[i] * dp[i];
+            for (int a4 = 0; a4 < 4; ++a4) {
+                const f32x4 nd = lds_load128f(stat, 32 * a4);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) dp[4 * a4 + e] = s[4 * a4 + e] * (dp[4 * a4 + e] + nd[e]);
+            }
             split_cols_product<kG>(dv, at, f, [&](int i) __attribute__((always_inline)) {
                 if (i < 12) cut.step(s, 1, i); else cut.step(dp, 0, i - 12);
                 if (i == 11) cut.take(f[1]);
