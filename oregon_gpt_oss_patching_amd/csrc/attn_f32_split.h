@@ -11,7 +11,7 @@
 // the four hi hi last: eight roundings at full size instead of 48.  And -delta, which is often almost all of dP, is added behind the products.
 //
 // What the split asks of the numbers.  Terms are exact while they stay normal and nothing overflows: inputs that are 0 or of magnitude
-// 2^-100 to 2^24 (SplitCheck); a workgroup that meets any other (infinities and NaN among them) takes the walk of attn_f32.h
+// 2^-100 to 2^24 (SplitCheck), and row statistics that go with them; a workgroup that meets any other (infinities and NaN among them) takes the walk of attn_f32.h
 // instead, within the same launch.  Weights are held as 2^24 P (0 or 2^-125 to 2^24: also the terms of denormal ones are) and so is dS.
 // (The factor is a product behind the exponential.  In its argument it would cost precision: a float near 24 is 2^-19 apart.)
 //
@@ -51,6 +51,7 @@ struct F32Split {
     static_assert(4 * kKvRecord <= kRowsLds && kRowsLds <= kDqLds && kRowsLds + kWaves * F32Dkdv::kStatBytes <= kDkdvLds, "two stages of two tiles; the general walk");
 };
 constexpr float kSplitScale = 0x1p24f, kSplitUnscale = 0x1p-24f;       // weights are held as 2^24 P
+constexpr float kSplitMostDelta = 0x1p54f;                             // what 64 products of numbers up to 2^24 and 2^24 reach
 // The weights are 2^24 exp2(x).  The bare exponential instruction flushes what is below 2^-126: whether a wavefront has none of that.
 __device__ __forceinline__ bool split_weights_normal(const f32x16 &x) {
     float lo = fminf(x[0], x[1]);
@@ -439,6 +440,8 @@ __global__ __launch_bounds__(512, 2) void attn_f32_split_dq_kernel(const KArgs a
         ndelta = -xhalf_sum(((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7])));
     }
     const float lse2 = a.lse[rid] * kLog2e;
+    // the statistics, too: dS must not overflow where it is held as 2^24 dS (a V outside the limits that only other workgroups see)
+    const bool stats_bad = live && !(fabsf(ndelta) <= kSplitMostDelta && fabsf(lse2) < INFINITY);
     // the unit's two wavefronts hold the same rows: one leaves Q and the statistics, the other dO
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks)
@@ -447,7 +450,7 @@ __global__ __launch_bounds__(512, 2) void attn_f32_split_dq_kernel(const KArgs a
             if (w & 1) *reinterpret_cast<bf16x8 *>(rec + (3 + p) * F32Split::kPlane + plane_chunk(l32, 2 * ks + half)) = gf[ks][p];
             else *reinterpret_cast<bf16x8 *>(rec + p * F32Split::kPlane + plane_chunk(l32, 2 * ks + half)) = qf[ks][p];
         }
-    const bool rows_bad = __builtin_amdgcn_ballot_w64(check.bad()) != 0ull;
+    const bool rows_bad = __builtin_amdgcn_ballot_w64(check.bad() || stats_bad) != 0ull;
     if (!(w & 1)) {
         reinterpret_cast<float *>(rec + F32Split::kStatOff)[lane] = live ? (half ? lse2 : ndelta) : 0.0f;
         if (lane == 0) a.split_q_bad[rec_i] = rows_bad;

@@ -1,6 +1,7 @@
 """GPU tests of float32 attention on the bf16 matrix pipes (operands as three bf16 terms): edges of tiles, groups and parts, no further
 from float64 than the fp32 matrix instruction, and the numbers the terms do not hold."""
 import ctypes
+import math
 
 import pytest
 import torch
@@ -123,3 +124,24 @@ def test_numbers_that_three_terms_do_not_hold(A, which, value):
         ok = torch.isfinite(y)
         x, y = x[ok].double(), y[ok].double()
         assert float((x - y).norm()) <= 2e-5 * float(y.norm()), name
+
+
+@pytest.mark.parametrize("which,value", [("v", float("inf")), ("v", -1e37), ("lse", -float("inf")), ("lse", float("inf"))])
+def test_row_statistics_that_three_terms_do_not_hold(A, which, value):
+    """A number that only the last row sees makes that row's delta infinite or large, or its lse is infinite: workgroups whose own operands are
+    ordinary still get what the fp32 instruction gives."""
+    q, k, v, sinks, d_out = (t.to(DEV) for t in E.make_inputs(7800, 1, 64, 8, 352, 64, torch.float32))
+    for t in (q[0, :, -1], d_out[0, -1]):
+        t.abs_()                                           # (what reaches dK has one sign: infinite or large, not NaN)
+    if which == "v":
+        v[0, 2, -1, 7] = value
+    o, lse = A.attention_forward(q, k, v, sinks, SCALE)
+    if which == "lse":
+        lse[0, 5, -1] = value
+    new, old = (A.attention_backward(q, k, v, sinks, o, lse, d_out, SCALE, split=split) for split in (False, True))
+    if which == "v" and math.isfinite(value):              # (an infinite one is NaN times nothing in the rows that share its tile, either way)
+        assert not torch.isnan(old[1][0, 2, :300]).any() and float(old[1][0, 2, :300].abs().min()) > 1e20
+    for name, x, y in zip(("dq", "dk", "dv", "dsinks"), new, old):
+        assert torch.equal(torch.isfinite(x), torch.isfinite(y)) and torch.equal(torch.isnan(x), torch.isnan(y)), name
+        ok = torch.isfinite(y)
+        assert bool(((x - y)[ok].abs() <= 1e-4 * y[ok].abs() + 2e-4).all()), name
