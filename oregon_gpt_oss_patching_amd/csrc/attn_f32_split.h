@@ -335,15 +335,15 @@ __global__ __launch_bounds__(512, 2) void attn_f32_split_fwd_kernel(const KArgs 
     SplitCheck check;
     const bool keys_bad = walk.bad(a, wk.b, wk.g);
     bf16x8 qf[4][3];
-    split_row(qf, t.q + (int64_t)wk.b * a.qs.b + (int64_t)wk.head * a.qs.h + (int64_t)min(row, a.Sq - 1) * a.qs.s, row < a.Sq, half, check);
+    int pos;
+    unsigned win;
+    wk.row_info(a, q_offset, row, pos, win);
+    split_row(qf, t.q + (int64_t)wk.b * a.qs.b + (int64_t)wk.head * a.qs.h + (int64_t)min(row, a.Sq - 1) * a.qs.s, pos >= 0, half, check);      // (what a padded row holds must not matter)
     wait_vmcnt<0>();
     if (__syncthreads_or(keys_bad || check.bad())) {
         f32_fwd_rows<2, F32Split::kWaves>(a, smem);
         return;
     }
-    int pos;
-    unsigned win;
-    wk.row_info(a, q_offset, row, pos, win);
     TileLaneOffsets at = tile_offsets_at(make_tile_offsets(lane), walk.lds + (w & 1) * F32Split::kKvRecord);
     const float c = a.scale_log2;
     float m = fast_max(sink_logit(a, wk.head) * kLog2e, kNoLogit), l = 0.0f;

@@ -48,3 +48,19 @@ def test_long_rows_dk_dv_of_padded_rows(A, s, lens):
     for a, b in zip(got[0][1:3], got[1][1:3]):             # dK, dV
         for row, n in enumerate(lens):
             assert torch.isfinite(b[row, :, :n]).all() and torch.equal(a[row, :, :n], b[row, :, :n])
+
+
+@pytest.mark.parametrize("s,w,lens", [(320, None, [200, 97]), (333, 100, [1, 320]), (257, None, [256, 225])])
+@pytest.mark.parametrize("value", [float("nan"), 1e30])
+def test_float32_padded_rows(A, value, s, w, lens):
+    """Also numbers that three bf16 terms do not hold: the rows that exist keep their bits."""
+    print(f"case S={s} W={w} lens={lens} value={value}", flush=True)
+    q, k, v, sinks, d_out = (t.to(DEV) for t in E.make_inputs(9950 + s, 2, 64, 8, s, 64, torch.float32))
+    got = []
+    for x in (_padded_with(0.0, lens, q, k, v, d_out), _padded_with(value, lens, q, k, v, d_out)):
+        o, lse = A.attention_forward(*x[:3], sinks, SCALE, w, 0, lens)
+        got.append((o, lse) + A.attention_backward(*x[:3], sinks, o, lse, x[3], SCALE, w, 0, lens)[:3])
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+    for b, n in enumerate(lens):
+        assert not got[1][0][b, n:].any()
