@@ -162,9 +162,11 @@ size_t gptoss_attn_bwd_workspace_bytes(const gptoss_attn_params *params);
 size_t gptoss_attn_fwd_workspace_bytes(const gptoss_attn_params *params);
 
 /*
- * Bytes of scratch with which float32 calls run on the bf16 matrix pipes, every operand cut into three bf16 terms (no less precise, about
- * twice as fast; 0 where the call has no such route): for gptoss_attn_fwd_scratch (backward == 0) or gptoss_attn_bwd_scratch
- * (backward != 0).  Not part of gptoss_attn_workspace_bytes.  Host-only.
+ * Bytes of scratch with which float32 calls run on the bf16 matrix pipes, every operand cut into three bf16 terms (no further from float64
+ * on the operands the tests try, 1.5 times as fast at 1024 tokens; 0 where the call has no such route): for gptoss_attn_fwd_scratch (backward == 0) or gptoss_attn_bwd_scratch
+ * (backward != 0).  At most 321 MiB: longer calls take their batch rows and KV heads some at a time over the same bytes, and where one KV
+ * head of one row does not fit (backward: beyond 38 000 tokens under eight query heads), the call has no such route.  Not part of
+ * gptoss_attn_workspace_bytes.  Host-only.
  */
 size_t gptoss_attn_split_bytes(const gptoss_attn_params *params, int backward);
 
@@ -244,7 +246,8 @@ int gptoss_attn_bwd_sinks(const gptoss_attn_params *params, int sinks_dtype, int
 
 /*
  * The same with scratch besides `delta`: `scratch` (16-byte aligned) holds `scratch_bytes` bytes, gptoss_attn_split_bytes(params, 1) for
- * float32 calls.  With NULL or less it is gptoss_attn_bwd_sinks.
+ * float32 calls.  With NULL or less it is gptoss_attn_bwd_sinks.  A call that takes that route (gptoss_attn_split_bytes is not 0 and the scratch
+ * holds as much) needs 2 * B * H * Sq floats of `delta` and no more.
  */
 int gptoss_attn_bwd_scratch(const gptoss_attn_params *params, int sinks_dtype, int dsinks_dtype, void *scratch, size_t scratch_bytes, void *stream);
 

@@ -219,8 +219,10 @@ def attention_backward(q, k, v, sinks, o, lse, d_o, sm_scale, window=None, q_off
     dsinks = torch.empty((h,), dtype=torch.float32, device=q.device) if need_dsinks else None
     with torch.cuda.device(q.device):
         p = _base_params(q, k, v, sinks32, sl, sm_scale, window, q_offset, ds, qod)
-        # scratch: [-delta; lse*log2e], then the dK/dV partial sums of key blocks cut into slices
-        delta = torch.empty((_lib.load().gptoss_attn_bwd_workspace_bytes(p) // 4,), dtype=torch.float32, device=q.device)
+        # scratch: [-delta; lse*log2e], then the dK/dV partial sums of key blocks cut into slices; the records of float32 operands are a
+        # scratch of their own, and the first is then the row statistics alone
+        need = 0 if split else _lib.load().gptoss_attn_split_bytes(p, 1)
+        delta = torch.empty((2 * b * h * sq if need else _lib.load().gptoss_attn_bwd_workspace_bytes(p) // 4,), dtype=torch.float32, device=q.device)
         p.o, p.lse = o.data_ptr(), lse.data_ptr()
         _set(p.o_stride, _strides_bhs(o, "bshd"))
         p.d_o = d_o.data_ptr()
@@ -235,7 +237,6 @@ def attention_backward(q, k, v, sinks, o, lse, d_o, sm_scale, window=None, q_off
             for name in ("gptoss_attn_bwd_preprocess", "gptoss_attn_bwd_dkdv", "gptoss_attn_bwd_dq"):
                 _lib.call(name, p, _stream(q))
         else:
-            need = _lib.load().gptoss_attn_split_bytes(p, 1)
             scratch = torch.empty((need // 4,), dtype=torch.float32, device=q.device) if need else None
             _lib.call("gptoss_attn_bwd_scratch", p, _stream(q), _lib.DTYPE_FP32, _lib.DTYPE_FP32, scratch.data_ptr() if need else None, need)
     return dq, dk, dv, dsinks

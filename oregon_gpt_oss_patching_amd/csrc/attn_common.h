@@ -69,6 +69,7 @@ struct KArgs {
     uint32_t *split_kv_bad, *split_q_bad;
     int split_steps, split_slots;
     float *split_partial;
+    int split_b0, split_nb, split_g0, split_ng;      // the batch rows and KV heads of this launch (the records are theirs alone)
 };
 
 // The sink logits and their gradient in the type the caller's parameter has: a conversion of 64 numbers was a launch of its own

@@ -153,11 +153,13 @@ struct F32QueryWork {
     // unit i of the workgroup: KV head fastest (its K / V stay in one XCD's L2), then the heads of the group, longest key loops first
     static __device__ __forceinline__ F32Unit unit(const KArgs &a, int i) {
         F32Unit u;
-        const int g = (int)(blockIdx.x % a.G);
-        int n = (int)(blockIdx.x / a.G) * (NW / KS) + i;
+        constexpr bool kSome = NW == 8;        // attn_f32_split.h: some of the batch rows and KV heads
+        const int G = kSome ? a.split_ng : a.G, B = kSome ? a.split_nb : a.B;
+        const int g = (int)(blockIdx.x % G) + (kSome ? a.split_g0 : 0);
+        int n = (int)(blockIdx.x / G) * (NW / KS) + i;
         u.head = g * a.r + n % a.r; n /= a.r;
-        const int bi = n % a.B, z = n / a.B, n_q = (a.Sq + 31) / 32;
-        u.b = rotated_batch_row(bi, z, a.B);
+        const int bi = n % B, z = n / B, n_q = (a.Sq + 31) / 32;
+        u.b = rotated_batch_row(bi, z, B) + (kSome ? a.split_b0 : 0);
         u.live = z < n_q;
         u.q0 = 32 * max(n_q - 1 - z, 0);
         return u;

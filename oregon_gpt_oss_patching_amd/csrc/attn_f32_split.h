@@ -21,7 +21,8 @@
 // for dK/dV.  A workgroup is eight wavefronts, one workgroup per compute unit: forward and dQ take four heads x 32 rows, two
 // wavefronts each, which walk the key tiles in turn; dK/dV takes four blocks of 32 keys, two wavefronts each, which walk the query
 // tiles in turn.  Both add their shares in LDS.  A step stages two tiles (48 KB), the next step's pair under way meanwhile, one
-// barrier per step.
+// barrier per step.  Where the records of all batch rows and KV heads would take too much memory, the launches are repeated for some of them
+// at a time, over the same scratch (f32_split_plan).
 //
 // What bounds it (S = 1024, 64 query heads on 8 KV heads, full causal; fp32 instruction / this): forward 101 / 61 us, dQ 134 / 85, dK/dV
 // 176 / 95, the whole call 413 / 259; S = 4096 5350 / 3280.  The matrix pipes are busy 43, 46 and 55 % of the cycles: about eight
@@ -262,12 +263,15 @@ __device__ __forceinline__ void split_copy(uint32_t dst, const char *src, int la
     for (int i = 0; i < F32Split::kWaveCopy / 1024; ++i) lds_dma16(dst + i * 1024, src + i * 1024, (uint32_t)(lane * 16));     // (one lane offset for all of them)
 }
 
+// where the records and the partial sums of a batch row's KV head stand among those of the launch
+__device__ __forceinline__ int64_t split_row_of(const KArgs &a, int b, int g) { return (int64_t)(b - a.split_b0) * a.split_ng + (g - a.split_g0); }
+
 // ---- K and V as records ------------------------------------------------------------------------------------
 // One workgroup per (batch, KV head, 32 keys).  Keys that nobody sees (past the tensor, a padded row's length, the last query) are
 // zeros.  Bound by memory: 10 bytes moved per number.
 __global__ __launch_bounds__(256) void attn_f32_split_kv_kernel(const KArgs a) {
     const F32Ptrs t = f32_ptrs(a);
-    const int nt = (a.Skv + 31) / 32, tile = (int)(blockIdx.x % nt), bg = (int)(blockIdx.x / nt), b = bg / a.G, g = bg % a.G;
+    const int nt = (a.Skv + 31) / 32, tile = (int)(blockIdx.x % nt), bg = (int)(blockIdx.x / nt), b = a.split_b0 + bg / a.split_ng, g = a.split_g0 + bg % a.split_ng;
     const int which = threadIdx.x >> 7, r = (threadIdx.x >> 2) & 31, part = threadIdx.x & 3, key = 32 * tile + r;
     int64_t end = min((int64_t)a.Skv, (int64_t)query_offset(a) + a.Sq);
     if (a.seqlens) end = min(end, (int64_t)a.seqlens[b]);
@@ -297,15 +301,18 @@ __global__ __launch_bounds__(256) void attn_f32_split_kv_kernel(const KArgs a) {
 // The key tiles of a forward / dQ workgroup: all four units stand at the same rows, wavefront w takes tile 2 step + w % 2 of them.
 struct SplitKeyWalk {
     const char *rec;
+    const uint32_t *rec_bad;
     int nt, t_lo, n, w, lane;
     uint32_t lds;
     __device__ __forceinline__ SplitKeyWalk(const KArgs &a, int b, int g, int t_lo_, int n_, int w_, int lane_, const char *smem)
         : nt((a.Skv + 31) / 32), t_lo(t_lo_), n(n_), w(w_), lane(lane_), lds(lds_addr(smem)) {
-        rec = a.split_kv + (int64_t)(b * a.G + g) * nt * F32Split::kKvRecord;
+        const int64_t first = split_row_of(a, b, g) * nt;
+        rec = a.split_kv + first * F32Split::kKvRecord;
+        rec_bad = a.split_kv_bad + first;
     }
-    __device__ __forceinline__ bool bad(const KArgs &a, int b, int g) const {
+    __device__ __forceinline__ bool bad() const {
         uint32_t x = 0;
-        for (int i = threadIdx.x; i < n; i += 64 * F32Split::kWaves) x |= a.split_kv_bad[(int64_t)(b * a.G + g) * nt + t_lo + i];
+        for (int i = threadIdx.x; i < n; i += 64 * F32Split::kWaves) x |= rec_bad[t_lo + i];
         return x != 0;
     }
     __device__ __forceinline__ int steps() const { return (n + 1) >> 1; }
@@ -333,7 +340,7 @@ __global__ __launch_bounds__(512, 2) void attn_f32_split_fwd_kernel(const KArgs 
     const SplitKeyWalk walk(a, wk.b, wk.g, wk.t_lo, wk.n, w, lane, smem);
     if (walk.n > 0) walk.request(0);
     SplitCheck check;
-    const bool keys_bad = walk.bad(a, wk.b, wk.g);
+    const bool keys_bad = walk.bad();
     bf16x8 qf[4][3];
     int pos;
     unsigned win;
@@ -418,7 +425,7 @@ __global__ __launch_bounds__(512, 2) void attn_f32_split_dq_kernel(const KArgs a
     const SplitKeyWalk walk(a, wk.b, wk.g, wk.t_lo, wk.n, w, lane, smem);
     if (walk.n > 0) walk.request(0);
     const int64_t total = (int64_t)a.B * a.H * a.Sq, rid = ((int64_t)wk.b * a.H + wk.head) * a.Sq + rowc;
-    const int64_t rec_i = ((int64_t)wk.b * a.H + wk.head) * ((a.Sq + 31) / 32) + wk.q0 / 32;
+    const int64_t rec_i = (split_row_of(a, wk.b, wk.g) * a.r + (wk.head - wk.g * a.r)) * ((a.Sq + 31) / 32) + wk.q0 / 32;
     char *const rec = a.split_q + rec_i * F32Split::kQRecord;
     const float *grow = t.d_o + (int64_t)wk.b * a.dos.b + (int64_t)wk.head * a.dos.h + (int64_t)rowc * a.dos.s;
     SplitCheck check;
@@ -468,7 +475,7 @@ __global__ __launch_bounds__(512, 2) void attn_f32_split_dq_kernel(const KArgs a
         kept.put(kept_g(2, ks), gf[ks][2]);
         if (kept_q(2, ks) >= 0) kept.put(kept_q(2, ks), qf[ks][2]);
     }
-    const bool keys_bad = walk.bad(a, wk.b, wk.g);
+    const bool keys_bad = walk.bad();
     if (!live) ndelta = 0.0f;
     wait_vmcnt<0>();
     if (__syncthreads_or(keys_bad || rows_bad)) {
@@ -535,9 +542,10 @@ __global__ __launch_bounds__(512, 2) void attn_f32_split_dkdv_kernel(const KArgs
     const F32Ptrs t = f32_ptrs(a);
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, half = lane >> 5;
     int bid = blockIdx.x;
-    const int g = bid % a.G; bid /= a.G;
-    const int bi = bid % a.B, slot = bid / a.B;
-    const int b = rotated_batch_row(bi, slot, a.B);
+    const int g = bid % a.split_ng + a.split_g0; bid /= a.split_ng;
+    const int bi = bid % a.split_nb, slot = bid / a.split_nb;
+    const int b = rotated_batch_row(bi, slot, a.split_nb) + a.split_b0;
+    const int64_t bg = split_row_of(a, b, g);
     int block = 0, part = slot;
     for (int n; part >= (n = split_block_parts(a.Sq, a.window, a.r, block, a.split_steps)); ++block) part -= n;
     const int J0 = C::kKeys * block, j0 = J0 + 32 * (w & 3), key = j0 + l32;
@@ -545,9 +553,9 @@ __global__ __launch_bounds__(512, 2) void attn_f32_split_dkdv_kernel(const KArgs
     const F32TileSpan span = f32_tiles_of_keys(a, 0, b, J0, C::kKeys, lane);
     const int t_hi = __builtin_amdgcn_readfirstlane(span.t_hi), t_lo = span.t_lo;
     const int all = ((t_hi - t_lo + 1) >> 1) * a.r, s0 = part * a.split_steps, n_steps = max(0, min(a.split_steps, all - s0));
-    float *const partial = a.split_partial ? a.split_partial + (((int64_t)b * a.G + g) * a.split_slots + slot) * (2 * C::kKeys * kD) : nullptr;
+    float *const partial = a.split_partial ? a.split_partial + (bg * a.split_slots + slot) * (2 * C::kKeys * kD) : nullptr;
 
-    const char *const qrec = a.split_q + ((int64_t)b * a.H + (int64_t)g * a.r) * nqt * C::kQRecord;
+    const char *const qrec = a.split_q + bg * a.r * nqt * C::kQRecord;
     const uint32_t lds = lds_addr(smem);
     auto request = [&](int step) __attribute__((always_inline)) {
         const int s = s0 + step, tile = min(t_lo + 2 * (s / a.r) + (w >> 2), nqt - 1);
@@ -561,12 +569,12 @@ __global__ __launch_bounds__(512, 2) void attn_f32_split_dkdv_kernel(const KArgs
     uint32_t bad = 0;
     if (n_steps > 0) {
         const int ta = t_lo + 2 * (s0 / a.r), tb = min(t_hi, t_lo + 2 * ((s0 + n_steps - 1) / a.r + 1)), per = tb - ta;
-        for (int i = tid; i < per * a.r; i += 64 * C::kWaves) bad |= a.split_q_bad[((int64_t)b * a.H + (int64_t)g * a.r + i / per) * nqt + ta + i % per];
-        if (tid < 4 && J0 / 32 + tid < nt) bad |= a.split_kv_bad[(int64_t)(b * a.G + g) * nt + J0 / 32 + tid];
+        for (int i = tid; i < per * a.r; i += 64 * C::kWaves) bad |= a.split_q_bad[(bg * a.r + i / per) * nqt + ta + i % per];
+        if (tid < 4 && J0 / 32 + tid < nt) bad |= a.split_kv_bad[bg * nt + J0 / 32 + tid];
     }
     bf16x8 kf[4][3], vf[4][3];     // B operands of S and dP
     {
-        const char *kv = a.split_kv + ((int64_t)(b * a.G + g) * nt + min(j0 / 32, nt - 1)) * C::kKvRecord;
+        const char *kv = a.split_kv + (bg * nt + min(j0 / 32, nt - 1)) * C::kKvRecord;
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks)
 #pragma unroll
@@ -704,11 +712,12 @@ __global__ __launch_bounds__(256) void attn_f32_split_reduce_kernel(const KArgs 
     if ((int)blockIdx.x < heads) { dsinks_of_head<256>(a, blockIdx.x, red); return; }
     using C = F32Split;
     const F32Ptrs t = f32_ptrs(a);
-    const int64_t rows = (int64_t)a.B * a.G * a.Skv, idx = (int64_t)(blockIdx.x - heads) * 256 + threadIdx.x;
+    const int64_t rows = (int64_t)a.split_nb * a.split_ng * a.Skv, idx = (int64_t)(blockIdx.x - heads) * 256 + threadIdx.x;
     if (idx >= 2 * rows * 16) return;
     const int which = idx >= rows * 16, ch = (int)(idx & 15);
     const int64_t row = (idx - (int64_t)which * rows * 16) >> 4;
-    const int key = (int)(row % a.Skv), bg = (int)(row / a.Skv), g = bg % a.G, b = bg / a.G, block = key / C::kKeys;
+    const int key = (int)(row % a.Skv), bg = (int)(row / a.Skv), block = key / C::kKeys;
+    const int g = a.split_g0 + bg % a.split_ng, b = a.split_b0 + bg / a.split_ng;
     int slot = 0;
     for (int i = 0; i < block; ++i) slot += split_block_parts(a.Sq, a.window, a.r, i, a.split_steps);
     const int n = split_block_parts(a.Sq, a.window, a.r, block, a.split_steps);

@@ -96,6 +96,7 @@ KArgs make_args(const gptoss_attn_params *p, SinkTypes ty) {
     a.split_kv_bad = a.split_q_bad = nullptr;
     a.split_steps = a.split_slots = 0;
     a.split_partial = nullptr;
+    a.split_b0 = a.split_nb = a.split_g0 = a.split_ng = 0;
     return a;
 }
 
@@ -309,44 +310,56 @@ bool f32_split_route(const gptoss_attn_params *p, bool bwd) {
     if (window > 0 && window < 384 && wgs > 400) return false;
     return p->Sq >= 192 && (wgs >= 160 || (wgs >= 128 && p->Skv >= 2048));
 }
-// Steps per dK/dV workgroup: the count whose rounds of workgroups take the least time on 256 compute units, one workgroup each (so that
-// the scratch does not depend on the device), a workgroup's start and end counted as three steps; more than four rounds even out.
+// Steps per dK/dV workgroup, `rows` batch rows and KV heads at once: the count whose rounds of workgroups take the least time on 256 compute units, one
+// workgroup each (so that the scratch does not depend on the device), a workgroup's start and end counted as three steps.  At most four
+// rounds: each workgroup of a cut key block leaves 64 KB.
 struct F32SplitParts { int steps, slots; bool cut; };
-F32SplitParts f32_split_parts(const gptoss_attn_params *p) {
+F32SplitParts f32_split_parts(const gptoss_attn_params *p, int64_t rows) {
     const int window = effective_window(p), r = p->H / p->G, blocks = (p->Skv + F32Split::kKeys - 1) / F32Split::kKeys;
-    const int64_t rows = (int64_t)p->G * p->B, cus = 256;
+    const int64_t cus = 256;
     const int most = split_block_steps(p->Sq, window, r, 0);
-    if (rows * blocks > 8 * cus) return {most, blocks, false};
-    int64_t all = 0;
-    for (int i = 0; i < blocks; ++i) all += split_block_steps(p->Sq, window, r, i);
     F32SplitParts best{most, blocks, false};
     int64_t best_cost = 0;
     for (int steps = most; steps >= 4; steps -= 1 + steps / 32) {
         int slots = 0;
         for (int i = 0; i < blocks; ++i) slots += split_block_parts(p->Sq, window, r, i, steps);
         const int64_t wgs = rows * slots;
-        const int64_t cost = wgs <= 4 * cus ? 4 * ((wgs + cus - 1) / cus) * (steps + 3) : 4 * (rows * all + 3 * wgs) / cus + 3 * steps;
+        if (wgs > 4 * cus) break;
+        const int64_t cost = ((wgs + cus - 1) / cus) * (steps + 3);
         if (steps == most || cost < best_cost) { best = {steps, slots, slots > blocks}; best_cost = cost; }
     }
     return best;
 }
-// The scratch: which K / V records are bad, these records; for the backward the same of Q / dO, then the parts' sums.
-struct F32SplitScratch { size_t kv_bad, kv, q_bad, q, partial, bytes; F32SplitParts parts; };
-F32SplitScratch f32_split_scratch(const gptoss_attn_params *p, bool bwd) {
+// How a call runs: nb batch rows by ng KV heads at a time, and what is where in the scratch: which K / V records are bad, these records; for
+// the backward the same of Q / dO, then the parts' sums.  The records are one and a half to two and a half times as large as what they are made of, and
+// the scratch is the caller's memory: kF32SplitRecords bytes of them at most (and 64 MB of parts' sums), in even shares; a KV head of one row
+// that needs more has no such route.  Forward + backward of 64 heads on 8 KV heads, everything at once / so, us (and MB at the peak, outputs
+// included; the left figures with terms cut off instead of rounded, 1.5 % faster at 1024 tokens): 4096 tokens 3200 (529) / 3275 (450), window 512 985 / 1010, 4 x 2000 3415 (913) / 3499
+// (579), 8192 12070 (1046) / 12310 (604), 16384 47300 (2106) / 49400 (911).  128 MB: window 512 another 7 % slower, the others alike.
+constexpr size_t kF32SplitRecords = (size_t)256 << 20;
+struct F32SplitPlan { int nb, ng; size_t kv, q_bad, q, partial, bytes; F32SplitParts parts; };
+F32SplitPlan f32_split_plan(const gptoss_attn_params *p, bool bwd) {
     auto up = [](size_t n) { return (n + 255) & ~(size_t)255; };
-    F32SplitScratch s{};
-    const size_t n_kv = (size_t)p->B * p->G * ((p->Skv + 31) / 32), n_q = (size_t)p->B * p->H * ((p->Sq + 31) / 32);
-    s.kv = up(4 * n_kv);
-    s.bytes = s.kv + n_kv * F32Split::kKvRecord;
+    auto share = [](int n, size_t most) { const int times = (int)((n + most - 1) / most); return (n + times - 1) / times; };
+    F32SplitPlan s{};
+    if (!f32_split_route(p, bwd)) return s;
+    const size_t n_kv = (size_t)(p->Skv + 31) / 32, n_q = (size_t)(p->H / p->G) * ((p->Sq + 31) / 32);      // of a KV head
+    const size_t most = kF32SplitRecords / (n_kv * F32Split::kKvRecord + (bwd ? n_q * F32Split::kQRecord : 0));
+    if (most == 0) return s;
+    s.nb = most > (size_t)p->G ? share(p->B, most / p->G) : 1;
+    s.ng = share(p->G, most);
+    const size_t rows = (size_t)s.nb * s.ng;
+    s.kv = up(4 * rows * n_kv);
+    s.bytes = s.kv + rows * n_kv * F32Split::kKvRecord;
     if (!bwd) return s;
     s.q_bad = s.bytes;
-    s.q = s.q_bad + up(4 * n_q);
-    s.partial = s.q + n_q * F32Split::kQRecord;
-    s.parts = f32_split_parts(p);
-    s.bytes = s.partial + (s.parts.cut ? (size_t)p->B * p->G * s.parts.slots * (2 * F32Split::kKeys * kD * sizeof(float)) : 0);
+    s.q = s.q_bad + up(4 * rows * n_q);
+    s.partial = s.q + rows * n_q * F32Split::kQRecord;
+    s.parts = f32_split_parts(p, (int64_t)rows);
+    s.bytes = s.partial + (s.parts.cut ? rows * s.parts.slots * (2 * F32Split::kKeys * kD * sizeof(float)) : 0);
     return s;
 }
-void f32_split_args(KArgs &a, const F32SplitScratch &s, void *scratch) {
+void f32_split_args(KArgs &a, const F32SplitPlan &s, void *scratch) {
     char *base = static_cast<char *>(scratch);
     a.split_kv_bad = reinterpret_cast<uint32_t *>(base);
     a.split_kv = base + s.kv;
@@ -355,6 +368,18 @@ void f32_split_args(KArgs &a, const F32SplitScratch &s, void *scratch) {
     a.split_steps = s.parts.steps;
     a.split_slots = s.parts.slots;
     a.split_partial = s.parts.cut ? reinterpret_cast<float *>(base + s.partial) : nullptr;
+}
+// step(last) for every share of the batch rows and KV heads, set in `a`
+template <typename Step>
+int f32_split_shares(KArgs &a, const F32SplitPlan &s, Step step) {
+    for (a.split_b0 = 0; a.split_b0 < a.B; a.split_b0 += s.nb)
+        for (a.split_g0 = 0; a.split_g0 < a.G; a.split_g0 += s.ng) {
+            a.split_nb = s.nb < a.B - a.split_b0 ? s.nb : a.B - a.split_b0;
+            a.split_ng = s.ng < a.G - a.split_g0 ? s.ng : a.G - a.split_g0;
+            const int rc = step(a.split_b0 + s.nb >= a.B && a.split_g0 + s.ng >= a.G);
+            if (rc) return rc;
+        }
+    return GPTOSS_ATTN_OK;
 }
 
 // One launch.  hipLaunchKernel reports this launch's own status, so an error some earlier call of the
@@ -489,27 +514,34 @@ int launch_window_bwd(const gptoss_attn_params *p, hipStream_t st, bool seam_sum
     return e == hipSuccess ? GPTOSS_ATTN_OK : static_cast<int>(e);
 }
 
-int launch_f32_split_kv(const KArgs &a, hipStream_t st) { return launch(attn_f32_split_kv_kernel, (int64_t)a.B * a.G * ((a.Skv + 31) / 32), 256, st, a); }
-int64_t f32_split_grid(const KArgs &a) { return (int64_t)a.G * (a.r / 4) * a.B * ((a.Sq + 31) / 32); }
+int launch_f32_split_kv(const KArgs &a, hipStream_t st) { return launch(attn_f32_split_kv_kernel, (int64_t)a.split_nb * a.split_ng * ((a.Skv + 31) / 32), 256, st, a); }
+int64_t f32_split_grid(const KArgs &a) { return (int64_t)a.split_ng * (a.r / 4) * a.split_nb * ((a.Sq + 31) / 32); }
 
-int launch_f32_split_fwd(const gptoss_attn_params *p, hipStream_t st, SinkTypes ty, void *scratch) {
+int launch_f32_split_fwd(const gptoss_attn_params *p, hipStream_t st, SinkTypes ty, const F32SplitPlan &plan, void *scratch) {
     KArgs a = make_args(p, ty);
-    f32_split_args(a, f32_split_scratch(p, false), scratch);
-    int rc = lds_attribute<&attn_f32_split_fwd_kernel>(F32Split::kRowsLds);
-    if (rc || (rc = launch_f32_split_kv(a, st))) return rc;
-    return launch(attn_f32_split_fwd_kernel, f32_split_grid(a), 512, st, a, F32Split::kRowsLds);
+    f32_split_args(a, plan, scratch);
+    const int rc = lds_attribute<&attn_f32_split_fwd_kernel>(F32Split::kRowsLds);
+    if (rc) return rc;
+    return f32_split_shares(a, plan, [&](bool) {
+        const int s = launch_f32_split_kv(a, st);
+        return s ? s : launch(attn_f32_split_fwd_kernel, f32_split_grid(a), 512, st, a, F32Split::kRowsLds);
+    });
 }
 
-int launch_f32_split_bwd(const gptoss_attn_params *p, hipStream_t st, SinkTypes ty, void *scratch) {
+int launch_f32_split_bwd(const gptoss_attn_params *p, hipStream_t st, SinkTypes ty, const F32SplitPlan &plan, void *scratch) {
     KArgs a = make_args(p, ty);
-    f32_split_args(a, f32_split_scratch(p, true), scratch);
+    f32_split_args(a, plan, scratch);
     int rc = lds_attribute<&attn_f32_split_dq_kernel>(F32Split::kDqLds);
-    if (rc || (rc = lds_attribute<&attn_f32_split_dkdv_kernel>(F32Split::kDkdvLds)) || (rc = launch_f32_split_kv(a, st))) return rc;
-    if ((rc = launch(attn_f32_split_dq_kernel, f32_split_grid(a), 512, st, a, F32Split::kDqLds))) return rc;
-    if (!a.split_partial && a.dsinks && (rc = launch(attn_bwd_dsinks_kernel, a.H, 1024, st, a))) return rc;
-    rc = launch(attn_f32_split_dkdv_kernel, (int64_t)a.G * a.B * a.split_slots, 512, st, a, F32Split::kDkdvLds);
-    if (rc || !a.split_partial) return rc;
-    return launch_reduce(attn_f32_split_reduce_kernel, (int64_t)2 * a.B * a.G * a.Skv * 16, st, a, a.dsinks != nullptr);
+    if (rc || (rc = lds_attribute<&attn_f32_split_dkdv_kernel>(F32Split::kDkdvLds))) return rc;
+    return f32_split_shares(a, plan, [&](bool last) {
+        int s = launch_f32_split_kv(a, st);
+        if (s || (s = launch(attn_f32_split_dq_kernel, f32_split_grid(a), 512, st, a, F32Split::kDqLds))) return s;
+        const bool with_dsinks = last && a.dsinks;         // (every row's statistics are there)
+        if (!a.split_partial && with_dsinks && (s = launch(attn_bwd_dsinks_kernel, a.H, 1024, st, a))) return s;
+        s = launch(attn_f32_split_dkdv_kernel, (int64_t)a.split_ng * a.split_nb * a.split_slots, 512, st, a, F32Split::kDkdvLds);
+        if (s || !a.split_partial) return s;
+        return launch_reduce(attn_f32_split_reduce_kernel, (int64_t)2 * a.split_nb * a.split_ng * a.Skv * 16, st, a, with_dsinks);
+    });
 }
 
 template <int NQB, int NW>
@@ -649,7 +681,7 @@ size_t gptoss_attn_workspace_bytes(const gptoss_attn_params *p) {
 }
 
 size_t gptoss_attn_split_bytes(const gptoss_attn_params *p, int backward) {
-    return p && f32_split_route(p, backward != 0) ? f32_split_scratch(p, backward != 0).bytes : 0;
+    return p ? f32_split_plan(p, backward != 0).bytes : 0;
 }
 
 // scratch: see gptoss_attn_fwd_scratch (NULL or too little: the keys are not cut)
@@ -670,8 +702,8 @@ static int forward(const gptoss_attn_params *p, void *stream, SinkTypes ty, void
         return launch(attn_decode_combine_kernel, ((int64_t)a.B * a.G * pairs + 3) / 4, 256, st, a);
     }
     if (p->dtype == GPTOSS_ATTN_FP32) {
-        const size_t records = gptoss_attn_split_bytes(p, 0);
-        if (records && scratch && scratch_bytes >= records) return launch_f32_split_fwd(p, st, ty, scratch);
+        const F32SplitPlan plan = f32_split_plan(p, false);
+        if (plan.bytes && scratch && scratch_bytes >= plan.bytes) return launch_f32_split_fwd(p, st, ty, plan, scratch);
         const int ks = f32_key_splits(a);
         const int64_t grid32 = f32_grid(a, ks);
         return ks == 4 ? launch(attn_f32_fwd_kernel<4>, grid32, 256, st, a) : ks == 2 ? launch(attn_f32_fwd_kernel<2>, grid32, 256, st, a) : launch(attn_f32_fwd_kernel<1>, grid32, 256, st, a);
@@ -817,8 +849,10 @@ static int bwd_all(const gptoss_attn_params *p, void *stream, bool whole_blocks,
     int rc = gptoss_attn_validate(p, 1);
     if (rc) return rc;
     if (!aligned16(scratch)) return GPTOSS_ATTN_ERR_ALIGNMENT;
-    const size_t records = gptoss_attn_split_bytes(p, 1);
-    if (records && scratch && scratch_bytes >= records) return launch_f32_split_bwd(p, static_cast<hipStream_t>(stream), ty, scratch);
+    if (scratch) {
+        const F32SplitPlan plan = f32_split_plan(p, true);
+        if (plan.bytes && scratch_bytes >= plan.bytes) return launch_f32_split_bwd(p, static_cast<hipStream_t>(stream), ty, plan, scratch);
+    }
     if (window_single_pass(p)) return launch_window_bwd(p, static_cast<hipStream_t>(stream), !whole_blocks, ty);
     rc = launch_dq(p, stream, 1);
     if (rc) return rc;

@@ -176,8 +176,10 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> bwd(const Tensor &q, const Tensor &k,
     Tensor dq = at::empty({b, h, s, d}, q.options()), dk = at::empty(k.sizes(), k.options()), dv = at::empty(v.sizes(), v.options());
     const bool bf16_dsinks = dsinks_as_sinks && c.sinks_dtype == GPTOSS_ATTN_BF16;
     Tensor dsinks = at::empty({need_dsinks ? h : 0}, lse.options().dtype(bf16_dsinks ? at::kBFloat16 : at::kFloat));
-    // scratch: the row statistics, then the dK/dV partial sums of split key blocks or the window kernel's shares
-    Tensor scratch = at::empty({static_cast<int64_t>(gptoss_attn_bwd_workspace_bytes(&c.p) / sizeof(float))}, lse.options());
+    // scratch: the row statistics, then the dK/dV partial sums of split key blocks or the window kernel's shares; the records of float32
+    // operands as bf16 terms are a scratch of their own, and with them the first is two floats per row
+    const size_t records = gptoss_attn_split_bytes(&c.p, 1);
+    Tensor scratch = at::empty({records ? 2 * b * h * s : static_cast<int64_t>(gptoss_attn_bwd_workspace_bytes(&c.p) / sizeof(float))}, lse.options());
     gptoss_attn_params &p = c.p;
     p.o = const_cast<void *>(o.const_data_ptr());             // (read only here)
     p.lse = const_cast<float *>(lse.const_data_ptr<float>());
@@ -192,7 +194,6 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> bwd(const Tensor &q, const Tensor &k,
     set(p.dq_stride, dq, false);
     set(p.dk_stride, dk, false);
     set(p.dv_stride, dv, false);
-    const size_t records = gptoss_attn_split_bytes(&c.p, 1);        // (float32 operands as bf16 terms)
     const Tensor split = records ? at::empty({static_cast<int64_t>(records / sizeof(float))}, lse.options()) : Tensor();
     check("gptoss_attn_bwd", gptoss_attn_bwd_scratch(&c.p, c.sinks_dtype, bf16_dsinks ? GPTOSS_ATTN_BF16 : GPTOSS_ATTN_FP32,
                                                      records ? split.data_ptr() : nullptr, records, stream_of(c)));

@@ -61,3 +61,22 @@ def test_backward_scratch_of_the_call_itself():
                 p = _params(dtype, 2, 64, 8, sq, sq, window, **ptrs)
                 assert 24 * 2 * 64 * sq <= exact(p) <= bound(p)
     assert exact(_params(sq=0)) == 0 and lib.gptoss_attn_bwd_workspace_bytes(None) == 0
+
+
+@pytest.mark.parametrize("backward", [0, 1])
+def test_float32_scratch_is_bounded(backward):
+    """Records of some batch rows and KV heads at a time: never more than 256 MiB of them (and 64 MiB of partial sums), however long the call; of all
+    at once where that is less."""
+    lib = _lib.load()
+    sizes = lambda **kw: lib.gptoss_attn_split_bytes(ctypes.byref(_params(dtype=1, **kw)), backward)
+    for b, (h, g), s in itertools.product((1, 2, 3, 16, 64), ((64, 8), (8, 1), (32, 8), (96, 8)), (192, 1024, 3001, 4096, 16384, 32768)):
+        n = sizes(b=b, h=h, g=g, sq=s, skv=s)
+        tiles = -(-s // 32)
+        record = tiles * (24576 + (h // g * 24832 if backward else 0))             # of one KV head
+        if b * (h // 4) * tiles >= 160 and record <= 256 << 20:
+            assert 0 < n <= 321 << 20, (b, h, g, s, n)
+            if b * g * record <= 256 << 20:
+                assert n >= b * g * record
+            else:
+                assert n >= 64 << 20                                                # (not one at a time where several fit)
+    assert sizes(b=1, h=64, g=8, sq=1 << 19, skv=1 << 19) == 0

@@ -145,3 +145,28 @@ def test_row_statistics_that_three_terms_do_not_hold(A, which, value):
         assert torch.equal(torch.isfinite(x), torch.isfinite(y)) and torch.equal(torch.isnan(x), torch.isnan(y)), name
         ok = torch.isfinite(y)
         assert bool(((x - y)[ok].abs() <= 1e-4 * y[ok].abs() + 2e-4).all()), name
+
+
+@pytest.mark.parametrize("b,h,g,s,w,lens,docs", [
+    (1, 64, 8, 5000, None, None, None),                        # four KV heads at a time
+    (10, 64, 8, 1056, None, [1056, 700, 1, 0, 1055, 32, 33, 900, 1024, 1056], None),     # four batch rows at a time, then two
+    (1, 28, 7, 15360, 500, None, None),                        # four KV heads, then three
+    (3, 64, 8, 1700, None, None, [1, 932, 767]),               # two batch rows, then one
+])
+def test_some_rows_and_heads_at_a_time(A, b, h, g, s, w, lens, docs):
+    """Calls whose records do not fit the scratch at once give what the fp32 instruction gives, and forward and dQ what each batch row gives by itself."""
+    from oregon_gpt_oss_patching_amd import _lib
+    from oregon_gpt_oss_patching_amd import attention_kernel as ak
+    print(f"case B={b} H={h} G={g} S={s} W={w} lens={lens} docs={docs}", flush=True)
+    inp = list(E.make_inputs(7900 + s, b, h, g, s, 64, torch.float32))
+    p = ak._base_params(*(t.to(DEV) for t in inp[:4]), None, SCALE, w, 0, None)
+    assert b * g * -(-s // 32) * (24576 + h // g * 24832) > _lib.load().gptoss_attn_split_bytes(ctypes.byref(p), 1) > 0
+    new, old = _both(A, inp, w, lens, docs)
+    for name, x, y in zip(("o", "lse", "dq", "dk", "dv"), new, old):
+        # (each no further from float64 than 2e-5 of the result: 7e-7 at the most in test_no_further_from_float64_than_the_fp32_instruction)
+        assert float((x - y).double().norm()) <= 2e-5 * float(y.double().norm()), name
+    assert bool(((new[5] - old[5]).abs() <= 1e-4 * old[5].abs() + 1e-3).all())
+    for i in range(b if b > 1 else 0):
+        row = [t[i:i + 1] if t.dim() == 4 else t for t in inp]
+        one, _ = _both(A, row, w, [lens[i]] if lens else None, docs)
+        assert torch.equal(one[0], new[0][i:i + 1]) and torch.equal(one[1], new[1][i:i + 1]) and torch.equal(one[2], new[2][i:i + 1]), i
