@@ -239,7 +239,7 @@ __device__ __forceinline__ void f32_fwd_merge(const KArgs &a, const F32Ptrs &t, 
     __syncthreads();
 #pragma unroll
     for (int pass = 0; pass < 8 / KS; ++pass) {                     // a pass takes NW / 8 units
-        const int u16 = (threadIdx.x >> 4) + 4 * NW * pass, i = u16 >> 5, r = u16 & 31, ch = threadIdx.x & 15;
+        const int i = 4 * NW * pass / 32, r = (threadIdx.x >> 4) + 4 * NW * pass % 32, ch = threadIdx.x & 15;
         const F32Unit u = W::unit(a, i);
         const float sink = sink_logit(a, u.head) * kLog2e;
         float mm = fast_max(sink, kNoLogit);
@@ -388,17 +388,29 @@ __device__ __forceinline__ F32TileSpan f32_tiles_of_keys(const KArgs &a, int q_o
     x.t_hi = max(x.t_lo, (row_hi + 31) / 32);
     return x;
 }
-// Step `it` of a walk over (query tile, head): `each` consecutive tiles of a head, the heads of the group, the tiles after these.
-// Tiles outside [t_from, t_to) have no row that sees the keys and are passed over.
-struct F32Walk {
-    int t0, t_end, each, first, n_it, t_from, t_to;
-    __device__ __forceinline__ int tile(int it, int r) const { return t0 + each * ((first + it / each) / r) + it % each; }
-    __device__ __forceinline__ int head(int it, int r) const { return (first + it / each) % r; }
+// Step `it` of a walk over (query tile, head): the heads of the group tile by tile, all of them with rows that see the keys.
+struct F32TileWalk {
+    int t0, n_it;
+    __device__ __forceinline__ int tile(int it, int r) const { return t0 + it / r; }
+    __device__ __forceinline__ int readable_tile(int it, int r) const { return tile(it, r); }
+    __device__ __forceinline__ int head(int it, int r) const { return it % r; }
+    __device__ __forceinline__ bool sees(int) const { return true; }
+};
+// The same by pairs of tiles (both of a head, the heads of the group, the pair after these) from step `first` on, for one of several key blocks:
+// tiles outside [t_from, t_to) have no row that sees its keys and are passed over, one past the last is read as that one.  (A type of its own: with both walks
+// in one, attn_f32_dkdv_kernel divided by a run-time number more often per request and step; forward + backward of 1000 rows of 8 heads on one KV head 148.9 us
+// instead of 148.0, of 64 on 8 with a window of 128 144.5 instead of 143.0.)
+struct F32PairWalk {
+    int t0, t_end, first, n_it, t_from, t_to;
+    __device__ __forceinline__ int tile(int it, int r) const { return t0 + 2 * ((first + it / 2) / r) + it % 2; }
+    __device__ __forceinline__ int readable_tile(int it, int r) const { return min(tile(it, r), t_end - 1); }
+    __device__ __forceinline__ int head(int it, int r) const { return (first + it / 2) % r; }
+    __device__ __forceinline__ bool sees(int tile) const { return tile >= t_from && tile < t_to; }
 };
 // dK, dV of 32 keys from j0 over a walk (its steps dealt to the NW wavefronts in turn); out: fp32 partial sums, rows of 64 floats, or
 // NULL for the scaled results
-template <int NW>
-__device__ __forceinline__ void f32_dkdv_keys(const KArgs &a, char *smem, int g, int b, int j0, const F32Walk walk, float *out_k, float *out_v) {
+template <int NW, typename Walk>
+__device__ __forceinline__ void f32_dkdv_keys(const KArgs &a, char *smem, int g, int b, int j0, const Walk walk, float *out_k, float *out_v) {
     using C = F32Dkdv;
     const int q_offset = query_offset(a);
     const F32Ptrs t = f32_ptrs(a);
@@ -424,13 +436,13 @@ __device__ __forceinline__ void f32_dkdv_keys(const KArgs &a, char *smem, int g,
     const uint32_t ssm = lds_addr(smem) + NW * 2 * F32Tile::kBytes + w * C::kStatBytes;
     const F32Offsets lo = make_f32_offsets(lane);
     const float c = a.scale_log2;
-    // requests for step `it`: the Q tile; the dO tile and the row statistics (a tile past the last one re-reads that one)
+    // requests for step `it`: the Q tile; the dO tile and the row statistics
     auto request_q = [&](int it) __attribute__((always_inline)) {
-        const int q0 = 32 * min(walk.tile(it, a.r), walk.t_end - 1), head = g * a.r + walk.head(it, a.r);
+        const int q0 = 32 * walk.readable_tile(it, a.r), head = g * a.r + walk.head(it, a.r);
         f32_copy_tile(qsm, t.q + (int64_t)b * a.qs.b + (int64_t)head * a.qs.h + (int64_t)q0 * a.qs.s, (int)a.qs.s, a.Sq - 1 - q0, lane);
     };
     auto request_g = [&](int it) __attribute__((always_inline)) {
-        const int q0 = 32 * min(walk.tile(it, a.r), walk.t_end - 1), head = g * a.r + walk.head(it, a.r);
+        const int q0 = 32 * walk.readable_tile(it, a.r), head = g * a.r + walk.head(it, a.r);
         f32_copy_tile(gsm, t.d_o + (int64_t)b * a.dos.b + (int64_t)head * a.dos.h + (int64_t)q0 * a.dos.s, (int)a.dos.s, a.Sq - 1 - q0, lane);
         lds_dma4(ssm, a.delta + ((int64_t)b * a.H + head) * a.Sq, ((half ? (uint32_t)total : 0u) + (uint32_t)min(q0 + l32, a.Sq - 1)) * 4u);
     };
@@ -439,7 +451,7 @@ __device__ __forceinline__ void f32_dkdv_keys(const KArgs &a, char *smem, int g,
     for (int it = w; it < n_it; it += NW) {
         const int tile = walk.tile(it, a.r), q0 = 32 * tile;
         const bool more = it + NW < n_it;
-        if (tile < walk.t_from || tile >= walk.t_to) {
+        if (!walk.sees(tile)) {
             GPTOSS_F32_WAIT(0);
             if (more) { request_g(it + NW); request_q(it + NW); }
             continue;
@@ -489,7 +501,7 @@ __device__ __forceinline__ void f32_dkdv_keys(const KArgs &a, char *smem, int g,
     __syncthreads();
 #pragma unroll
     for (int pass = 0; pass < 16 / NW; ++pass) {
-        const int row = (tid >> 4) + 4 * NW * pass, which = row >> 5, r = row & 31, ch = tid & 15, j = j0 + r;
+        const int which = 4 * NW * pass / 32, r = (tid >> 4) + 4 * NW * pass % 32, ch = tid & 15, j = j0 + r;
         f32x4 x = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int k = 0; k < NW; ++k) {
@@ -519,7 +531,7 @@ __global__ __launch_bounds__(256, 2) void attn_f32_dkdv_kernel(const KArgs a) {
     const int b = rotated_batch_row(bi, kblk, a.B), j0 = 32 * kblk;
     const F32TileSpan span = f32_tiles_of_keys(a, query_offset(a), b, j0, 32, threadIdx.x & 63);
     const int n_tiles = span.t_hi - span.t_lo, slice = (n_tiles + a.dkdv_parts - 1) / a.dkdv_parts;
-    const F32Walk walk{span.t_lo + part * slice, span.t_hi, 1, 0, max(0, min(slice, n_tiles - part * slice)) * a.r, span.t_lo, span.t_hi};
+    const F32TileWalk walk{span.t_lo + part * slice, max(0, min(slice, n_tiles - part * slice)) * a.r};
     const int64_t tensor = (int64_t)a.B * a.G * a.Skv * kD;
     float *out = a.dkdv_parts > 1 ? a.dkdv_partial + 2 * part * tensor + (((int64_t)b * a.G + g) * a.Skv + j0) * kD : nullptr;
     f32_dkdv_keys<4>(a, smem, g, b, j0, walk, out, out ? out + tensor : nullptr);
@@ -561,7 +573,7 @@ __device__ __forceinline__ void f32_dq_merge(const KArgs &a, const F32Ptrs &t, c
     __syncthreads();
 #pragma unroll
     for (int pass = 0; pass < 8 / KS; ++pass) {
-        const int u16 = (threadIdx.x >> 4) + 4 * NW * pass, i = u16 >> 5, r = u16 & 31, ch = threadIdx.x & 15;
+        const int i = 4 * NW * pass / 32, r = (threadIdx.x >> 4) + 4 * NW * pass % 32, ch = threadIdx.x & 15;
         const F32Unit u = W::unit(a, i);
         f32x4 x = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll

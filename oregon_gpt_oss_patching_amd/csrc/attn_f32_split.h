@@ -598,7 +598,7 @@ __global__ __launch_bounds__(512, 2) void attn_f32_split_dkdv_kernel(const KArgs
     if (__syncthreads_or(bad != 0)) {
         for (int k = 0; k < 4 && J0 + 32 * k < a.Skv; ++k) {
             const F32TileSpan own = f32_tiles_of_keys(a, 0, b, J0 + 32 * k, 32, lane);
-            const F32Walk walk{t_lo, t_hi, 2, s0, 2 * n_steps, own.t_lo, own.t_hi};
+            const F32PairWalk walk{t_lo, t_hi, s0, 2 * n_steps, own.t_lo, own.t_hi};
             float *out = partial ? partial + 32 * k * kD : nullptr;
             f32_dkdv_keys<C::kWaves>(a, smem, g, b, J0 + 32 * k, walk, out, out ? out + C::kKeys * kD : nullptr);
             __syncthreads();
