@@ -312,21 +312,33 @@ bool f32_split_route(const gptoss_attn_params *p, bool bwd) {
 }
 // Steps per dK/dV workgroup, `rows` batch rows and KV heads at once: the count whose rounds of workgroups take the least time on 256 compute units, one
 // workgroup each (so that the scratch does not depend on the device), a workgroup's start and end counted as three steps.  At most four
-// rounds: each workgroup of a cut key block leaves 64 KB.
+// rounds: each workgroup of a cut key block leaves 64 KB.  Of the counts from the longest walk's down to four, a thirty-second apart, the smallest
+// that needs no more than k rounds is the best of k rounds: found by halving, as the caller asks for the scratch's size and the call itself asks again
+// (all counts one by one / so, 1024 tokens 1.1 / 0.4 us, 4096 4.0 / 2.0, 16384 17 / 8).
 struct F32SplitParts { int steps, slots; bool cut; };
 F32SplitParts f32_split_parts(const gptoss_attn_params *p, int64_t rows) {
     const int window = effective_window(p), r = p->H / p->G, blocks = (p->Skv + F32Split::kKeys - 1) / F32Split::kKeys;
     const int64_t cus = 256;
-    const int most = split_block_steps(p->Sq, window, r, 0);
-    F32SplitParts best{most, blocks, false};
-    int64_t best_cost = 0;
-    for (int steps = most; steps >= 4; steps -= 1 + steps / 32) {
+    int steps[640], n = 0;                                 // (from 2^31 down: 609)
+    for (int x = split_block_steps(p->Sq, window, r, 0); n == 0 || x >= 4; x -= 1 + x / 32) steps[n++] = x;
+    auto slots_of = [&](int i) {
         int slots = 0;
-        for (int i = 0; i < blocks; ++i) slots += split_block_parts(p->Sq, window, r, i, steps);
-        const int64_t wgs = rows * slots;
-        if (wgs > 4 * cus) break;
-        const int64_t cost = ((wgs + cus - 1) / cus) * (steps + 3);
-        if (steps == most || cost < best_cost) { best = {steps, slots, slots > blocks}; best_cost = cost; }
+        for (int k = 0; k < blocks; ++k) slots += split_block_parts(p->Sq, window, r, k, steps[i]);
+        return slots;
+    };
+    F32SplitParts best{steps[0], blocks, false};
+    int64_t rounds = (rows * blocks + cus - 1) / cus, best_cost = rounds * (steps[0] + 3);
+    for (int first = 0; rounds <= 4; ++rounds) {
+        int last = first, slots = 0;                       // the last count of at most so many rounds, from `first` on
+        for (int lo = first, hi = n - 1; lo <= hi;) {
+            const int mid = (lo + hi) / 2, m = slots_of(mid);
+            if (rows * m <= rounds * cus) { last = mid; slots = m; lo = mid + 1; } else hi = mid - 1;
+        }
+        if (slots && rounds * (steps[last] + 3) < best_cost) {
+            best = {steps[last], slots, slots > blocks};
+            best_cost = rounds * (steps[last] + 3);
+        }
+        first = last;
     }
     return best;
 }

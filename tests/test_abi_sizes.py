@@ -80,3 +80,29 @@ def test_float32_scratch_is_bounded(backward):
             else:
                 assert n >= 64 << 20                                                # (not one at a time where several fit)
     assert sizes(b=1, h=64, g=8, sq=1 << 19, skv=1 << 19) == 0
+
+
+def test_float32_dkdv_workgroups():
+    """The steps per dK/dV workgroup, through the partial sums' share of the scratch: the best of all counts, tried one by one."""
+    lib = _lib.load()
+    def steps_of(s, window, r, block):
+        lo = 128 * block
+        hi = min(s, lo + 127 + window) if window else s
+        return ((-(-hi // 32) - lo // 32 + 1) // 2) * r
+    for (h, g), s, window in itertools.product(((64, 8), (8, 1), (12, 3), (96, 8)), (320, 700, 1024, 2500, 4095, 6000), (0, 129, 500)):
+        if h // 4 * -(-s // 32) < 160 or (0 < window < 384 and h // 4 * -(-s // 32) > 400):
+            continue
+        walks = [steps_of(s, window, h // g, i) for i in range(-(-s // 128))]
+        best, steps = None, walks[0]
+        while steps >= 4 or best is None:
+            slots = sum(max(1, -(-w // steps)) for w in walks)
+            rounds = -(-g * slots // 256)
+            if rounds <= 4 and (best is None or rounds * (steps + 3) < best[0]):
+                best = (rounds * (steps + 3), slots)
+            steps -= 1 + steps // 32
+        tiles, up = -(-s // 32), lambda n: (n + 255) // 256 * 256
+        records = up(4 * g * tiles) + g * tiles * 24576 + up(4 * h * tiles) + h * tiles * 24832
+        if records > 256 << 20:
+            continue
+        sums = g * best[1] * 65536 if best[1] > len(walks) else 0
+        assert lib.gptoss_attn_split_bytes(ctypes.byref(_params(dtype=1, h=h, g=g, sq=s, skv=s, window=window)), 1) == records + sums, (h, g, s, window)
