@@ -803,8 +803,8 @@ static int launch_dkdv(const gptoss_attn_params *p, void *stream, bool whole_blo
     if (dkdv64_route(p, a.dkdv_parts)) {
         const int64_t blocks = (int64_t)a.B * ((a.Skv + Dkdv64::BN - 1) / Dkdv64::BN);      // of a KV head
         // padded and packed rows, and several rows of one length whose blocks would stay whole otherwise: pieces by the walks' lengths,
-        // at most as many as there are slots for partial sums (Dkdv64Plan)
-        const bool by_lengths = a.dkdv_parts > 1 && (a.seqlens || a.doc_start || (a.B > 1 && a.Sq < 4096 && many_key_blocks(p)));
+        // at most as many as there are slots for partial sums (Dkdv64Plan; the kernels hold kMaxBlocks lengths, nearly twice what dkdv_parts_for leaves)
+        const bool by_lengths = a.dkdv_parts > 1 && blocks <= Dkdv64Plan::kMaxBlocks && (a.seqlens || a.doc_start || (a.B > 1 && a.Sq < 4096 && many_key_blocks(p)));
         if (by_lengths) a.dkdv_slots = (int)((int64_t)a.dkdv_parts * a.B * a.Skv / Dkdv64::BN);
         const int64_t grid64 = a.G * (by_lengths ? a.dkdv_slots : blocks * a.dkdv_parts);
         const bool plain = !by_lengths && !a.seqlens && !a.doc_start && a.Sq % kTile == 0;
