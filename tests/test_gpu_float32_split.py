@@ -126,6 +126,49 @@ def test_numbers_that_three_terms_do_not_hold(A, which, value):
         assert float((x - y).norm()) <= 2e-5 * float(y.norm()), name
 
 
+@pytest.mark.parametrize("b,s,w,lens,docs,row,at", [
+    (2, 333, None, [150, 333], None, 0, 140),                  # the number in the last tile of a padded row
+    (2, 333, None, [333, 150], None, 0, 200),
+    (1, 700, None, None, [5, 300, 32, 363], 0, 200),           # in a document in the middle
+    (1, 333, 100, None, None, 0, 200),                         # seen by a few tiles
+    (1, 1056, None, None, None, 0, 900),                       # parts of 20 steps on eight heads: they start inside a pair of tiles
+    (1, 2600, 500, None, None, 0, 64),
+])
+@pytest.mark.parametrize("which,value", [("k", float("inf")), ("v", 1e30), ("v", float("nan")), ("q", 1e-35), ("d_out", 1e-34), ("q", 3e7)])
+def test_such_numbers_in_padded_packed_windowed_and_long_rows(A, which, value, b, s, w, lens, docs, row, at):
+    """Row by row and column by column, so that a huge number hides nothing but itself."""
+    print(f"case {which}={value} B={b} S={s} W={w} lens={lens} docs={docs}", flush=True)
+    inp = dict(zip(("q", "k", "v", "sinks", "d_out"), E.make_inputs(7750 + s, b, 64, 8, s, 64, torch.float32)))
+    t = inp[which]
+    (t[row, at, 5] if which == "d_out" else t[row, 2, at])[7] = value
+    if lens:
+        inp["d_out"] = inp["d_out"] * (torch.arange(s).view(1, s) < torch.tensor(lens).view(b, 1)).view(b, s, 1, 1)
+    _alike(*_both(A, tuple(inp.values()), w, lens, docs))
+
+
+def _alike(new, old):
+    for name, x, y in zip(("o", "lse", "dq", "dk", "dv"), new, old):
+        assert torch.equal(torch.isfinite(x), torch.isfinite(y)) and torch.equal(torch.isnan(x), torch.isnan(y)), name
+        ok = torch.isfinite(y)
+        x, y = (torch.where(ok, t, 0.0).double() for t in (x, y))
+        if name == "lse":
+            assert bool(((x - y).abs() <= 2e-5 * (1 + y.abs())).all())
+            continue
+        # 2e-5 of the row's and of the column's size, as everywhere; a row that is much smaller than most (its products cancel): of those
+        rows, off = y.norm(dim=-1), (x - y).norm(dim=-1)
+        assert bool((off <= 2e-5 * (rows + rows.median())).all()), (name, float((off / (rows + rows.median())).max()))
+        y, off = (t.reshape(-1, 64).norm(dim=0) for t in (y, x - y))
+        assert bool((off <= 2e-5 * y).all()), (name, float((off / y).max()))
+
+
+@pytest.mark.parametrize("sq,skv,w", [(330, 777, None), (256, 2049, None), (330, 777, 100)])
+@pytest.mark.parametrize("which,value,at", [("k", float("inf"), 600), ("v", 1e30, 600), ("v", float("nan"), 40), ("q", 1e-35, 17)])
+def test_such_numbers_behind_a_cache(A, which, value, at, sq, skv, w):
+    inp = dict(zip(("q", "k", "v", "sinks", "d_out"), E.make_inputs(7760 + sq, 1, 64, 8, sq, 64, torch.float32, skv=skv)))
+    inp[which][0, 2, at, 7] = value
+    _alike(*_both(A, tuple(inp.values()), w, start=skv - sq, backward=False))
+
+
 @pytest.mark.parametrize("which,value", [("v", float("inf")), ("v", -1e37), ("lse", -float("inf")), ("lse", float("inf"))])
 def test_row_statistics_that_three_terms_do_not_hold(A, which, value):
     """A number that only the last row sees makes that row's delta infinite or large, or its lse is infinite: workgroups whose own operands are
