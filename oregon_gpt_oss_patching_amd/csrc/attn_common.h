@@ -70,6 +70,7 @@ struct KArgs {
     int split_steps, split_slots;
     float *split_partial;
     int split_b0, split_nb, split_g0, split_ng;      // the batch rows and KV heads of this launch (the records are theirs alone)
+    int split_tiles;     // K / V records of a KV head: 32 keys each, those that some query sees
 };
 
 // The sink logits and their gradient in the type the caller's parameter has: a conversion of 64 numbers was a launch of its own

@@ -266,14 +266,23 @@ __device__ __forceinline__ void split_copy(uint32_t dst, const char *src, int la
 // where the records and the partial sums of a batch row's KV head stand among those of the launch
 __device__ __forceinline__ int64_t split_row_of(const KArgs &a, int b, int g) { return (int64_t)(b - a.split_b0) * a.split_ng + (g - a.split_g0); }
 
+// The first 32 keys with a record: behind a cache a window's queries see the last ones only (256 queries on 16384 keys, window 128: forward with
+// a record for every key 71 us).  The host counts split_tiles of them (split_key_tiles).
+__device__ __forceinline__ int split_first_tile(const KArgs &a, int q_offset) { return a.window > 0 ? max(0, q_offset - a.window + 1) / 32 : 0; }
+// from the tile of the first query's first key to that of the last query, wherever the queries stand in these
+__host__ __device__ inline int split_key_tiles(int Sq, int Skv, int window) {
+    const int64_t all = ((int64_t)Skv + 31) / 32, seen = ((int64_t)Sq + window - 2) / 32 + 2;
+    return (int)(window > 0 && seen < all ? seen : all);
+}
 // ---- K and V as records ------------------------------------------------------------------------------------
 // One workgroup per (batch, KV head, 32 keys).  Keys that nobody sees (past the tensor, a padded row's length, the last query) are
 // zeros.  Bound by memory: 10 bytes moved per number.
 __global__ __launch_bounds__(256) void attn_f32_split_kv_kernel(const KArgs a) {
     const F32Ptrs t = f32_ptrs(a);
-    const int nt = (a.Skv + 31) / 32, tile = (int)(blockIdx.x % nt), bg = (int)(blockIdx.x / nt), b = a.split_b0 + bg / a.split_ng, g = a.split_g0 + bg % a.split_ng;
+    const int q_offset = query_offset(a);
+    const int nt = a.split_tiles, tile = split_first_tile(a, q_offset) + (int)(blockIdx.x % nt), bg = (int)(blockIdx.x / nt), b = a.split_b0 + bg / a.split_ng, g = a.split_g0 + bg % a.split_ng;
     const int which = threadIdx.x >> 7, r = (threadIdx.x >> 2) & 31, part = threadIdx.x & 3, key = 32 * tile + r;
-    int64_t end = min((int64_t)a.Skv, (int64_t)query_offset(a) + a.Sq);
+    int64_t end = min((int64_t)a.Skv, (int64_t)q_offset + a.Sq);
     if (a.seqlens) end = min(end, (int64_t)a.seqlens[b]);
     const float *row = which == 0 ? t.k + (int64_t)b * a.ks.b + (int64_t)g * a.ks.h + (int64_t)key * a.ks.s
                                   : t.v + (int64_t)b * a.vs.b + (int64_t)g * a.vs.h + (int64_t)key * a.vs.s;
@@ -302,11 +311,13 @@ __global__ __launch_bounds__(256) void attn_f32_split_kv_kernel(const KArgs a) {
 struct SplitKeyWalk {
     const char *rec;
     const uint32_t *rec_bad;
-    int nt, t_lo, n, w, lane;
+    int t_end, t_lo, n, w, lane;
     uint32_t lds;
-    __device__ __forceinline__ SplitKeyWalk(const KArgs &a, int b, int g, int t_lo_, int n_, int w_, int lane_, const char *smem)
-        : nt((a.Skv + 31) / 32), t_lo(t_lo_), n(n_), w(w_), lane(lane_), lds(lds_addr(smem)) {
-        const int64_t first = split_row_of(a, b, g) * nt;
+    __device__ __forceinline__ SplitKeyWalk(const KArgs &a, int q_offset, int b, int g, int t_lo_, int n_, int w_, int lane_, const char *smem)
+        : t_lo(t_lo_), n(n_), w(w_), lane(lane_), lds(lds_addr(smem)) {
+        const int t_first = split_first_tile(a, q_offset);
+        t_end = t_first + a.split_tiles;
+        const int64_t first = split_row_of(a, b, g) * a.split_tiles - t_first;       // (tile 0's)
         rec = a.split_kv + first * F32Split::kKvRecord;
         rec_bad = a.split_kv_bad + first;
     }
@@ -318,7 +329,7 @@ struct SplitKeyWalk {
     __device__ __forceinline__ int steps() const { return (n + 1) >> 1; }
     // (the tile behind the last one, if there is none, is the last one again)
     __device__ __forceinline__ void request(int step) const {
-        const int tile = min(t_lo + 2 * step + (w >> 2), nt - 1);
+        const int tile = min(t_lo + 2 * step + (w >> 2), t_end - 1);
         split_copy(lds + ((step & 1) * 2 + (w >> 2)) * F32Split::kKvRecord + (w & 3) * F32Split::kWaveCopy,
                    rec + (int64_t)tile * F32Split::kKvRecord + (w & 3) * F32Split::kWaveCopy, lane);
     }
@@ -337,7 +348,7 @@ __global__ __launch_bounds__(512, 2) void attn_f32_split_fwd_kernel(const KArgs 
     const F32Ptrs t = f32_ptrs(a);
     const F32QueryWork<2, F32Split::kWaves> wk(a, t, q_offset, smem);
     const int lane = wk.lane, w = wk.w, l32 = lane & 31, half = lane >> 5, row = wk.q0 + l32;
-    const SplitKeyWalk walk(a, wk.b, wk.g, wk.t_lo, wk.n, w, lane, smem);
+    const SplitKeyWalk walk(a, q_offset, wk.b, wk.g, wk.t_lo, wk.n, w, lane, smem);
     if (walk.n > 0) walk.request(0);
     SplitCheck check;
     const bool keys_bad = walk.bad();
@@ -422,7 +433,7 @@ __global__ __launch_bounds__(512, 2) void attn_f32_split_dq_kernel(const KArgs a
     const int lane = wk.lane, w = wk.w, l32 = lane & 31, half = lane >> 5, row = wk.q0 + l32;
     const bool row_ok = row < a.Sq, live = row_ok && row < wk.q_len;       // (what a padded row holds must not matter)
     const int rowc = min(row, a.Sq - 1);
-    const SplitKeyWalk walk(a, wk.b, wk.g, wk.t_lo, wk.n, w, lane, smem);
+    const SplitKeyWalk walk(a, 0, wk.b, wk.g, wk.t_lo, wk.n, w, lane, smem);
     if (walk.n > 0) walk.request(0);
     const int64_t total = (int64_t)a.B * a.H * a.Sq, rid = ((int64_t)wk.b * a.H + wk.head) * a.Sq + rowc;
     const int64_t rec_i = (split_row_of(a, wk.b, wk.g) * a.r + (wk.head - wk.g * a.r)) * ((a.Sq + 31) / 32) + wk.q0 / 32;

@@ -96,7 +96,7 @@ KArgs make_args(const gptoss_attn_params *p, SinkTypes ty) {
     a.split_kv_bad = a.split_q_bad = nullptr;
     a.split_steps = a.split_slots = 0;
     a.split_partial = nullptr;
-    a.split_b0 = a.split_nb = a.split_g0 = a.split_ng = 0;
+    a.split_b0 = a.split_nb = a.split_g0 = a.split_ng = a.split_tiles = 0;
     return a;
 }
 
@@ -297,17 +297,21 @@ int64_t f32_grid(const KArgs &a, int ks) {
 // ---- float32 on the bf16 matrix pipes (attn_f32_split.h) -----------------------------------------
 // Taken where the caller has scratch for the records, four consecutive heads share a KV head (the four units of a workgroup then stand
 // at the same rows), the backward for self-attention without an offset, and where it is the faster one: it costs a launch and fills the
-// chip with workgroups of eight wavefronts.  fp32 instruction / this, us a call, 64 query heads on 8 KV heads, forward + backward: 8 x 128
-// rows 121 / 123, 256 95 / 104, 320 101 / 96, 448 139 / 106, 1024 413 / 254, 4096 5350 / 3280; 8 heads on one KV head 1024 (64 workgroups) 150 /
-// 145, 2048 on two (128) 263 / 225; a window of 128 is a handful of tiles per workgroup, whose start and end then decide: 320
-// 111 / 106, 640 132 / 120, 1024 (512 workgroups) 148 / 151, 2048 254 / 268; of 512, 1024 rows 382 / 228.  Queries on a cache: 1 on
-// 2048 47 / 88, 64 x 4 on 4096 158 / 174, 256 on 4096 155 / 139, 1024 on 8192 1119 / 614.
+// chip with workgroups of eight wavefronts, one per compute unit.  Self-attention takes it in both directions or in neither (with lse of the one and S of the other
+// dQ of operands next to a bf16 number was 1.09 times as far from float64 as with the fp32 instruction alone).  fp32 instruction / this, us in a graph, 64 query heads on 8 KV heads,
+// forward and backward: 320 rows 23 + 82 / 25 + 70, 448 33 + 110 / 31 + 80, 1024 100 + 310 / 66 + 200, 4096 5320 / 3120; 8 heads on one KV head 2048 rows (128 workgroups)
+// 63 + 249 / 79 + 165; a window is a handful of tiles per workgroup, whose start and end then decide: of 128, 320 rows 22 + 88 / 21 + 63, 640 33 + 103 / 35 + 91, 800 (400 workgroups)
+// 36 + 107 / 39 + 102, 1024 147 / 150; of 383, 800 63 + 220 / 50 + 136; of 64, 448 21 + 69 / 20 + 61, but 640 26 + 74 / 33 + 83.
+// Queries on a cache, forward: 256 (128 workgroups) on 2048 80 / 84, on 4096 154 / 154, on 16384 600 / 566; 320 on 1024 59 / 48, 1024 on 8192 1121 / 647; with a window of 128, 320 on
+// 16384 23 / 21, 448 26 / 22, 576 34 / 36, 256 (128 workgroups) 15 / 21; of 64, 320 17 / 19, 448 21 / 20; of 192, 576 43 / 41; of 400, 800 76 / 56.
 bool f32_split_route(const gptoss_attn_params *p, bool bwd) {
     if (p->dtype != GPTOSS_ATTN_FP32 || p->B <= 0 || p->G <= 0 || p->H <= 0 || p->H % p->G || (p->H / p->G) % 4 || p->Skv <= 0) return false;
-    if (bwd && (p->Sq != p->Skv || p->q_offset != 0 || p->q_offset_dev)) return false;
+    const bool self = p->Sq == p->Skv && p->q_offset == 0 && !p->q_offset_dev;       // (both directions take it, or neither)
+    if (bwd && !self) return false;
     const int64_t wgs = (int64_t)(p->H / 4) * p->B * (((int64_t)p->Sq + 31) / 32);
     const int window = effective_window(p);
-    if (window > 0 && window < 384 && wgs > 400) return false;
+    if (window > 0 && window < 384 && wgs > (!self && window < 160 ? 256 : 400)) return false;
+    if (!self && window > 0) return p->Sq >= 192 && wgs >= (window < 96 ? 224 : 160);
     return p->Sq >= 192 && (wgs >= 160 || (wgs >= 128 && p->Skv >= 2048));
 }
 // Steps per dK/dV workgroup, `rows` batch rows and KV heads at once: the count whose rounds of workgroups take the least time on 256 compute units, one
@@ -349,13 +353,14 @@ F32SplitParts f32_split_parts(const gptoss_attn_params *p, int64_t rows) {
 // included; the left figures with terms cut off instead of rounded, 1.5 % faster at 1024 tokens): 4096 tokens 3200 (529) / 3275 (450), window 512 985 / 1010, 4 x 2000 3415 (913) / 3499
 // (579), 8192 12070 (1046) / 12310 (604), 16384 47300 (2106) / 49400 (911).  128 MB: window 512 another 7 % slower, the others alike.
 constexpr size_t kF32SplitRecords = (size_t)256 << 20;
-struct F32SplitPlan { int nb, ng; size_t kv, q_bad, q, partial, bytes; F32SplitParts parts; };
+struct F32SplitPlan { int nb, ng, tiles; size_t kv, q_bad, q, partial, bytes; F32SplitParts parts; };
 F32SplitPlan f32_split_plan(const gptoss_attn_params *p, bool bwd) {
     auto up = [](size_t n) { return (n + 255) & ~(size_t)255; };
     auto share = [](int n, size_t most) { const int times = (int)((n + most - 1) / most); return (n + times - 1) / times; };
     F32SplitPlan s{};
     if (!f32_split_route(p, bwd)) return s;
-    const size_t n_kv = (size_t)(p->Skv + 31) / 32, n_q = (size_t)(p->H / p->G) * ((p->Sq + 31) / 32);      // of a KV head
+    s.tiles = split_key_tiles(p->Sq, p->Skv, effective_window(p));
+    const size_t n_kv = (size_t)s.tiles, n_q = (size_t)(p->H / p->G) * ((p->Sq + 31) / 32);      // of a KV head
     const size_t most = kF32SplitRecords / (n_kv * F32Split::kKvRecord + (bwd ? n_q * F32Split::kQRecord : 0));
     if (most == 0) return s;
     s.nb = most > (size_t)p->G ? share(p->B, most / p->G) : 1;
@@ -377,6 +382,7 @@ void f32_split_args(KArgs &a, const F32SplitPlan &s, void *scratch) {
     a.split_kv = base + s.kv;
     a.split_q_bad = reinterpret_cast<uint32_t *>(base + s.q_bad);
     a.split_q = base + s.q;
+    a.split_tiles = s.tiles;
     a.split_steps = s.parts.steps;
     a.split_slots = s.parts.slots;
     a.split_partial = s.parts.cut ? reinterpret_cast<float *>(base + s.partial) : nullptr;
@@ -526,7 +532,7 @@ int launch_window_bwd(const gptoss_attn_params *p, hipStream_t st, bool seam_sum
     return e == hipSuccess ? GPTOSS_ATTN_OK : static_cast<int>(e);
 }
 
-int launch_f32_split_kv(const KArgs &a, hipStream_t st) { return launch(attn_f32_split_kv_kernel, (int64_t)a.split_nb * a.split_ng * ((a.Skv + 31) / 32), 256, st, a); }
+int launch_f32_split_kv(const KArgs &a, hipStream_t st) { return launch(attn_f32_split_kv_kernel, (int64_t)a.split_nb * a.split_ng * a.split_tiles, 256, st, a); }
 int64_t f32_split_grid(const KArgs &a) { return (int64_t)a.split_ng * (a.r / 4) * a.split_nb * ((a.Sq + 31) / 32); }
 
 int launch_f32_split_fwd(const gptoss_attn_params *p, hipStream_t st, SinkTypes ty, const F32SplitPlan &plan, void *scratch) {

@@ -106,3 +106,13 @@ def test_float32_dkdv_workgroups():
             continue
         sums = g * best[1] * 65536 if best[1] > len(walks) else 0
         assert lib.gptoss_attn_split_bytes(ctypes.byref(_params(dtype=1, h=h, g=g, sq=s, skv=s, window=window)), 1) == records + sums, (h, g, s, window)
+
+
+def test_float32_window_on_a_cache():
+    """Records of the keys that the window's queries see: however long the cache is, the same scratch.  Few workgroups or a small window: none."""
+    lib = _lib.load()
+    size = lambda sq, skv, window, **kw: lib.gptoss_attn_split_bytes(ctypes.byref(_params(1, 1, 64, 8, sq, skv, window, q_offset=skv - sq, **kw)), 0)
+    assert size(448, 2000, 128) == size(448, 32768, 128) == size(448, 1 << 20, 128) > 0
+    assert size(448, 448 + 64, 128) == size(448, 480 + 32, 128) <= size(448, 2000, 128)
+    assert size(256, 16384, 128) == size(320, 16384, 64) == size(576, 16384, 128) == 0
+    assert size(576, 16384, 192) > 0 and size(320, 16384, 0) > size(320, 4096, 0) > 0

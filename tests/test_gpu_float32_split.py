@@ -213,3 +213,33 @@ def test_some_rows_and_heads_at_a_time(A, b, h, g, s, w, lens, docs):
         row = [t[i:i + 1] if t.dim() == 4 else t for t in inp]
         one, _ = _both(A, row, w, [lens[i]] if lens else None, docs)
         assert torch.equal(one[0], new[0][i:i + 1]) and torch.equal(one[1], new[1][i:i + 1]) and torch.equal(one[2], new[2][i:i + 1]), i
+
+
+@pytest.mark.parametrize("sq,skv,w,start", [
+    (330, 5000, 100, 4670), (330, 5000, 100, 131), (330, 5000, 100, 99), (330, 5000, 100, 1), (330, 5000, 100, 0),
+    (321, 4100, 500, 3779),
+    (320, 4099, 129, 2000),            # keys behind the last query
+    (330, 600, 100, 500),              # queries behind the last key
+    (330, 600, 100, 1200),             # none of them sees one
+])
+@pytest.mark.parametrize("on_device", [False, True])
+def test_windows_behind_a_cache(A, sq, skv, w, start, on_device):
+    """Records of the keys that some query sees, and of no others: the walks meet the right ones wherever the queries stand."""
+    from oregon_gpt_oss_patching_amd import _lib
+    from oregon_gpt_oss_patching_amd import attention_kernel as ak
+    q, k, v, sinks, _ = (t.to(DEV) for t in E.make_inputs(7950 + start, 2, 32, 4, sq, 64, torch.float32, skv=skv))
+    k[:, :, :max(0, start - w + 1)] = float("nan")             # (nobody sees them)
+    at = torch.tensor([start], dtype=torch.int32, device=DEV) if on_device else None
+    new = A.attention_forward(q, k, v, sinks, SCALE, w, 0 if on_device else start, q_offset_dev=at)
+    p = ak._base_params(q, k, v, sinks, None, SCALE, w, start, None)
+    o, lse = torch.empty_like(new[0]), torch.empty_like(new[1])
+    p.o, p.lse = o.data_ptr(), lse.data_ptr()
+    ak._set(p.o_stride, ak._strides_bhs(o, "bshd"))
+    assert 0 < _lib.load().gptoss_attn_split_bytes(ctypes.byref(p), 0) <= 2 * 4 * (24576 + 4) * ((sq + w) // 32 + 2) + 256
+    if start > w:
+        k[:, :, :start - w + 1] = 0.0                          # (the other kernel multiplies what shares a tile, masked)
+    _lib.call("gptoss_attn_fwd", p, torch.cuda.current_stream().cuda_stream)
+    assert bool(torch.isfinite(o).all())
+    # each no further from float64 than 2e-5 of the result (1.3e-6 at the most in test_chunks_behind_a_cache)
+    assert float((new[0] - o).double().norm()) <= 2e-5 * float(o.double().norm())
+    assert float((new[1] - lse).abs().max()) <= 2e-5
