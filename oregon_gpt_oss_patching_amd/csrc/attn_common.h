@@ -69,6 +69,7 @@ struct KArgs {
     uint32_t *split_kv_bad, *split_q_bad;
     int split_steps, split_slots;
     float *split_partial;
+    int *split_plan;     // padded and packed rows whose key blocks are cut: first slot and number of parts of every block, by the dK/dV kernel
     int split_b0, split_nb, split_g0, split_ng;      // the batch rows and KV heads of this launch (the records are theirs alone)
     int split_tiles;     // K / V records of a KV head: 32 keys each, those that some query sees
 };

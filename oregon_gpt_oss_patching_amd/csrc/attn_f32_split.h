@@ -546,6 +546,82 @@ __host__ __device__ inline int split_block_parts(int Sq, int window, int r, int 
     const int n = (split_block_steps(Sq, window, r, block) + steps - 1) / steps;
     return n < 1 ? 1 : n;
 }
+// Padded rows and packed documents (split_plan) have shorter walks, which only the device knows: the host's parts of them would be many short ones of the first
+// blocks and one long one of the last.  A row's workgroups then divide its walks themselves, into parts of the number of steps that takes the fewest rounds as the
+// host counts them, and need no more slots than the host counted.  Backward of 64 heads, us, fp32 instruction / the host's parts / so: 4096 tokens in documents of 100 332 / 515 / 365, of 250 541 / 630 / 455, of 700 1037 / 860 / 740, of 1000 1465 / 1060 / 890; 1024 tokens of 100 108 / 156 / 115, of 1000 350 / 210 / 213; 8 heads on one KV
+// head, 4096 of 200 98 / 208 / 84; two rows of 1024 padded to 100 and 150 91 / 162 / 113.  (What is left of documents of 100 is the start of a workgroup per 128 keys and four
+// heads, which dQ and the forward have too.)
+struct SplitPart { int block, number, steps; };            // (block -1: there is nothing left for this workgroup)
+__device__ __forceinline__ int split_walk_steps(const KArgs &a, int b, int block) {
+    const int len = a.seqlens ? max(0, min(a.Sq, a.seqlens[b])) : a.Sq, lo = F32Split::kKeys * block, last = min(lo + F32Split::kKeys, len) - 1;
+    if (last < lo) return 0;
+    int end = a.window > 0 ? min(len, last + a.window) : len;
+    if (a.doc_start) {                                     // the first row that does not see the block's last key
+        const int32_t *row = a.doc_start + (int64_t)b * a.Sq;
+        int from = last + 1;
+        while (from < end) {
+            const int x = (from + end) >> 1;
+            if (row[x] > last) end = x; else from = x + 1;
+        }
+    }
+    return (((end + 31) / 32 - lo / 32 + 1) >> 1) * a.r;
+}
+template <bool SHORT>
+__device__ __forceinline__ SplitPart split_part(const KArgs &a, int b, int64_t bg, int slot, int lane) {
+    const int blocks = (a.Skv + F32Split::kKeys - 1) / F32Split::kKeys;
+    if (!SHORT || !a.split_plan) {
+        int block = 0;
+        for (int n; slot >= (n = split_block_parts(a.Sq, a.window, a.r, block, a.split_steps)); ++block) slot -= n;
+        return {block, slot, a.split_steps};
+    }
+    int all = 0, most = 0, mine = 0;
+    for (int i = lane; i < blocks; i += 64) {
+        mine = split_walk_steps(a, b, i);
+        all += mine;
+        most = max(most, mine);
+    }
+#pragma unroll
+    for (int d = 1; d < 64; d *= 2) { all += __shfl_xor(all, d); most = max(most, __shfl_xor(most, d)); }
+    // rows like this one that make up the launch's work, about: a long row among short ones has more of the chip
+    int rows = a.split_nb * a.split_ng;
+    if (a.seqlens && a.split_nb > 1) {
+        auto size = [&](int row) __attribute__((always_inline)) { const float n = (float)max(1, min(a.Sq, a.seqlens[row])); return a.window > 0 ? n : n * n; };
+        float sum = 0.0f;
+        for (int i = lane; i < a.split_nb; i += 64) sum += size(a.split_b0 + i);
+#pragma unroll
+        for (int d = 1; d < 64; d *= 2) sum += __shfl_xor(sum, d);
+        rows = (int)fminf((float)a.split_ng * sum / size(b), 0x1p14f);
+    }
+    int steps = a.split_steps, cost = (rows * a.split_slots + 255) / 256 * (steps + 3);
+    auto consider = [&](int rounds, int x) __attribute__((always_inline)) { if (rounds * (x + 3) < cost) { cost = rounds * (x + 3); steps = x; } };
+    consider((rows * blocks + 255) / 256, max(most, 1));
+    for (int k = 1; k <= 4; ++k) {
+        const int n = min(a.split_slots, k * 256 / max(rows, 1)) - blocks;       // (each block may leave one part that is not full)
+        if (n > 0) consider(k, max(1, (all + n - 1) / n));
+    }
+    steps = __builtin_amdgcn_readfirstlane(steps);
+    int first = 0;
+    for (int i0 = 0; i0 < blocks; i0 += 64) {
+        if (blocks > 64) mine = i0 + lane < blocks ? split_walk_steps(a, b, i0 + lane) : 0;
+        const int n = i0 + lane < blocks ? max(1, (mine + steps - 1) / steps) : 0;
+        int upto = n;
+#pragma unroll
+        for (int d = 1; d < 64; d *= 2) { const int x = __shfl_up(upto, d); upto += lane >= d ? x : 0; }
+        const uint64_t past = __builtin_amdgcn_ballot_w64(first + upto > slot);
+        if (past) {
+            const int i = __builtin_ctzll(past), parts = __builtin_amdgcn_readlane(n, i), number = slot - (first + __builtin_amdgcn_readlane(upto, i) - parts);
+            if (number == 0 && threadIdx.x == 0) {         // (for the sum)
+                a.split_plan[2 * (bg * blocks + i0 + i)] = slot;
+                a.split_plan[2 * (bg * blocks + i0 + i) + 1] = parts;
+            }
+            return {i0 + i, number, steps};
+        }
+        first += __builtin_amdgcn_readlane(upto, 63);
+    }
+    return {-1, 0, 0};
+}
+// SHORT: padded rows or packed documents (an instantiation: 1024 rows without either 2 us slower with both)
+template <bool SHORT>
 __global__ __launch_bounds__(512, 2) void attn_f32_split_dkdv_kernel(const KArgs a) {
     extern __shared__ __attribute__((aligned(1024))) char f32_split_lds[];
     char *const smem = f32_split_lds;
@@ -557,13 +633,15 @@ __global__ __launch_bounds__(512, 2) void attn_f32_split_dkdv_kernel(const KArgs
     const int bi = bid % a.split_nb, slot = bid / a.split_nb;
     const int b = rotated_batch_row(bi, slot, a.split_nb) + a.split_b0;
     const int64_t bg = split_row_of(a, b, g);
-    int block = 0, part = slot;
-    for (int n; part >= (n = split_block_parts(a.Sq, a.window, a.r, block, a.split_steps)); ++block) part -= n;
+    const SplitPart part = split_part<SHORT>(a, b, bg, slot, lane);
+    const int block = part.block;
+    if (SHORT && block < 0) return;
     const int J0 = C::kKeys * block, j0 = J0 + 32 * (w & 3), key = j0 + l32;
     const int nt = (a.Skv + 31) / 32, nqt = (a.Sq + 31) / 32;
     const F32TileSpan span = f32_tiles_of_keys(a, 0, b, J0, C::kKeys, lane);
     const int t_hi = __builtin_amdgcn_readfirstlane(span.t_hi), t_lo = span.t_lo;
-    const int all = ((t_hi - t_lo + 1) >> 1) * a.r, s0 = part * a.split_steps, n_steps = max(0, min(a.split_steps, all - s0));
+    const int all = ((t_hi - t_lo + 1) >> 1) * a.r;
+    const int s0 = part.number * part.steps, n_steps = max(0, min(part.steps, all - s0));
     float *const partial = a.split_partial ? a.split_partial + (bg * a.split_slots + slot) * (2 * C::kKeys * kD) : nullptr;
 
     const char *const qrec = a.split_q + bg * a.r * nqt * C::kQRecord;
@@ -575,6 +653,22 @@ __global__ __launch_bounds__(512, 2) void attn_f32_split_dkdv_kernel(const KArgs
         split_copy(dst + (w & 3) * C::kWaveCopy, src + (w & 3) * C::kWaveCopy, lane);
         if ((w & 3) == 3) lds_dma4(dst + C::kStatOff, src + C::kStatOff, (uint32_t)(lane * 4));
     };
+    // the rows from `lim` on do not see the lane's key: they do not exist, or belong to a later document (found once: with the document starts read per tile and every
+    // tile masked, the backward of 4096 tokens in documents of 100 490 us instead of 475, of 400 672 instead of 639)
+    int lim = span.row_lim, all_see = lim;                 // (all_see: no key of the wavefront has less)
+    if (SHORT && a.doc_start) {
+        const int32_t *row = a.doc_start + (int64_t)b * a.Sq;
+        int lo = min(key, lim), hi = max(lo, min(lim, 32 * t_hi));
+        while (__builtin_amdgcn_ballot_w64(lo < hi) != 0ull) {
+            const int x = (lo + hi) >> 1;
+            const bool past = row[min(x, a.Sq - 1)] > key;
+            if (lo < hi) { if (past) hi = x; else lo = x + 1; }
+        }
+        lim = all_see = lo;
+#pragma unroll
+        for (int d = 1; d < 32; d *= 2) all_see = min(all_see, __shfl_xor(all_see, d));
+    }
+    all_see = __builtin_amdgcn_readfirstlane(all_see);
     if (n_steps > 0) request(0);
     // numbers the split does not take, among the block's keys or the rows of the walk
     uint32_t bad = 0;
@@ -621,7 +715,6 @@ __global__ __launch_bounds__(512, 2) void attn_f32_split_dkdv_kernel(const KArgs
     for (int i = 0; i < 16; ++i) { dk[0][i] = dk[1][i] = 0.0f; dv[0][i] = dv[1][i] = 0.0f; }
     const int kv_len = a.seqlens ? min(a.Skv, a.seqlens[b]) : a.Skv;
     const int weff = a.window ? a.window : 0x3fffffff;
-    const int32_t *dsrow = a.doc_start ? a.doc_start + (int64_t)b * a.Sq : nullptr;
     TileLaneOffsets at = tile_offsets_at(make_tile_offsets(lane), lds + (w >> 2) * C::kQRecord);
     uint32_t stat = lds + (w >> 2) * C::kQRecord + C::kStatOff + 16 * half;
     const float c = a.scale_log2;
@@ -650,7 +743,7 @@ __global__ __launch_bounds__(512, 2) void attn_f32_split_dkdv_kernel(const KArgs
                 if (i >= 12) cut.step(s, 0, i - 12);
                 if (i == 23) cut.take(f[0]);
             };
-            const bool interior = j0 + 31 <= q0 && q0 + 31 - weff < j0 && j0 + 32 <= kv_len && q0 + 32 <= span.row_lim && !dsrow;
+            const bool interior = j0 + 31 <= q0 && q0 + 31 - weff < j0 && j0 + 32 <= kv_len && q0 + 32 <= all_see;
             if (interior && split_weights_normal(s)) {
                 split_rows_product<kG, true>(dp, at, vf, kept, kept_v, [&](int i) __attribute__((always_inline)) {
                     if (i < 16) s[i] = split_weight(s[i]);
@@ -662,13 +755,9 @@ __global__ __launch_bounds__(512, 2) void attn_f32_split_dkdv_kernel(const KArgs
                     // visible: 0 <= row - key < width (hidden from the compiler, which would keep sixteen lane-dependent numbers for it)
                     int first = q0 + 4 * half;
                     asm volatile("" : "+v"(first));
-                    const unsigned width = key < kv_len ? (unsigned)max(0, min(weff, span.row_lim - key)) : 0u;
+                    const unsigned width = key < kv_len ? (unsigned)max(0, min(weff, lim - key)) : 0u;
 #pragma unroll
                     for (int i = 0; i < 16; ++i) s[i] = (unsigned)(first - key + crow(i, 0)) < width ? s[i] : 0.0f;
-                    if (dsrow) {
-#pragma unroll
-                        for (int i = 0; i < 16; ++i) s[i] = key >= dsrow[min(first + crow(i, 0), a.Sq - 1)] ? s[i] : 0.0f;
-                    }
                 }
                 split_rows_product<kG, true>(dp, at, vf, kept, kept_v, cut_first);
             }
@@ -729,9 +818,15 @@ __global__ __launch_bounds__(256) void attn_f32_split_reduce_kernel(const KArgs 
     const int64_t row = (idx - (int64_t)which * rows * 16) >> 4;
     const int key = (int)(row % a.Skv), bg = (int)(row / a.Skv), block = key / C::kKeys;
     const int g = a.split_g0 + bg % a.split_ng, b = a.split_b0 + bg / a.split_ng;
-    int slot = 0;
-    for (int i = 0; i < block; ++i) slot += split_block_parts(a.Sq, a.window, a.r, i, a.split_steps);
-    const int n = split_block_parts(a.Sq, a.window, a.r, block, a.split_steps);
+    int slot = 0, n;
+    if (a.split_plan) {
+        const int *plan = a.split_plan + 2 * ((int64_t)bg * ((a.Skv + C::kKeys - 1) / C::kKeys) + block);
+        slot = plan[0];
+        n = plan[1];
+    } else {
+        for (int i = 0; i < block; ++i) slot += split_block_parts(a.Sq, a.window, a.r, i, a.split_steps);
+        n = split_block_parts(a.Sq, a.window, a.r, block, a.split_steps);
+    }
     const float *src = a.split_partial + ((int64_t)bg * a.split_slots + slot) * (2 * C::kKeys * kD) + (which * C::kKeys + key % C::kKeys) * kD + 4 * ch;
     f32x4 x = {0.0f, 0.0f, 0.0f, 0.0f};
     for (int i = 0; i < n; ++i) {

@@ -96,6 +96,7 @@ KArgs make_args(const gptoss_attn_params *p, SinkTypes ty) {
     a.split_kv_bad = a.split_q_bad = nullptr;
     a.split_steps = a.split_slots = 0;
     a.split_partial = nullptr;
+    a.split_plan = nullptr;
     a.split_b0 = a.split_nb = a.split_g0 = a.split_ng = a.split_tiles = 0;
     return a;
 }
@@ -353,7 +354,7 @@ F32SplitParts f32_split_parts(const gptoss_attn_params *p, int64_t rows) {
 // included; the left figures with terms cut off instead of rounded, 1.5 % faster at 1024 tokens): 4096 tokens 3200 (529) / 3275 (450), window 512 985 / 1010, 4 x 2000 3415 (913) / 3499
 // (579), 8192 12070 (1046) / 12310 (604), 16384 47300 (2106) / 49400 (911).  128 MB: window 512 another 7 % slower, the others alike.
 constexpr size_t kF32SplitRecords = (size_t)256 << 20;
-struct F32SplitPlan { int nb, ng, tiles; size_t kv, q_bad, q, partial, bytes; F32SplitParts parts; };
+struct F32SplitPlan { int nb, ng, tiles; size_t kv, q_bad, q, plan, partial, bytes; F32SplitParts parts; };
 F32SplitPlan f32_split_plan(const gptoss_attn_params *p, bool bwd) {
     auto up = [](size_t n) { return (n + 255) & ~(size_t)255; };
     auto share = [](int n, size_t most) { const int times = (int)((n + most - 1) / most); return (n + times - 1) / times; };
@@ -371,8 +372,9 @@ F32SplitPlan f32_split_plan(const gptoss_attn_params *p, bool bwd) {
     if (!bwd) return s;
     s.q_bad = s.bytes;
     s.q = s.q_bad + up(4 * rows * n_q);
-    s.partial = s.q + rows * n_q * F32Split::kQRecord;
+    s.plan = s.q + rows * n_q * F32Split::kQRecord;
     s.parts = f32_split_parts(p, (int64_t)rows);
+    s.partial = s.plan + (s.parts.cut ? up(2 * sizeof(int) * rows * ((p->Skv + F32Split::kKeys - 1) / F32Split::kKeys)) : 0);
     s.bytes = s.partial + (s.parts.cut ? rows * s.parts.slots * (2 * F32Split::kKeys * kD * sizeof(float)) : 0);
     return s;
 }
@@ -386,6 +388,7 @@ void f32_split_args(KArgs &a, const F32SplitPlan &s, void *scratch) {
     a.split_steps = s.parts.steps;
     a.split_slots = s.parts.slots;
     a.split_partial = s.parts.cut ? reinterpret_cast<float *>(base + s.partial) : nullptr;
+    a.split_plan = s.parts.cut && (a.seqlens || a.doc_start) ? reinterpret_cast<int *>(base + s.plan) : nullptr;
 }
 // step(last) for every share of the batch rows and KV heads, set in `a`
 template <typename Step>
@@ -550,13 +553,14 @@ int launch_f32_split_bwd(const gptoss_attn_params *p, hipStream_t st, SinkTypes 
     KArgs a = make_args(p, ty);
     f32_split_args(a, plan, scratch);
     int rc = lds_attribute<&attn_f32_split_dq_kernel>(F32Split::kDqLds);
-    if (rc || (rc = lds_attribute<&attn_f32_split_dkdv_kernel>(F32Split::kDkdvLds))) return rc;
+    const bool lengths = a.seqlens || a.doc_start;
+    if (rc || (rc = lengths ? lds_attribute<&attn_f32_split_dkdv_kernel<true>>(F32Split::kDkdvLds) : lds_attribute<&attn_f32_split_dkdv_kernel<false>>(F32Split::kDkdvLds))) return rc;
     return f32_split_shares(a, plan, [&](bool last) {
         int s = launch_f32_split_kv(a, st);
         if (s || (s = launch(attn_f32_split_dq_kernel, f32_split_grid(a), 512, st, a, F32Split::kDqLds))) return s;
         const bool with_dsinks = last && a.dsinks;         // (every row's statistics are there)
         if (!a.split_partial && with_dsinks && (s = launch(attn_bwd_dsinks_kernel, a.H, 1024, st, a))) return s;
-        s = launch(attn_f32_split_dkdv_kernel, (int64_t)a.split_ng * a.split_nb * a.split_slots, 512, st, a, F32Split::kDkdvLds);
+        s = launch(lengths ? attn_f32_split_dkdv_kernel<true> : attn_f32_split_dkdv_kernel<false>, (int64_t)a.split_ng * a.split_nb * a.split_slots, 512, st, a, F32Split::kDkdvLds);
         if (s || !a.split_partial) return s;
         return launch_reduce(attn_f32_split_reduce_kernel, (int64_t)2 * a.split_nb * a.split_ng * a.Skv * 16, st, a, with_dsinks);
     });

@@ -104,7 +104,7 @@ def test_float32_dkdv_workgroups():
         records = up(4 * g * tiles) + g * tiles * 24576 + up(4 * h * tiles) + h * tiles * 24832
         if records > 256 << 20:
             continue
-        sums = g * best[1] * 65536 if best[1] > len(walks) else 0
+        sums = up(8 * g * len(walks)) + g * best[1] * 65536 if best[1] > len(walks) else 0      # (and where each block's stand)
         assert lib.gptoss_attn_split_bytes(ctypes.byref(_params(dtype=1, h=h, g=g, sq=s, skv=s, window=window)), 1) == records + sums, (h, g, s, window)
 
 

@@ -21,7 +21,7 @@ def _both(A, inp, window, seqlens=None, docs=None, start=0, backward=True):
     from oregon_gpt_oss_patching_amd import attention_kernel as ak
     q, k, v, sinks, d_out = (t.to(DEV) for t in inp)
     lens = None if seqlens is None else torch.tensor(seqlens, dtype=torch.int32, device=DEV)
-    ds = None if docs is None else E.doc_start_from_lengths([docs] * q.shape[0], q.shape[2]).to(DEV).to(torch.int32)
+    ds = docs.to(DEV) if torch.is_tensor(docs) else None if docs is None else E.doc_start_from_lengths([docs] * q.shape[0], q.shape[2]).to(DEV).to(torch.int32)
     p = ak._base_params(q, k, v, sinks, lens, SCALE, window, start, ds)
     o, lse = A.attention_forward(q, k, v, sinks, SCALE, window, start, lens, ds)
     o2, lse2 = torch.empty_like(o), torch.empty_like(lse)
@@ -154,9 +154,11 @@ def _alike(new, old):
         if name == "lse":
             assert bool(((x - y).abs() <= 2e-5 * (1 + y.abs())).all())
             continue
-        # 2e-5 of the row's and of the column's size, as everywhere; a row that is much smaller than most (its products cancel): of those
+        # 2e-5 of the row's and of the column's size, as everywhere; a row that is much smaller than most (its products cancel): of those (which are not
+        # the zeros of padding)
         rows, off = y.norm(dim=-1), (x - y).norm(dim=-1)
-        assert bool((off <= 2e-5 * (rows + rows.median())).all()), (name, float((off / (rows + rows.median())).max()))
+        most = rows[rows > 0].median()
+        assert bool((off <= 2e-5 * (rows + most)).all()), (name, float((off / (rows + most)).max()))
         y, off = (t.reshape(-1, 64).norm(dim=0) for t in (y, x - y))
         assert bool((off <= 2e-5 * y).all()), (name, float((off / y).max()))
 
@@ -243,3 +245,28 @@ def test_windows_behind_a_cache(A, sq, skv, w, start, on_device):
     # each no further from float64 than 2e-5 of the result (1.3e-6 at the most in test_chunks_behind_a_cache)
     assert float((new[0] - o).double().norm()) <= 2e-5 * float(o.double().norm())
     assert float((new[1] - lse).abs().max()) <= 2e-5
+
+
+@pytest.mark.parametrize("b,h,g,s,w,lens,docs", [
+    (1, 64, 8, 1030, None, None, [100] * 10 + [30]),
+    (1, 64, 8, 700, None, None, [1] * 700),                    # every walk a single pair of tiles
+    (1, 8, 1, 4100, None, None, [200] * 20 + [100]),           # many parts for few workgroups
+    (1, 8, 1, 9000, None, None, [3, 1500, 1, 1, 40, 4000, 128, 127, 3200]),      # more key blocks than lanes
+    (1, 8, 1, 4100, 500, None, [700, 1400, 2000]),
+    (2, 64, 8, 1024, None, [100, 150], None),
+    (9, 32, 4, 513, None, [513, 0, 1, 32, 33, 128, 129, 40, 200], None),         # one long row among short ones
+    (3, 8, 1, 2500, None, [2500, 1200, 7], [900, 900, 700]),
+    (1, 64, 8, 1030, None, None, "sliding"),                   # starts that move with the row
+])
+def test_walks_shortened_by_padding_and_documents(A, b, h, g, s, w, lens, docs):
+    """dK / dV of key blocks whose walks are divided on the device: every step once, in slots that are there."""
+    print(f"case B={b} H={h} G={g} S={s} W={w} lens={lens} docs={docs}", flush=True)
+    if docs == "sliding":
+        docs = (torch.arange(s) - 70).clamp(min=0).to(torch.int32).view(1, s).repeat(b, 1)
+    inp = list(E.make_inputs(8000 + s, b, h, g, s, 64, torch.float32))
+    if lens:
+        inp[4] = inp[4] * (torch.arange(s).view(1, s) < torch.tensor(lens).view(b, 1)).view(b, s, 1, 1)
+    new, old = _both(A, inp, w, lens, docs)
+    _alike(new, old)
+    again, _ = _both(A, inp, w, lens, docs)
+    assert all(torch.equal(x, y) for x, y in zip(new, again))
