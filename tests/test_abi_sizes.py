@@ -116,3 +116,10 @@ def test_float32_window_on_a_cache():
     assert size(448, 448 + 64, 128) == size(448, 480 + 32, 128) <= size(448, 2000, 128)
     assert size(256, 16384, 128) == size(320, 16384, 64) == size(576, 16384, 128) == 0
     assert size(576, 16384, 192) > 0 and size(320, 16384, 0) > size(320, 4096, 0) > 0
+
+
+def test_float32_shares_are_even():
+    """Three rows of 2000 tokens, nineteen of whose twenty-four KV heads fit: twelve and twelve, not two rows and one."""
+    lib = _lib.load()
+    size = lib.gptoss_attn_split_bytes(ctypes.byref(_params(1, 3, 64, 8, 2000, 2000)), 1)
+    assert 12 * 63 * (24576 + 8 * 24832) <= size < 12 * 63 * (24576 + 8 * 24832) + (65 << 20)

@@ -194,9 +194,10 @@ def test_row_statistics_that_three_terms_do_not_hold(A, which, value):
 
 @pytest.mark.parametrize("b,h,g,s,w,lens,docs", [
     (1, 64, 8, 5000, None, None, None),                        # four KV heads at a time
-    (10, 64, 8, 1056, None, [1056, 700, 1, 0, 1055, 32, 33, 900, 1024, 1056], None),     # four batch rows at a time, then two
+    (10, 64, 8, 1056, None, [1056, 700, 1, 0, 1055, 32, 33, 900, 1024, 1056], None),     # three KV heads of all rows at a time, then two
     (1, 28, 7, 15360, 500, None, None),                        # four KV heads, then three
-    (3, 64, 8, 1700, None, None, [1, 932, 767]),               # two batch rows, then one
+    (3, 64, 8, 1700, None, None, [1, 932, 767]),               # four KV heads of all rows at a time
+    (8, 16, 2, 5000, 500, [5000, 3, 4999, 0, 2500, 5000, 4000, 33], None),      # three batch rows at a time, then two
 ])
 def test_some_rows_and_heads_at_a_time(A, b, h, g, s, w, lens, docs):
     """Calls whose records do not fit the scratch at once give what the fp32 instruction gives, and forward and dQ what each batch row gives by itself."""
