@@ -20,8 +20,10 @@ def _takes_pieces(b, h, g, s, lens, docs):
     p.B, p.H, p.G, p.Sq, p.Skv, p.D, p.scale = b, h, g, s, s, 64, 0.125
     p.seqlens, p.doc_start = 256 if lens else None, 256 if docs else None
     blocks = b * g * -(-s // 128)
-    room = _lib.load().gptoss_attn_bwd_workspace_bytes(ctypes.byref(p)) > 24 * b * h * s + 16
-    return room and (blocks > 512 or s >= 2048) and bool(lens or docs or (b > 1 and s < 4096 and blocks > 512))
+    parts = (_lib.load().gptoss_attn_bwd_workspace_bytes(ctypes.byref(p)) - 24 * b * h * s) // (512 * b * g * s)
+    if docs and not lens and h // g <= 4 and b * g * -(-s // 256) * parts <= 256:
+        return False                                           # (equal shares that run all at once)
+    return parts > 1 and (blocks > 512 or s >= 2048) and bool(lens or docs or (b > 1 and s < 4096 and blocks > 512))
 
 
 @pytest.mark.parametrize("b,h,g,s,lens,docs", [
@@ -49,3 +51,9 @@ def test_too_many_rows_for_pieces(A):
 def test_several_rows_of_one_length(A, b, h, g, s):
     assert _takes_pieces(b, h, g, s, None, None)
     _check(A, b, h, g, s, None, None)
+
+
+@pytest.mark.parametrize("b,h,g,s,docs", [(1, 8, 2, 2300, [1, 1, 2040, 2, 256]), (1, 16, 4, 2048, [300] * 6 + [248]), (2, 8, 2, 2048, [100] * 20 + [48])])
+def test_packed_rows_of_few_heads_in_equal_shares(A, b, h, g, s, docs):
+    assert not _takes_pieces(b, h, g, s, None, docs)
+    _check(A, b, h, g, s, None, docs)
