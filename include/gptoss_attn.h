@@ -59,7 +59,8 @@ extern "C" {
 enum gptoss_attn_dtype {
     GPTOSS_ATTN_BF16 = 0, /* 2-byte bfloat16 tensors, bf16 MFMA products, fp32 accumulation: the fast path */
     GPTOSS_ATTN_FP32 = 1  /* 4-byte float tensors, fp32 MFMA products (the reference's fp32 mode,
-                             attention_kernel.py is dtype-generic), at a sixteenth of the bf16 matrix rate */
+                             attention_kernel.py is dtype-generic), at a sixteenth of the bf16 matrix rate;
+                             larger calls with scratch: gptoss_attn_split_bytes */
 };
 
 enum gptoss_attn_status {

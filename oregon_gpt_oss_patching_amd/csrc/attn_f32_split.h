@@ -24,8 +24,8 @@
 // barrier per step.  Where the records of all batch rows and KV heads would take too much memory, the launches are repeated for some of them
 // at a time, over the same scratch (f32_split_plan).
 //
-// What bounds it (S = 1024, 64 query heads on 8 KV heads, full causal; fp32 instruction / this): forward 101 / 61 us, dQ 134 / 85, dK/dV
-// 176 / 95, the whole call 413 / 259; S = 4096 5350 / 3280.  The matrix pipes are busy 43, 46 and 55 % of the cycles: about eight
+// What bounds it (S = 1024, 64 query heads on 8 KV heads, full causal; fp32 instruction / this): forward 101 / 58 us, dQ 134 / 83, dK/dV
+// 176 / 94, the whole call 413 / 270; S = 4096 5320 / 3120.  The matrix pipes are busy 42, 45 and 53 % of the cycles: about eight
 // vector instructions per MFMA in the forward (cutting the weights is 88 of a tile's 290), and the two wavefronts of a SIMD start each step together.
 // Error against float64 (relative 2-norm, S = 1024, fp32 instruction / this), N(0, 1): O 3.0e-7 / 1.3e-7, lse 4.8e-8 / 4.8e-8, dQ 4.4e-7 / 3.4e-7, dK
 // 6.0e-7 / 5.1e-7, dV 5.9e-7 / 5.1e-7; all operands in [1, 1 + 2^-7], where dP - delta cancels: dQ 2.2e-3 / 2.1e-3, dK 1.24e-5 / 1.15e-5; powers of two

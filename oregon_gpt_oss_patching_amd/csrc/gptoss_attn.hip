@@ -302,7 +302,8 @@ int64_t f32_grid(const KArgs &a, int ks) {
 // dQ of operands next to a bf16 number was 1.09 times as far from float64 as with the fp32 instruction alone).  fp32 instruction / this, us in a graph, 64 query heads on 8 KV heads,
 // forward and backward: 320 rows 23 + 82 / 25 + 70, 448 33 + 110 / 31 + 80, 1024 100 + 310 / 66 + 200, 4096 5320 / 3120; 8 heads on one KV head 2048 rows (128 workgroups)
 // 63 + 249 / 79 + 165; a window is a handful of tiles per workgroup, whose start and end then decide: of 128, 320 rows 22 + 88 / 21 + 63, 640 33 + 103 / 35 + 91, 800 (400 workgroups)
-// 36 + 107 / 39 + 102, 1024 147 / 150; of 383, 800 63 + 220 / 50 + 136; of 64, 448 21 + 69 / 20 + 61, but 640 26 + 74 / 33 + 83.
+// 36 + 107 / 39 + 102, 1024 147 / 150; of 383, 800 63 + 220 / 50 + 136; of 64, 448 21 + 69 / 20 + 61, but 640 26 + 74 / 33 + 83
+// (windows below 96 would rather have the line at 256 workgroups).
 // Queries on a cache, forward: 256 (128 workgroups) on 2048 80 / 84, on 4096 154 / 154, on 16384 600 / 566; 320 on 1024 59 / 48, 1024 on 8192 1121 / 647; with a window of 128, 320 on
 // 16384 23 / 21, 448 26 / 22, 576 34 / 36, 256 (128 workgroups) 15 / 21; of 64, 320 17 / 19, 448 21 / 20; of 192, 576 43 / 41; of 400, 800 76 / 56.
 bool f32_split_route(const gptoss_attn_params *p, bool bwd) {
@@ -875,7 +876,8 @@ int gptoss_attn_bwd_dq(const gptoss_attn_params *p, void *stream) { return launc
 
 // The whole backward: the dQ kernel computes the row statistics on the way (no separate
 // pass over O and dO), then dK/dV and dSinks read them from the scratch buffer.  The results are
-// bit-identical to gptoss_attn_bwd_preprocess + gptoss_attn_bwd_dkdv + gptoss_attn_bwd_dq.
+// bit-identical to gptoss_attn_bwd_preprocess + gptoss_attn_bwd_dkdv + gptoss_attn_bwd_dq, but for the two routes in front: float32 with
+// scratch (attn_f32_split.h) and the single-pass window kernel agree with these within the rounding of their sums.
 static int bwd_all(const gptoss_attn_params *p, void *stream, bool whole_blocks, SinkTypes ty, void *scratch = nullptr, size_t scratch_bytes = 0) {
     int rc = gptoss_attn_validate(p, 1);
     if (rc) return rc;
