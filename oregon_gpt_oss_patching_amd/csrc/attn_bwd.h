@@ -106,33 +106,6 @@ __global__ __launch_bounds__(1024) void attn_bwd_dsinks_kernel(const KArgs a) {
     dsinks_of_head<1024>(a, blockIdx.x, red);
 }
 
-// ---------------------------------------------------------------------------------
-// dS exchange through LDS (fused backward).  The dS tile is key-major: key row r of the
-// workgroup occupies 128 bytes (64 query-row columns in bf16), chunk-swizzled by swz(r).
-// A lane of an owner wavefront (key row r, half = lane / 32) holds, per 16-row step u of the
-// 32-row block qb, the B fragment dsf: elements 0..3 are rows 16u + 4*half + 0..3, elements 4..7
-// rows 16u + 8 + 4*half + 0..3, i.e. two 8-byte pieces in the logical chunks 4*qb + 2*u and
-// 4*qb + 2*u + 1 of its key row, at byte 8*half of the chunk.  With the row's swizzle folded into
-// the base address the chunk selection is one XOR with an immediate.
-__device__ __forceinline__ uint32_t ds_store_addr(uint32_t tile, int keyrow, int half) {
-    return tile + keyrow * kRowBytes + (swz(keyrow) << 4) + 8 * half;
-}
-__device__ __forceinline__ void ds_store(uint32_t base, int qb, int u, const bf16x8 dsf) {
-    typedef __attribute__((address_space(3))) bf16x4 lds_bf16x4;
-    bf16x4 p0, p1;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) { p0[e] = dsf[e]; p1[e] = dsf[4 + e]; }
-    *reinterpret_cast<lds_bf16x4 *>((uintptr_t)(base ^ ((4 * qb + 2 * u) << 4))) = p0;
-    *reinterpret_cast<lds_bf16x4 *>((uintptr_t)(base ^ ((4 * qb + 2 * u + 1) << 4))) = p1;
-}
-__device__ __forceinline__ void ds_store_zero(uint32_t base, int qb) {
-    bf16x8 z;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) z[e] = (bf16)0.0f;
-    ds_store(base, qb, 0, z);
-    ds_store(base, qb, 1, z);
-}
-
 // ---- MFMAs whose accumulator lives in the AGPR half of the register file -----------------------------
 // A kernel that runs one wavefront per SIMD has 512 registers per lane, 256 of them AGPRs, which only
 // MFMAs (and copies) can touch.  The compiler keeps all MFMA results of a kernel in one kind of register;
@@ -177,40 +150,17 @@ __device__ __forceinline__ void agpr_accumulators_settled(f32x16 (&dk)[2][2], f3
 // lane's key), or a huge negative number for a dead key, so that pair (row r, key)
 // is visible iff 0 <= dbase + r < weff, tested with one unsigned compare; rows at
 // or beyond `row_lim` (relative to the tile) do not exist.
-// STORE_DS (needs NB == 1): the bf16 dS values of the tile are also written to LDS, key-major: the
-// lane's key row starts at ds_out (which already holds the row's swizzle, see ds_store_addr), one
-// 128-byte row of 64 query-row columns per key, 16-byte chunks XOR-swizzled like every staged
-// tile.  A 32-row block that is skipped stores zeros.  The wavefronts that form dQ read it back
-// with the transposing fragment reads.
-// SPLIT: the row statistics are staged in the split form (split_row_stats) and enter through one more
-// step of the S and dP contractions; stat_lane then addresses the 16 bytes of row l32 of block 0.
-template <bool MASKED, bool DOCS, int NB, bool STORE_DS = false, bool SPLIT = false>
+// The row statistics are staged in the split form (split_row_stats) and enter through one more
+// step of the S and dP contractions; stat_lane addresses the 16 bytes of row l32 of block 0.
+template <bool MASKED, bool DOCS, int NB>
 __device__ __forceinline__ void dkdv_tile(uint32_t qsm, uint32_t gsm, uint32_t stat_lane, const TileLaneOffsets &lo,
                                           const bf16x8 (&kf)[NB][4], const bf16x8 (&vf)[NB][4],
                                           f32x16 (&dk)[NB][2], f32x16 (&dv)[NB][2], float c, int half,
                                           const int (&dbase)[NB], unsigned weff, int row_lim, int krel,
-                                          uint32_t ds_lane, const int (&jkey)[NB], uint32_t ds_out = 0) {
-    static_assert(!STORE_DS || NB == 1, "the dS store is written for one 32-key block per wavefront");
-    // masked variant, per lane and tile: pair (row r, key) is visible iff 0 <= dbase + r < weff and
-    // r < row_lim.  With r = rc + 4*half (rc a compile-time constant per accumulator register) that is
-    // (unsigned)(dbh + rc) < width with dbh = dbase + 4*half, width = max(0, min(weff, dbh + row_lim - 4*half)):
-    // one add, one compare, one select per element.  Used by the single-pass window kernel, where
-    // two tiles out of three are masked (window layer, S = 16384: -6 %); the dK/dV kernel, whose
-    // masked tiles are the few on the diagonal of a full-causal layer, keeps the plain form (the
-    // folded one costs it 17 registers and 4 % on that layer).
-    int dbh[NB];
-    unsigned width[NB];
-    if (MASKED && STORE_DS) {
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-            dbh[nb] = dbase[nb] + 4 * half;
-            width[nb] = (unsigned)max(0, min((int)weff, dbh[nb] + max(row_lim, -8) - 4 * half));
-        }
-    }
+                                          uint32_t ds_lane, const int (&jkey)[NB]) {
     bf16x8 b_stat_s, b_stat_dp;
-    if constexpr (SPLIT) stat_step_operands(half, b_stat_s, b_stat_dp);
-    // qsm / gsm: LDS byte addresses of the staged Q and dO tiles; stat_lane (not SPLIT): address of this
-    // lane's first lse2 value (rows 4*half..), -delta sits kTile floats further on.
+    stat_step_operands(half, b_stat_s, b_stat_dp);
+    // qsm / gsm: LDS byte addresses of the staged Q and dO tiles.
     // DOCS (packed rows): ds_lane addresses the staged document starts of the same rows, jkey
     // is the lane's key index; a key before its query's document start is invisible.
     // krel (masked variant only): (first key of the wavefront) - (first query position of the
@@ -219,30 +169,17 @@ __device__ __forceinline__ void dkdv_tile(uint32_t qsm, uint32_t gsm, uint32_t s
 #pragma unroll
     for (int qb = 0; qb < 2; ++qb) {
         if (MASKED && ((32 * qb + 31 < krel) || (32 * qb > krel + 32 * NB - 1 + (int)weff - 1) || (32 * qb >= row_lim))) {
-            if constexpr (STORE_DS) ds_store_zero(ds_out, qb);
             continue;
         }
         f32x16 s[NB], dp[NB];
-        if constexpr (SPLIT) {
-            // the statistics step: S starts at -lse / scale, dP at -delta of the rows
-            const bf16x8 a_stat = as_bf16x8(lds_load128(stat_lane, 32 * qb * 16));
+        // the statistics step: S starts at -lse / scale, dP at -delta of the rows
+        const bf16x8 a_stat = as_bf16x8(lds_load128(stat_lane, 32 * qb * 16));
 #pragma unroll
-            for (int nb = 0; nb < NB; ++nb) {
+        for (int nb = 0; nb < NB; ++nb) {
 #pragma unroll
-                for (int i = 0; i < 16; ++i) { s[nb][i] = 0.0f; dp[nb][i] = 0.0f; }
-                s[nb] = mfma_bf16(a_stat, b_stat_s, s[nb]);
-                dp[nb] = mfma_bf16(a_stat, b_stat_dp, dp[nb]);
-            }
-        } else {
-            // the dP accumulators start at -delta of their rows, so the MFMAs deliver dP - delta
-#pragma unroll
-            for (int a4 = 0; a4 < 4; ++a4) {
-                const f32x4 nd = lds_load128f(stat_lane, (kTile + 32 * qb + 8 * a4) * 4);
-#pragma unroll
-                for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) { s[nb][4 * a4 + e] = 0.0f; dp[nb][4 * a4 + e] = nd[e]; }
-            }
+            for (int i = 0; i < 16; ++i) { s[nb][i] = 0.0f; dp[nb][i] = 0.0f; }
+            s[nb] = mfma_bf16(a_stat, b_stat_s, s[nb]);
+            dp[nb] = mfma_bf16(a_stat, b_stat_dp, dp[nb]);
         }
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
@@ -256,8 +193,6 @@ __device__ __forceinline__ void dkdv_tile(uint32_t qsm, uint32_t gsm, uint32_t s
         }
 #pragma unroll
         for (int a4 = 0; a4 < 4; ++a4) {
-            f32x4 lv = {0.0f, 0.0f, 0.0f, 0.0f};
-            if constexpr (!SPLIT) lv = lds_load128f(stat_lane, (32 * qb + 8 * a4) * 4);
             u32x4 dsr = {0u, 0u, 0u, 0u};
             if (MASKED && DOCS) dsr = lds_load128(ds_lane, (32 * qb + 8 * a4) * 4);
 #pragma unroll
@@ -265,15 +200,10 @@ __device__ __forceinline__ void dkdv_tile(uint32_t qsm, uint32_t gsm, uint32_t s
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const int i = 4 * a4 + e;
-                    float pe = fast_exp2(SPLIT ? s[nb][i] * c : fmaf(s[nb][i], c, -lv[e]));
+                    float pe = fast_exp2(s[nb][i] * c);
                     if (MASKED) {
-                        bool vis;
-                        if constexpr (STORE_DS) {
-                            vis = (unsigned)(dbh[nb] + (32 * qb + 8 * a4 + e)) < width[nb];
-                        } else {
-                            const int r = 32 * qb + 8 * a4 + 4 * half + e;
-                            vis = ((unsigned)(dbase[nb] + r) < weff) & (r < row_lim);
-                        }
+                        const int r = 32 * qb + 8 * a4 + 4 * half + e;
+                        bool vis = ((unsigned)(dbase[nb] + r) < weff) & (r < row_lim);
                         if (DOCS) vis = vis & (jkey[nb] >= (int)dsr[e]);
                         pe = vis ? pe : 0.0f;
                     }
@@ -292,7 +222,6 @@ __device__ __forceinline__ void dkdv_tile(uint32_t qsm, uint32_t gsm, uint32_t s
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb) {
                 const bf16x8 pf = cfrag(s[nb], u), dsf = cfrag(dp[nb], u);
-                if constexpr (STORE_DS) ds_store(ds_out, qb, u, dsf);
 #pragma unroll
                 for (int dblk = 0; dblk < 2; ++dblk) {
                     dv[nb][dblk] = mfma_bf16(agt[dblk], pf, dv[nb][dblk]);
@@ -514,7 +443,7 @@ __global__ __launch_bounds__(NW * 64, (NB == 1 ? 2 : 1)) void attn_bwd_dkdv_kern
         }
         if (skip) return;
         if (interior) {
-            dkdv_tile<false, false, NB, false, true>(qsm, gsm, stat_lane, lo, kf, vf, dk, dv, c, half, dead, 0u, 0, 0, 0u, jkey);
+            dkdv_tile<false, false, NB>(qsm, gsm, stat_lane, lo, kf, vf, dk, dv, c, half, dead, 0u, 0, 0, 0u, jkey);
         } else {
             int dbase[NB];
 #pragma unroll
@@ -523,7 +452,7 @@ __global__ __launch_bounds__(NW * 64, (NB == 1 ? 2 : 1)) void attn_bwd_dkdv_kern
                 dbase[nb] = (j < kv_len) ? pos0 - j : -0x40000000;
             }
             const int row_lim = (int)min((int64_t)kTile, min((int64_t)a.Sq, (int64_t)q_len - q_offset) - i0);
-            dkdv_tile<true, DOCS, NB, false, true>(qsm, gsm, stat_lane, lo, kf, vf, dk, dv, c, half, dbase, (unsigned)weff, row_lim,
+            dkdv_tile<true, DOCS, NB>(qsm, gsm, stat_lane, lo, kf, vf, dk, dv, c, half, dbase, (unsigned)weff, row_lim,
                                       wj0 - pos0, ds_lane, jkey);
         }
     };

@@ -59,9 +59,9 @@ struct KArgs {
     int dkdv_steps;      // > 0: attn_bwd_dkdv_kernel cuts its walks into pieces of so many (query tile, head) steps (DkdvPieces), dkdv_slots of them per batch row and KV head
     int kv_splits;       // forward: workgroups that share one query block, each taking a slice of its keys
     float *fwd_partial;  // kv_splits > 1: fp32 partial results of the slices
-    int chunk_tiles;     // single-pass window backward: 64-row query tiles per workgroup
-    float *dsink_partial; // single-pass window backward: dSinks partial sums, [B][chunk][H][2]
-    float *boundary_partial; // single-pass window backward: fp32 dK / dV shares of the tiles on chunk seams, or NULL
+    int chunk_blocks;    // single-pass window backward: 32-row query blocks per workgroup
+    float *dsink_partial; // single-pass window backward: dSinks partial sums, [B][chunk][H]
+    float *boundary_partial; // single-pass window backward: fp32 dK / dV shares of the blocks on chunk seams, or NULL
     bool sinks_bf16, dsinks_bf16;
     // float32 on the bf16 matrix pipes (attn_f32_split.h): records of K / V and of Q / dO, which of them hold numbers the split does
     // not take, steps per dK/dV workgroup, parts of all key blocks of a row, their partial sums (or NULL)

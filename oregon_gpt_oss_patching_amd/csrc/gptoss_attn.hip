@@ -89,7 +89,7 @@ KArgs make_args(const gptoss_attn_params *p, SinkTypes ty) {
     a.dkdv_steps = 0;
     a.kv_splits = 1;
     a.fwd_partial = nullptr;
-    a.chunk_tiles = 0;
+    a.chunk_blocks = 0;
     a.dsink_partial = nullptr;
     a.boundary_partial = nullptr;
     a.split_kv = a.split_q = nullptr;
@@ -467,19 +467,18 @@ int compute_units() {
     return n;
 }
 
-// Query tiles per workgroup, 2 to 16: the count whose rounds of workgroups (one per compute unit at a time) take the least time,
-// a workgroup's own start counted as a quarter of a tile; of equals the larger (fewer seams).
-// (An equal share per compute unit, rounded down, left 2 x 3001 tokens of 8 KV heads with 384 workgroups of two tiles, two rounds
-// of which the second is half empty; 256 of three: window layer 146 -> 124 us, 5 x 2100 tokens 250 -> 210, 32 heads 2 x 3001 107 -> 87.)
-int window_chunk_tiles(const gptoss_attn_params *p, int cus) {
-    const int64_t n_tiles = (p->Sq + kTile - 1) / kTile, rows = (int64_t)p->G * p->B;
+// Query blocks per workgroup, 4 to 32: the count whose rounds of workgroups (one per compute unit at a time) take the least time,
+// a workgroup's own start counted as four steps; of equals the larger (fewer seams).
+int window_chunk_blocks(const gptoss_attn_params *p, int cus) {
+    const int64_t n_blocks = (p->Sq + WinCfg::kRows - 1) / WinCfg::kRows, rows = (int64_t)p->G * p->B;
+    const int pairs = (p->H / p->G + 1) / 2;
     if (cus <= 0) cus = 256;
-    int best = 2;
+    int best = WinCfg::kBack;
     int64_t best_cost = 0;
-    for (int c = 2; c <= 16; ++c) {
-        const int64_t rounds = (rows * ((n_tiles + c - 1) / c) + cus - 1) / cus, cost = rounds * (4 * c + 1);
-        if (c == 2 || cost <= best_cost) { best = c; best_cost = cost; }
-        if (c >= n_tiles) break;
+    for (int c = WinCfg::kBack; c <= 32; ++c) {
+        const int64_t rounds = (rows * ((n_blocks + c - 1) / c) + cus - 1) / cus, cost = rounds * (pairs * c + 4);
+        if (c == WinCfg::kBack || cost <= best_cost) { best = c; best_cost = cost; }
+        if (c >= n_blocks) break;
     }
     return best;
 }
@@ -500,37 +499,37 @@ int lds_attribute(int bytes) {
     return GPTOSS_ATTN_OK;
 }
 
-// Scratch of the single-pass window backward: dSinks partial sums [B][chunk][H][2], then (rounded up
-// to 16 bytes) the fp32 dK / dV shares of the two key tiles on each seam between chunks.
-struct WindowScratch { int chunk_tiles, n_chunks; size_t sink_bytes, seam_bytes; };
+// Scratch of the single-pass window backward: dSinks partial sums [B][chunk][H] (room for two words each: the size that callers have known), then (rounded up
+// to 16 bytes) the fp32 dK / dV shares of the four key blocks on each seam between chunks.
+struct WindowScratch { int chunk_blocks, n_chunks; size_t sink_bytes, seam_bytes; };
 
-WindowScratch window_scratch_for(const gptoss_attn_params *p, int chunk_tiles) {
+WindowScratch window_scratch_for(const gptoss_attn_params *p, int chunk_blocks) {
     WindowScratch w;
-    w.chunk_tiles = chunk_tiles;
-    const int n_tiles = (p->Sq + kTile - 1) / kTile;
-    w.n_chunks = (n_tiles + w.chunk_tiles - 1) / w.chunk_tiles;
-    w.sink_bytes = (((size_t)p->B * w.n_chunks * p->H * WinCfg::NHELP * sizeof(float)) + 15) & ~(size_t)15;
-    w.seam_bytes = (size_t)p->B * p->G * (w.n_chunks - 1) * 2 * 2 * (2 * kTile * kD) * sizeof(float);
+    w.chunk_blocks = chunk_blocks;
+    const int n_blocks = (p->Sq + WinCfg::kRows - 1) / WinCfg::kRows;
+    w.n_chunks = (n_blocks + w.chunk_blocks - 1) / w.chunk_blocks;
+    w.sink_bytes = (((size_t)p->B * w.n_chunks * p->H * 2 * sizeof(float)) + 15) & ~(size_t)15;
+    w.seam_bytes = (size_t)p->B * p->G * (w.n_chunks - 1) * WinCfg::kBack * 2 * (2 * WinCfg::kRows * kD) * sizeof(float);
     return w;
 }
 
-WindowScratch window_scratch(const gptoss_attn_params *p, int cus) { return window_scratch_for(p, window_chunk_tiles(p, cus)); }
+WindowScratch window_scratch(const gptoss_attn_params *p, int cus) { return window_scratch_for(p, window_chunk_blocks(p, cus)); }
 
 // seam_sums: neighbouring chunks exchange fp32 shares through the scratch (needs window_scratch bytes);
-// otherwise each chunk walks two query tiles past its end and nothing but the dSinks sums is kept.
+// otherwise each chunk walks four query blocks past its end and nothing but the dSinks sums is kept.
 int launch_window_bwd(const gptoss_attn_params *p, hipStream_t st, bool seam_sums, SinkTypes ty) {
     int rc = lds_attribute<&attn_bwd_window_kernel>(WinCfg::kLdsBytes);
     if (rc) return rc;
     KArgs a = make_args(p, ty);
     const WindowScratch ws = window_scratch(p, compute_units());
-    a.chunk_tiles = ws.chunk_tiles;
+    a.chunk_blocks = ws.chunk_blocks;
     a.dsink_partial = p->delta;
     if (seam_sums && ws.n_chunks > 1)
         a.boundary_partial = reinterpret_cast<float *>(reinterpret_cast<char *>(p->delta) + ws.sink_bytes);
     rc = launch(attn_bwd_window_kernel, (int64_t)a.G * a.B * ws.n_chunks, 64 * WinCfg::NWAVES, st, a, WinCfg::kLdsBytes);
     if (rc) return rc;
-    // seam tiles and dSinks in one small launch
-    const int64_t seam_chunks = a.boundary_partial ? (int64_t)a.B * a.G * (ws.n_chunks - 1) * 2 * 2 * kTile * 8 : 0;
+    // seam blocks and dSinks in one small launch
+    const int64_t seam_chunks = a.boundary_partial ? (int64_t)a.B * a.G * (ws.n_chunks - 1) * WinCfg::kBack * 2 * WinCfg::kRows * 8 : 0;
     const int seam_blocks = (int)((seam_chunks + 255) / 256);
     const int sink_blocks = a.dsinks ? a.H : 0;
     if (seam_blocks + sink_blocks == 0) return GPTOSS_ATTN_OK;
@@ -684,7 +683,7 @@ static size_t bwd_bytes(const gptoss_attn_params *p, int parts) {
             // gptoss_attn_bwd takes this route and lays its own scratch over the same bytes.  The layout
             // follows the compute-unit count of the device that is current at launch time; the size
             // returned is that of the shortest chunks (the most seams), which covers every device.
-            const WindowScratch ws = window_scratch_for(p, 2);
+            const WindowScratch ws = window_scratch_for(p, WinCfg::kBack);
             if (ws.sink_bytes + ws.seam_bytes > n) n = ws.sink_bytes + ws.seam_bytes;
         }
     }
