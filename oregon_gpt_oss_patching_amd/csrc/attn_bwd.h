@@ -7,6 +7,7 @@
 //                           and walks every (query head of the group, query
 //                           tile) that can see them                      (:199-212)
 //   attn_bwd_dq_kernel      Q-outer, same shape as the forward kernel    (:206-217)
+//   attn_bwd_both_kernel    the last two in one launch, for small problems
 #pragma once
 #include <type_traits>
 
@@ -269,8 +270,8 @@ struct DkdvPieces {
 };
 
 // NB = 32-key blocks per wavefront; DOCS = packed rows (doc_start given); PIECES: DkdvPieces (an instantiation: the slices' one is 4 % slower with both)
-template <int NW, int NB, bool DOCS, bool PIECES = false>
-__global__ __launch_bounds__(NW * 64, (NB == 1 ? 2 : 1)) void attn_bwd_dkdv_kernel(const KArgs a) {
+template <int NW, int NB, bool DOCS, bool PIECES>
+__device__ __forceinline__ void dkdv_workgroup(const KArgs &a, int bid) {
     const int q_offset = query_offset(a);
     static_assert(NW == 4, "the asynchronous tile copy is written for 4 wavefronts");
     constexpr int NS = 3;              // LDS stages: tiles are requested two iterations ahead
@@ -283,7 +284,6 @@ __global__ __launch_bounds__(NW * 64, (NB == 1 ? 2 : 1)) void attn_bwd_dkdv_kern
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int l32 = lane & 31, half = lane >> 5;
 
-    int bid = blockIdx.x;
     const int g = bid % a.G; bid /= a.G;
     const int bi = bid % a.B; bid /= a.B;
     int part, kt;
@@ -520,6 +520,9 @@ __global__ __launch_bounds__(NW * 64, (NB == 1 ? 2 : 1)) void attn_bwd_dkdv_kern
     }
 }
 
+template <int NW, int NB, bool DOCS, bool PIECES = false>
+__global__ __launch_bounds__(NW * 64, (NB == 1 ? 2 : 1)) void attn_bwd_dkdv_kernel(const KArgs a) { dkdv_workgroup<NW, NB, DOCS, PIECES>(a, blockIdx.x); }
+
 // ---------------------------------------------------------------------------------
 // Sum of the dK / dV partials of a split key block, in part order (bit-reproducible), scaled and
 // rounded to the output type.  One thread per 16-byte output chunk: (tensor, b, g, key, 8 columns).
@@ -673,7 +676,7 @@ __device__ __forceinline__ void dq_tile(uint32_t ksm, uint32_t vsm, const TileLa
 }
 
 template <int HPB, int NQB, bool FUSE_DELTA>   // FUSE_DELTA: also produce the row statistics of the wavefront's own rows
-__global__ __launch_bounds__(256, (NQB == 1 ? 3 : 2)) void attn_bwd_dq_kernel(const KArgs a) {
+__device__ __forceinline__ void dq_workgroup(const KArgs &a, int bid) {
     const int q_offset = query_offset(a);
     constexpr int QSUB = 4 / HPB;
     constexpr int WM = 32 * NQB;
@@ -690,7 +693,6 @@ __global__ __launch_bounds__(256, (NQB == 1 ? 3 : 2)) void attn_bwd_dq_kernel(co
     auto fresh_lane = []() __attribute__((always_inline)) { return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)); };
 
     const int n_hc = (a.r + HPB - 1) / HPB;
-    int bid = blockIdx.x;
     const int g = bid % a.G; bid /= a.G;
     const int hc = bid % n_hc; bid /= n_hc;
     const int bi = bid % a.B; bid /= a.B;
@@ -865,6 +867,18 @@ __global__ __launch_bounds__(256, (NQB == 1 ? 3 : 2)) void attn_bwd_dq_kernel(co
             __builtin_amdgcn_wave_barrier();
         }
     }
+}
+
+template <int HPB, int NQB, bool FUSE_DELTA>
+__global__ __launch_bounds__(256, (NQB == 1 ? 3 : 2)) void attn_bwd_dq_kernel(const KArgs a) { dq_workgroup<HPB, NQB, FUSE_DELTA>(a, blockIdx.x); }
+
+// dQ and dK/dV side by side: the first workgroups are attn_bwd_dkdv_kernel's, the others attn_bwd_dq_kernel's (32-row wavefronts), with the same bits.  Either alone is a
+// chain of latencies, 7 us and 1.1 to 1.9 per (query tile, head) or key tile of its longest walk, which leaves most of a compute unit idle; the row statistics, which dQ forms on
+// its way for the dK/dV kernel otherwise, come from attn_bwd_delta_kernel here (4 us).  Taken where everything fits the chip at once (both_route).
+template <bool DOCS, bool PIECES>
+__global__ __launch_bounds__(256, 2) void attn_bwd_both_kernel(const KArgs a, int dkdv_workgroups) {
+    if ((int)blockIdx.x < dkdv_workgroups) dkdv_workgroup<4, 1, DOCS, PIECES>(a, blockIdx.x);
+    else dq_workgroup<4, 1, false>(a, blockIdx.x - dkdv_workgroups);
 }
 
 }  // namespace gptoss

@@ -194,6 +194,30 @@ void dkdv_pieces_for(const gptoss_attn_params *p, KArgs &a) {
     }
 }
 
+// workgroups of the forward / dQ launch: (KV head, chunk of HPB query heads, batch, query tile)
+int64_t q_outer_grid(const KArgs &a, int hpb, int qb) {
+    const int bm = 32 * qb * (4 / hpb);
+    const int n_hc = (a.r + hpb - 1) / hpb;
+    return (int64_t)a.G * n_hc * a.B * ((a.Sq + bm - 1) / bm);
+}
+// Workgroups of attn_bwd_dkdv_kernel.
+int64_t dkdv_grid(const KArgs &a) {
+    return (int64_t)a.G * a.B * (a.dkdv_steps ? a.dkdv_slots : a.dkdv_parts * ((a.Skv + kDkdvKeys - 1) / kDkdvKeys));
+}
+bool window_single_pass(const gptoss_attn_params *p);
+// dQ and dK/dV in one launch (attn_bwd_both_kernel) behind one for the row statistics, instead of one after the other: where their workgroups, two to a compute
+// unit of a 256-CU part, are few enough to run side by side.  `a` has the backward's dkdv_parts; gets its pieces.  Whole backward, us in a graph, one after the
+// other / side by side (workgroups): 8 heads on one KV head 300 tokens 34 / 27 (29), 1300 70 / 47 (161), 2000 96 / 63 (248), 2 x 1500 78 / 56 (368), 4 x 1000 61 / 53 (500),
+// 4 x 2000 114 / 119 (992); 8 on two 2 x 1500 74 / 67 (500), 4 x 1000 58 / 56 (744); 32 on four 700 49 / 34 (320), 1500 90 / 79 (736), 2000 114 / 118 (992); 64 on eight 256 30 / 27
+// (192), 512 37 / 36 (480), 2 x 383 41.7 / 41.3 (656), 768 53.4 / 53.3 (720), 1024 66 / 78 (1000): two full rounds, of which the second holds the longest walks.  Against the
+// 64-key kernel (2048 tokens and more) and for padded and packed rows the line is lower: 8 heads on one 2500 tokens 137 / 77 (318), 4000 169 / 111 (506), padded
+// 2 x 2500 131 / 111 (636), padded 2 x 3000 147 / 148 (760); on two 2500 110 / 94 (478), 4000 131 / 147 (762), in three documents 89 / 93.
+bool both_route(const gptoss_attn_params *p, KArgs &a) {
+    if (p->dtype != GPTOSS_ATTN_BF16 || a.r < 4 || window_single_pass(p)) return false;
+    dkdv_pieces_for(p, a);
+    return q_outer_grid(a, 4, 1) + dkdv_grid(a) <= (p->Skv >= 2048 || p->seqlens || p->doc_start ? 640 : 768);
+}
+
 // Full-causal self-attention goes to attn_bwd_dkdv64_kernel (64 keys per wavefront, one wavefront per SIMD)
 // when the shape is the one it is written for (bf16, no window, no offset, Sq == Skv; right-padded batch rows and packed
 // documents are fine) and there is enough of it: more than
@@ -202,7 +226,7 @@ void dkdv_pieces_for(const gptoss_attn_params *p, KArgs &a) {
 // 32-key kernel would get, so the scratch is the same; -15 % at S = 2048 ... 8192).
 // (The kernel walks Q, dO and the row statistics of one KV head's group of query heads with 32-bit byte
 // offsets from the group's first row: head strides must not be negative and the group's span must stay
-// below 2^31 bytes; anything else takes the 32-key kernel.)
+// below 2^31 bytes; anything else takes the 32-key kernel, and so does what fits both_route.)
 bool walk_fits_32_bits(const gptoss_attn_strides &s, int64_t heads, int64_t rows) {
     return s.h >= 0 && ((heads - 1) * s.h + rows * s.s) * 2 < ((int64_t)1 << 31);
 }
@@ -212,6 +236,11 @@ bool dkdv64_route(const gptoss_attn_params *p, int parts) {
     if (!walk_fits_32_bits(p->q_stride, heads, p->Sq) || !walk_fits_32_bits(p->do_stride, heads, p->Sq) ||
         heads * p->Sq * 16 >= ((int64_t)1 << 31))
         return false;
+    if (parts > 1) {
+        KArgs a = make_args(p, {});
+        a.dkdv_parts = parts;
+        if (both_route(p, a)) return false;
+    }
     return p->dtype == GPTOSS_ATTN_BF16 && effective_window(p) == 0 && p->q_offset == 0 && !p->q_offset_dev && p->Sq == p->Skv &&
            p->Sq >= kTile && (blocks > 512 || (parts > 1 && p->Skv >= 2048));
 }
@@ -578,13 +607,6 @@ int launch_decode(int64_t workgroups, hipStream_t st, const KArgs &a) {
     return rc ? rc : launch(attn_decode_kernel<NQB, NW>, workgroups, 64 * NW, st, a, lds);
 }
 
-// workgroups of the forward / dQ launch: (KV head, chunk of HPB query heads, batch, query tile)
-int64_t q_outer_grid(const KArgs &a, int hpb, int qb) {
-    const int bm = 32 * qb * (4 / hpb);
-    const int n_hc = (a.r + hpb - 1) / hpb;
-    return (int64_t)a.G * n_hc * a.B * ((a.Sq + bm - 1) / bm);
-}
-
 // one launch of a synthetic instruction stream (mfma_rate.h): one workgroup per compute unit
 template <int MIX>
 int64_t launch_stream_probe(int waves_per_simd, int iters, float *sink, hipStream_t st) {
@@ -797,6 +819,11 @@ int gptoss_attn_bwd_preprocess(const gptoss_attn_params *p, void *stream) {
     return s;
 }
 
+static int launch_dkdv_sum(const KArgs &a, hipStream_t st, bool with_dsinks) {
+    if (a.dkdv_steps) return launch_reduce(attn_bwd_dkdv_pieces_reduce_kernel, (int64_t)2 * a.B * a.G * ((a.Skv + 31) / 32) * 256, st, a, with_dsinks);
+    return launch_reduce(attn_bwd_dkdv_reduce_kernel, (int64_t)2 * a.B * a.G * a.Skv * 8, st, a, with_dsinks);
+}
+
 // The dK/dV launch (and the sum of the partials when key blocks are cut).  whole_blocks: never cut a
 // key block, so that nothing beyond the row statistics is kept in the scratch.  with_dsinks: dSinks too, from the row statistics.
 static int launch_dkdv(const gptoss_attn_params *p, void *stream, bool whole_blocks, bool with_dsinks, SinkTypes ty) {
@@ -833,13 +860,27 @@ static int launch_dkdv(const gptoss_attn_params *p, void *stream, bool whole_blo
         return launch_reduce(attn_bwd_dkdv_reduce_kernel, (int64_t)2 * a.B * a.G * a.Skv * 8, st, a, with_dsinks);
     }
     dkdv_pieces_for(p, a);
-    const int64_t grid = (int64_t)a.G * a.B * (a.dkdv_steps ? a.dkdv_slots : a.dkdv_parts * ((a.Skv + kDkdvKeys - 1) / kDkdvKeys));
+    const int64_t grid = dkdv_grid(a);
     const int s = a.doc_start ? launch(attn_bwd_dkdv_kernel<kDkdvWaves, kDkdvNB, true>, grid, 64 * kDkdvWaves, st, a)
                  : a.dkdv_steps ? launch(attn_bwd_dkdv_kernel<kDkdvWaves, kDkdvNB, false, true>, grid, 64 * kDkdvWaves, st, a)
                               : launch(attn_bwd_dkdv_kernel<kDkdvWaves, kDkdvNB, false>, grid, 64 * kDkdvWaves, st, a);
     if (s || a.dkdv_parts == 1) return s;
-    if (a.dkdv_steps) return launch_reduce(attn_bwd_dkdv_pieces_reduce_kernel, (int64_t)2 * a.B * a.G * ((a.Skv + 31) / 32) * 256, st, a, with_dsinks);
-    return launch_reduce(attn_bwd_dkdv_reduce_kernel, (int64_t)2 * a.B * a.G * a.Skv * 8, st, a, with_dsinks);
+    return launch_dkdv_sum(a, st, with_dsinks);
+}
+
+// dQ and dK/dV side by side, behind the row statistics.
+static int launch_both(KArgs &a, hipStream_t st) {
+    int s = launch(attn_bwd_delta_kernel, ((int64_t)a.B * a.H * a.Sq + 127) / 128, 256, st, a);
+    if (s) return s;
+    const void *kernel = a.doc_start    ? reinterpret_cast<const void *>(attn_bwd_both_kernel<true, false>)
+                         : a.dkdv_steps ? reinterpret_cast<const void *>(attn_bwd_both_kernel<false, true>)
+                                        : reinterpret_cast<const void *>(attn_bwd_both_kernel<false, false>);
+    int first = (int)dkdv_grid(a);
+    void *args[] = {&a, &first};
+    const hipError_t e = hipLaunchKernel(kernel, dim3((unsigned)(first + q_outer_grid(a, 4, 1))), dim3(256), args, 0, st);
+    if (e != hipSuccess) return static_cast<int>(e);
+    if (a.dkdv_parts > 1) return launch_dkdv_sum(a, st, a.dsinks != nullptr);
+    return a.dsinks ? launch(attn_bwd_dsinks_kernel, a.H, 1024, st, a) : GPTOSS_ATTN_OK;
 }
 
 int gptoss_attn_bwd_dkdv(const gptoss_attn_params *p, void *stream) { return launch_dkdv(p, stream, false, false, {}); }
@@ -886,6 +927,12 @@ static int bwd_all(const gptoss_attn_params *p, void *stream, bool whole_blocks,
         if (plan.bytes && scratch_bytes >= plan.bytes) return launch_f32_split_bwd(p, static_cast<hipStream_t>(stream), ty, plan, scratch);
     }
     if (window_single_pass(p)) return launch_window_bwd(p, static_cast<hipStream_t>(stream), !whole_blocks, ty);
+    if (!whole_blocks) {
+        KArgs a = make_args(p, ty);
+        a.dkdv_parts = dkdv_parts_for(p, p->seqlens != nullptr, p->doc_start != nullptr);
+        a.dkdv_partial = reinterpret_cast<float *>(reinterpret_cast<char *>(p->delta) + stats_bytes(p));
+        if (both_route(p, a)) return launch_both(a, static_cast<hipStream_t>(stream));
+    }
     rc = launch_dq(p, stream, 1);
     if (rc) return rc;
     return launch_dkdv(p, stream, whole_blocks, p->dsinks != nullptr, ty);
