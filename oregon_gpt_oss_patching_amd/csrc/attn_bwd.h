@@ -22,28 +22,30 @@ namespace gptoss {
 // pass stores lse*log2(e) in the second half of the scratch buffer, which is what
 // the dQ and dSinks kernels feed to exp2, and both statistics once more in the split form the
 // dK/dV kernels take (split_row_stats).
-__global__ __launch_bounds__(256) void attn_bwd_delta_kernel(const KArgs a) {
+// (32-bit row numbers where they suffice: in front of few rows the 64-bit divisions took longer than the loads.)
+template <typename Int>
+__device__ __forceinline__ void delta_rows(const KArgs &a, Int total) {
     constexpr int kRowsPerThread = 4;                      // independent 128-bit loads in flight per tensor
-    const int64_t total = (int64_t)a.B * a.H * a.Sq;       // rows, indexed (b*H + h)*Sq + s
     const int c = threadIdx.x & 7;
-    const int64_t rid0 = (int64_t)blockIdx.x * (32 * kRowsPerThread) + (threadIdx.x >> 3);
+    const Int rid0 = (Int)blockIdx.x * (32 * kRowsPerThread) + (threadIdx.x >> 3);
     u32x4 ov[kRowsPerThread], gv[kRowsPerThread];
+    float lse[kRowsPerThread];
 #pragma unroll
     for (int k = 0; k < kRowsPerThread; ++k) {
-        const int64_t rid = rid0 + 32 * k;
+        const Int rid = rid0 + 32 * k;
         ov[k] = u32x4{0u, 0u, 0u, 0u};
         gv[k] = u32x4{0u, 0u, 0u, 0u};
+        lse[k] = 0.0f;
         if (rid < total) {
-            const int s = (int)(rid % a.Sq);
-            const int bh = (int)(rid / a.Sq);
-            const int h = bh % a.H, b = bh / a.H;
+            const Int bh = rid / (Int)a.Sq, s = rid - bh * (Int)a.Sq, b = bh / (Int)a.H, h = bh - b * (Int)a.H;
             ov[k] = *reinterpret_cast<const u32x4 *>(a.o + (int64_t)b * a.os.b + (int64_t)h * a.os.h + (int64_t)s * a.os.s + c * 8);
             gv[k] = *reinterpret_cast<const u32x4 *>(a.d_o + (int64_t)b * a.dos.b + (int64_t)h * a.dos.h + (int64_t)s * a.dos.s + c * 8);
+            lse[k] = a.lse[rid];
         }
     }
 #pragma unroll
     for (int k = 0; k < kRowsPerThread; ++k) {
-        const int64_t rid = rid0 + 32 * k;
+        const Int rid = rid0 + 32 * k;
         const bf16x8 of = as_bf16x8(ov[k]), gf = as_bf16x8(gv[k]);
         float acc = 0.0f;
 #pragma unroll
@@ -53,10 +55,14 @@ __global__ __launch_bounds__(256) void attn_bwd_delta_kernel(const KArgs a) {
         acc += __shfl_xor(acc, 4);
         if (c == 0 && rid < total) {
             a.delta[rid] = -acc;                          // stored negated: it seeds the dP accumulators
-            a.delta[total + rid] = a.lse[rid] * kLog2e;   // second half of the scratch: lse in log2 units
-            a.split[rid] = split_row_stats(a.lse[rid], a.scale, -acc);
+            a.delta[total + rid] = lse[k] * kLog2e;       // second half of the scratch: lse in log2 units
+            a.split[rid] = split_row_stats(lse[k], a.scale, -acc);
         }
     }
+}
+__global__ __launch_bounds__(256) void attn_bwd_delta_kernel(const KArgs a) {
+    const int64_t total = (int64_t)a.B * a.H * a.Sq;       // rows, indexed (b*H + h)*Sq + s
+    if (total < ((int64_t)1 << 30)) delta_rows(a, (uint32_t)total); else delta_rows(a, total);
 }
 
 // ---------------------------------------------------------------------------------
