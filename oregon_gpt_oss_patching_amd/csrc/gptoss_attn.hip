@@ -844,13 +844,18 @@ static int launch_dkdv(const gptoss_attn_params *p, void *stream, bool whole_blo
     }
     if (dkdv64_route(p, a.dkdv_parts)) {
         const int64_t blocks = (int64_t)a.B * ((a.Skv + Dkdv64::BN - 1) / Dkdv64::BN);      // of a KV head
-        // padded and packed rows, and several rows of one length whose blocks would stay whole otherwise: pieces by the walks' lengths,
+        // padded and packed rows, several rows of one length whose blocks would stay whole otherwise, and few enough equal shares that the longest of them decides:
+        // pieces by the walks' lengths,
         // at most as many as there are slots for partial sums (Dkdv64Plan; the kernels hold kMaxBlocks lengths, nearly twice what dkdv_parts_for leaves)
         // (not packed rows of up to four heads per KV head whose equal shares run all at once: these are four heads of a tile or two, and finding the lengths takes
         // longer than the better division saves.  Backward of 8 heads on two KV heads, equal shares / by lengths, us: 4096 tokens in documents of 100 43 / 50, of 300 54 / 58, of
         // 3000 132 / 135, of 95, 1502 and 222 94 / 92; 8192 (512 shares) of 300 82 / 67; eight heads on one, 4096 of 300 62 / 59)
+        // (Few shares, rows of one length, the same in a graph: 8 heads on one KV head 6000 tokens 293 / 263 (192 shares), 8000 337 / 294 (256), 16 on one 5000 358 / 324, 32 on four
+        // 2200 142 / 130 (288), 8 on two 5000 201 / 195 (320); 32 on four 3000 187 / 195 (384), 8 on one 12000 567 / 587 (376), 2 x 6000 343 / 370 (384): with several rounds
+        // the shares even out by themselves, and equal ones keep in step.)
         const bool one_round = !a.seqlens && a.doc_start && a.r <= 4 && a.G * blocks * a.dkdv_parts <= 256;
-        const bool by_lengths = a.dkdv_parts > 1 && blocks <= Dkdv64Plan::kMaxBlocks && !one_round && (a.seqlens || a.doc_start || (a.B > 1 && a.Sq < 4096 && many_key_blocks(p)));
+        const bool by_lengths = a.dkdv_parts > 1 && blocks <= Dkdv64Plan::kMaxBlocks && !one_round &&
+                                (a.seqlens || a.doc_start || (a.B > 1 && a.Sq < 4096 && many_key_blocks(p)) || a.G * blocks * a.dkdv_parts <= 320);
         if (by_lengths) a.dkdv_slots = (int)((int64_t)a.dkdv_parts * a.B * a.Skv / Dkdv64::BN);
         const int64_t grid64 = a.G * (by_lengths ? a.dkdv_slots : blocks * a.dkdv_parts);
         const bool plain = !by_lengths && !a.seqlens && !a.doc_start && a.Sq % kTile == 0;
