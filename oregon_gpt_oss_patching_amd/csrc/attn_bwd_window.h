@@ -67,7 +67,7 @@ struct WinCfg {
     static constexpr int kLdsBytes = kLogitOff + kMaxGroup * 4;
     static_assert(NSLOT * kMergeBytes == kStatOff - kStageOff, "behind the walk every slot has a merge buffer");
     static_assert(kDsOff % 128 == 0 && kTransitOff % 128 == 0, "swizzled tiles start on 128-byte boundaries");
-    static_assert(kRows * kLS * 2 <= kMergeBytes, "an owner's output stage is its merge buffer");
+    static_assert(kRows * kLS * 2 <= kMergeBytes / 2, "an owner's output stage is its merge buffer");
     static_assert(kLdsBytes <= 160 * 1024, "one workgroup per CU");
 };
 
@@ -494,52 +494,59 @@ __global__ __launch_bounds__(WinCfg::NWAVES * 64, 1) void attn_bwd_window_kernel
             vf[ks] = as_bf16x8(zv);
         }
     }
-    // unscaled sums as accumulator quads of 64 lanes, dK then dV: group 1's on their way to group 0's owner of the same slot, and the shares of seam blocks
-    auto leave_sums = [&](auto *buf) __attribute__((always_inline)) {
-        f32x4 *q = reinterpret_cast<f32x4 *>(buf) + fresh_lane();
+    // Unscaled sums of one tensor as accumulator quads of 64 lanes: on their way to the owner of the same slot in the other group, and the shares of seam blocks.
+    // (A group's tensor is chosen value by value: chosen by branches, the accumulators end up in memory.)
+    constexpr int kHalf = C::kMergeBytes / 2;
+    auto quad = [&](bool of_dv, int dblk, int a4) __attribute__((always_inline)) {
+        f32x4 x;
 #pragma unroll
-        for (int dblk = 0; dblk < 2; ++dblk)
-#pragma unroll
-            for (int a4 = 0; a4 < 4; ++a4) {
-                f32x4 xk, xv;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) { xk[e] = dk[dblk][4 * a4 + e]; xv[e] = dv[dblk][4 * a4 + e]; }
-                q[(4 * dblk + a4) * 64] = xk;
-                q[(8 + 4 * dblk + a4) * 64] = xv;
-            }
+        for (int e = 0; e < 4; ++e) x[e] = of_dv ? dv[dblk][4 * a4 + e] : dk[dblk][4 * a4 + e];
+        return x;
     };
-    // fp32 share of a seam block: [b][g][seam][block 0..3][workgroup before / after the seam], accumulator quads of 64 lanes as above
+    // into a slot's merge buffer: group 1's dK, group 0's dV
+    auto exchange = [&](char *buf) __attribute__((always_inline)) {
+        f32x4 *q = reinterpret_cast<f32x4 *>(buf + (grp ? 0 : kHalf)) + fresh_lane();
+#pragma unroll
+        for (int j = 0; j < 8; ++j) q[j * 64] = quad(grp == 0, j >> 2, j & 3);
+    };
+    // fp32 share of a seam block: [b][g][seam][block 0..3][workgroup before / after the seam], dK then dV, accumulator quads of 64 lanes as above
     auto seam_share = [&](int seam, int block, int side) {
         return a.boundary_partial + (((((int64_t)b * a.G + g) * (n_chunks - 1) + seam) * C::kBack + block) * 2 + side) * (2 * kRows * kD);
     };
-    // group 0: dK / dV of the key block held, group 1's sums in `buf` added: written out if it is complete, left as this workgroup's share if
+    // One tensor of the key block held (group 0: dK, group 1: dV), the other group's sums in `buf` added: written out if it is complete, left as this workgroup's share if
     // it sits on a seam, dropped if it belongs to the neighbour (recomputation mode).  `buf` then stages the rows.
     auto flush = [&](char *buf) __attribute__((always_inline)) {
         if (my_kb < 0 || (!seam_sums && (my_kb < u0 || my_kb >= u1))) return;
         const int ln = fresh_lane();
-        const f32x4 *q = reinterpret_cast<const f32x4 *>(buf) + ln;
+        char *const half_buf = buf + (grp ? kHalf : 0);
+        const f32x4 *q = reinterpret_cast<const f32x4 *>(half_buf) + ln;
+        f32x16 sum[2];
 #pragma unroll
-        for (int dblk = 0; dblk < 2; ++dblk)
+        for (int dblk = 0; dblk < 2; ++dblk) {
+            f32x4 x[4];
 #pragma unroll
-            for (int h2 = 0; h2 < 2; ++h2) {
-                f32x4 x[4];
+            for (int j = 0; j < 4; ++j) x[j] = q[(4 * dblk + j) * 64];
 #pragma unroll
-                for (int j = 0; j < 4; ++j) x[j] = q[((j & 1) * 8 + 4 * dblk + 2 * h2 + (j >> 1)) * 64];
+            for (int j = 0; j < 4; ++j) {
+                const f32x4 own = quad(grp == 1, dblk, j);
 #pragma unroll
-                for (int j = 0; j < 2; ++j)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) { dk[dblk][8 * h2 + 4 * j + e] += x[2 * j][e]; dv[dblk][8 * h2 + 4 * j + e] += x[2 * j + 1][e]; }
-                asm volatile("" ::: "memory");             // (four reads at a time: all sixteen would spill what the walk holds)
+                for (int e = 0; e < 4; ++e) sum[dblk][4 * j + e] = own[e] + x[j][e];
             }
-        if (seam_sums) {
-            if (my_kb < u0) { leave_sums(seam_share(chunk - 1, my_kb - (u0 - C::kBack), 1)); return; }
-            if (my_kb >= u1 - C::kBack && u1 < n_blocks) { leave_sums(seam_share(chunk, my_kb - (u1 - C::kBack), 0)); return; }
+            asm volatile("" ::: "memory");                     // (four reads at a time: all eight would spill what the walk holds)
+        }
+        float *share = nullptr;
+        if (seam_sums && my_kb < u0) share = seam_share(chunk - 1, my_kb - (u0 - C::kBack), 1);
+        else if (seam_sums && my_kb >= u1 - C::kBack && u1 < n_blocks) share = seam_share(chunk, my_kb - (u1 - C::kBack), 0);
+        if (share) {
+            f32x4 *to = reinterpret_cast<f32x4 *>(share + grp * (kRows * kD)) + ln;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) to[j * 64] = f32x4{sum[j >> 2][4 * (j & 3)], sum[j >> 2][4 * (j & 3) + 1], sum[j >> 2][4 * (j & 3) + 2], sum[j >> 2][4 * (j & 3) + 3]};
+            return;
         }
         const int r0 = my_kb * kRows;
-        const int nvalid = a.Skv - r0;
-        bf16 *const out_stage = reinterpret_cast<bf16 *>(buf);
-        window_store_rows(out_stage, dk, a.scale, a.dk + (int64_t)b * a.dks.b + (int64_t)g * a.dks.h + (int64_t)r0 * a.dks.s, (int)a.dks.s, nvalid, ln);
-        window_store_rows(out_stage, dv, 1.0f, a.dv + (int64_t)b * a.dvs.b + (int64_t)g * a.dvs.h + (int64_t)r0 * a.dvs.s, (int)a.dvs.s, nvalid, ln);
+        const Strides &st = grp ? a.dvs : a.dks;
+        window_store_rows(reinterpret_cast<bf16 *>(half_buf), sum, grp ? 1.0f : a.scale, (grp ? a.dv : a.dk) + (int64_t)b * st.b + (int64_t)g * st.h + (int64_t)r0 * st.s, (int)st.s,
+                          a.Skv - r0, ln);
     };
 
     const float c = a.scale_log2;
@@ -578,7 +585,7 @@ __global__ __launch_bounds__(WinCfg::NWAVES * 64, 1) void attn_bwd_window_kernel
     for (;;) {
         begin();
         if (u > u0) {
-            if (grp == 0) flush(lds + C::kMergeOff);           // the block held so far
+            flush(lds + C::kMergeOff);                         // the block held so far
             kb += C::NSLOT;
             my_kb = u < u1 ? u : -1;
             const uint32_t from = transit_base + (u & 1) * (2 * C::kBlockBytes) - at_stage;
@@ -619,13 +626,13 @@ __global__ __launch_bounds__(WinCfg::NWAVES * 64, 1) void attn_bwd_window_kernel
             next();
         }
         if (u == u_end) break;
-        if (grp == 1) leave_sums(lds + C::kMergeOff);
+        exchange(lds + C::kMergeOff);
     }
     __syncthreads();                                           // hands the last dS blocks over; nobody reads a stage any more
     char *const last = lds + C::kStageOff + slot * C::kMergeBytes;
-    if (grp == 1) leave_sums(last);
+    exchange(last);
     __syncthreads();
-    if (grp == 0) flush(last);
+    flush(last);
 }
 
 // ---------------------------------------------------------------------------------
