@@ -157,7 +157,7 @@ size_t gptoss_attn_bwd_workspace_bytes(const gptoss_attn_params *params);
 
 /*
  * Bytes of scratch gptoss_attn_fwd_scratch can use for this call (0 for most): few queries on a long key / value cache (a decoding
- * step, a short piece of a prompt) are cut over the keys, and the slices leave fp32 partial results there.  Never more than
+ * step, a short piece of a prompt) and long rows of few heads are cut over the keys, and the slices leave fp32 partial results there.  Never more than
  * gptoss_attn_workspace_bytes.  Host-only.
  */
 size_t gptoss_attn_fwd_workspace_bytes(const gptoss_attn_params *params);
@@ -186,7 +186,7 @@ int gptoss_attn_fwd(const gptoss_attn_params *params, void *stream);
 int gptoss_attn_fwd_sinks(const gptoss_attn_params *params, int sinks_dtype, void *stream);
 
 /*
- * The same with scratch of the caller's for few queries on a long cache: `scratch` (16-byte aligned) holds `scratch_bytes` bytes, which
+ * The same with scratch of the caller's for few queries on a long cache or long rows of few heads: `scratch` (16-byte aligned) holds `scratch_bytes` bytes, which
  * no other call may use until this one has run.  With NULL, or with fewer bytes than gptoss_attn_fwd_workspace_bytes gives
  * for the same block, the same kernel walks each row's keys uncut, as the two calls above do (O then agrees to one bf16 rounding).
  * float32 calls take gptoss_attn_split_bytes(params, 0) bytes; with less they run on the fp32 matrix instruction, as the two calls above do.

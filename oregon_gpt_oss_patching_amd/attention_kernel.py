@@ -191,7 +191,7 @@ def attention_forward(q, k, v, sinks, sm_scale, window=None, q_offset=0, seqlens
         p = _base_params(q, k, v, sinks32, sl, sm_scale, window, q_offset, ds, qod)
         p.o, p.lse = o.data_ptr(), lse.data_ptr()
         _set(p.o_stride, _strides_bhs(o, "bshd"))
-        # partial results of few queries' rows, cut over their keys; records of float32 operands
+        # partial results of few queries' or few heads' rows, cut over their keys; records of float32 operands
         need = max(_lib.load().gptoss_attn_fwd_workspace_bytes(p), _lib.load().gptoss_attn_split_bytes(p, 0))
         scratch = torch.empty((need // 4,), dtype=torch.float32, device=q.device) if need else None
         _lib.call("gptoss_attn_fwd_scratch", p, _stream(q), _lib.DTYPE_FP32, scratch.data_ptr() if need else None, need)

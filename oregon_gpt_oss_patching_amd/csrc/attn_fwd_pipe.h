@@ -49,10 +49,10 @@ struct FwdPipe {
 // keys 181 -> 135 us a call; 2 x 3001 tokens 164 -> 160 us, 1 x 1000 33.6 -> 25.2, 2 x 383 16.1 -> 14.8; seven documents in 8192 tokens
 // 185 -> 180 (without letting the other documents' rows run along, every tile of such a workgroup being an exact
 // step: 230).
-// Few queries on a long cache leave most of the chip idle (100 queries on 4096 keys: 32 workgroups).  With kv_splits > 1 a query block's
+// Few queries on a long cache, or few heads, leave most of the chip idle (100 queries on 4096 keys: 32 workgroups).  With kv_splits > 1 a query block's
 // key tiles are cut into that many consecutive shares, one workgroup each, which leave their unnormalised rows with (reference,
 // sum) in the scratch; attn_fwd_combine_kernel adds them in share order.  Each share freezes a reference of its own (100 queries on 4096 keys
-// of 64 heads: 62 -> 30 us, the sum included).
+// of 64 heads: 62 -> 30 us, the sum included; 4000 tokens of 8 heads 60 -> 41).
 template <bool GENERAL, bool DOCS = false>       // DOCS: packed documents (needs GENERAL)
 __global__ __launch_bounds__(256, 2) void attn_fwd_pipe_kernel(const KArgs a) {
     constexpr int NS = FwdPipe::NS;

@@ -254,19 +254,23 @@ bool fwd_pipe_plain(const gptoss_attn_params *p) {
     return p->Sq == p->Skv && p->Sq % kTile == 0 && !p->seqlens && !p->doc_start && p->q_offset == 0 && !p->q_offset_dev;
 }
 
-// Shares of the keys per query block where new queries on a cache (fewer queries than keys, no packing) are too few to fill the chip: two
-// workgroups per compute unit of a 256-CU part, at least eight tiles each.  From the shapes alone, so that the scratch does not
-// depend on where the queries stand.  64 query heads on 8 KV heads: 100 queries on 4096 keys 62 -> 30 us, 300 on 12000 167 -> 82
+// Shares of the keys per query block where the workgroups are too few to fill the chip (no packing): two
+// per compute unit of a 256-CU part, at least eight tiles each.  From the shapes alone, so that the scratch (35 MB at most, 69 for the longest rows) does not
+// depend on where the queries stand.  New queries on a cache, 64 query heads on 8 KV heads: 100 queries on 4096 keys 62 -> 30 us, 300 on 12000 167 -> 82
 // (four tiles each: 37 us and 83); 8 heads on one KV head: 300 on 12000 164 -> 34 (more than sixteen shares: 36), 1000 on 17000 231 -> 57.
-// Two shares are not worth the sum: 1024 on 8192 134 -> 137.
+// Two shares are not worth the sum: 1024 on 8192 134 -> 137.  Self-attention, where the sum is over more rows (us in a graph): on up to four groups of four heads from 20 tiles on, 8 heads on
+// one KV head 1300 tokens 23.4 -> 21.3, 2000 33 -> 23, 4000 60 -> 41, 8000 113 -> 96, 2 x 1300 23.8 -> 23.1, 2 x 3000 48 -> 43; not 2 x 1024 19.2 -> 20.4, on six groups 3 x 1600
+// 28 -> 31, 3 x 2560 41 -> 46, on eight 4 x 1000 21 -> 23, 32 heads on four 2000 37 -> 41.  Rows of 128 tiles and more: four workgroups per unit, 8200 117 -> 91, 12000 191 -> 164
+// (with two it would stay whole), 16384 309 -> 275, but 4000 60 -> 46.
 int fwd_pipe_splits(const gptoss_attn_params *p) {
-    if (p->Skv <= p->Sq) return 1;
-    const int64_t wgs = (int64_t)p->G * (p->H / p->G / 4) * p->B * ((p->Sq + kTile - 1) / kTile);
+    const bool self = p->Skv <= p->Sq;
+    const int64_t groups = (int64_t)p->G * (p->H / p->G / 4) * p->B, wgs = groups * ((p->Sq + kTile - 1) / kTile);
     const int64_t tiles = (p->Skv + kTile - 1) / kTile;
-    int64_t n = 512 / wgs;
+    if (self && (groups > 4 || tiles < 20)) return 1;
+    int64_t n = (self && tiles >= 128 ? 1024 : 512) / wgs;
     if (n > tiles / 8) n = tiles / 8;
     if (n > 16) n = 16;
-    return n < 3 ? 1 : (int)n;
+    return n < (self ? 2 : 3) ? 1 : (int)n;
 }
 
 // The one-pass forward of sliding-window layers (attn_fwd_window.h): a window of 32, 64, 96 or 128 keys, all four wavefronts of

@@ -147,7 +147,7 @@ std::tuple<Tensor, Tensor> fwd(const Tensor &q, const Tensor &k, const Tensor &v
     c.p.o = o.data_ptr();
     c.p.lse = lse.data_ptr<float>();
     set(c.p.o_stride, o, true);
-    // partial results of few queries' rows, cut over their keys; records of float32 operands
+    // partial results of few queries' or few heads' rows, cut over their keys; records of float32 operands
     const size_t need = c.p.dtype == GPTOSS_ATTN_FP32 ? gptoss_attn_split_bytes(&c.p, 0) : gptoss_attn_fwd_workspace_bytes(&c.p);
     const Tensor scratch = need ? at::empty({static_cast<int64_t>(need / sizeof(float))}, lse.options()) : Tensor();
     check("gptoss_attn_fwd", gptoss_attn_fwd_scratch(&c.p, c.sinks_dtype, need ? scratch.data_ptr() : nullptr, need, stream_of(c)));
