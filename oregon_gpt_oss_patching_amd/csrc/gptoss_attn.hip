@@ -136,13 +136,19 @@ bool many_key_blocks(const gptoss_attn_params *p) { return (int64_t)p->G * p->B 
 // rather have two: 340 / 359, 526 / 513, 864 / 902, 904 / 919.)
 int dkdv_parts_for(const gptoss_attn_params *p, bool padded, bool packed) {
     if (p->dtype == GPTOSS_ATTN_FP32) {
-        // a workgroup per 32 keys, two per compute unit: about four workgroups per unit of a 256-CU part, so that the long
-        // first key blocks of a row do not decide the time
-        const int64_t blocks = (int64_t)p->G * p->B * ((p->Skv + 31) / 32), tiles = (p->Sq + 31) / 32;
-        int64_t parts = effective_window(p) > 0 ? 1 : 1024 / blocks;
+        // A workgroup per 32 keys, two per compute unit at a time.  Up to four slices and a thousand workgroups, so that the long first key blocks of a row do not decide the time;
+        // more where that is not two per unit of a 256-CU part: the longest walk, 1.2 us a step, is all there is to such a launch (backward, us in a graph, at most four slices / these: 8 heads
+        // on one KV head 300 tokens 55 / 38, 1000 122 / 76, 2 x 1000 134 / 111, on two 1000 83 / 73 (with a thousand workgroups here too 82), 64 on eight 150 45 / 36).  A window's walk is cut by the
+        // same rule, into three or more: of 128 8 heads on one 400 tokens 73 / 34, 64 on eight 500 95 / 82; into two 900 108 / 110.
+        const int64_t blocks = (int64_t)p->G * p->B * ((p->Skv + 31) / 32), all = (p->Sq + 31) / 32;
+        const int window = effective_window(p);
+        const int64_t tiles = window > 0 && (window + 62) / 32 + 1 < all ? (window + 62) / 32 + 1 : all;        // that see a block
+        int64_t parts = window > 0 ? 1 : 1024 / blocks;
+        if (parts > 4) parts = 4;
+        if (512 / blocks > (window > 0 ? 2 : parts)) parts = 512 / blocks;
         if (parts > tiles * (p->H / p->G) / 8) parts = tiles * (p->H / p->G) / 8;
         if (parts > tiles) parts = tiles;
-        if (parts > 4) parts = 4;
+        if (parts > 16) parts = 16;
         return parts < 1 ? 1 : (int)parts;
     }
     if (p->dtype != GPTOSS_ATTN_BF16) return 1;
