@@ -337,18 +337,17 @@ __global__ __launch_bounds__(256, 2) void attn_f32_fwd_kernel(const KArgs a) {
 }
 
 // ---- backward step 1: -delta and lse*log2(e) into the scratch (same layout as the bf16 path) ----
-__global__ __launch_bounds__(256) void attn_f32_delta_kernel(const KArgs a) {
+template <typename Int>
+__device__ __forceinline__ void f32_delta_rows(const KArgs &a, Int total) {
     const F32Ptrs t = f32_ptrs(a);
-    const int64_t total = (int64_t)a.B * a.H * a.Sq;
     const int c = threadIdx.x & 15;                                   // 16 lanes x 16 bytes = one 256-byte row
-    const int64_t rid = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
-    float acc = 0.0f;
+    const Int rid = (Int)blockIdx.x * 16 + (threadIdx.x >> 4);
+    float acc = 0.0f, lse = 0.0f;
     if (rid < total) {
-        const int s = (int)(rid % a.Sq);
-        const int bh = (int)(rid / a.Sq);
-        const int h = bh % a.H, b = bh / a.H;
+        const Int bh = rid / (Int)a.Sq, s = rid - bh * (Int)a.Sq, b = bh / (Int)a.H, h = bh - b * (Int)a.H;
         const f32x4 ov = *reinterpret_cast<const f32x4 *>(t.o + (int64_t)b * a.os.b + (int64_t)h * a.os.h + (int64_t)s * a.os.s + 4 * c);
         const f32x4 gv = *reinterpret_cast<const f32x4 *>(t.d_o + (int64_t)b * a.dos.b + (int64_t)h * a.dos.h + (int64_t)s * a.dos.s + 4 * c);
+        lse = a.lse[rid];
 #pragma unroll
         for (int e = 0; e < 4; ++e) acc = fmaf(ov[e], gv[e], acc);
     }
@@ -358,8 +357,12 @@ __global__ __launch_bounds__(256) void attn_f32_delta_kernel(const KArgs a) {
     acc += __shfl_xor(acc, 8);
     if (c == 0 && rid < total) {
         a.delta[rid] = -acc;
-        a.delta[total + rid] = a.lse[rid] * kLog2e;
+        a.delta[total + rid] = lse * kLog2e;
     }
+}
+__global__ __launch_bounds__(256) void attn_f32_delta_kernel(const KArgs a) {
+    const int64_t total = (int64_t)a.B * a.H * a.Sq;
+    if (total < ((int64_t)1 << 30)) f32_delta_rows(a, (uint32_t)total); else f32_delta_rows(a, total);
 }
 
 // ---- backward step 2: dK, dV ------------------------------------------------------------
@@ -522,9 +525,7 @@ __device__ __forceinline__ void f32_dkdv_keys(const KArgs &a, char *smem, int g,
         }
     }
 }
-__global__ __launch_bounds__(256, 2) void attn_f32_dkdv_kernel(const KArgs a) {
-    __shared__ __attribute__((aligned(1024))) char smem[F32Dkdv::kLdsBytes];
-    int bid = blockIdx.x;
+__device__ __forceinline__ void f32_dkdv_workgroup(const KArgs &a, char *smem, int bid) {
     const int g = bid % a.G; bid /= a.G;
     const int bi = bid % a.B; bid /= a.B;
     const int part = bid % a.dkdv_parts, kblk = bid / a.dkdv_parts;       // ascending: most work first
@@ -535,6 +536,10 @@ __global__ __launch_bounds__(256, 2) void attn_f32_dkdv_kernel(const KArgs a) {
     const int64_t tensor = (int64_t)a.B * a.G * a.Skv * kD;
     float *out = a.dkdv_parts > 1 ? a.dkdv_partial + 2 * part * tensor + (((int64_t)b * a.G + g) * a.Skv + j0) * kD : nullptr;
     f32_dkdv_keys<4>(a, smem, g, b, j0, walk, out, out ? out + tensor : nullptr);
+}
+__global__ __launch_bounds__(256, 2) void attn_f32_dkdv_kernel(const KArgs a) {
+    __shared__ __attribute__((aligned(1024))) char smem[F32Dkdv::kLdsBytes];
+    f32_dkdv_workgroup(a, smem, blockIdx.x);
 }
 
 // The slices' partial sums, added in slice order.  One thread per 16-byte output chunk.
@@ -665,6 +670,15 @@ template <int KS, bool FUSE_DELTA>
 __global__ __launch_bounds__(256, 2) void attn_f32_dq_kernel(const KArgs a) {
     __shared__ __attribute__((aligned(1024))) char smem[8 * F32Tile::kBytes];
     f32_dq_rows<KS, FUSE_DELTA, 4>(a, smem);
+}
+
+// dQ (the first workgroups) and dK/dV side by side behind the row statistics, where all of them run at once: the float32 counterpart of attn_bwd_both_kernel, with the bits
+// of the two launches.
+__global__ __launch_bounds__(256, 2) void attn_f32_both_kernel(const KArgs a, int dq_workgroups) {
+    static_assert(F32Dkdv::kLdsBytes >= 8 * F32Tile::kBytes, "one array for both");
+    __shared__ __attribute__((aligned(1024))) char smem[F32Dkdv::kLdsBytes];
+    if ((int)blockIdx.x < dq_workgroups) f32_dq_rows<4, false, 4>(a, smem);
+    else f32_dkdv_workgroup(a, smem, blockIdx.x - dq_workgroups);
 }
 
 }  // namespace gptoss

@@ -883,6 +883,24 @@ static int launch_dkdv(const gptoss_attn_params *p, void *stream, bool whole_blo
     return launch_dkdv_sum(a, st, with_dsinks);
 }
 
+// The same for float32: dQ's workgroups come first.  Two launches / one, us as above (workgroups): 8 heads on one KV head 300 tokens 38 / 24, 1000 76 / 67 (730), 1500 141 / 102 (846), on
+// two 500 41 / 31, 2 x 700 76 / 61 (792), 2 x 1000 111 / 104 (1024); 64 on eight 64 29 / 22, 150 36 / 30 (520); window 128, 8 on one 400 34 / 23.  Not 4 x 700 122 / 132 (1144); rows of a
+// few tiles start and end rather than walk, 64 on eight 180 39.7 / 40.6 (672), 2 x 100 37 / 38 (768).
+static int64_t f32_dkdv_grid(const KArgs &a) { return (int64_t)a.B * a.G * a.dkdv_parts * ((a.Skv + 31) / 32); }
+static bool f32_both_route(const KArgs &a, int dtype) {
+    return dtype == GPTOSS_ATTN_FP32 && f32_key_splits(a) == 4 && f32_grid(a, 4) + f32_dkdv_grid(a) <= (a.Sq > 256 ? 1024 : 640);
+}
+static int launch_f32_both(KArgs &a, hipStream_t st) {
+    int s = launch(attn_f32_delta_kernel, ((int64_t)a.B * a.H * a.Sq + 15) / 16, 256, st, a);
+    if (s) return s;
+    int first = (int)f32_grid(a, 4);
+    void *args[] = {&a, &first};
+    const hipError_t e = hipLaunchKernel(reinterpret_cast<const void *>(attn_f32_both_kernel), dim3((unsigned)(first + f32_dkdv_grid(a))), dim3(256), args, 0, st);
+    if (e != hipSuccess) return static_cast<int>(e);
+    if (a.dkdv_parts > 1) return launch_reduce(attn_f32_dkdv_reduce_kernel, (int64_t)2 * a.B * a.G * a.Skv * 16, st, a, a.dsinks != nullptr);
+    return a.dsinks ? launch(attn_bwd_dsinks_kernel, a.H, 1024, st, a) : GPTOSS_ATTN_OK;
+}
+
 // dQ and dK/dV side by side, behind the row statistics.
 static int launch_both(KArgs &a, hipStream_t st) {
     int s = launch(attn_bwd_delta_kernel, ((int64_t)a.B * a.H * a.Sq + 127) / 128, 256, st, a);
@@ -946,6 +964,7 @@ static int bwd_all(const gptoss_attn_params *p, void *stream, bool whole_blocks,
         KArgs a = make_args(p, ty);
         a.dkdv_parts = dkdv_parts_for(p, p->seqlens != nullptr, p->doc_start != nullptr);
         a.dkdv_partial = reinterpret_cast<float *>(reinterpret_cast<char *>(p->delta) + stats_bytes(p));
+        if (f32_both_route(a, p->dtype)) return launch_f32_both(a, static_cast<hipStream_t>(stream));
         if (both_route(p, a)) return launch_both(a, static_cast<hipStream_t>(stream));
     }
     rc = launch_dq(p, stream, 1);
