@@ -264,7 +264,11 @@ bool fwd_pipe_plain(const gptoss_attn_params *p) {
 // per compute unit of a 256-CU part, at least eight tiles each.  From the shapes alone, so that the scratch (35 MB at most, 69 for the longest rows) does not
 // depend on where the queries stand.  New queries on a cache, 64 query heads on 8 KV heads: 100 queries on 4096 keys 62 -> 30 us, 300 on 12000 167 -> 82
 // (four tiles each: 37 us and 83); 8 heads on one KV head: 300 on 12000 164 -> 34 (more than sixteen shares: 36), 1000 on 17000 231 -> 57.
-// Two shares are not worth the sum: 1024 on 8192 134 -> 137.  Self-attention, where the sum is over more rows (us in a graph): on up to four groups of four heads from 20 tiles on, 8 heads on
+// Two shares are not worth the sum where they just fill the chip: 1024 on 8192 134 -> 137.  More workgroups than compute units, but not two each, make some units take twice as long as
+// the others (a unit is no faster with two): shares that end with a full or half full round of two per unit even that out on long caches, three for 257 to 341 workgroups, two to 384; us, whole / in
+// shares: 1088 on 6000 144 / 128, 1268 on 4000 97 / 97, on 16000 398 / 319, 1344 on 7000 173 / 155, 1500 on 9000 228 / 211, on 4000 99 / 101, 1600 on 16000 (400 workgroups, two) 412 / 437; and four for 171 to 192,
+// 704 on 16000 219 / 190, on 5000 75 / 77, 768 on 16000 220 / 200, 32 heads on four 1600 (200) on 9000 130 / 143.
+// Self-attention, where the sum is over more rows (us in a graph): on up to four groups of four heads from 20 tiles on, 8 heads on
 // one KV head 1300 tokens 23.4 -> 21.3, 2000 33 -> 23, 4000 60 -> 41, 8000 113 -> 96, 2 x 1300 23.8 -> 23.1, 2 x 3000 48 -> 43; not 2 x 1024 19.2 -> 20.4, on six groups 3 x 1600
 // 28 -> 31, 3 x 2560 41 -> 46, on eight 4 x 1000 21 -> 23, 32 heads on four 2000 37 -> 41.  Rows of 128 tiles and more: four workgroups per unit, 8200 117 -> 91, 12000 191 -> 164
 // (with two it would stay whole), 16384 309 -> 275, but 4000 60 -> 46.
@@ -276,6 +280,11 @@ int fwd_pipe_splits(const gptoss_attn_params *p) {
     int64_t n = (self && tiles >= 128 ? 1024 : 512) / wgs;
     if (n > tiles / 8) n = tiles / 8;
     if (n > 16) n = 16;
+    if (!self && n < 3 && tiles >= 96) {
+        if (wgs > 256) n = wgs <= 1024 / 3 ? 3 : wgs <= 768 / 2 ? 2 : 1;
+        else n = wgs <= 768 / 4 && tiles >= 128 ? 4 : 1;
+        return (int)n;
+    }
     return n < (self ? 2 : 3) ? 1 : (int)n;
 }
 
