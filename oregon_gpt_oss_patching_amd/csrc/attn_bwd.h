@@ -531,19 +531,18 @@ __global__ __launch_bounds__(NW * 64, (NB == 1 ? 2 : 1)) void attn_bwd_dkdv_kern
 
 // ---------------------------------------------------------------------------------
 // Sum of the dK / dV partials of a split key block, in part order (bit-reproducible), scaled and
-// rounded to the output type.  One thread per 16-byte output chunk: (tensor, b, g, key, 8 columns).
+// rounded to the output type.  One thread per 16-byte output chunk: a block of threads is 32 keys of one tensor.
 // The first `heads` blocks produce dSinks (a launch of their own took 4.5 to 11 us; here they run beside the sums).
 __global__ __launch_bounds__(256) void attn_bwd_dkdv_reduce_kernel(const KArgs a, int heads) {
     __shared__ float red[1024];
     if ((int)blockIdx.x < heads) { dsinks_of_head<256>(a, blockIdx.x, red); return; }
-    const int64_t rows = (int64_t)a.B * a.G * a.Skv;
-    const int64_t tensor = rows * kD;
-    const int64_t idx = (int64_t)(blockIdx.x - heads) * 256 + threadIdx.x;   // chunk index over both tensors
-    if (idx >= 2 * rows * 8) return;
-    const int which = (int)(idx / (rows * 8));                            // 0 = dK, 1 = dV
-    const int64_t rem = idx - (int64_t)which * rows * 8;
-    const int64_t row = rem >> 3;
-    const int c8 = (int)(rem & 7) * 8;
+    int bid = blockIdx.x - heads;                                         // (g changes fastest, as where the partials were written: the same XCD's L2)
+    const int g = bid % a.G; bid /= a.G;
+    const int which = bid & 1; bid >>= 1;                                 // 0 = dK, 1 = dV
+    const int key_blocks = (a.Skv + 31) / 32, k32 = bid % key_blocks, b = bid / key_blocks;
+    const int c8 = (threadIdx.x & 7) * 8, key = 32 * k32 + (threadIdx.x >> 3);
+    if (key >= a.Skv) return;
+    const int64_t tensor = (int64_t)a.B * a.G * a.Skv * kD, row = ((int64_t)b * a.G + g) * a.Skv + key;
     const float *src = a.dkdv_partial + (int64_t)which * tensor + row * kD + c8;
     f32x4 lo = {0.0f, 0.0f, 0.0f, 0.0f}, hi = {0.0f, 0.0f, 0.0f, 0.0f};
     for (int part = 0; part < a.dkdv_parts; ++part) {
@@ -556,9 +555,6 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_reduce_kernel(const KArgs a
     bf16x8 out;
 #pragma unroll
     for (int e = 0; e < 4; ++e) { out[e] = (bf16)(lo[e] * mul); out[4 + e] = (bf16)(hi[e] * mul); }
-    const int key = (int)(row % a.Skv);
-    const int bg = (int)(row / a.Skv);
-    const int g = bg % a.G, b = bg / a.G;
     const Strides &st = which == 0 ? a.dks : a.dvs;
     bf16 *dst = (which == 0 ? a.dk : a.dv) + (int64_t)b * st.b + (int64_t)g * st.h + (int64_t)key * st.s + c8;
     union { bf16x8 v; u32x4 u; } cv;
@@ -571,9 +567,9 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_pieces_reduce_kernel(const 
     __shared__ float red[1024];
     if ((int)blockIdx.x < heads) { dsinks_of_head<256>(a, blockIdx.x, red); return; }
     int bid = blockIdx.x - heads;
+    const int g = bid % a.G; bid /= a.G;
     const int which = bid & 1; bid >>= 1;                                 // 0 = dK, 1 = dV
-    const int key_blocks = (a.Skv + 31) / 32, k32 = bid % key_blocks; bid /= key_blocks;
-    const int g = bid % a.G, b = bid / a.G;
+    const int key_blocks = (a.Skv + 31) / 32, k32 = bid % key_blocks, b = bid / key_blocks;
     const int kt = k32 >> 2, w = k32 & 3, chunk = threadIdx.x & 7, row = threadIdx.x >> 3, key = 32 * k32 + row;
     const int mine = DkdvPieces::of(a.Sq, a.r, a.dkdv_steps, threadIdx.x & 63);
     int base = 0;

@@ -840,7 +840,7 @@ int gptoss_attn_bwd_preprocess(const gptoss_attn_params *p, void *stream) {
 
 static int launch_dkdv_sum(const KArgs &a, hipStream_t st, bool with_dsinks) {
     if (a.dkdv_steps) return launch_reduce(attn_bwd_dkdv_pieces_reduce_kernel, (int64_t)2 * a.B * a.G * ((a.Skv + 31) / 32) * 256, st, a, with_dsinks);
-    return launch_reduce(attn_bwd_dkdv_reduce_kernel, (int64_t)2 * a.B * a.G * a.Skv * 8, st, a, with_dsinks);
+    return launch_reduce(attn_bwd_dkdv_reduce_kernel, (int64_t)2 * a.B * a.G * ((a.Skv + 31) / 32) * 256, st, a, with_dsinks);
 }
 
 // The dK/dV launch (and the sum of the partials when key blocks are cut).  whole_blocks: never cut a
@@ -881,7 +881,7 @@ static int launch_dkdv(const gptoss_attn_params *p, void *stream, bool whole_blo
         const int s = plain ? launch(attn_bwd_dkdv64_kernel<false>, grid64, 256, st, a) : launch(attn_bwd_dkdv64_kernel<true>, grid64, 256, st, a);
         if (s || a.dkdv_parts == 1) return s;
         if (by_lengths) return launch_reduce(attn_bwd_dkdv64_reduce_kernel, a.G * blocks * 16 * 256, st, a, with_dsinks);
-        return launch_reduce(attn_bwd_dkdv_reduce_kernel, (int64_t)2 * a.B * a.G * a.Skv * 8, st, a, with_dsinks);
+        return launch_reduce(attn_bwd_dkdv_reduce_kernel, (int64_t)2 * a.B * a.G * ((a.Skv + 31) / 32) * 256, st, a, with_dsinks);
     }
     dkdv_pieces_for(p, a);
     const int64_t grid = dkdv_grid(a);
