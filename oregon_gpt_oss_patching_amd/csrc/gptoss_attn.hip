@@ -213,13 +213,14 @@ int64_t dkdv_grid(const KArgs &a) {
 bool window_single_pass(const gptoss_attn_params *p);
 // dQ and dK/dV in one launch (attn_bwd_both_kernel) behind one for the row statistics, instead of one after the other: where their workgroups, two to a compute
 // unit of a 256-CU part, are few enough to run side by side.  `a` has the backward's dkdv_parts; gets its pieces.  Whole backward, us in a graph, one after the
-// other / side by side (workgroups): 8 heads on one KV head 300 tokens 34 / 27 (29), 1300 70 / 47 (161), 2000 96 / 63 (248), 2 x 1500 78 / 56 (368), 4 x 1000 61 / 53 (500),
-// 4 x 2000 114 / 119 (992); 8 on two 2 x 1500 74 / 67 (500), 4 x 1000 58 / 56 (744); 32 on four 700 49 / 34 (320), 1500 90 / 79 (736), 2000 114 / 118 (992); 64 on eight 256 30 / 27
-// (192), 512 37 / 36 (480), 2 x 383 41.7 / 41.3 (656), 768 53.4 / 53.3 (720), 1024 66 / 78 (1000): two full rounds, of which the second holds the longest walks.  Against the
-// 64-key kernel (2048 tokens and more) and for padded and packed rows the line is lower: 8 heads on one 2500 tokens 137 / 77 (318), 4000 169 / 111 (506), padded
-// 2 x 2500 131 / 111 (636), padded 2 x 3000 147 / 148 (760); on two 2500 110 / 94 (478), 4000 131 / 147 (762), in three documents 89 / 93.
+// other / side by side (workgroups): 8 heads on one KV head 300 tokens 34 / 26 (29), 1300 70 / 45 (161), 2000 96 / 61 (248), 2 x 1500 78 / 54 (368), 4 x 1000 61 / 50 (500),
+// 4 x 2000 114 / 119 (992); 8 on two 2 x 1500 74 / 65 (500), 4 x 1000 58 / 54 (744); 32 on four 700 49 / 32 (320), 1500 90 / 76 (736), 2000 114 / 118 (992); 64 on eight 256 30 / 25
+// (192), 512 37 / 34 (480), 2 x 383 42 / 39 (656), 768 53 / 50 (720), 1024 66 / 78 (1000): two full rounds, of which the second holds the longest walks.  Padded 2 x 1500 92 / 54, documents of
+// 700, 300 and 500 67 / 52.  Against the 64-key kernel (2048 tokens and more) and for padded and packed rows the line is lower: 8 heads on one 2500 tokens 137 / 75 (318), 4000 169 / 110
+// (506); on two 2500 110 / 92 (478), 4000 131 / 147 (762), in three documents 89 / 93.
 bool both_route(const gptoss_attn_params *p, KArgs &a) {
     if (p->dtype != GPTOSS_ATTN_BF16 || a.r < 4 || window_single_pass(p)) return false;
+    if (p->seqlens && p->Skv >= 2048) return false;        // (attn_bwd_dkdv64_kernel reads no row of the padding, attn_bwd_dkdv_kernel those that share a tile)
     dkdv_pieces_for(p, a);
     return q_outer_grid(a, 4, 1) + dkdv_grid(a) <= (p->Skv >= 2048 || p->seqlens || p->doc_start ? 640 : 768);
 }
