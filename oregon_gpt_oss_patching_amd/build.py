@@ -59,7 +59,7 @@ def build_torch_ops(verbose: bool = False) -> str:
           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
           "-isystem", os.path.join(root, "include"), "-isystem", os.path.join(root, "include", "torch", "csrc", "api", "include"),
           "-isystem", os.path.join(rocm, "include"), "-isystem", sysconfig.get_paths()["include"], "-o", TORCH_LIBRARY, TORCH_SOURCE,
-          "-L" + os.path.join(root, "lib"), "-lc10", "-ltorch_cpu", "-lc10_hip", "-L" + _HERE, "-lgptoss_attn", "-Wl,-rpath,$ORIGIN"], verbose)
+          "-L" + os.path.join(root, "lib"), "-lc10", "-ltorch_cpu", "-lc10_hip", "-ltorch_hip", "-L" + _HERE, "-lgptoss_attn", "-Wl,-rpath,$ORIGIN"], verbose)
     return TORCH_LIBRARY
 
 

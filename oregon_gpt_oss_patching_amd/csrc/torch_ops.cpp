@@ -10,6 +10,7 @@
 // whatever the size; the same calls through this file take 60 to 90 us for two rows of 383 tokens, 88 for a sliding-window layer of
 // 4096, of which 64 and 83 are kernels, and a decoding step 13 us instead of 44).  This file is built against torch; the kernels are not.
 #include <ATen/ATen.h>
+#include <ATen/hip/EmptyTensor.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <pybind11/pybind11.h>
@@ -62,6 +63,11 @@ void check_inputs(const Tensor &q, const Tensor &k, const Tensor &v, const OptTe
     }
     require_on(q, "k", k);
     require_on(q, "v", v);
+}
+
+// Memory for a result or for scratch, without the dispatcher: every value of it is written before it is read.  A call's allocations are a tenth of its host time.
+Tensor new_tensor(at::IntArrayRef sizes, at::ScalarType dtype, const Tensor &like) {
+    return Tensor(at::detail::empty_cuda(sizes, dtype, like.device(), std::nullopt));
 }
 
 void set(gptoss_attn_strides &s, const Tensor &t, bool bshd) {
@@ -142,14 +148,14 @@ std::tuple<Tensor, Tensor> fwd(const Tensor &q, const Tensor &k, const Tensor &v
     const c10::OptionalDeviceGuard guard(q.device());
     Call c;
     fill(c, q, k, v, sinks, sm_scale, window, q_offset, seqlens, doc_start, q_offset_dev);
-    Tensor o = at::empty({q.size(0), q.size(2), q.size(1), q.size(3)}, q.options());
-    Tensor lse = at::empty({q.size(0), q.size(1), q.size(2)}, q.options().dtype(at::kFloat));
+    Tensor o = new_tensor({q.size(0), q.size(2), q.size(1), q.size(3)}, q.scalar_type(), q);
+    Tensor lse = new_tensor({q.size(0), q.size(1), q.size(2)}, at::kFloat, q);
     c.p.o = o.data_ptr();
     c.p.lse = lse.data_ptr<float>();
     set(c.p.o_stride, o, true);
     // partial results of few queries' or few heads' rows, cut over their keys; records of float32 operands
     const size_t need = c.p.dtype == GPTOSS_ATTN_FP32 ? gptoss_attn_split_bytes(&c.p, 0) : gptoss_attn_fwd_workspace_bytes(&c.p);
-    const Tensor scratch = need ? at::empty({static_cast<int64_t>(need / sizeof(float))}, lse.options()) : Tensor();
+    const Tensor scratch = need ? new_tensor({static_cast<int64_t>(need / sizeof(float))}, at::kFloat, q) : Tensor();
     check("gptoss_attn_fwd", gptoss_attn_fwd_scratch(&c.p, c.sinks_dtype, need ? scratch.data_ptr() : nullptr, need, stream_of(c)));
     return {o, lse};
 }
@@ -173,13 +179,13 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> bwd(const Tensor &q, const Tensor &k,
     TORCH_CHECK(lse_.sizes() == at::IntArrayRef({b, h, s}), "lse must be (B, H, S) = ", at::IntArrayRef({b, h, s}), ", got ", lse_.sizes());
     const Tensor o = row_contiguous(o_, 1), d_o = row_contiguous(d_o_, 1), lse = lse_.contiguous();
 
-    Tensor dq = at::empty({b, h, s, d}, q.options()), dk = at::empty(k.sizes(), k.options()), dv = at::empty(v.sizes(), v.options());
+    Tensor dq = new_tensor({b, h, s, d}, q.scalar_type(), q), dk = new_tensor(k.sizes(), k.scalar_type(), q), dv = new_tensor(v.sizes(), v.scalar_type(), q);
     const bool bf16_dsinks = dsinks_as_sinks && c.sinks_dtype == GPTOSS_ATTN_BF16;
-    Tensor dsinks = at::empty({need_dsinks ? h : 0}, lse.options().dtype(bf16_dsinks ? at::kBFloat16 : at::kFloat));
+    Tensor dsinks = new_tensor({need_dsinks ? h : 0}, bf16_dsinks ? at::kBFloat16 : at::kFloat, q);
     // scratch: the row statistics, then the dK/dV partial sums of split key blocks or the window kernel's shares; the records of float32
     // operands as bf16 terms are a scratch of their own, and with them the first is two floats per row
     const size_t records = gptoss_attn_split_bytes(&c.p, 1);
-    Tensor scratch = at::empty({records ? 2 * b * h * s : static_cast<int64_t>(gptoss_attn_bwd_workspace_bytes(&c.p) / sizeof(float))}, lse.options());
+    Tensor scratch = new_tensor({records ? 2 * b * h * s : static_cast<int64_t>(gptoss_attn_bwd_workspace_bytes(&c.p) / sizeof(float))}, at::kFloat, q);
     gptoss_attn_params &p = c.p;
     p.o = const_cast<void *>(o.const_data_ptr());             // (read only here)
     p.lse = const_cast<float *>(lse.const_data_ptr<float>());
@@ -194,7 +200,7 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> bwd(const Tensor &q, const Tensor &k,
     set(p.dq_stride, dq, false);
     set(p.dk_stride, dk, false);
     set(p.dv_stride, dv, false);
-    const Tensor split = records ? at::empty({static_cast<int64_t>(records / sizeof(float))}, lse.options()) : Tensor();
+    const Tensor split = records ? new_tensor({static_cast<int64_t>(records / sizeof(float))}, at::kFloat, q) : Tensor();
     check("gptoss_attn_bwd", gptoss_attn_bwd_scratch(&c.p, c.sinks_dtype, bf16_dsinks ? GPTOSS_ATTN_BF16 : GPTOSS_ATTN_FP32,
                                                      records ? split.data_ptr() : nullptr, records, stream_of(c)));
     return {dq, dk, dv, dsinks};
@@ -252,7 +258,8 @@ struct AttentionFunction : public torch::autograd::Function<AttentionFunction> {
         // a first-order backward needs no autograd bookkeeping; under create_graph the operator records that it has no second derivative
         std::optional<at::AutoDispatchBelowADInplaceOrView> below;
         if (!at::GradMode::is_enabled()) below.emplace();
-        auto [dq, dk, dv, dsinks] = call_bwd(q, saved[1], saved[2], optional_of(sinks), saved[4], saved[5], grads[0].to(q.scalar_type()),
+        auto [dq, dk, dv, dsinks] = call_bwd(q, saved[1], saved[2], optional_of(sinks), saved[4], saved[5],
+                                             grads[0].scalar_type() == q.scalar_type() ? grads[0] : grads[0].to(q.scalar_type()),
                                              ctx->saved_data["sm_scale"].toDouble(), ctx->saved_data["window"].toSymInt(),
                                              ctx->saved_data["q_offset"].toSymInt(), optional_of(saved[6]), optional_of(saved[7]), need_dsinks,
                                              optional_of(saved[8]), true);
@@ -261,7 +268,10 @@ struct AttentionFunction : public torch::autograd::Function<AttentionFunction> {
             dk = dk.to(at::kHalf);
             dv = dv.to(at::kHalf);
         }
-        return {dq, dk, dv, need_dsinks ? dsinks.to(sinks.scalar_type()).view_as(sinks) : Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+        // (a logit per head in one dimension, as a rule: dsinks is what it has to be)
+        if (!need_dsinks) dsinks = Tensor();
+        else if (dsinks.scalar_type() != sinks.scalar_type() || sinks.dim() != 1) dsinks = dsinks.to(sinks.scalar_type()).view_as(sinks);
+        return {dq, dk, dv, dsinks, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
     }
 };
 
