@@ -874,13 +874,14 @@ __device__ __forceinline__ void dq_workgroup(const KArgs &a, int bid) {
 template <int HPB, int NQB, bool FUSE_DELTA>
 __global__ __launch_bounds__(256, (NQB == 1 ? 3 : 2)) void attn_bwd_dq_kernel(const KArgs a) { dq_workgroup<HPB, NQB, FUSE_DELTA>(a, blockIdx.x); }
 
-// dQ and dK/dV side by side: the first workgroups are attn_bwd_dkdv_kernel's, the others attn_bwd_dq_kernel's (32-row wavefronts), with the same bits.  Either alone is a
+// dQ and dK/dV side by side: from dkdv_at on the workgroups are attn_bwd_dkdv_kernel's, from dq_at on attn_bwd_dq_kernel's (32-row wavefronts), with the same bits.  Either alone is a
 // chain of latencies, 7 us and 1.1 to 1.9 per (query tile, head) or key tile of its longest walk, which leaves most of a compute unit idle; the row statistics, which dQ forms on
 // its way for the dK/dV kernel otherwise, come from attn_bwd_delta_kernel here (4 us).  Taken where everything fits the chip at once (both_route).
 template <bool DOCS, bool PIECES>
-__global__ __launch_bounds__(256, 2) void attn_bwd_both_kernel(const KArgs a, int dkdv_workgroups) {
-    if ((int)blockIdx.x < dkdv_workgroups) dkdv_workgroup<4, 1, DOCS, PIECES>(a, blockIdx.x);
-    else dq_workgroup<4, 1, false>(a, blockIdx.x - dkdv_workgroups);
+__global__ __launch_bounds__(256, 2) void attn_bwd_both_kernel(const KArgs a, int dkdv_at, int dq_at) {
+    const int bid = blockIdx.x;
+    if (dkdv_at > dq_at ? bid >= dkdv_at : bid < dq_at) dkdv_workgroup<4, 1, DOCS, PIECES>(a, bid - dkdv_at);
+    else dq_workgroup<4, 1, false>(a, bid - dq_at);
 }
 
 }  // namespace gptoss

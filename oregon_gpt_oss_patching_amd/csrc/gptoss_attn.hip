@@ -217,12 +217,18 @@ bool window_single_pass(const gptoss_attn_params *p);
 // 4 x 2000 114 / 119 (992); 8 on two 2 x 1500 74 / 65 (500), 4 x 1000 58 / 54 (744); 32 on four 700 49 / 32 (320), 1500 90 / 76 (736), 2000 114 / 118 (992); 64 on eight 256 30 / 25
 // (192), 512 37 / 34 (480), 2 x 383 42 / 39 (656), 768 53 / 50 (720), 1024 66 / 78 (1000): two full rounds, of which the second holds the longest walks.  Padded 2 x 1500 92 / 54, documents of
 // 700, 300 and 500 67 / 52.  Against the 64-key kernel (2048 tokens and more) and for padded and packed rows the line is lower: 8 heads on one 2500 tokens 137 / 75 (318), 4000 169 / 110
-// (506); on two 2500 110 / 92 (478), 4000 131 / 147 (762), in three documents 89 / 93.
-bool both_route(const gptoss_attn_params *p, KArgs &a) {
-    if (p->dtype != GPTOSS_ATTN_BF16 || a.r < 4 || window_single_pass(p)) return false;
-    if (p->seqlens && p->Skv >= 2048) return false;        // (attn_bwd_dkdv64_kernel reads no row of the padding, attn_bwd_dkdv_kernel those that share a tile)
+// (506).
+// dK/dV's workgroups start first, or dQ's, which are the longest where a KV head has one chunk of four heads, and in long rows that are more than two per unit: dK/dV's / dQ's first, 8 heads
+// on two 1500 tokens twice 66 / 57, 2500 92 / 74 (one after the other 112), 3000 118 / 85 (125), 4000 146 / 120 (127), documents of 2000 and 1000 87 / 75 (95), but 8 x 500 39 / 43; on one 5000
+// 188 / 174 (231), 6000 251 / 232 (264), 2 x 3000 147 / 137 (151), but 4000 (506) 109 / 115, 3 x 2048 (768) 99 / 110 (104), documents of 1700, 1300 and 2500 117 / 143.
+struct BothRoute { bool taken, dq_first; };
+BothRoute both_route(const gptoss_attn_params *p, KArgs &a) {
+    if (p->dtype != GPTOSS_ATTN_BF16 || a.r < 4 || window_single_pass(p)) return {false, false};
+    if (p->seqlens && p->Skv >= 2048) return {false, false};    // (attn_bwd_dkdv64_kernel reads no row of the padding, attn_bwd_dkdv_kernel those that share a tile)
     dkdv_pieces_for(p, a);
-    return q_outer_grid(a, 4, 1) + dkdv_grid(a) <= (p->Skv >= 2048 || p->seqlens || p->doc_start ? 640 : 768);
+    const int64_t all = q_outer_grid(a, 4, 1) + dkdv_grid(a);
+    const bool one_chunk = a.r == 4 && p->Sq >= 1024, rows_differ = p->seqlens || p->doc_start, longer = p->Skv >= 2048 && !rows_differ;
+    return {all <= (rows_differ && !(one_chunk && p->doc_start) ? 640 : p->Skv >= 2048 ? 767 : 768), one_chunk || (longer && all > 512)};
 }
 
 // Full-causal self-attention goes to attn_bwd_dkdv64_kernel (64 keys per wavefront, one wavefront per SIMD)
@@ -246,7 +252,7 @@ bool dkdv64_route(const gptoss_attn_params *p, int parts) {
     if (parts > 1) {
         KArgs a = make_args(p, {});
         a.dkdv_parts = parts;
-        if (both_route(p, a)) return false;
+        if (both_route(p, a).taken) return false;
     }
     return p->dtype == GPTOSS_ATTN_BF16 && effective_window(p) == 0 && p->q_offset == 0 && !p->q_offset_dev && p->Sq == p->Skv &&
            p->Sq >= kTile && (blocks > 512 || (parts > 1 && p->Skv >= 2048));
@@ -912,15 +918,15 @@ static int launch_f32_both(KArgs &a, hipStream_t st) {
 }
 
 // dQ and dK/dV side by side, behind the row statistics.
-static int launch_both(KArgs &a, hipStream_t st) {
+static int launch_both(KArgs &a, hipStream_t st, bool dq_first) {
     int s = launch(attn_bwd_delta_kernel, ((int64_t)a.B * a.H * a.Sq + 127) / 128, 256, st, a);
     if (s) return s;
     const void *kernel = a.doc_start    ? reinterpret_cast<const void *>(attn_bwd_both_kernel<true, false>)
                          : a.dkdv_steps ? reinterpret_cast<const void *>(attn_bwd_both_kernel<false, true>)
                                         : reinterpret_cast<const void *>(attn_bwd_both_kernel<false, false>);
-    int first = (int)dkdv_grid(a);
-    void *args[] = {&a, &first};
-    const hipError_t e = hipLaunchKernel(kernel, dim3((unsigned)(first + q_outer_grid(a, 4, 1))), dim3(256), args, 0, st);
+    int dkdv = (int)dkdv_grid(a), dq = (int)q_outer_grid(a, 4, 1), dkdv_at = dq_first ? dq : 0, dq_at = dq_first ? 0 : dkdv;
+    void *args[] = {&a, &dkdv_at, &dq_at};
+    const hipError_t e = hipLaunchKernel(kernel, dim3((unsigned)(dkdv + dq)), dim3(256), args, 0, st);
     if (e != hipSuccess) return static_cast<int>(e);
     if (a.dkdv_parts > 1) return launch_dkdv_sum(a, st, a.dsinks != nullptr);
     return a.dsinks ? launch(attn_bwd_dsinks_kernel, a.H, 1024, st, a) : GPTOSS_ATTN_OK;
@@ -975,7 +981,8 @@ static int bwd_all(const gptoss_attn_params *p, void *stream, bool whole_blocks,
         a.dkdv_parts = dkdv_parts_for(p, p->seqlens != nullptr, p->doc_start != nullptr);
         a.dkdv_partial = reinterpret_cast<float *>(reinterpret_cast<char *>(p->delta) + stats_bytes(p));
         if (f32_both_route(a, p->dtype)) return launch_f32_both(a, static_cast<hipStream_t>(stream));
-        if (both_route(p, a)) return launch_both(a, static_cast<hipStream_t>(stream));
+        const BothRoute both = both_route(p, a);
+        if (both.taken) return launch_both(a, static_cast<hipStream_t>(stream), both.dq_first);
     }
     rc = launch_dq(p, stream, 1);
     if (rc) return rc;

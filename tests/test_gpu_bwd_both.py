@@ -25,6 +25,10 @@ _CASES = [
     (2, 8, 1, 2100, 2100, None, [2100, 999], None),
     (1, 8, 1, 900, 900, None, None, [1, 63, 500, 336]),  # documents
     (1, 8, 1, 2200, 2200, None, None, [100, 1400, 700]),
+    (1, 8, 2, 1024, 1024, None, None, None),             # dQ first: one chunk of heads, a row in front of the line, packed, long rows of two
+    (1, 8, 2, 1023, 1023, None, None, None),
+    (1, 8, 2, 2600, 2600, None, None, [1000, 1599, 1]),
+    (1, 8, 1, 4400, 4400, None, None, None),
     (1, 8, 2, 500, 500, 200, None, None),                # windows the single-pass kernel does not take
     (1, 8, 2, 500, 500, 130, None, [170, 330]),
     (1, 8, 1, 400, 400, 100, None, [250, 150]),
