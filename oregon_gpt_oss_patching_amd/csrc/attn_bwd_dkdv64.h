@@ -664,8 +664,12 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv64_kernel(const KArgs a) 
     }
 }
 
-// The partial sums of the cut key blocks, in the order of their pieces, scaled and rounded; sixteen workgroups per block, a thread
-// per 16-byte output chunk.  The first `heads` workgroups produce dSinks.
+// The partial sums of the cut key blocks, in the order of their pieces, scaled and rounded; kChunks 16-byte output chunks per thread, 16 / kChunks workgroups per
+// block.  What bounds it: finding the pieces, about 5 us, which every workgroup does for itself: four chunks where one would be many workgroups (launch, us, one / four: 4 x 4096
+// tokens padded to 3309, 1968, 1554 and 4079 22.2 / 12.7, 8192 in seven documents 19.0 / 11.4, 5 x 2265 16.1 / 10.8, but 8000 of 8 heads, 512 workgroups, 12.6 / 17.0, and the whole call of 96 key blocks 332 / 333).  The first `heads`
+// workgroups produce dSinks.
+constexpr int dkdv64_reduce_chunks(int64_t key_blocks) { return key_blocks > 128 ? 4 : 1; }
+template <int kChunks>
 __global__ __launch_bounds__(256) void attn_bwd_dkdv64_reduce_kernel(const KArgs a, int heads) {
     __shared__ int lds[Dkdv64Plan::kMaxBlocks];
     __shared__ float red[1024];
@@ -673,29 +677,45 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv64_reduce_kernel(const KArgs
     const int tid = threadIdx.x, lane = tid & 63, nblk = a.B * ((a.Skv + Dkdv64::BN - 1) / Dkdv64::BN);
     int bid = blockIdx.x - heads;
     const int g = bid % a.G; bid /= a.G;
-    const int chunk = (bid & 15) * 256 + tid, block = bid >> 4, kt = block / a.B, b = block % a.B;
+    const int first = bid % (16 / kChunks) * (kChunks * 256) + tid, block = bid / (16 / kChunks), kt = block / a.B, b = block % a.B;
     Dkdv64Plan::lengths(a, nblk, lds, tid);
     const Dkdv64Plan plan(a, lds, nblk, a.dkdv_slots, lane);
     const int n = plan.cuts(lds[block]);
     if (n == 0) return;
-    const int which = chunk >> 11, key = (chunk >> 3) & (Dkdv64::BN - 1), c8 = (chunk & 7) * 8, j = kt * Dkdv64::BN + key;
-    const bool live = j < a.Skv;               // (the counting takes whole wavefronts)
-    const float *src = a.dkdv_partial + (int64_t)g * a.dkdv_slots * kDkdv64Slot + (which * Dkdv64::BN + key) * kD + c8;       // (a slot holds all 256 keys)
-    float x[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+    // chunk = (tensor, key, eight columns), the order in which a slot holds them (all 256 keys)
+    const float *src = a.dkdv_partial + (int64_t)g * a.dkdv_slots * kDkdv64Slot + first * 8;
+    float x[kChunks][8];
+#pragma unroll
+    for (int c = 0; c < kChunks; ++c)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[c][e] = 0.0f;
     int before = 0;                            // full pieces of smaller number
     for (int i = 0; i <= n; ++i) {
         const float *p = src + (int64_t)(i < n ? before + plan.count_cut(i, block) : plan.full + plan.count_cut(0, block)) * kDkdv64Slot;
         if (i < n) before += plan.count_cut(i, nblk);
-        const f32x4 y = *reinterpret_cast<const f32x4 *>(p), z = *reinterpret_cast<const f32x4 *>(p + 4);
+        f32x4 y[kChunks], z[kChunks];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) { x[e] += y[e]; x[4 + e] += z[e]; }
+        for (int c = 0; c < kChunks; ++c) {
+            y[c] = *reinterpret_cast<const f32x4 *>(p + c * 2048);
+            z[c] = *reinterpret_cast<const f32x4 *>(p + c * 2048 + 4);
+        }
+#pragma unroll
+        for (int c = 0; c < kChunks; ++c)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) { x[c][e] += y[c][e]; x[c][4 + e] += z[c][e]; }
     }
+    const int which = first >> 11;             // (a workgroup's chunks are of one tensor)
     const float mul = which == 0 ? a.scale : 1.0f;
-    union { bf16x8 v; u32x4 u; } out;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) out.v[e] = (bf16)(x[e] * mul);
     const Strides &st = which == 0 ? a.dks : a.dvs;
-    if (live) *reinterpret_cast<u32x4 *>((which == 0 ? a.dk : a.dv) + (int64_t)b * st.b + (int64_t)g * st.h + (int64_t)j * st.s + c8) = out.u;
+    bf16 *dst = (which == 0 ? a.dk : a.dv) + (int64_t)b * st.b + (int64_t)g * st.h + (tid & 7) * 8;
+#pragma unroll
+    for (int c = 0; c < kChunks; ++c) {
+        const int j = kt * Dkdv64::BN + (((first + c * 256) >> 3) & (Dkdv64::BN - 1));
+        union { bf16x8 v; u32x4 u; } out;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) out.v[e] = (bf16)(x[c][e] * mul);
+        if (j < a.Skv) *reinterpret_cast<u32x4 *>(dst + (int64_t)j * st.s) = out.u;
+    }
 }
 
 }  // namespace gptoss

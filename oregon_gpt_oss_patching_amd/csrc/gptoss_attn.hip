@@ -887,7 +887,9 @@ static int launch_dkdv(const gptoss_attn_params *p, void *stream, bool whole_blo
         const bool plain = !by_lengths && !a.seqlens && !a.doc_start && a.Sq % kTile == 0;
         const int s = plain ? launch(attn_bwd_dkdv64_kernel<false>, grid64, 256, st, a) : launch(attn_bwd_dkdv64_kernel<true>, grid64, 256, st, a);
         if (s || a.dkdv_parts == 1) return s;
-        if (by_lengths) return launch_reduce(attn_bwd_dkdv64_reduce_kernel, a.G * blocks * 16 * 256, st, a, with_dsinks);
+        if (by_lengths)
+            return dkdv64_reduce_chunks(a.G * blocks) == 4 ? launch_reduce(attn_bwd_dkdv64_reduce_kernel<4>, a.G * blocks * 4 * 256, st, a, with_dsinks)
+                                                           : launch_reduce(attn_bwd_dkdv64_reduce_kernel<1>, a.G * blocks * 16 * 256, st, a, with_dsinks);
         return launch_reduce(attn_bwd_dkdv_reduce_kernel, (int64_t)2 * a.B * a.G * ((a.Skv + 31) / 32) * 256, st, a, with_dsinks);
     }
     dkdv_pieces_for(p, a);
