@@ -10,8 +10,8 @@
 //   * five "owners".  Owner p holds, as MFMA B operands in registers, the K and V rows of the one live key block kb with
 //     kb % 5 == p and its group's dK / dV accumulators of that block.  Per step an owner does one 32 x 32 block
 //     (window_block: S = Q K^T, dP = dO V^T, P, dS, dV^T += dO^T P, dK^T += Q^T dS) and leaves the bf16 dS block in LDS,
-//     key-major.  When the walk moves on to query block u, key block u-5 is complete: group 1's owner has left its sums in
-//     LDS, group 0's adds them and writes dK / dV out, and both take over key block u.
+//     key-major.  When the walk moves on to query block u, key block u-5 is complete: its two owners have exchanged
+//     one tensor each through LDS, group 0's adds and writes dK, group 1's dV, and both take over key block u.
 //   * one "helper".  One step AHEAD of the owners it forms the row statistics -lse / scale and -rowsum(dO*O) of the
 //     group's 32 rows (dO from the staged tile, O rows it reads itself) and leaves them in LDS; one step BEHIND them it turns
 //     the dS blocks into dQ^T = K^T dS^T over all 160 live keys (K^T fragments resident in its registers) and writes the finished
@@ -38,7 +38,9 @@
 // fragments under way.  Whole backward, us, six owners with 64-row tiles and two helpers (two wavefronts per SIMD, one head per step) / so: 16384 tokens of 64
 // heads on 8 KV heads 204 / 176, 2 x 3001 77 / 68, 4096 56.5 / 51.5.  What bounds it: all the copies, loads and stores without the owners' arithmetic take 134 us at 16384
 // (660 MB, 4.9 TB/s), everything but the tiles' copies 128 us (1.8 us a step; matrix pipe 30 % busy, LDS 33 %), and a workgroup per compute unit lays
-// the one over the other only in part.  The merge of the two groups' sums and the results' way out are 14 us of it, once in five blocks per owner.
+// the one over the other only in part.  The merge of the two groups' sums and the results' way out, once in
+// five blocks per owner, were 14 us of it with one owner per block doing both tensors and are 11 with one tensor each (whole call, 16384 tokens 256 / 253, 2 x 3001 105.7 / 104.8).  A block's start and end
+// cost about one step: 4096 tokens are four blocks of four steps per workgroup, 29 of 48 us.
 #pragma once
 #include <type_traits>
 
@@ -244,7 +246,7 @@ __global__ __launch_bounds__(WinCfg::NWAVES * 64, 1) void attn_bwd_window_kernel
     // key block that slot p holds while the walk is at query block u: the one of u-4 .. u that is congruent to p modulo 5
     auto block_of_slot = [](int p, int u) { return u - ((u - p) % C::NSLOT + C::NSLOT) % C::NSLOT; };
 
-    // ---- copies of the walk's Q / dO tiles: wavefronts 5 to 8 (owners of group 1, which write no results), one (group, tensor) each,
+    // ---- copies of the walk's Q / dO tiles: wavefronts 5 to 8 (owners of group 1), one (group, tensor) each,
     // four 16-byte-per-lane instructions per step; K / V of the next key block: wavefront 9 ----
     constexpr int kWaveTile0 = C::NSLOT, kWaveTransit = C::NSLOT + 4;
     const bool copies = w >= kWaveTile0 && w < kWaveTile0 + 4;
@@ -569,7 +571,7 @@ __global__ __launch_bounds__(WinCfg::NWAVES * 64, 1) void attn_bwd_window_kernel
         at_stage = to;
     };
     auto copy_ahead = [&]() __attribute__((always_inline)) {
-        // (one step per query block: group 0 may still be reading the sums that group 1 left)
+        // (one step per query block: the other group may still be reading the sums that this one left)
         if (pairs == 1) __syncthreads();
         if (w == kWaveTransit && hp == 0 && u + 1 < u1) issue_transit(u + 1);
         if (copies && it + NS - 1 < n_it) issue(it + NS - 1);
