@@ -55,6 +55,9 @@ struct WinCfg {
     static constexpr int kMaxWindow = 128;
     static constexpr int kBack = kMaxWindow / kRows;                       // key blocks in front of a query block's own that it sees
     static constexpr int kMaxGroup = 16;                                   // query heads per KV head
+    // The weights are exp(scale * (S - lse / scale)), whose quotient has to stay finite.  Smaller scales take this one's weights: a sum of up to 128 exponentials and a
+    // sink has an lse below 2^11 (or no room beside its sink), and S is nothing beside it up to 2^100.
+    static constexpr float kMinScale = 0x1p-116f;
     static constexpr int kBlockBytes = kRows * kRowBytes;                  // 4 KB: a block's rows of one tensor
     static constexpr int kMergeBytes = 2 * 2 * 16 * 64 * 4;                // an owner's dK and dV accumulators
     static constexpr int kStageOff = 0;                                    // [NS][group][Q, dO][4 KB]; behind the walk four merge buffers
@@ -335,7 +338,7 @@ __global__ __launch_bounds__(WinCfg::NWAVES * 64, 1) void attn_bwd_window_kernel
         const char *o_at = reinterpret_cast<const char *>(a.o + (int64_t)b * a.os.b + head0 * a.os.h + row_0 * a.os.s);
         const char *lse_at = reinterpret_cast<const char *>(a.lse + ((int64_t)b * a.H + head0) * a.Sq + row_0);
         const char *dq_at = reinterpret_cast<const char *>(a.dq + (int64_t)b * a.dqs.b + head0 * a.dqs.h + row_0 * a.dqs.s);
-        const float inv_scale = 1.0f / a.scale;
+        const float inv_scale = 1.0f / fmaxf(a.scale, C::kMinScale);
         // O half rows + lse of this lane's row of a walk position (rows past the end of the tensor re-read the last one)
         u32x4 pre_o[4];
         float pre_lse = 0.0f;

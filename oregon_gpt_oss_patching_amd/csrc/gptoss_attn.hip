@@ -577,6 +577,7 @@ int launch_window_bwd(const gptoss_attn_params *p, hipStream_t st, bool seam_sum
     if (rc) return rc;
     KArgs a = make_args(p, ty);
     const WindowScratch ws = window_scratch(p, compute_units());
+    a.scale_log2 = (p->scale > WinCfg::kMinScale ? p->scale : WinCfg::kMinScale) * kLog2e;
     a.chunk_blocks = ws.chunk_blocks;
     a.dsink_partial = p->delta;
     if (seam_sums && ws.n_chunks > 1)
