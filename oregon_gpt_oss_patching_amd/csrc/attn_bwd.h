@@ -275,17 +275,30 @@ struct DkdvPieces {
     }
 };
 
+// Staging memory of a dK/dV and of a dQ workgroup.  The kernel declares it and hands it over: the kernel that holds both kinds gives them the same bytes.
+template <bool DOCS>
+struct DkdvLds {
+    static constexpr int NS = 3;       // LDS stages: tiles are requested two iterations ahead
+    char tile[NS][2][kStageTileBytes];                    // Q, dO
+    u32x4 stat[NS][kTile];                                // split row statistics of the staged rows
+    int32_t doc[DOCS ? NS : 1][kTile];                    // document starts of the staged rows
+};
+struct DqLds {
+    static constexpr int NS = 3;
+    char tile[NS][2][kStageTileBytes];                    // K, V
+};
+
 // NB = 32-key blocks per wavefront; DOCS = packed rows (doc_start given); PIECES: DkdvPieces (an instantiation: the slices' one is 4 % slower with both)
 template <int NW, int NB, bool DOCS, bool PIECES>
-__device__ __forceinline__ void dkdv_workgroup(const KArgs &a, int bid) {
+__device__ __forceinline__ void dkdv_workgroup(const KArgs &a, int bid, DkdvLds<DOCS> &lds) {
     const int q_offset = query_offset(a);
     static_assert(NW == 4, "the asynchronous tile copy is written for 4 wavefronts");
-    constexpr int NS = 3;              // LDS stages: tiles are requested two iterations ahead
+    constexpr int NS = DkdvLds<DOCS>::NS;
     constexpr int WK = 32 * NB;        // keys per wavefront
     constexpr int BN = WK * NW;        // keys per workgroup
-    __shared__ __attribute__((aligned(16))) char smem[NS][2][kStageTileBytes];
-    __shared__ __attribute__((aligned(16))) u32x4 sstat[NS][kTile];               // split row statistics of the staged rows
-    __shared__ __attribute__((aligned(16))) int32_t sdoc[DOCS ? NS : 1][kTile];   // document starts of the staged rows
+    auto &smem = lds.tile;
+    auto &sstat = lds.stat;
+    auto &sdoc = lds.doc;
 
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int l32 = lane & 31, half = lane >> 5;
@@ -527,7 +540,10 @@ __device__ __forceinline__ void dkdv_workgroup(const KArgs &a, int bid) {
 }
 
 template <int NW, int NB, bool DOCS, bool PIECES = false>
-__global__ __launch_bounds__(NW * 64, (NB == 1 ? 2 : 1)) void attn_bwd_dkdv_kernel(const KArgs a) { dkdv_workgroup<NW, NB, DOCS, PIECES>(a, blockIdx.x); }
+__global__ __launch_bounds__(NW * 64, (NB == 1 ? 2 : 1)) void attn_bwd_dkdv_kernel(const KArgs a) {
+    __shared__ __attribute__((aligned(16))) DkdvLds<DOCS> lds;
+    dkdv_workgroup<NW, NB, DOCS, PIECES>(a, blockIdx.x, lds);
+}
 
 // ---------------------------------------------------------------------------------
 // Sum of the dK / dV partials of a split key block, in part order (bit-reproducible), scaled and
@@ -678,13 +694,13 @@ __device__ __forceinline__ void dq_tile(uint32_t ksm, uint32_t vsm, const TileLa
 }
 
 template <int HPB, int NQB, bool FUSE_DELTA>   // FUSE_DELTA: also produce the row statistics of the wavefront's own rows
-__device__ __forceinline__ void dq_workgroup(const KArgs &a, int bid) {
+__device__ __forceinline__ void dq_workgroup(const KArgs &a, int bid, DqLds &lds) {
     const int q_offset = query_offset(a);
     constexpr int QSUB = 4 / HPB;
     constexpr int WM = 32 * NQB;
     constexpr int BM = WM * QSUB;
-    constexpr int NS = 3;
-    __shared__ __attribute__((aligned(16))) char smem[NS][2][kStageTileBytes];
+    constexpr int NS = DqLds::NS;
+    auto &smem = lds.tile;
 
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int l32 = lane & 31, half = lane >> 5;
@@ -872,16 +888,23 @@ __device__ __forceinline__ void dq_workgroup(const KArgs &a, int bid) {
 }
 
 template <int HPB, int NQB, bool FUSE_DELTA>
-__global__ __launch_bounds__(256, (NQB == 1 ? 3 : 2)) void attn_bwd_dq_kernel(const KArgs a) { dq_workgroup<HPB, NQB, FUSE_DELTA>(a, blockIdx.x); }
+__global__ __launch_bounds__(256, (NQB == 1 ? 3 : 2)) void attn_bwd_dq_kernel(const KArgs a) {
+    __shared__ __attribute__((aligned(16))) DqLds lds;
+    dq_workgroup<HPB, NQB, FUSE_DELTA>(a, blockIdx.x, lds);
+}
 
-// dQ and dK/dV side by side: from dkdv_at on the workgroups are attn_bwd_dkdv_kernel's, from dq_at on attn_bwd_dq_kernel's (32-row wavefronts), with the same bits.  Either alone is a
-// chain of latencies, 7 us and 1.1 to 1.9 per (query tile, head) or key tile of its longest walk, which leaves most of a compute unit idle; the row statistics, which dQ forms on
-// its way for the dK/dV kernel otherwise, come from attn_bwd_delta_kernel here (4 us).  Taken where everything fits the chip at once (both_route).
+// dQ and dK/dV side by side: from dkdv_at on the workgroups are attn_bwd_dkdv_kernel's, from dq_at on attn_bwd_dq_kernel's (32-row
+// wavefronts), with the same bits.  Either alone is a chain of latencies, 7 us and 1.1 to 1.9 per (query tile, head) or key tile of its longest
+// walk, with most of a compute unit idle at its end; the row statistics, which dQ forms on its way for the dK/dV kernel
+// otherwise, come from attn_bwd_delta_kernel here (4 us).  Both kinds use the same bytes of LDS, so that a compute unit takes two
+// workgroups of any kind (with an array each, 101 KB, it took one: whole backward, us, 64 heads on 8 KV heads 2 x 383 tokens 41 / 34, 1024 74 / 56; 8
+// on one 6000 228 / 199, on two 4000 119 / 94, but 2500 76 / 82: its few long walks then share their units).
 template <bool DOCS, bool PIECES>
 __global__ __launch_bounds__(256, 2) void attn_bwd_both_kernel(const KArgs a, int dkdv_at, int dq_at) {
+    __shared__ __attribute__((aligned(16))) union { DkdvLds<DOCS> dkdv; DqLds dq; } lds;
     const int bid = blockIdx.x;
-    if (dkdv_at > dq_at ? bid >= dkdv_at : bid < dq_at) dkdv_workgroup<4, 1, DOCS, PIECES>(a, bid - dkdv_at);
-    else dq_workgroup<4, 1, false>(a, bid - dq_at);
+    if (dkdv_at > dq_at ? bid >= dkdv_at : bid < dq_at) dkdv_workgroup<4, 1, DOCS, PIECES>(a, bid - dkdv_at, lds.dkdv);
+    else dq_workgroup<4, 1, false>(a, bid - dq_at, lds.dq);
 }
 
 }  // namespace gptoss
