@@ -174,7 +174,7 @@ int dkdv_parts_for(const gptoss_attn_params *p, bool padded, bool packed) {
 }
 
 // Pieces of the 32-key kernel's walks (DkdvPieces) instead of equal slices of whole tiles: the shortest ones, of four steps or more, of which
-// there are no more than 512 (two workgroups per compute unit of a 256-CU part: all run at once and end together) and than the
+// there are no more than 512 (two workgroups per compute unit of a 256-CU part: in a launch of their own all run at once and end together) and than the
 // scratch has slots for.  Taken for one row where they are no longer than the longest slice, for several (whose tiles a piece that starts elsewhere does
 // not find in L2) where they are shorter.  dK/dV and the sum of its parts, us, slices / pieces: 2 x 383 tokens 29.8 / 26.9, 2 x 621 47.0 / 37.5,
 // 1 x 1024 47.0 / 41.5, 1 x 1900 95 / 83; not taken: 4 x 1000 (pieces as long as the slices) whole call 227 / 234, 3 x 1200 (longer)
@@ -206,31 +206,19 @@ int64_t q_outer_grid(const KArgs &a, int hpb, int qb) {
     const int n_hc = (a.r + hpb - 1) / hpb;
     return (int64_t)a.G * n_hc * a.B * ((a.Sq + bm - 1) / bm);
 }
+// 32-row query blocks per wavefront of the dQ kernel.  Short problems: 64-row workgroups (two per compute unit) would be few and
+// uneven (the key loops grow with the row index); 32-row wavefronts make twice as many, three per SIMD (measured, full causal, B = 1: dQ
+// 0.077 -> 0.066 ms at S = 2048, 0.240 -> 0.218 at S = 4096, equal from S = 8192 on, 6 % slower at S = 16384).
+int compute_units();
+int dq_query_blocks(const KArgs &a) {
+    const int qb = query_blocks_for(a.window);
+    return qb == 2 && q_outer_grid(a, hpb_for(a.r), 2) <= 4 * (int64_t)compute_units() ? 1 : qb;
+}
 // Workgroups of attn_bwd_dkdv_kernel.
 int64_t dkdv_grid(const KArgs &a) {
     return (int64_t)a.G * a.B * (a.dkdv_steps ? a.dkdv_slots : a.dkdv_parts * ((a.Skv + kDkdvKeys - 1) / kDkdvKeys));
 }
 bool window_single_pass(const gptoss_attn_params *p);
-// dQ and dK/dV in one launch (attn_bwd_both_kernel) behind one for the row statistics, instead of one after the other: where their workgroups, two to a compute
-// unit of a 256-CU part, are few enough to run side by side.  `a` has the backward's dkdv_parts; gets its pieces.  Whole backward, us in a graph, one after the
-// other / side by side (workgroups): 8 heads on one KV head 300 tokens 34 / 26 (29), 1300 70 / 45 (161), 2000 96 / 61 (248), 2 x 1500 78 / 54 (368), 4 x 1000 61 / 50 (500),
-// 4 x 2000 114 / 119 (992); 8 on two 2 x 1500 74 / 65 (500), 4 x 1000 58 / 54 (744); 32 on four 700 49 / 32 (320), 1500 90 / 76 (736), 2000 114 / 118 (992); 64 on eight 256 30 / 25
-// (192), 512 37 / 34 (480), 2 x 383 42 / 39 (656), 768 53 / 50 (720), 1024 66 / 78 (1000): two full rounds, of which the second holds the longest walks.  Padded 2 x 1500 92 / 54, documents of
-// 700, 300 and 500 67 / 52.  Against the 64-key kernel (2048 tokens and more) and for padded and packed rows the line is lower: 8 heads on one 2500 tokens 137 / 75 (318), 4000 169 / 110
-// (506).
-// dK/dV's workgroups start first, or dQ's, which are the longest where a KV head has one chunk of four heads, and in long rows that are more than two per unit: dK/dV's / dQ's first, 8 heads
-// on two 1500 tokens twice 66 / 57, 2500 92 / 74 (one after the other 112), 3000 118 / 85 (125), 4000 146 / 120 (127), documents of 2000 and 1000 87 / 75 (95), but 8 x 500 39 / 43; on one 5000
-// 188 / 174 (231), 6000 251 / 232 (264), 2 x 3000 147 / 137 (151), but 4000 (506) 109 / 115, 3 x 2048 (768) 99 / 110 (104), documents of 1700, 1300 and 2500 117 / 143.
-struct BothRoute { bool taken, dq_first; };
-BothRoute both_route(const gptoss_attn_params *p, KArgs &a) {
-    if (p->dtype != GPTOSS_ATTN_BF16 || a.r < 4 || window_single_pass(p)) return {false, false};
-    if (p->seqlens && p->Skv >= 2048) return {false, false};    // (attn_bwd_dkdv64_kernel reads no row of the padding, attn_bwd_dkdv_kernel those that share a tile)
-    dkdv_pieces_for(p, a);
-    const int64_t all = q_outer_grid(a, 4, 1) + dkdv_grid(a);
-    const bool one_chunk = a.r == 4 && p->Sq >= 1024, rows_differ = p->seqlens || p->doc_start, longer = p->Skv >= 2048 && !rows_differ;
-    return {all <= (rows_differ && !(one_chunk && p->doc_start) ? 640 : p->Skv >= 2048 ? 767 : 768), one_chunk || (longer && all > 512)};
-}
-
 // Full-causal self-attention goes to attn_bwd_dkdv64_kernel (64 keys per wavefront, one wavefront per SIMD)
 // when the shape is the one it is written for (bf16, no window, no offset, Sq == Skv; right-padded batch rows and packed
 // documents are fine) and there is enough of it: more than
@@ -243,19 +231,48 @@ BothRoute both_route(const gptoss_attn_params *p, KArgs &a) {
 bool walk_fits_32_bits(const gptoss_attn_strides &s, int64_t heads, int64_t rows) {
     return s.h >= 0 && ((heads - 1) * s.h + rows * s.s) * 2 < ((int64_t)1 << 31);
 }
-bool dkdv64_route(const gptoss_attn_params *p, int parts) {
+bool dkdv64_shape(const gptoss_attn_params *p, int parts) {
     const int64_t blocks = (int64_t)p->G * p->B * ((p->Skv + kDkdvKeys - 1) / kDkdvKeys);
     const int64_t heads = p->H / p->G;
     if (!walk_fits_32_bits(p->q_stride, heads, p->Sq) || !walk_fits_32_bits(p->do_stride, heads, p->Sq) ||
         heads * p->Sq * 16 >= ((int64_t)1 << 31))
         return false;
-    if (parts > 1) {
-        KArgs a = make_args(p, {});
-        a.dkdv_parts = parts;
-        if (both_route(p, a).taken) return false;
-    }
     return p->dtype == GPTOSS_ATTN_BF16 && effective_window(p) == 0 && p->q_offset == 0 && !p->q_offset_dev && p->Sq == p->Skv &&
            p->Sq >= kTile && (blocks > 512 || (parts > 1 && p->Skv >= 2048));
+}
+
+// dQ and dK/dV in one launch (attn_bwd_both_kernel), behind one for the row statistics, instead of one after the other.  `a` has the
+// backward's dkdv_parts; gets its pieces.
+// What it saves is the end of the first launch, where units wait for its longest walks, and the start of the second; what it adds
+// is the statistics' own launch, 4 us.  So the line is a number of rounds of workgroups, two per compute unit of a 256-CU part: six where the
+// same two kernels would run one after the other (dQ's with 32-row wavefronts), after which an end is little beside the rest (whole backward, us in a graph, one
+// after the other / side by side: 64 heads on 8 KV heads 512 tokens 38 / 31, 2 x 383 43 / 34, 1500 114 / 91, 2 x 1500 (2656 workgroups) 184 / 174, padded
+// 4 x 1000 (3072) 143 / 138); three where the other side has attn_bwd_dkdv64_kernel, whose steps are cheaper (8 heads on one 4000 155 / 112,
+// 10000 (1258) 495 / 441, 32 on four 3000 (1520) 188 / 178, 3500 (1776) 231 / 218, but 2 x 2048 (2048) 152 / 160, documents of 1500 to 2500
+// 1520: 143 / 141, 2048: 215 / 219).
+// Padded rows of 2048 tokens and more stay apart: attn_bwd_dkdv64_kernel reads no row of the padding, attn_bwd_dkdv_kernel those that
+// share a tile with rows that count.
+// Which of them starts first: pieces, and slices under a window, are of one length, and what starts last ends last: dQ's last
+// walks are short (dK/dV's / dQ's first: 64 on 8 2 x 383 34 / 40, 1500 91 / 101; window 200 98 / 124).  Where the walks of both shrink along the row the
+// longest one starts first: a step (query tile, head) of dK/dV takes 1.9 us, a key tile of dQ 1.1 (8 on two, slices of half a
+// row's steps, 4000 101 / 94, 8000 289 / 261, padded 4 x 1000 51 / 48; on one, of a row's, 4000 112 / 124, but 5000 171 / 151).
+constexpr int64_t kBothRound = 512;
+struct BothRoute { bool taken, dq_first; };
+BothRoute both_route(const gptoss_attn_params *p, KArgs &a) {
+    if (p->dtype != GPTOSS_ATTN_BF16 || a.r < 4 || window_single_pass(p) || dq_query_blocks(a) != 1) return {false, false};
+    if (p->seqlens && p->Skv >= 2048) return {false, false};
+    dkdv_pieces_for(p, a);
+    const int64_t rounds = dkdv64_shape(p, a.dkdv_parts) ? 3 : 6;
+    const int64_t q_tiles = (p->Sq + kTile - 1) / kTile, k_tiles = (p->Skv + kTile - 1) / kTile;
+    const int64_t slice = (q_tiles + a.dkdv_parts - 1) / a.dkdv_parts * a.r;
+    return {q_outer_grid(a, 4, 1) + dkdv_grid(a) <= rounds * kBothRound, !a.dkdv_steps && a.window == 0 && 11 * k_tiles > 19 * slice};
+}
+
+bool dkdv64_route(const gptoss_attn_params *p, int parts) {
+    if (!dkdv64_shape(p, parts)) return false;
+    KArgs a = make_args(p, {});
+    a.dkdv_parts = parts;
+    return parts == 1 || !both_route(p, a).taken;
 }
 
 // The hand-pipelined forward kernel (attn_fwd_pipe.h) takes full-causal rows whose groups of query heads fill its four
@@ -951,11 +968,7 @@ static int launch_dq(const gptoss_attn_params *p, void *stream, int fuse_delta) 
 #undef GPTOSS_LAUNCH_DQ
     }
     const int hpb = hpb_for(a.r);
-    int qb = query_blocks_for(a.window);
-    // short problems: 64-row workgroups (two per compute unit) would be few and uneven (the key loops grow with the row
-    // index); 32-row wavefronts make twice as many, three per SIMD (measured, full causal, B = 1: dQ 0.077 -> 0.066 ms
-    // at S = 2048, 0.240 -> 0.218 at S = 4096, equal from S = 8192 on, 6 % slower at S = 16384)
-    if (qb == 2 && q_outer_grid(a, hpb, 2) <= 4 * (int64_t)compute_units()) qb = 1;
+    const int qb = dq_query_blocks(a);
     const int64_t grid = q_outer_grid(a, hpb, qb);
 #define GPTOSS_LAUNCH_DQ(HPB, QB) \
     (fuse_delta ? launch(attn_bwd_dq_kernel<HPB, QB, true>, grid, 256, st, a) : launch(attn_bwd_dq_kernel<HPB, QB, false>, grid, 256, st, a))

@@ -34,6 +34,14 @@ _CASES = [
     (1, 8, 1, 400, 400, 100, None, [250, 150]),
     (1, 8, 2, 100, 450, None, None, None),               # queries behind earlier keys
     (2, 8, 2, 70, 200, 64, None, None),
+    (21, 64, 8, 160, 160, None, None, None),             # 1008 workgroups of 64 rows, so dQ has 32-row wavefronts
+    (22, 64, 8, 160, 160, None, None, None),             # 1056: 64-row ones, and one launch after the other
+    (8, 64, 8, 300, 300, 200, None, None),               # a window: under six rounds of 512 workgroups, and over
+    (16, 64, 8, 300, 300, 200, None, None),
+    (1, 32, 8, 2048, 2048, None, None, None),            # in the 64-key kernel's place: three rounds
+    (1, 32, 8, 2049, 2049, None, None, None),            # 1608
+    (2, 8, 2, 1500, 1500, None, [1500, 600], None),      # slices, dQ first
+    (4, 16, 2, 700, 700, 200, None, None),
 ]
 
 
