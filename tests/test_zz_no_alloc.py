@@ -100,8 +100,8 @@ def test_static_scratch_backward_matches_workspace_backward(window):
 ])
 def test_static_scratch_backward_other_routes(b, h, g, s, window, dtype, lens):
     """The routes the two-call test above does not take, each against gptoss_attn_bwd: float32 tensors,
-    right-padded rows in the single-pass window kernel's no-seam walk (every workgroup walks two query
-    tiles past its chunk and drops the dK/dV of the two tiles before it), and group sizes the
+    right-padded rows in the single-pass window kernel's no-seam walk (every workgroup walks four 32-row query
+    blocks past its chunk and drops the dK/dV of the four blocks before it), and group sizes the
     single-pass kernel does not take.  Padded positions must be exactly zero."""
     print(f"no-alloc backward: B={b} H={h} G={g} S={s} W={window} {dtype} lens={lens}", flush=True)
     ref, got, cut = _backward_both(b, h, g, s, window, 13, dtype, lens)
@@ -112,6 +112,29 @@ def test_static_scratch_backward_other_routes(b, h, g, s, window, dtype, lens):
             if n < s:
                 for t in got[:3]:
                     assert float(t[i, :, n:].abs().max()) == 0.0
+
+
+@pytest.mark.parametrize("b,h,g,s,window,lens", [
+    (1, 4, 2, 417, 128, None),                           # one pair of heads per block: the barrier of its own in every step; a last chunk of two blocks
+    (1, 4, 2, 545, 33, None),
+    (1, 2, 1, 1300, 128, None),                          # of one block
+    (1, 2, 1, 1100, 97, None),                           # of three
+    (2, 6, 2, 417, 128, None),                           # three heads: a step without a head for group 1
+    (1, 3, 1, 1300, 65, None),
+    (1, 5, 1, 545, 128, None),                           # five
+    (1, 10, 2, 1100, 128, None),
+    (2, 4, 2, 545, 128, [545, 130]),                     # padding in front of the walk's end, behind it, and in whole chunks
+    (2, 5, 1, 417, 128, [96, 417]),
+    (2, 3, 1, 1300, 128, [1, 1281]),
+])
+def test_static_scratch_window_walk(b, h, g, s, window, lens):
+    """The no-seam walk with one, two and three pairs of heads per block, even and odd numbers of heads, and last chunks of one to three blocks, shorter than the
+    four blocks that a walk goes past its chunk."""
+    print(f"no-alloc window backward: B={b} H={h} G={g} S={s} W={window} lens={lens}", flush=True)
+    ref, got, _ = _backward_both(b, h, g, s, window, 14, torch.bfloat16, lens)
+    _compare(ref, got, True)
+    for i, n in enumerate(lens or ()):
+        assert not any(t[i, :, n:].any() for t in got[:3])
 
 
 def test_static_scratch_refuses_what_does_not_fit():
