@@ -1,7 +1,7 @@
 // Single-pass backward for sliding-window layers (window <= 128): dQ, dK, dV and the dSinks
 // terms from ONE read of Q, dO, O, K, V, five GEMMs per (query block, key block) pair.  Stands in for
 // the reference's `_attn_bwd_precompute_D` + `_attn_bwd` (attention_kernel.py:102-217) on such
-// layers; results are bit-reproducible (no atomics, fixed summation orders).
+// layers; results are bit-reproducible (fixed summation orders; no word is added to by more than one lane).
 //
 // With a window of at most 128 a block u of 32 query rows sees the five 32-key blocks u-4 .. u, and a key block is seen by
 // the query blocks u .. u+4.  A workgroup owns a chunk of consecutive query blocks [u0, u1) of one KV head (all r query heads
@@ -27,7 +27,7 @@
 //     walk goes four query blocks past the chunk, for the sake of its last key blocks only, and
 //     drops the dK / dV of the key blocks before the chunk (the neighbour produces them the
 //     same way): recomputation instead of an exchange.
-// Both are free of atomics and bit-reproducible.
+// Both are bit-reproducible.
 //
 // One barrier per step hands over the staged Q / dO tiles (asynchronous global->LDS copies, four stages), the row
 // statistics of the next step and the dS blocks of the previous one (double buffered).  K / V rows of the next key block travel
@@ -61,7 +61,7 @@ struct WinCfg {
     static constexpr int kBlockBytes = kRows * kRowBytes;                  // 4 KB: a block's rows of one tensor
     static constexpr int kMergeBytes = 2 * 2 * 16 * 64 * 4;                // an owner's dK and dV accumulators
     static constexpr int kStageOff = 0;                                    // [NS][group][Q, dO][4 KB]; behind the walk four merge buffers
-    static constexpr int kMergeOff = kStageOff + NS * 2 * 2 * kBlockBytes; // group 1's accumulators of the block that is complete
+    static constexpr int kMergeOff = kStageOff + NS * 2 * 2 * kBlockBytes; // of the block that is complete: group 1's dK, group 0's dV
     static constexpr int kStatOff = kMergeOff + kMergeBytes;               // [2][group][-lse / scale, -delta][32] floats
     static constexpr int kDsOff = kStatOff + 2 * 2 * 2 * kRows * 4;        // [2][slot][32 keys][group][32 rows] bf16
     static constexpr int kDsBytes = NSLOT * kBlockBytes;
@@ -674,7 +674,7 @@ __global__ __launch_bounds__(256) void attn_bwd_window_finish_kernel(const KArgs
     const int g = bg % a.G, b = bg / a.G;
     const int row = ((seam + 1) * a.chunk_blocks - WinCfg::kBack + block) * WinCfg::kRows + key;
     if (row >= a.Skv) return;
-    // eight columns of a key: the quads of both halves of its lane pair (accumulator order, see leave_sums)
+    // eight columns of a key: the quads of both halves of its lane pair (accumulator order, see quad and seam_share)
     const float *before = a.boundary_partial + ((rest * WinCfg::kBack + block) * 2) * (2 * WinCfg::kRows * kD) + ((which * 8 + c8 / 8) * 64 + key) * 4;
     const float *after = before + 2 * WinCfg::kRows * kD;
     const float mul = which == 0 ? a.scale : 1.0f;

@@ -284,18 +284,18 @@ bool fwd_pipe_plain(const gptoss_attn_params *p) {
     return p->Sq == p->Skv && p->Sq % kTile == 0 && !p->seqlens && !p->doc_start && p->q_offset == 0 && !p->q_offset_dev;
 }
 
-// Shares of the keys per query block where the workgroups are too few to fill the chip (no packing): two
-// per compute unit of a 256-CU part, at least eight tiles each.  From the shapes alone, so that the scratch (35 MB at most, 69 for the longest rows) does not
-// depend on where the queries stand.  New queries on a cache, 64 query heads on 8 KV heads: 100 queries on 4096 keys 62 -> 30 us, 300 on 12000 167 -> 82
-// (four tiles each: 37 us and 83); 8 heads on one KV head: 300 on 12000 164 -> 34 (more than sixteen shares: 36), 1000 on 17000 231 -> 57.
-// Two shares are not worth the sum where they just fill the chip: 1024 on 8192 134 -> 137.  More workgroups than compute units, but not two each, make some units take twice as long as
-// the others (a unit is no faster with two): shares that end with a full or half full round of two per unit even that out on long caches, three for 257 to 341 workgroups, two to 384; us, whole / in
-// shares: 1088 on 6000 144 / 128, 1268 on 4000 97 / 97, on 16000 398 / 319, 1344 on 7000 173 / 155, 1500 on 9000 228 / 211, on 4000 99 / 101, 1600 on 16000 (400 workgroups, two) 412 / 437; and four for 171 to 192,
-// 704 on 16000 219 / 190, on 5000 75 / 77, 768 on 16000 220 / 200, 32 heads on four 1600 (200) on 9000 130 / 143.
-// Self-attention, where the sum is over more rows (us in a graph): on up to four groups of four heads from 20 tiles on, 8 heads on
-// one KV head 1300 tokens 23.4 -> 21.3, 2000 33 -> 23, 4000 60 -> 41, 8000 113 -> 96, 2 x 1300 23.8 -> 23.1, 2 x 3000 48 -> 43; not 2 x 1024 19.2 -> 20.4, on six groups 3 x 1600
-// 28 -> 31, 3 x 2560 41 -> 46, on eight 4 x 1000 21 -> 23, 32 heads on four 2000 37 -> 41.  Rows of 128 tiles and more: four workgroups per unit, 8200 117 -> 91, 12000 191 -> 164
-// (with two it would stay whole), 16384 309 -> 275, but 4000 60 -> 46.
+// Shares of the keys per query block where the workgroups (64 queries of four heads) are too few to fill the chip (no packing): two per compute
+// unit of a 256-CU part, at least eight tiles each, as a share starts and ends and is added.  From the shapes alone, so that the
+// scratch (68 KB a workgroup) does not depend on where the queries stand.  us, whole / in shares, 64 heads on 8 KV heads:
+//  * New queries on a cache, up to 512 workgroups in three shares and more (35 MB at most): 100 queries on 4096 keys 62 / 30, 300 on 12000
+//    167 / 82; two shares that just fill the chip are not worth their sum, 1024 on 8192 134 / 137.
+//  * More workgroups than compute units, but not two each, make some units take twice as long as the others (a unit is no faster with
+//    two).  On long caches shares end with a full or half full round of two per unit: three for 257 to 341 workgroups (69 MB), two to
+//    384 and four for 171 to 192 (52): 1268 queries on 16000 keys 398 / 319, on 4000 97 / 97; 1500 on 9000 228 / 211, on 4000 99 / 101; 704 on 16000
+//    219 / 190, on 5000 75 / 77; 400 workgroups 412 / 437, 200 of 32 heads 130 / 143.
+//  * Self-attention has more rows to add: up to four groups of four heads from 20 tiles on (8 heads on one KV head 1300 tokens 23.4 / 21.3,
+//    4000 60 / 41, but 2 x 1024 19.2 / 20.4, six groups of 1600 28 / 31), and four workgroups per unit from 128 tiles on (69 MB), whose walks differ
+//    most: 8200 tokens 117 / 91, 12000 191 / 164 (with two per unit whole), but 4000 60 / 46.
 int fwd_pipe_splits(const gptoss_attn_params *p) {
     const bool self = p->Skv <= p->Sq;
     const int64_t groups = (int64_t)p->G * (p->H / p->G / 4) * p->B, wgs = groups * ((p->Sq + kTile - 1) / kTile);
