@@ -54,9 +54,10 @@ struct Dkdv64 {
 // shares (dkdv_parts_for), one workgroup each; with padded rows or packed documents (dkdv_slots > 0) a KV head's blocks, of all batch
 // rows, are divided by their lengths, which only the device knows: a unit's share is L = (all tiles) / (units
 // of the KV head); walks longer than that are cut into pieces of L tiles from their end down, and the rest of each.  The pieces of L tiles start
-// first (the first ones of all blocks, then the second ones: neighbours walk the same Q and dO tiles), the rests follow, the longest first.  A walk that is not cut writes its result itself; the pieces of one that is leave fp32
-// partial sums, in slots of the scratch (attn_bwd_dkdv64_reduce_kernel adds them).  Every workgroup finds its own piece (the
-// blocks' lengths in LDS, then counting over a wavefront: about 2 us, documents 4).
+// first (the first ones of all blocks, then the second ones: neighbours walk the same Q and dO tiles), the rests follow, the longest first.
+// A walk that is not cut writes its result itself; the pieces of one that is leave fp32 partial sums, in slots of the scratch
+// (attn_bwd_dkdv64_reduce_kernel adds them).  Every workgroup finds its own piece (the blocks' lengths in LDS, then counting over a
+// wavefront: about 2 us, documents 4).
 // Equal shares leave padded and packed rows' short walks in as many pieces as the long ones', each with a start, an end and 128 KB of
 // partial sums of its own.  Forward + backward, us equal shares / pieces (64 query heads on 8 KV heads): 4 x 4096 padded to 3309 / 1968 / 1554 / 4079
 // 1400 / 1329, 2 x 5438 to 2212 / 2754 634 / 594; documents of 95 to 3067 in 8192 tokens 785 / 768, of 100 to 4000 in 12000 1450 / 1395;
@@ -664,10 +665,11 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkdv64_kernel(const KArgs a) 
     }
 }
 
-// The partial sums of the cut key blocks, in the order of their pieces, scaled and rounded; kChunks 16-byte output chunks per thread, 16 / kChunks workgroups per
-// block.  What bounds it: finding the pieces, about 5 us, which every workgroup does for itself: four chunks where one would be many workgroups (launch, us, one / four: 4 x 4096
-// tokens padded to 3309, 1968, 1554 and 4079 22.2 / 12.7, 8192 in seven documents 19.0 / 11.4, 5 x 2265 16.1 / 10.8, but 8000 of 8 heads, 512 workgroups, 12.6 / 17.0, and the whole call of 96 key blocks 332 / 333).  The first `heads`
-// workgroups produce dSinks.
+// The partial sums of the cut key blocks, in the order of their pieces, scaled and rounded; kChunks 16-byte output chunks per thread, 16 /
+// kChunks workgroups per block.  What bounds it: finding the pieces, about 5 us, which every workgroup does for itself: four chunks where
+// one would be many workgroups (launch, us, one / four: 4 x 4096 tokens padded to 3309, 1968, 1554 and 4079 22.2 / 12.7, 8192 in seven
+// documents 19.0 / 11.4, 5 x 2265 16.1 / 10.8, but 8000 of 8 heads, 512 workgroups, 12.6 / 17.0, and the whole call of 96 key blocks 332 /
+// 333).  The first `heads` workgroups produce dSinks.
 constexpr int dkdv64_reduce_chunks(int64_t key_blocks) { return key_blocks > 128 ? 4 : 1; }
 template <int kChunks>
 __global__ __launch_bounds__(256) void attn_bwd_dkdv64_reduce_kernel(const KArgs a, int heads) {

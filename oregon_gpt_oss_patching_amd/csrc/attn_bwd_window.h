@@ -55,8 +55,8 @@ struct WinCfg {
     static constexpr int kMaxWindow = 128;
     static constexpr int kBack = kMaxWindow / kRows;                       // key blocks in front of a query block's own that it sees
     static constexpr int kMaxGroup = 16;                                   // query heads per KV head
-    // The weights are exp(scale * (S - lse / scale)), whose quotient has to stay finite.  Smaller scales take this one's weights: a sum of up to 128 exponentials and a
-    // sink has an lse below 2^11 (or no room beside its sink), and S is nothing beside it up to 2^100.
+    // The weights are exp(scale * (S - lse / scale)), whose quotient has to stay finite.  Smaller scales take this one's weights: a sum of
+    // up to 128 exponentials and a sink has an lse below 2^11 (or no room beside its sink), and S is nothing beside it up to 2^100.
     static constexpr float kMinScale = 0x1p-116f;
     static constexpr int kBlockBytes = kRows * kRowBytes;                  // 4 KB: a block's rows of one tensor
     static constexpr int kMergeBytes = 2 * 2 * 16 * 64 * 4;                // an owner's dK and dV accumulators
@@ -499,7 +499,8 @@ __global__ __launch_bounds__(WinCfg::NWAVES * 64, 1) void attn_bwd_window_kernel
             vf[ks] = as_bf16x8(zv);
         }
     }
-    // Unscaled sums of one tensor as accumulator quads of 64 lanes: on their way to the owner of the same slot in the other group, and the shares of seam blocks.
+    // Unscaled sums of one tensor as accumulator quads of 64 lanes: on their way to the owner of the same slot in the other group, and the
+    // shares of seam blocks.
     // (A group's tensor is chosen value by value: chosen by branches, the accumulators end up in memory.)
     constexpr int kHalf = C::kMergeBytes / 2;
     auto quad = [&](bool of_dv, int dblk, int a4) __attribute__((always_inline)) {
@@ -518,8 +519,9 @@ __global__ __launch_bounds__(WinCfg::NWAVES * 64, 1) void attn_bwd_window_kernel
     auto seam_share = [&](int seam, int block, int side) {
         return a.boundary_partial + (((((int64_t)b * a.G + g) * (n_chunks - 1) + seam) * C::kBack + block) * 2 + side) * (2 * kRows * kD);
     };
-    // One tensor of the key block held (group 0: dK, group 1: dV), the other group's sums in `buf` added: written out if it is complete, left as this workgroup's share if
-    // it sits on a seam, dropped if it belongs to the neighbour (recomputation mode).  `buf` then stages the rows.
+    // One tensor of the key block held (group 0: dK, group 1: dV), the other group's sums in `buf` added: written out if it is complete,
+    // left as this workgroup's share if it sits on a seam, dropped if it belongs to the neighbour (recomputation mode).  `buf` then stages
+    // the rows.
     auto flush = [&](char *buf) __attribute__((always_inline)) {
         if (my_kb < 0 || (!seam_sums && (my_kb < u0 || my_kb >= u1))) return;
         const int ln = fresh_lane();

@@ -672,8 +672,8 @@ __global__ __launch_bounds__(256, 2) void attn_f32_dq_kernel(const KArgs a) {
     f32_dq_rows<KS, FUSE_DELTA, 4>(a, smem);
 }
 
-// dQ (the first workgroups) and dK/dV side by side behind the row statistics, where all of them run at once: the float32 counterpart of attn_bwd_both_kernel, with the bits
-// of the two launches.
+// dQ (the first workgroups) and dK/dV side by side behind the row statistics, where all of them run at once: the float32 counterpart of
+// attn_bwd_both_kernel, with the bits of the two launches.
 __global__ __launch_bounds__(256, 2) void attn_f32_both_kernel(const KArgs a, int dq_workgroups) {
     static_assert(F32Dkdv::kLdsBytes >= 8 * F32Tile::kBytes, "one array for both");
     __shared__ __attribute__((aligned(1024))) char smem[F32Dkdv::kLdsBytes];

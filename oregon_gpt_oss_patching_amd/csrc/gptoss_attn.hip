@@ -123,23 +123,26 @@ bool many_key_blocks(const gptoss_attn_params *p) { return (int64_t)p->G * p->B 
 // slices so that there are about a thousand workgroups, and sum the slices' fp32 partials afterwards.  A slice
 // keeps at least four query tiles of a sliding-window layer (windows of up to 321 keys stay whole, wider ones are cut) and at least
 // eight (query tile, head) steps of a full-causal one, which may be a single tile.  Up to 512 blocks the count is rounded
-// up (B = 2, S = 383: 78 us uncut, 25 + 5 us in six slices; unpadded short rows then take pieces of other lengths in the same scratch, dkdv_pieces_for).  Between 512 and 1024 blocks the first
-// key block of a long row (4096 rows and more) is still longer than the average compute unit's share: two slices; a
-// right-padded batch counts half, because its shorter rows leave the longest one alone (dK/dV of B = 4, S = 4096,
-// lengths 3309 / 1968 / 1554 / 4079: 715 us uncut, 589 in two slices; B = 2, S = 8192 / 4000: 1437 and 1216).  Several rows of 1280 tokens and
-// more (padded: 1024) get the same scratch, for pieces by the walks' lengths (Dkdv64Plan), which cut only the longest walks: whole backward and forward of 5 x 1600
-// 564 -> 514 us, 6 x 1500 610 -> 584, 3 x 3000 1074 -> 995, 7 x 1417 645 and 646, 8 x 1300 611 -> 602; but 9 x 1100 536 -> 547.  Packed rows: a walk ends with its document, so the longest document's first blocks stand out more, and
-// the host does not see the documents: four slices from 256 to 768 blocks of rows of 4096 keys and more.  Whole backward of one row of
-// 64 query heads, two slices / four, documents of up to 1500 tokens, up to 4096, 1500 to 6000, and ONE: 8192 tokens 367 / 373,
-// 602 / 568, 994 / 924, 1683 / 1689 us; 12288 (768 blocks) 554 / 557, 970 / 963, 1296 / 1254, 3826 / 3712; beyond the line 14000 571 / 593,
-// 872 / 866, 1508 / 1501, 4913 / 4875 and 16384 687 / 711, 928 / 941, 1623 / 1631, 6636 / 6690.  (Two rows of 4096, 512 blocks, would
-// rather have two: 340 / 359, 526 / 513, 864 / 902, 904 / 919.)
+// up (B = 2, S = 383: 78 us uncut, 25 + 5 us in six slices; unpadded short rows then take pieces of other lengths in the same scratch,
+// dkdv_pieces_for).  Between 512 and 1024 blocks the first key block of a long row (4096 rows and more) is still longer than the average
+// compute unit's share: two slices; a right-padded batch counts half, because its shorter rows leave the longest one alone (dK/dV of B = 4,
+// S = 4096, lengths 3309 / 1968 / 1554 / 4079: 715 us uncut, 589 in two slices; B = 2, S = 8192 / 4000: 1437 and 1216).  Several rows of
+// 1280 tokens and more (padded: 1024) get the same scratch, for pieces by the walks' lengths (Dkdv64Plan), which cut only the longest
+// walks: whole backward and forward of 5 x 1600 564 -> 514 us, 6 x 1500 610 -> 584, 3 x 3000 1074 -> 995, 7 x 1417 645 and 646, 8 x 1300
+// 611 -> 602; but 9 x 1100 536 -> 547.  Packed rows: a walk ends with its document, so the longest document's first blocks stand out more,
+// and the host does not see the documents: four slices from 256 to 768 blocks of rows of 4096 keys and more.  Whole backward of one row of
+// 64 query heads, two slices / four, documents of up to 1500 tokens, up to 4096, 1500 to 6000, and ONE: 8192 tokens 367 / 373, 602 / 568,
+// 994 / 924, 1683 / 1689 us; 12288 (768 blocks) 554 / 557, 970 / 963, 1296 / 1254, 3826 / 3712; beyond the line 14000 571 / 593, 872 / 866,
+// 1508 / 1501, 4913 / 4875 and 16384 687 / 711, 928 / 941, 1623 / 1631, 6636 / 6690.  (Two rows of 4096, 512 blocks, would rather have two:
+// 340 / 359, 526 / 513, 864 / 902, 904 / 919.)
 int dkdv_parts_for(const gptoss_attn_params *p, bool padded, bool packed) {
     if (p->dtype == GPTOSS_ATTN_FP32) {
-        // A workgroup per 32 keys, two per compute unit at a time.  Up to four slices and a thousand workgroups, so that the long first key blocks of a row do not decide the time;
-        // more where that is not two per unit of a 256-CU part: the longest walk, 1.2 us a step, is all there is to such a launch (backward, us in a graph, at most four slices / these: 8 heads
-        // on one KV head 300 tokens 55 / 38, 1000 122 / 76, 2 x 1000 134 / 111, on two 1000 83 / 73 (with a thousand workgroups here too 82), 64 on eight 150 45 / 36).  A window's walk is cut by the
-        // same rule, into three or more: of 128 8 heads on one 400 tokens 73 / 34, 64 on eight 500 95 / 82; into two 900 108 / 110.
+        // A workgroup per 32 keys, two per compute unit at a time.  Up to four slices and a thousand workgroups, so that the long first key
+        // blocks of a row do not decide the time; more where that is not two per unit of a 256-CU part: the longest walk, 1.2 us a step, is
+        // all there is to such a launch (backward, us in a graph, at most four slices / these: 8 heads on one KV head 300 tokens 55 / 38,
+        // 1000 122 / 76, 2 x 1000 134 / 111, on two 1000 83 / 73 (with a thousand workgroups here too 82), 64 on eight 150 45 / 36).  A
+        // window's walk is cut by the same rule, into three or more: of 128 8 heads on one 400 tokens 73 / 34, 64 on eight 500 95 / 82;
+        // into two 900 108 / 110.
         const int64_t blocks = (int64_t)p->G * p->B * ((p->Skv + 31) / 32), all = (p->Sq + 31) / 32;
         const int window = effective_window(p);
         const int64_t tiles = window > 0 && (window + 62) / 32 + 1 < all ? (window + 62) / 32 + 1 : all;        // that see a block
@@ -243,13 +246,13 @@ bool dkdv64_shape(const gptoss_attn_params *p, int parts) {
 
 // dQ and dK/dV in one launch (attn_bwd_both_kernel), behind one for the row statistics, instead of one after the other.  `a` has the
 // backward's dkdv_parts; gets its pieces.
-// What it saves is the end of the first launch, where units wait for its longest walks, and the start of the second; what it adds
-// is the statistics' own launch, 4 us.  So the line is a number of rounds of workgroups, two per compute unit of a 256-CU part: six where the
-// same two kernels would run one after the other (dQ's with 32-row wavefronts), after which an end is little beside the rest (whole backward, us in a graph, one
-// after the other / side by side: 64 heads on 8 KV heads 512 tokens 38 / 31, 2 x 383 43 / 34, 1500 114 / 91, 2 x 1500 (2656 workgroups) 184 / 174, padded
-// 4 x 1000 (3072) 143 / 138); three where the other side has attn_bwd_dkdv64_kernel, whose steps are cheaper (8 heads on one 4000 155 / 112,
-// 10000 (1258) 495 / 441, 32 on four 3000 (1520) 188 / 178, 3500 (1776) 231 / 218, but 2 x 2048 (2048) 152 / 160, documents of 1500 to 2500
-// 1520: 143 / 141, 2048: 215 / 219).
+// What it saves is the end of the first launch, where units wait for its longest walks, and the start of the second; what it adds is the
+// statistics' own launch, 4 us.  So the line is a number of rounds of workgroups, two per compute unit of a 256-CU part.  Six where the
+// same two kernels would run one after the other (dQ's with 32-row wavefronts), as an end is little beside so many rounds: whole backward,
+// us in a graph, one after the other / side by side (workgroups), 64 heads on 8 KV heads 512 tokens 38 / 31 (480), 2 x 383 43 / 34 (656),
+// 1500 114 / 91 (1248), 2 x 1500 184 / 174 (2656), padded 4 x 1000 143 / 138 (3072).  Three where the other side has
+// attn_bwd_dkdv64_kernel, whose steps are cheaper: 8 heads on one 4000 155 / 112 (506), 10000 495 / 441 (1258), 32 on four 3000 188 / 178
+// (1520), but 2 x 2048 152 / 160 (2048); documents of 500 to 2500 143 / 141 (1520), 215 / 219 (2048).
 // Padded rows of 2048 tokens and more stay apart: attn_bwd_dkdv64_kernel reads no row of the padding, attn_bwd_dkdv_kernel those that
 // share a tile with rows that count.
 // Which of them starts first: pieces, and slices under a window, are of one length, and what starts last ends last: dQ's last
@@ -335,9 +338,9 @@ int64_t decode_keys(const gptoss_attn_params *p) {
 }
 // The keys of a KV head walked by one workgroup of eight wavefronts, no slices to add and one launch less.  Where the cache comes from HBM
 // (us a call, sliced / whole, 8 query heads per KV head), B G = 8: 257 keys 12.5 / 10.6, 1024 12.4 / 11.1, 1500 12.4 / 13.6, 2049 12.4 / 16.7;
-// B G = 128: 1024 14.1 / 13.0, 2049 20.9 / 20.1, 4096 32.8 / 34.3, 8192 55.7 / 65.5; B G = 256: 1000 20.1 / 17.1; two column blocks, B G = 8: 600 12.6 / 11.7, 1000
-// 12.6 / 14.6.  (A cache that is still in the last-level cache moves the line up to 3000 keys, but a decoding step reads all layers'
-// weights between two calls on one cache.)  512 groups fill the chip unsliced.
+// B G = 128: 1024 14.1 / 13.0, 2049 20.9 / 20.1, 4096 32.8 / 34.3, 8192 55.7 / 65.5; B G = 256: 1000 20.1 / 17.1; two column blocks, B G =
+// 8: 600 12.6 / 11.7, 1000 12.6 / 14.6.  (A cache that is still in the last-level cache moves the line up to 3000 keys, but a decoding step
+// reads all layers' weights between two calls on one cache.)  512 groups fill the chip unsliced.
 bool decode_whole(const gptoss_attn_params *p) {
     const int64_t groups = (int64_t)p->B * p->G, pairs = (int64_t)p->Sq * (p->H / p->G);
     return groups < 512 && decode_keys(p) <= (pairs > 32 ? 640 : 1024);
@@ -370,14 +373,15 @@ int64_t f32_grid(const KArgs &a, int ks) {
 // ---- float32 on the bf16 matrix pipes (attn_f32_split.h) -----------------------------------------
 // Taken where the caller has scratch for the records, four consecutive heads share a KV head (the four units of a workgroup then stand
 // at the same rows), the backward for self-attention without an offset, and where it is the faster one: it costs a launch and fills the
-// chip with workgroups of eight wavefronts, one per compute unit.  Self-attention takes it in both directions or in neither (with lse of the one and S of the other
-// dQ of operands next to a bf16 number was 1.09 times as far from float64 as with the fp32 instruction alone).  fp32 instruction / this, us in a graph, 64 query heads on 8 KV heads,
-// forward and backward: 320 rows 23 + 82 / 25 + 70, 448 33 + 110 / 31 + 80, 1024 100 + 310 / 66 + 200, 4096 5320 / 3120; 8 heads on one KV head 2048 rows (128 workgroups)
-// 63 + 249 / 79 + 165; a window is a handful of tiles per workgroup, whose start and end then decide: of 128, 320 rows 22 + 88 / 21 + 63, 640 33 + 103 / 35 + 91, 800 (400 workgroups)
-// 36 + 107 / 39 + 102, 1024 147 / 150; of 383, 800 63 + 220 / 50 + 136; of 64, 448 21 + 69 / 20 + 61, but 640 26 + 74 / 33 + 83
-// (windows below 96 would rather have the line at 256 workgroups).
-// Queries on a cache, forward: 256 (128 workgroups) on 2048 80 / 84, on 4096 154 / 154, on 16384 600 / 566; 320 on 1024 59 / 48, 1024 on 8192 1121 / 647; with a window of 128, 320 on
-// 16384 23 / 21, 448 26 / 22, 576 34 / 36, 256 (128 workgroups) 15 / 21; of 64, 320 17 / 19, 448 21 / 20; of 192, 576 43 / 41; of 400, 800 76 / 56.
+// chip with workgroups of eight wavefronts, one per compute unit.  Self-attention takes it in both directions or in neither (with lse of
+// the one and S of the other dQ of operands next to a bf16 number was 1.09 times as far from float64 as with the fp32 instruction alone).
+// fp32 instruction / this, us in a graph, 64 query heads on 8 KV heads, forward and backward: 320 rows 23 + 82 / 25 + 70, 448 33 + 110 / 31
+// + 80, 1024 100 + 310 / 66 + 200, 4096 5320 / 3120; 8 heads on one KV head 2048 rows (128 workgroups) 63 + 249 / 79 + 165; a window is a
+// handful of tiles per workgroup, whose start and end then decide: of 128, 320 rows 22 + 88 / 21 + 63, 640 33 + 103 / 35 + 91, 800 (400
+// workgroups) 36 + 107 / 39 + 102, 1024 147 / 150; of 383, 800 63 + 220 / 50 + 136; of 64, 448 21 + 69 / 20 + 61, but 640 26 + 74 / 33 + 83
+// (windows below 96 would rather have the line at 256 workgroups). Queries on a cache, forward: 256 (128 workgroups) on 2048 80 / 84, on
+// 4096 154 / 154, on 16384 600 / 566; 320 on 1024 59 / 48, 1024 on 8192 1121 / 647; with a window of 128, 320 on 16384 23 / 21, 448 26 /
+// 22, 576 34 / 36, 256 (128 workgroups) 15 / 21; of 64, 320 17 / 19, 448 21 / 20; of 192, 576 43 / 41; of 400, 800 76 / 56.
 bool f32_split_route(const gptoss_attn_params *p, bool bwd) {
     if (p->dtype != GPTOSS_ATTN_FP32 || p->B <= 0 || p->G <= 0 || p->H <= 0 || p->H % p->G || (p->H / p->G) % 4 || p->Skv <= 0) return false;
     const bool self = p->Sq == p->Skv && p->q_offset == 0 && !p->q_offset_dev;       // (both directions take it, or neither)
@@ -424,8 +428,9 @@ F32SplitParts f32_split_parts(const gptoss_attn_params *p, int64_t rows) {
 // the backward the same of Q / dO, then the parts' sums.  The records are one and a half to two and a half times as large as what they are made of, and
 // the scratch is the caller's memory: kF32SplitRecords bytes of them at most (and 64 MB of parts' sums), in even shares; a KV head of one row
 // that needs more has no such route.  Forward + backward of 64 heads on 8 KV heads, everything at once / so, us (and MB at the peak, outputs
-// included; the left figures with terms cut off instead of rounded, 1.5 % faster at 1024 tokens): 4096 tokens 3200 (529) / 3275 (450), window 512 985 / 1010, 4 x 2000 3415 (913) / 3499
-// (579), 8192 12070 (1046) / 12310 (604), 16384 47300 (2106) / 49400 (911).  128 MB: window 512 another 7 % slower, the others alike.
+// included; the left figures with terms cut off instead of rounded, 1.5 % faster at 1024 tokens): 4096 tokens 3200 (529) / 3275 (450),
+// window 512 985 / 1010, 4 x 2000 3415 (913) / 3499 (579), 8192 12070 (1046) / 12310 (604), 16384 47300 (2106) / 49400 (911).  128 MB:
+// window 512 another 7 % slower, the others alike.
 constexpr size_t kF32SplitRecords = (size_t)256 << 20;
 struct F32SplitPlan { int nb, ng, tiles; size_t kv, q_bad, q, plan, partial, bytes; F32SplitParts parts; };
 F32SplitPlan f32_split_plan(const gptoss_attn_params *p, bool bwd) {
@@ -888,15 +893,16 @@ static int launch_dkdv(const gptoss_attn_params *p, void *stream, bool whole_blo
     }
     if (dkdv64_route(p, a.dkdv_parts)) {
         const int64_t blocks = (int64_t)a.B * ((a.Skv + Dkdv64::BN - 1) / Dkdv64::BN);      // of a KV head
-        // padded and packed rows, several rows of one length whose blocks would stay whole otherwise, and few enough equal shares that the longest of them decides:
-        // pieces by the walks' lengths,
-        // at most as many as there are slots for partial sums (Dkdv64Plan; the kernels hold kMaxBlocks lengths, nearly twice what dkdv_parts_for leaves)
-        // (not packed rows of up to four heads per KV head whose equal shares run all at once: these are four heads of a tile or two, and finding the lengths takes
-        // longer than the better division saves.  Backward of 8 heads on two KV heads, equal shares / by lengths, us: 4096 tokens in documents of 100 43 / 50, of 300 54 / 58, of
-        // 3000 132 / 135, of 95, 1502 and 222 94 / 92; 8192 (512 shares) of 300 82 / 67; eight heads on one, 4096 of 300 62 / 59)
-        // (Few shares, rows of one length, the same in a graph: 8 heads on one KV head 6000 tokens 293 / 263 (192 shares), 8000 337 / 294 (256), 16 on one 5000 358 / 324, 32 on four
-        // 2200 142 / 130 (288), 8 on two 5000 201 / 195 (320); 32 on four 3000 187 / 195 (384), 8 on one 12000 567 / 587 (376), 2 x 6000 343 / 370 (384): with several rounds
-        // the shares even out by themselves, and equal ones keep in step.)
+        // padded and packed rows, several rows of one length whose blocks would stay whole otherwise, and few enough equal shares that the
+        // longest of them decides: pieces by the walks' lengths, at most as many as there are slots for partial sums (Dkdv64Plan; the
+        // kernels hold kMaxBlocks lengths, nearly twice what dkdv_parts_for leaves) (not packed rows of up to four heads per KV head whose
+        // equal shares run all at once: these are four heads of a tile or two, and finding the lengths takes longer than the better
+        // division saves.  Backward of 8 heads on two KV heads, equal shares / by lengths, us: 4096 tokens in documents of 100 43 / 50, of
+        // 300 54 / 58, of 3000 132 / 135, of 95, 1502 and 222 94 / 92; 8192 (512 shares) of 300 82 / 67; eight heads on one, 4096 of 300 62
+        // / 59) (Few shares, rows of one length, the same in a graph: 8 heads on one KV head 6000 tokens 293 / 263 (192 shares), 8000 337 /
+        // 294 (256), 16 on one 5000 358 / 324, 32 on four 2200 142 / 130 (288), 8 on two 5000 201 / 195 (320); 32 on four 3000 187 / 195
+        // (384), 8 on one 12000 567 / 587 (376), 2 x 6000 343 / 370 (384): with several rounds the shares even out by themselves, and equal
+        // ones keep in step.)
         const bool one_round = !a.seqlens && a.doc_start && a.r <= 4 && a.G * blocks * a.dkdv_parts <= 256;
         const bool by_lengths = a.dkdv_parts > 1 && blocks <= Dkdv64Plan::kMaxBlocks && !one_round &&
                                 (a.seqlens || a.doc_start || (a.B > 1 && a.Sq < 4096 && many_key_blocks(p)) || a.G * blocks * a.dkdv_parts <= 320);
@@ -919,9 +925,10 @@ static int launch_dkdv(const gptoss_attn_params *p, void *stream, bool whole_blo
     return launch_dkdv_sum(a, st, with_dsinks);
 }
 
-// The same for float32: dQ's workgroups come first.  Two launches / one, us as above (workgroups): 8 heads on one KV head 300 tokens 38 / 24, 1000 76 / 67 (730), 1500 141 / 102 (846), on
-// two 500 41 / 31, 2 x 700 76 / 61 (792), 2 x 1000 111 / 104 (1024); 64 on eight 64 29 / 22, 150 36 / 30 (520); window 128, 8 on one 400 34 / 23.  Not 4 x 700 122 / 132 (1144); rows of a
-// few tiles start and end rather than walk, 64 on eight 180 39.7 / 40.6 (672), 2 x 100 37 / 38 (768).
+// The same for float32: dQ's workgroups come first.  Two launches / one, us as above (workgroups): 8 heads on one KV head 300 tokens 38 /
+// 24, 1000 76 / 67 (730), 1500 141 / 102 (846), on two 500 41 / 31, 2 x 700 76 / 61 (792), 2 x 1000 111 / 104 (1024); 64 on eight 64 29 /
+// 22, 150 36 / 30 (520); window 128, 8 on one 400 34 / 23.  Not 4 x 700 122 / 132 (1144); rows of a few tiles start and end rather than
+// walk, 64 on eight 180 39.7 / 40.6 (672), 2 x 100 37 / 38 (768).
 static int64_t f32_dkdv_grid(const KArgs &a) { return (int64_t)a.B * a.G * a.dkdv_parts * ((a.Skv + 31) / 32); }
 static bool f32_both_route(const KArgs &a, int dtype) {
     return dtype == GPTOSS_ATTN_FP32 && f32_key_splits(a) == 4 && f32_grid(a, 4) + f32_dkdv_grid(a) <= (a.Sq > 256 ? 1024 : 640);
